@@ -93,7 +93,8 @@ struct FinalBwdParams
     float* d_feat;            // [C][H][W], written
     _Float16* dpre;           // [H][W][npad], written
     float* part;              // [gridDim.x][4 * (4 + CS) + 4] sums of this launch's workgroups (WGRAD)
-    int chunks;               // ceil(pixels / kFinalPixelsPerBlock)
+    int chunks;               // of one image: ceil(pixels / kFinalPixelsPerBlock)
+    int batch;                // images, one after the other in every array
 };
 
 // One pass over the pixels of the finest level: dL/d in[0], the gated block's pre-activation gradients and, when
@@ -162,6 +163,11 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[k][i] = 0.f;
 
+    // the arrays of the image at hand
+    const float *d_out = p.d_out, *feat = p.feat;
+    const _Float16* pre = p.pre;
+    float* d_feat       = p.d_feat;
+    _Float16* dpre      = p.dpre;
     struct Loaded
     {
         float g[4], x[NI];
@@ -171,17 +177,23 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
     {
         Loaded l;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) l.g[k] = (valid && k < p.cout) ? p.d_out[k * plane + pix] : 0.f;
+        for (int k = 0; k < 4; ++k) l.g[k] = (valid && k < p.cout) ? d_out[k * plane + pix] : 0.f;
 #pragma unroll
-        for (int j = 0; j < NI; ++j) l.x[j] = (WGRAD && valid && has_img[j]) ? p.feat[(size_t)(g + LPP * j) * plane + pix] : 0.f;
+        for (int j = 0; j < NI; ++j) l.x[j] = (WGRAD && valid && has_img[j]) ? feat[(size_t)(g + LPP * j) * plane + pix] : 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) l.mine[i] = _Float16(0.f);
-        if (valid && in_row) l.mine = *reinterpret_cast<const half8*>(p.pre + pix * p.npad + 8 * g);
+        if (valid && in_row) l.mine = *reinterpret_cast<const half8*>(pre + pix * p.npad + 8 * g);
         return l;
     };
     constexpr int STEP = 4 * PPW;  // pixels per iteration of the workgroup
-    for (int chunk = blockIdx.x; chunk < p.chunks; chunk += gridDim.x)
+    for (int item = blockIdx.x; item < p.chunks * p.batch; item += gridDim.x)
     {
+        const int image = item / p.chunks, chunk = item - image * p.chunks;
+        d_out  = p.d_out + (size_t)image * p.cout * plane;
+        feat   = p.feat + (size_t)image * p.c_feat * plane;
+        d_feat = p.d_feat + (size_t)image * p.c_feat * plane;
+        pre    = p.pre + (size_t)image * plane * p.npad;
+        dpre   = p.dpre + (size_t)image * plane * p.npad;
         const size_t p1 = std::min(plane, (size_t)(chunk + 1) * kFinalPixelsPerBlock);
         size_t base     = (size_t)chunk * kFinalPixelsPerBlock + wave * PPW;
         Loaded next     = load(base + sub, base + sub < p1);
@@ -221,7 +233,7 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
             // a feature lane stores the feature gradients of the eight channels: its own four, then the partner's
             const half8 out = is_f ? half8{keep[0], keep[1], keep[2], keep[3], got[0], got[1], got[2], got[3]}
                                    : half8{got[0], got[1], got[2], got[3], keep[0], keep[1], keep[2], keep[3]};
-            if (valid && in_row) *reinterpret_cast<half8*>(p.dpre + pix * p.npad + 8 * g) = out;
+            if (valid && in_row) *reinterpret_cast<half8*>(dpre + pix * p.npad + 8 * g) = out;
 #pragma unroll
             for (int j = 0; j < NI; ++j)
             {
@@ -230,7 +242,7 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
                     float d = 0.f;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) d = __builtin_fmaf(wimg[k][j], cur.g[k], d);
-                    p.d_feat[(size_t)(g + LPP * j) * plane + pix] = d;
+                    d_feat[(size_t)(g + LPP * j) * plane + pix] = d;
                 }
             }
             if (WGRAD)
@@ -329,12 +341,19 @@ struct BwdDataParams
     const _Float16* wt;    // [9][NN][KC]
     float* d_feat;         // [C][H][W], accumulated
     _Float16* d_in;        // [H][W][NN] or nullptr (start block: nothing below)
+    int first_image;       // images of a batch: the grid's z dimension, one after the other in every array
 };
 
 // CI = image channels the kernel has room for (4, 8 or 16): positions [0, C) of the block input are the level's image.
 template <int KC, int NN, int THREADS, int CI>
-__global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(const BwdDataParams p)
+__global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
 {
+    {
+        const size_t pixels = (size_t)(p.first_image + blockIdx.z) * p.H * p.W;
+        p.dpre += pixels * KC;
+        p.d_feat += pixels * p.c_feat;
+        p.d_in = p.d_in ? p.d_in + pixels * NN : nullptr;
+    }
     constexpr int MB = 16 / (THREADS / 64);  // 16-pixel row blocks of a wavefront: two rows of the tile, or one
     constexpr int ROW    = KC + kLdsChanPad;
     constexpr int GROUPS = KC / 8;
@@ -436,6 +455,7 @@ struct UpAdjointParams
     const _Float16* pre;   // [Hb][Wb][npad]
     float* d_feat;         // [C][Hb][Wb], written
     _Float16* dpre;        // [Hb][Wb][npad], written
+    int first_image;       // images of a batch: the grid's y dimension
 };
 
 // weight with which finer row / column `dst` reads coarser row / column `src`
@@ -451,8 +471,16 @@ __device__ __forceinline__ float up2_weight(int dst, int fine_size, int src, int
 // SHIFT = (2 C) % 8: the block outputs of the coarser level start at position 2 C of the finer block's input, which is
 // a multiple of 8 halves only for C = 4; otherwise a group of eight outputs straddles two aligned groups of positions.
 template <int SHIFT>
-__global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(const UpAdjointParams p)
+__global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p)
 {
+    if (const size_t image = p.first_image + blockIdx.y; image > 0)
+    {
+        const size_t coarse = image * p.Hb * p.Wb;
+        p.d_in += image * p.H * p.W * p.cin_fine;
+        p.pre += coarse * p.npad;
+        p.dpre += coarse * p.npad;
+        p.d_feat += coarse * p.c_feat;
+    }
     const int half   = p.npad / 2;
     const int C      = p.c_feat;
     // the coarser level's image sits at positions [C, 2C) of the finer block's input: the aligned groups of eight
@@ -613,7 +641,8 @@ struct BwdWeightParams
 {
     int H, W, Hb, Wb;
     int c_feat, cb_store;
-    int tiles_x, tiles;
+    int tiles_x, tiles;  // tiles of one image
+    int batch;           // images, one after the other in every array
     const float* feat;
     const float* feat_below;
     const _Float16* act_below;
@@ -756,8 +785,25 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     };
     const int act_groups = p.cb_store / 8;
     const int per_pixel  = IQ + act_groups;
+    // the images of the batch are walked as one run of tiles: a workgroup keeps its sums from one image to the next
+    // (image after image, every image paid for a set of partial sums of its own and for a last round of its own)
+    const float *feat = p.feat, *feat_below = p.feat_below;
+    const _Float16 *act_below = p.act_below, *dpre = p.dpre;
+    auto of_image = [&](int& tile)
+    {
+        const int image = p.batch > 1 ? tile / p.tiles : 0;
+        tile -= image * p.tiles;
+        feat = p.feat + (size_t)image * C * p.H * p.W;
+        dpre = p.dpre + (size_t)image * p.H * p.W * NPAD;
+        if (has_below)
+        {
+            feat_below = p.feat_below + (size_t)image * C * p.Hb * p.Wb;
+            act_below  = p.act_below + (size_t)image * p.Hb * p.Wb * p.cb_store;
+        }
+    };
     auto issue_loads = [&](int tile, TileLoads& r)
     {
+        of_image(tile);
         const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
         const int x0 = tx * kConvTileW, y0 = ty * kConvTileH;
         const int by0 = y0 / 2 - 1, bx0 = x0 / 2 - 1;
@@ -770,7 +816,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             const int y = y0 + py - 1, x = x0 + px - 1;
             const bool in = item < kConvPatchH * kConvPatchW && y >= 0 && y < p.H && x >= 0 && x < p.W;
 #pragma unroll
-            for (int c = 0; c < CI; ++c) r.feat[k][c] = (in && c < C) ? p.feat[c * plane + (size_t)y * p.W + x] : 0.f;
+            for (int c = 0; c < CI; ++c) r.feat[k][c] = (in && c < C) ? feat[c * plane + (size_t)y * p.W + x] : 0.f;
         }
         if (has_below)
         {
@@ -789,11 +835,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
                     {
                         float f[4];
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) f[c] = 4 * q + c < C ? p.feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
+                        for (int c = 0; c < 4; ++c) f[c] = 4 * q + c < C ? feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
                         r.below[k] = make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
                     }
                     else
-                        r.below[k] = *reinterpret_cast<const uint4*>(p.act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ));
+                        r.below[k] = *reinterpret_cast<const uint4*>(act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ));
                 }
             }
         }
@@ -806,7 +852,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
 #pragma unroll
             for (int i = 0; i < 8; ++i) r.dpre[k][i] = _Float16(0.f);
             if (tp < kConvTileH * kConvTileW && y < p.H && x < p.W)
-                r.dpre[k] = *reinterpret_cast<const half8*>(p.dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
+                r.dpre[k] = *reinterpret_cast<const half8*>(dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
         }
     };
     // this level's image into channels [0, C) of a patch pixel (the channels [C, 8) follow from the upsampling, or are
@@ -915,7 +961,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
                 const bool in = y >= 0 && y < p.H && x >= 0 && x < p.W;
                 float v[CI];
 #pragma unroll
-                for (int c = 0; c < CI; ++c) v[c] = (in && c < C) ? p.feat[c * plane + (size_t)y * p.W + x] : 0.f;
+                for (int c = 0; c < CI; ++c) v[c] = (in && c < C) ? feat[c * plane + (size_t)y * p.W + x] : 0.f;
                 put_image(item, v);
             }
         }
@@ -931,12 +977,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
                 {
                     float v[4];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) v[c] = 4 * q + c < C ? p.feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
+                    for (int c = 0; c < 4; ++c) v[c] = 4 * q + c < C ? feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
                     put_below_image(bp, q, v);
                 }
                 else
                 {
-                    put_below_act(bp, q, *reinterpret_cast<const uint4*>(p.act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ)));
+                    put_below_act(bp, q, *reinterpret_cast<const uint4*>(act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ)));
                 }
             }
         }
@@ -947,7 +993,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             half8 v;
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = _Float16(0.f);
-            if (y < p.H && x < p.W) v = *reinterpret_cast<const half8*>(p.dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
+            if (y < p.H && x < p.W) v = *reinterpret_cast<const half8*>(dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
             *reinterpret_cast<half8*>(s_d + (size_t)tp * DS + 8 * g) = v;
         }
     };
@@ -966,9 +1012,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     // with 64 input channels and more than 64 pre-activations the accumulators leave no registers for a tile in flight
     constexpr bool kPrefetch = !(CIN == 64 && NPAD > 64);
     TileLoads cur;
-    if (kPrefetch && (int)blockIdx.x < p.tiles) issue_loads(blockIdx.x, cur);
-    for (int tile = blockIdx.x; tile < p.tiles; tile += gridDim.x)
+    const int tiles = p.tiles * p.batch;
+    if (kPrefetch && (int)blockIdx.x < tiles) issue_loads(blockIdx.x, cur);
+    for (int tile0 = blockIdx.x; tile0 < tiles; tile0 += gridDim.x)
     {
+        int tile = tile0;
+        of_image(tile);
         const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
         const int x0 = tx * kConvTileW, y0 = ty * kConvTileH;
         const int by0 = y0 / 2 - 1, bx0 = x0 / 2 - 1;
@@ -977,7 +1026,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             stream_stage1(x0, y0, by0, bx0);
         else
             commit_loads(cur);
-        if (kPrefetch && tile + (int)gridDim.x < p.tiles) issue_loads(tile + gridDim.x, cur);  // travels during stage 2 and the taps
+        if (kPrefetch && tile0 + (int)gridDim.x < tiles) issue_loads(tile0 + gridDim.x, cur);  // travels during stage 2 and the taps
         if (has_below)
         {
             __syncthreads();
@@ -1191,7 +1240,7 @@ __global__ __launch_bounds__(256) void reduce_weight_grad_kernel(const ReduceTab
 namespace
 {
 template <int KC, int NN, int CI>
-hipError_t launch_bwd_data(const BwdDataParams& p, hipStream_t stream)
+hipError_t launch_bwd_data(const BwdDataParams& p, int batch, hipStream_t stream)
 {
     // the patch and the staged taps of the weights
     const size_t lds_in  = ((size_t)kConvPatchH * kConvPatchW * (KC + kLdsChanPad) + ConvTapStage<KC, NN, 512>::LDS_HALVES) * sizeof(_Float16);
@@ -1201,17 +1250,22 @@ hipError_t launch_bwd_data(const BwdDataParams& p, hipStream_t stream)
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_data_kernel<KC, NN, THREADS, CI>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH);
-    hipLaunchKernelGGL((conv_bwd_data_kernel<KC, NN, THREADS, CI>), grid, dim3(THREADS), lds, stream, p);
+    for (int b = 0; b < batch; b += kMaxGridImages)
+    {
+        BwdDataParams q = p;
+        q.first_image   = b;
+        dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH, std::min(batch - b, kMaxGridImages));
+        hipLaunchKernelGGL((conv_bwd_data_kernel<KC, NN, THREADS, CI>), grid, dim3(THREADS), lds, stream, q);
+    }
     return hipGetLastError();
 }
 
-hipError_t dispatch_bwd_data(const BwdDataParams& p, int npad, int cin_pad, hipStream_t stream)
+hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int cin_pad, hipStream_t stream)
 {
 #define TRIPS_BD(KC_, NN_)                                                                   \
     if (npad == KC_ && cin_pad == NN_)                                                       \
-        return p.c_feat <= 4 ? launch_bwd_data<KC_, NN_, 4>(p, stream)                       \
-                             : p.c_feat <= 8 ? launch_bwd_data<KC_, NN_, 8>(p, stream) : launch_bwd_data<KC_, NN_, 16>(p, stream);
+        return p.c_feat <= 4 ? launch_bwd_data<KC_, NN_, 4>(p, batch, stream)                       \
+                             : p.c_feat <= 8 ? launch_bwd_data<KC_, NN_, 8>(p, batch, stream) : launch_bwd_data<KC_, NN_, 16>(p, batch, stream);
     TRIPS_BD(32, 32) TRIPS_BD(64, 32) TRIPS_BD(96, 32) TRIPS_BD(128, 32)
     TRIPS_BD(32, 64) TRIPS_BD(64, 64) TRIPS_BD(96, 64) TRIPS_BD(128, 64)
 #undef TRIPS_BD
@@ -1298,25 +1352,25 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     const int K           = d.num_output_channels;
     const int ci          = C <= 4 ? 4 : C <= 8 ? 8 : 16;  // image channels the kernels are built with room for
 
-    auto act_ptr = [&](int level, int b)
+    auto act_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<const _Float16*>(sv + l.saved_act_off) + (size_t)b * l.H * l.W * l.cout_store;
+        return reinterpret_cast<const _Float16*>(sv + l.saved_act_off);
     };
-    auto pre_ptr = [&](int level, int b)
+    auto pre_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<const _Float16*>(sv + l.saved_pre_off) + (size_t)b * l.H * l.W * l.npad;
+        return reinterpret_cast<const _Float16*>(sv + l.saved_pre_off);
     };
-    auto dpre_ptr = [&](int level, int b)
+    auto dpre_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<_Float16*>(ws + l.dpre_off) + (size_t)b * l.H * l.W * l.npad;
+        return reinterpret_cast<_Float16*>(ws + l.dpre_off);
     };
-    auto din_ptr = [&](int level, int b)
+    auto din_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<_Float16*>(ws + l.din_off) + (size_t)b * l.H * l.W * l.cin_pad;
+        return reinterpret_cast<_Float16*>(ws + l.din_off);
     };
     auto fill = [&](float* p, int n)
     {
@@ -1349,24 +1403,23 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         ProfScope ps(prof, "unet_bwd_final", stream);
         const LevelPlan& lv = np.lv[0];
         const size_t plane  = (size_t)lv.H * lv.W;
-        for (int b = 0; b < d.batch; ++b)
+        FinalBwdParams p;
+        std::memset(&p, 0, sizeof(p));
+        p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cact_store = lv.cout_store, p.cout = K, p.npad = lv.npad;
+        p.scale    = grad_scale;
+        p.feat     = inputs[0];
+        p.pre      = pre_ptr(0);
+        p.weight   = weights->final_weight;
+        p.d_out    = d_output;
+        p.d_feat   = grads->inputs[0];
+        p.dpre     = dpre_ptr(0);
+        p.chunks   = (int)((plane + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
+        p.batch    = d.batch;
+        p.part     = reinterpret_cast<float*>(ws + np.final_part_off);
+        const bool wgrad = grads->final_weight || grads->final_bias;
+        const int chunks = wgrad ? np.final_groups : p.chunks * p.batch;
+        switch (lv.cout_store)
         {
-            FinalBwdParams p;
-            std::memset(&p, 0, sizeof(p));
-            p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cact_store = lv.cout_store, p.cout = K, p.npad = lv.npad;
-            p.scale    = grad_scale;
-            p.feat     = inputs[0] + (size_t)b * C * plane;
-            p.pre      = pre_ptr(0, b);
-            p.weight   = weights->final_weight;
-            p.d_out    = d_output + (size_t)b * K * plane;
-            p.d_feat   = grads->inputs[0] + (size_t)b * C * plane;
-            p.dpre     = dpre_ptr(0, b);
-            p.chunks   = (int)((plane + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
-            p.part     = reinterpret_cast<float*>(ws + np.final_part_off) + (size_t)b * np.final_groups * (4 * (ci + lv.cout_store) + 4);
-            const bool wgrad = grads->final_weight || grads->final_bias;
-            const int chunks = wgrad ? np.final_groups : p.chunks;
-            switch (lv.cout_store)
-            {
 #define TRIPS_FW_CI(CS_, CI_)                                                                                     \
     if (wgrad)                                                                                                    \
         hipLaunchKernelGGL((final_backward_kernel<CS_, true, CI_>), dim3(chunks), dim3(256), 0, stream, p);       \
@@ -1376,27 +1429,26 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     case CS_:                        \
         if (ci == 4)                 \
         {                            \
-            TRIPS_FW_CI(CS_, 4)      \
+        TRIPS_FW_CI(CS_, 4)      \
         }                            \
         else if (ci == 8)            \
         {                            \
-            TRIPS_FW_CI(CS_, 8)      \
+        TRIPS_FW_CI(CS_, 8)      \
         }                            \
         else                         \
         {                            \
-            TRIPS_FW_CI(CS_, 16)     \
+        TRIPS_FW_CI(CS_, 16)     \
         }                            \
         break;
-                TRIPS_FW(8) TRIPS_FW(16) TRIPS_FW(24) TRIPS_FW(32) TRIPS_FW(40) TRIPS_FW(48) TRIPS_FW(56) TRIPS_FW(64)
+            TRIPS_FW(8) TRIPS_FW(16) TRIPS_FW(24) TRIPS_FW(32) TRIPS_FW(40) TRIPS_FW(48) TRIPS_FW(56) TRIPS_FW(64)
 #undef TRIPS_FW
 #undef TRIPS_FW_CI
-                default: return set_error(TRIPS_ERR_UNSUPPORTED, "block output stride %d", lv.cout_store);
-            }
+            default: return set_error(TRIPS_ERR_UNSUPPORTED, "block output stride %d", lv.cout_store);
         }
         if (grads->final_weight || grads->final_bias)
         {
             hipLaunchKernelGGL(final_reduce_kernel, dim3(K * (C + lv.cout) + K), dim3(256), 0, stream,
-                               reinterpret_cast<const float*>(ws + np.final_part_off), d.batch * np.final_groups, ci + lv.cout_store, ci, C,
+                               reinterpret_cast<const float*>(ws + np.final_part_off), np.final_groups, ci + lv.cout_store, ci, C,
                                lv.cout, K, grads->final_weight, grads->final_bias);
         }
     }
@@ -1411,79 +1463,76 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         const bool below    = i < L - 1;
         {
             ProfScope ps(prof, kWeightNames[i], stream);
-            for (int b = 0; b < d.batch; ++b)
-            {
-                BiasGradParams bp;
-                bp.pixels    = plane;
-                bp.npad      = lv.npad;
-                bp.cout      = lv.cout;
-                bp.scale_inv = scale_inv;
-                bp.dpre      = dpre_ptr(i, b);
-                bp.d_bias_f  = grads->feature_bias[i];
-                bp.d_bias_m  = grads->mask_bias[i];
-                const bool want_w = grads->feature_weight[i] || grads->mask_weight[i];
-                if ((bp.d_bias_f || bp.d_bias_m) && !want_w)  // otherwise the weight-gradient kernel sums them on its way
-                    hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((plane + kBiasChunk - 1) / kBiasChunk)), dim3(256), 0, stream, bp);
+            BiasGradParams bp;
+            bp.pixels    = plane * d.batch;
+            bp.npad      = lv.npad;
+            bp.cout      = lv.cout;
+            bp.scale_inv = scale_inv;
+            bp.dpre      = dpre_ptr(i);
+            bp.d_bias_f  = grads->feature_bias[i];
+            bp.d_bias_m  = grads->mask_bias[i];
+            const bool want_w = grads->feature_weight[i] || grads->mask_weight[i];
+            if ((bp.d_bias_f || bp.d_bias_m) && !want_w)  // otherwise the weight-gradient kernel sums them on its way
+                hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((bp.pixels + kBiasChunk - 1) / kBiasChunk)), dim3(256), 0, stream, bp);
 
-                BwdWeightParams wp;
-                std::memset(&wp, 0, sizeof(wp));
-                wp.H = lv.H, wp.W = lv.W, wp.c_feat = C;
-                wp.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
-                wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
-                wp.feat    = inputs[i] + (size_t)b * C * plane;
-                wp.dpre    = dpre_ptr(i, b);
-                wp.part    = reinterpret_cast<float*>(ws + lv.part_off) + (size_t)b * lv.groups * 9 * lv.npad * lv.cin_pad;
-                if (bp.d_bias_f || bp.d_bias_m)
-                    wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off) + (size_t)b * lv.groups * lv.npad;
-                if (below)
-                {
-                    const LevelPlan& lb = np.lv[i + 1];
-                    wp.Hb = lb.H, wp.Wb = lb.W, wp.cb_store = lb.cout_store;
-                    wp.feat_below = inputs[i + 1] + (size_t)b * C * lb.H * lb.W;
-                    wp.act_below  = act_ptr(i + 1, b);
-                }
-                if (grads->feature_weight[i] || grads->mask_weight[i])
-                {
-                    hipError_t e = dispatch_bwd_weight(wp, lv.cin_pad, lv.npad, lv.groups, stream);
-                    if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
-                }
+            BwdWeightParams wp;
+            std::memset(&wp, 0, sizeof(wp));
+            wp.H = lv.H, wp.W = lv.W, wp.c_feat = C;
+            wp.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
+            wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
+            wp.batch   = d.batch;
+            wp.feat    = inputs[i];
+            wp.dpre    = dpre_ptr(i);
+            wp.part    = reinterpret_cast<float*>(ws + lv.part_off);
+            if (bp.d_bias_f || bp.d_bias_m) wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off);
+            if (below)
+            {
+                const LevelPlan& lb = np.lv[i + 1];
+                wp.Hb = lb.H, wp.Wb = lb.W, wp.cb_store = lb.cout_store;
+                wp.feat_below = inputs[i + 1];
+                wp.act_below  = act_ptr(i + 1);
+            }
+            if (want_w)
+            {
+                hipError_t e = dispatch_bwd_weight(wp, lv.cin_pad, lv.npad, lv.groups, stream);
+                if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
             }
         }
         {
             ProfScope ps(prof, kDataNames[i], stream);
-            for (int b = 0; b < d.batch; ++b)
+            BwdDataParams dp;
+            dp.H = lv.H, dp.W = lv.W, dp.c_feat = C;
+            dp.scale_inv = scale_inv;
+            dp.dpre      = dpre_ptr(i);
+            dp.wt        = reinterpret_cast<const _Float16*>(ws + lv.wt_off);
+            dp.d_feat    = grads->inputs[i];
+            dp.d_in      = below ? din_ptr(i) : nullptr;
+            hipError_t e = dispatch_bwd_data(dp, d.batch, lv.npad, lv.cin_pad, stream);
+            if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
+            if (below)
             {
-                BwdDataParams dp;
-                dp.H = lv.H, dp.W = lv.W, dp.c_feat = C;
-                dp.scale_inv = scale_inv;
-                dp.dpre      = dpre_ptr(i, b);
-                dp.wt        = reinterpret_cast<const _Float16*>(ws + lv.wt_off);
-                dp.d_feat    = grads->inputs[i] + (size_t)b * C * plane;
-                dp.d_in      = below ? din_ptr(i, b) : nullptr;
-                hipError_t e = dispatch_bwd_data(dp, lv.npad, lv.cin_pad, stream);
-                if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
-                if (below)
+                const LevelPlan& lb = np.lv[i + 1];
+                UpAdjointParams up;
+                up.H = lv.H, up.W = lv.W, up.Hb = lb.H, up.Wb = lb.W;
+                up.cin_fine  = lv.cin_pad;
+                up.c_feat    = C;
+                up.cout      = lb.cout;
+                up.npad      = lb.npad;
+                up.scale_inv = scale_inv;
+                up.d_in      = din_ptr(i);
+                up.pre       = pre_ptr(i + 1);
+                up.d_feat    = grads->inputs[i + 1];
+                up.dpre      = dpre_ptr(i + 1);
+                const size_t items = (size_t)lb.H * lb.W * ((2 * C - 1) / 8 - C / 8 + 1 + lb.npad / 16);
+                for (up.first_image = 0; up.first_image < d.batch; up.first_image += kMaxGridImages)
                 {
-                    const LevelPlan& lb = np.lv[i + 1];
-                    UpAdjointParams up;
-                    up.H = lv.H, up.W = lv.W, up.Hb = lb.H, up.Wb = lb.W;
-                    up.cin_fine  = lv.cin_pad;
-                    up.c_feat    = C;
-                    up.cout      = lb.cout;
-                    up.npad      = lb.npad;
-                    up.scale_inv = scale_inv;
-                    up.d_in      = din_ptr(i, b);
-                    up.pre       = pre_ptr(i + 1, b);
-                    up.d_feat    = grads->inputs[i + 1] + (size_t)b * C * lb.H * lb.W;
-                    up.dpre      = dpre_ptr(i + 1, b);
-                    const size_t items = (size_t)lb.H * lb.W * ((2 * C - 1) / 8 - C / 8 + 1 + lb.npad / 16);
-                    const int blocks   = (int)std::min<size_t>((items + 255) / 256, 1u << 20);
+                    const dim3 blocks((unsigned)std::min<size_t>((items + 255) / 256, 1u << 20), std::min(d.batch - up.first_image, kMaxGridImages));
                     switch ((2 * C) & 7)
                     {
-                        case 0: hipLaunchKernelGGL(up2_adjoint_gate_kernel<0>, dim3(blocks), dim3(256), 0, stream, up); break;
-                        case 2: hipLaunchKernelGGL(up2_adjoint_gate_kernel<2>, dim3(blocks), dim3(256), 0, stream, up); break;
-                        case 4: hipLaunchKernelGGL(up2_adjoint_gate_kernel<4>, dim3(blocks), dim3(256), 0, stream, up); break;
-                        default: hipLaunchKernelGGL(up2_adjoint_gate_kernel<6>, dim3(blocks), dim3(256), 0, stream, up); break;
+                        case 0: hipLaunchKernelGGL(up2_adjoint_gate_kernel<0>, blocks, dim3(256), 0, stream, up); break;
+                        case 2: hipLaunchKernelGGL(up2_adjoint_gate_kernel<2>, blocks, dim3(256), 0, stream, up); break;
+                        case 4: hipLaunchKernelGGL(up2_adjoint_gate_kernel<4>, blocks, dim3(256), 0, stream, up); break;
+                        default: hipLaunchKernelGGL(up2_adjoint_gate_kernel<6>, blocks, dim3(256), 0, stream, up); break;
                     }
                 }
             }
@@ -1504,7 +1553,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             ReduceLevel& r = rt.lv[n++];
             r.part      = reinterpret_cast<const float*>(ws + lv.part_off);
             r.sliced    = reinterpret_cast<float*>(ws + lv.sliced_off);
-            r.groups    = d.batch * lv.groups;
+            r.groups    = lv.groups;
             r.total     = 9 * lv.npad * lv.cin_pad;
             r.cout = lv.cout, r.cin_real = lv.cin_real, r.cin_pad = lv.cin_pad, r.npad = lv.npad;
             r.d_wf = grads->feature_weight[i], r.d_wm = grads->mask_weight[i];

@@ -21,6 +21,7 @@ constexpr int kBelowW      = kConvTileW / 2 + 2;
 constexpr int kFinalPixelsPerBlock = 512;   // pixels a workgroup of the 1x1 convolution's backward takes at a time
 constexpr int kUnetMaxImageChannels = 16;  // channels of the splat images (the descriptor widths of the splat: 3, 4, 6, 8, 16)
 constexpr int kFinalPartFloats     = 4 * (kUnetMaxImageChannels + 64) + 4;  // its partial sums: [4 outputs][<= 16 image + <= 64 block channels], 4 biases
+constexpr int kMaxGridImages = 32768;  // images of a batch that one launch takes (the y and z dimensions of a grid end at 65535)
 constexpr int kLdsChanPad  = 8;  // halves added to every LDS row so that 16 lanes reading 16 bytes hit 64 distinct banks
 
 // source row / column and weight of torch's bilinear upsampling with scale_factor 2, align_corners = false
@@ -210,8 +211,8 @@ struct LevelPlan
     size_t din_off;     // gradient of the block input [B][H][W][cin_pad] fp16
     size_t part_off;    // partial weight gradients [groups][9][npad][cin_pad] fp32
     size_t sliced_off;  // partial sums of the partials [16][9][npad][cin_pad] fp32
-    size_t bias_part_off;  // per-workgroup sums of the pre-activation gradients [batch * groups][npad] fp32
-    int groups;         // persistent workgroups of the weight-gradient kernel (per image)
+    size_t bias_part_off;  // per-workgroup sums of the pre-activation gradients [groups][npad] fp32
+    int groups;         // persistent workgroups of the weight-gradient kernel, for all images of the batch
 };
 
 struct NetPlan
@@ -221,7 +222,7 @@ struct NetPlan
     size_t saved_bytes;     // saved state
     size_t backward_bytes;  // backward workspace
     size_t final_part_off;  // backward workspace: per-workgroup sums of the 1x1 convolution's weight and bias gradients
-    int final_groups;       // persistent workgroups of the finest level's first backward kernel (per image)
+    int final_groups;       // persistent workgroups of the finest level's first backward kernel, for all images of the batch
 };
 
 inline int check_unet_desc(const TripsUnetDesc* d)
@@ -306,25 +307,25 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         bw += align256(pixels * lv.npad * sizeof(_Float16));
         lv.din_off = bw;
         bw += align256(pixels * lv.cin_pad * sizeof(_Float16));
-        const int tiles = ((lv.W + kConvTileW - 1) / kConvTileW) * ((lv.H + kConvTileH - 1) / kConvTileH);
+        const long long tiles = (long long)d.batch * ((lv.W + kConvTileW - 1) / kConvTileW) * ((lv.H + kConvTileH - 1) / kConvTileH);
         // persistent workgroups of the weight-gradient kernel: as many as are resident at once (two per CU for the
         // smallest shape, else one); every further one would only add a set of partial sums to write and reduce
         const int resident = (lv.cin_pad * lv.npad <= 1024 ? 2 : 1) * 256;
-        lv.groups          = tiles < resident ? tiles : resident;
+        lv.groups          = tiles < resident ? (int)tiles : resident;
         lv.part_off     = bw;
-        bw += align256((size_t)d.batch * lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
+        bw += align256((size_t)lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
         lv.sliced_off = bw;
         bw += align256((size_t)16 * 9 * lv.npad * lv.cin_pad * sizeof(float));
         lv.bias_part_off = bw;
-        bw += align256((size_t)d.batch * lv.groups * lv.npad * sizeof(float));
+        bw += align256((size_t)lv.groups * lv.npad * sizeof(float));
     }
     {
-        const size_t chunks = ((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock;
+        const size_t chunks = d.batch * (((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
         // as many workgroups as are resident at once (three per CU at the kernel's 160 registers) walk the chunks: a
         // second, partly filled round of one-chunk workgroups cost a third of the kernel's time
         np.final_groups     = chunks < 768 ? (int)chunks : 768;
         np.final_part_off   = bw;
-        bw += align256((size_t)d.batch * np.final_groups * kFinalPartFloats * sizeof(float));
+        bw += align256((size_t)np.final_groups * kFinalPartFloats * sizeof(float));
     }
     np.saved_bytes    = sv;
     np.backward_bytes = bw;

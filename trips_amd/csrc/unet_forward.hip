@@ -45,6 +45,9 @@ struct ConvParams
     const float* final_b;     // [final_cout]
     float* final_out;         // [final_cout][H][W]
     int final_cout;
+    // the images of a batch are the grid's z dimension: the first one's number, elements from one image to the next
+    int first_image;
+    size_t feat_stride, feat_below_stride, act_below_stride, out_stride, pre_stride, final_stride;
 };
 
 // A loaded value that is only needed under a condition is otherwise loaded under that condition by the compiler, in a
@@ -55,8 +58,16 @@ __device__ __forceinline__ void loaded(uint4& v) { asm volatile("" : "+v"(v.x), 
 
 // CI: image channels the kernel has room for (4, 8 or 16; C <= CI)
 template <int CIN, int NPAD, int THREADS, int CI>
-__global__ __launch_bounds__(THREADS) void gated_conv3x3_kernel(const ConvParams p)
+__global__ __launch_bounds__(THREADS) void gated_conv3x3_kernel(ConvParams p)
 {
+    // All images of a batch are one launch: the coarse levels of a 512 x 512 crop are 4 to 64 tiles, and image after
+    // image they took the latency of a tile each (four crops, five levels of 32: 256 us in 20 launches).
+    {
+        const size_t b = p.first_image + blockIdx.z;
+        p.feat += b * p.feat_stride, p.feat_below += b * p.feat_below_stride, p.act_below += b * p.act_below_stride;
+        p.out = p.out ? p.out + b * p.out_stride : nullptr, p.pre = p.pre ? p.pre + b * p.pre_stride : nullptr;
+        p.final_out = p.final_out ? p.final_out + b * p.final_stride : nullptr;
+    }
     constexpr int IQ = CI / 4;  // 16-byte items that carry the image of a pixel of the level below
     constexpr int MB = 16 / (THREADS / 64);  // 16-pixel row blocks of a wavefront: two rows of the tile, or one
     constexpr int ROW  = CIN + kLdsChanPad;  // halves per patch pixel in LDS
@@ -492,7 +503,7 @@ __global__ __launch_bounds__(256) void pack_conv_weights_kernel(const PackTable 
 namespace
 {
 template <int CIN, int NPAD, int CI>
-hipError_t launch_conv(const ConvParams& p, hipStream_t stream)
+hipError_t launch_conv(const ConvParams& p, int batch, hipStream_t stream)
 {
     constexpr int ROW  = CIN + kLdsChanPad;
     constexpr int IPAD = CI > kLdsChanPad ? CI : kLdsChanPad;
@@ -506,37 +517,42 @@ hipError_t launch_conv(const ConvParams& p, hipStream_t stream)
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gated_conv3x3_kernel<CIN, NPAD, THREADS, CI>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH);
-    hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, NPAD, THREADS, CI>), grid, dim3(THREADS), lds, stream, p);
+    for (int b = 0; b < batch; b += kMaxGridImages)
+    {
+        ConvParams q = p;
+        q.first_image = b;
+        dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH, std::min(batch - b, kMaxGridImages));
+        hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, NPAD, THREADS, CI>), grid, dim3(THREADS), lds, stream, q);
+    }
     return hipGetLastError();
 }
 
 template <int CI>
-hipError_t dispatch_conv_ci(const ConvParams& p, int cin_pad, int npad, hipStream_t stream)
+hipError_t dispatch_conv_ci(const ConvParams& p, int batch, int cin_pad, int npad, hipStream_t stream)
 {
     if (cin_pad == 32)
     {
-        if (npad == 32) return launch_conv<32, 32, CI>(p, stream);
-        if (npad == 64) return launch_conv<32, 64, CI>(p, stream);
-        if (npad == 96) return launch_conv<32, 96, CI>(p, stream);
-        if (npad == 128) return launch_conv<32, 128, CI>(p, stream);
+        if (npad == 32) return launch_conv<32, 32, CI>(p, batch, stream);
+        if (npad == 64) return launch_conv<32, 64, CI>(p, batch, stream);
+        if (npad == 96) return launch_conv<32, 96, CI>(p, batch, stream);
+        if (npad == 128) return launch_conv<32, 128, CI>(p, batch, stream);
     }
     else
     {
-        if (npad == 32) return launch_conv<64, 32, CI>(p, stream);
-        if (npad == 64) return launch_conv<64, 64, CI>(p, stream);
-        if (npad == 96) return launch_conv<64, 96, CI>(p, stream);
-        if (npad == 128) return launch_conv<64, 128, CI>(p, stream);
+        if (npad == 32) return launch_conv<64, 32, CI>(p, batch, stream);
+        if (npad == 64) return launch_conv<64, 64, CI>(p, batch, stream);
+        if (npad == 96) return launch_conv<64, 96, CI>(p, batch, stream);
+        if (npad == 128) return launch_conv<64, 128, CI>(p, batch, stream);
     }
     return hipErrorInvalidValue;
 }
 
 // (the kernel is built for 4, 8 and 16 image channels; fewer use the next size up)
-hipError_t dispatch_conv(const ConvParams& p, int cin_pad, int npad, hipStream_t stream)
+hipError_t dispatch_conv(const ConvParams& p, int batch, int cin_pad, int npad, hipStream_t stream)
 {
-    if (p.c_feat <= 4) return dispatch_conv_ci<4>(p, cin_pad, npad, stream);
-    if (p.c_feat <= 8) return dispatch_conv_ci<8>(p, cin_pad, npad, stream);
-    return dispatch_conv_ci<16>(p, cin_pad, npad, stream);
+    if (p.c_feat <= 4) return dispatch_conv_ci<4>(p, batch, cin_pad, npad, stream);
+    if (p.c_feat <= 8) return dispatch_conv_ci<8>(p, batch, cin_pad, npad, stream);
+    return dispatch_conv_ci<16>(p, batch, cin_pad, npad, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -600,11 +616,10 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
     char* sv           = reinterpret_cast<char*>(saved);
     Profiler* prof     = ctx->prof.enabled ? &ctx->prof : nullptr;
     // block outputs live in the saved state when there is one (the backward reads them), else in the workspace
-    auto act_ptr = [&](int level, int b)
+    auto act_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        char* base         = sv ? sv + l.saved_act_off : ws + l.act_off;
-        return reinterpret_cast<_Float16*>(base) + (size_t)b * l.H * l.W * l.cout_store;
+        return reinterpret_cast<_Float16*>(sv ? sv + l.saved_act_off : ws + l.act_off);
     };
 
     if (!d.weights_packed)
@@ -628,41 +643,44 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
     {
         const LevelPlan& lv = np.lv[i];
         ProfScope ps(prof, kLevelNames[i], stream);
-        for (int b = 0; b < d.batch; ++b)
+        ConvParams p;
+        std::memset(&p, 0, sizeof(p));
+        p.H           = lv.H;
+        p.W           = lv.W;
+        p.c_feat      = C;
+        p.cout        = lv.cout;
+        p.cout_store  = lv.cout_store;
+        p.feat        = inputs[i];
+        p.feat_stride = (size_t)C * lv.H * lv.W;
+        p.wpack       = reinterpret_cast<const _Float16*>(ws + lv.wpack_off);
+        p.bias        = reinterpret_cast<const float*>(ws + lv.bias_off);
+        // (nobody reads the finest block's output again: its 1x1 runs in the same kernel, and the backward takes
+        // it from the pre-activations)
+        p.out        = i == 0 ? nullptr : act_ptr(i);
+        p.out_stride = (size_t)lv.H * lv.W * lv.cout_store;
+        p.pre        = sv ? reinterpret_cast<_Float16*>(sv + lv.saved_pre_off) : nullptr;
+        p.pre_stride = (size_t)lv.H * lv.W * lv.npad;
+        if (i < L - 1)
         {
-            ConvParams p;
-            std::memset(&p, 0, sizeof(p));
-            p.H          = lv.H;
-            p.W          = lv.W;
-            p.c_feat     = C;
-            p.cout       = lv.cout;
-            p.cout_store = lv.cout_store;
-            p.feat       = inputs[i] + (size_t)b * C * lv.H * lv.W;
-            p.wpack      = reinterpret_cast<const _Float16*>(ws + lv.wpack_off);
-            p.bias       = reinterpret_cast<const float*>(ws + lv.bias_off);
-            // (nobody reads the finest block's output again: its 1x1 runs in the same kernel, and the backward takes
-            // it from the pre-activations)
-            p.out        = i == 0 ? nullptr : act_ptr(i, b);
-            p.pre        = sv ? reinterpret_cast<_Float16*>(sv + lv.saved_pre_off) + (size_t)b * lv.H * lv.W * lv.npad : nullptr;
-            if (i < L - 1)
-            {
-                const LevelPlan& lb = np.lv[i + 1];
-                p.Hb         = lb.H;
-                p.Wb         = lb.W;
-                p.cb_store   = lb.cout_store;
-                p.feat_below = inputs[i + 1] + (size_t)b * C * lb.H * lb.W;
-                p.act_below  = act_ptr(i + 1, b);
-            }
-            if (i == 0)
-            {
-                p.final_w    = weights->final_weight;
-                p.final_b    = weights->final_bias;
-                p.final_out  = output + (size_t)b * d.num_output_channels * lv.H * lv.W;
-                p.final_cout = d.num_output_channels;
-            }
-            hipError_t e = dispatch_conv(p, lv.cin_pad, lv.npad, stream);
-            if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "gated conv launch (level %d): %s", i, hipGetErrorString(e));
+            const LevelPlan& lb = np.lv[i + 1];
+            p.Hb                = lb.H;
+            p.Wb                = lb.W;
+            p.cb_store          = lb.cout_store;
+            p.feat_below        = inputs[i + 1];
+            p.feat_below_stride = (size_t)C * lb.H * lb.W;
+            p.act_below         = act_ptr(i + 1);
+            p.act_below_stride  = (size_t)lb.H * lb.W * lb.cout_store;
         }
+        if (i == 0)
+        {
+            p.final_w      = weights->final_weight;
+            p.final_b      = weights->final_bias;
+            p.final_out    = output;
+            p.final_stride = (size_t)d.num_output_channels * lv.H * lv.W;
+            p.final_cout   = d.num_output_channels;
+        }
+        hipError_t e = dispatch_conv(p, d.batch, lv.cin_pad, lv.npad, stream);
+        if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "gated conv launch (level %d): %s", i, hipGetErrorString(e));
     }
     return TRIPS_OK;
 }
