@@ -69,10 +69,9 @@ __global__ __launch_bounds__(256) void pack_conv_weights_T_kernel(const PackTTab
     for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256)
     {
         const int n = i % npad, c = (i / npad) % cin_pad, tap = i / (npad * cin_pad);
-        const int half = npad / 2;
-        const int o    = n < half ? n : n - half;
-        float v        = 0.f;
-        if (o < cout && c < cin_real) v = (n < half ? wf : wm)[((size_t)o * cin_real + c) * 9 + (8 - tap)];
+        const int o = preact_channel(n);
+        float v     = 0.f;
+        if (o < cout && c < cin_real) v = (preact_is_mask(n) ? wm : wf)[((size_t)o * cin_real + c) * 9 + (8 - tap)];
         wt[i] = _Float16(v);
     }
 }
@@ -84,7 +83,7 @@ __global__ __launch_bounds__(256) void fill_f32_kernel(float* __restrict__ p, fl
 
 struct FinalBwdParams
 {
-    int H, W, c_feat, cact, cact_store, cout, npad;
+    int H, W, c_feat, cact, cout, npad;
     float scale;
     const float* feat;        // [C][H][W]
     const _Float16* pre;      // [H][W][npad]
@@ -103,16 +102,15 @@ struct FinalBwdParams
 // workgroups up: atomics of a thousand workgroups on these few addresses would serialise in one L2 channel).
 // (The library is compiled without contraction of products and sums; this kernel is bound by its arithmetic
 // instructions, and its sums are written as fused multiply-adds.)
-// CS = halves per pixel of the block output.
 // CI = image channels the kernel has room for (4, 8 or 16).
-template <int CS, bool WGRAD, int CI>
+template <int NPAD, bool WGRAD, int CI>
 __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParams p)
 {
+    constexpr int CS   = NPAD / 2;  // block outputs, padded
     constexpr int MAXC = CI + CS;
-    // LPP lanes share a pixel, one per 16 bytes of its pre-activation row (feature groups first, then mask groups),
-    // so that a wavefront reads and writes whole lines of the channels-innermost arrays. The feature and the mask
-    // lane of a channel group exchange their values with one cross-lane read.
-    constexpr int LPP = CS <= 16 ? 4 : CS <= 32 ? 8 : 16;
+    // LPP lanes share a pixel, one per 16 bytes of its pre-activation row (the features and the masks of four channels),
+    // so that a wavefront reads and writes whole lines of the channels-innermost arrays.
+    constexpr int LPP = NPAD <= 32 ? 4 : NPAD <= 64 ? 8 : 16;
     constexpr int PPW = 64 / LPP;  // pixels per wavefront and iteration
     __shared__ float s_w[4 * MAXC];
     __shared__ float s_sum[4 * MAXC + 4];
@@ -129,20 +127,13 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
     const size_t plane = (size_t)p.H * p.W;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane % LPP, sub = lane / LPP;
-    const int hg       = p.npad / 16;                    // 16-byte groups in each half of a pre-activation row
-    const bool is_f    = g < hg;
-    const bool in_row  = g < 2 * hg;                     // lanes past the row idle (rows of 96 halves on 16 lanes)
-    const int ch0      = 8 * (is_f ? g : g - hg);        // first of this lane's 8 channels
-    const int partner  = is_f ? lane + hg : lane - hg;   // the lane with the other half of the same channels
+    const bool in_row = g < NPAD / 8;  // lanes past the row idle (rows of 96 halves on 16 lanes)
+    const int c0      = 4 * g;         // first of this lane's four channels
     // ... and the image channels g, g + LPP, ... (one each for up to LPP image channels)
     constexpr int NI = (CI + LPP - 1) / LPP;
     bool has_img[NI];
 #pragma unroll
     for (int j = 0; j < NI; ++j) has_img[j] = g + LPP * j < p.c_feat;
-    // The feature lane and the mask lane of a group hold the same eight channels once they have exchanged their values:
-    // the feature lane works out the first four (gradients of both pre-activations, the block's output), the mask lane
-    // the other four, and they exchange what the other one stores.
-    const int c0 = ch0 + (is_f ? 0 : 4);  // first of the four channels this lane works out
     float wj[4][4], wimg[4][NI];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -150,7 +141,7 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
 #pragma unroll
         for (int j = 0; j < NI; ++j) wimg[k][j] = has_img[j] ? s_w[k * MAXC + g + LPP * j] : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wj[k][i] = (in_row && c0 + i < CS) ? s_w[k * MAXC + CI + c0 + i] : 0.f;
+        for (int i = 0; i < 4; ++i) wj[k][i] = in_row ? s_w[k * MAXC + CI + c0 + i] : 0.f;
     }
     float acc[4][4];
     float acc_img[4][NI], accb[4] = {0.f, 0.f, 0.f, 0.f};
@@ -182,7 +173,7 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
         for (int j = 0; j < NI; ++j) l.x[j] = (WGRAD && valid && has_img[j]) ? feat[(size_t)(g + LPP * j) * plane + pix] : 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) l.mine[i] = _Float16(0.f);
-        if (valid && in_row) l.mine = *reinterpret_cast<const half8*>(pre + pix * p.npad + 8 * g);
+        if (valid && in_row) l.mine = *reinterpret_cast<const half8*>(pre + pix * NPAD + 8 * g);
         return l;
     };
     constexpr int STEP = 4 * PPW;  // pixels per iteration of the workgroup
@@ -203,15 +194,8 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
             const bool valid = pix < p1;
             const Loaded cur = next;
             if (base + STEP < p1) next = load(pix + STEP, pix + STEP < p1);  // in flight while this pixel is worked on
-            // the other half (mask values for a feature lane and the reverse) of the same 8 channels
-            typedef int intx4 __attribute__((ext_vector_type(4)));
-            intx4 raw = __builtin_bit_cast(intx4, cur.mine), oth;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) oth[q] = __shfl(raw[q], partner);
-            const half8 other = __builtin_bit_cast(half8, oth);
-            const half8 f8 = is_f ? cur.mine : other, m8 = is_f ? other : cur.mine;
-            half4 keep, give;  // what this lane stores of its four channels, and what its partner stores of them
-            float v[4];        // the block's output as the forward's 1x1 convolution read it (fp16)
+            half8 out;   // gradients of the four features, then of the four masks
+            float v[4];  // the block's output as the forward's 1x1 convolution read it (fp16)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
             {
@@ -219,21 +203,12 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
 #pragma unroll
                 for (int k = 0; k < 4; ++k) da = __builtin_fmaf(wj[k][i], cur.g[k], da);
                 float df, dm, a;
-                gate_backward(da * p.scale, float(is_f ? f8[i] : f8[4 + i]), float(is_f ? m8[i] : m8[4 + i]), df, dm, a);
-                keep[i] = _Float16(is_f ? df : dm);
-                give[i] = _Float16(is_f ? dm : df);
-                v[i]    = (valid && in_row && c0 + i < p.cact) ? float(_Float16(a)) : 0.f;
+                gate_backward(da * p.scale, float(cur.mine[i]), float(cur.mine[4 + i]), df, dm, a);
+                out[i]     = _Float16(df);
+                out[4 + i] = _Float16(dm);
+                v[i]       = (valid && c0 + i < p.cact) ? float(_Float16(a)) : 0.f;
             }
-            typedef int intx2 __attribute__((ext_vector_type(2)));
-            const intx2 give_raw = __builtin_bit_cast(intx2, give);
-            intx2 got_raw;
-            got_raw[0] = __shfl(give_raw[0], partner);
-            got_raw[1] = __shfl(give_raw[1], partner);
-            const half4 got = __builtin_bit_cast(half4, got_raw);
-            // a feature lane stores the feature gradients of the eight channels: its own four, then the partner's
-            const half8 out = is_f ? half8{keep[0], keep[1], keep[2], keep[3], got[0], got[1], got[2], got[3]}
-                                   : half8{got[0], got[1], got[2], got[3], keep[0], keep[1], keep[2], keep[3]};
-            if (valid && in_row) *reinterpret_cast<half8*>(dpre + pix * p.npad + 8 * g) = out;
+            if (valid && in_row) *reinterpret_cast<half8*>(dpre + pix * NPAD + 8 * g) = out;
 #pragma unroll
             for (int j = 0; j < NI; ++j)
             {
@@ -286,7 +261,7 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
         for (int i = 0; i < 4; ++i)
         {
             const float v = fold(acc[k][i]);
-            if (lane < LPP && in_row && c0 + i < CS) atomicAdd(&s_sum[k * MAXC + CI + c0 + i], v);
+            if (lane < LPP && in_row) atomicAdd(&s_sum[k * MAXC + CI + c0 + i], v);
         }
     }
     __syncthreads();
@@ -501,8 +476,10 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
         for (int i = 0; i < 8; ++i) f8[i] = m8[i] = _Float16(0.f);
         if (q >= ig)
         {
-            f8 = *reinterpret_cast<const half8*>(p.pre + bp * p.npad + ch0);
-            m8 = *reinterpret_cast<const half8*>(p.pre + bp * p.npad + half + ch0);
+            const half8 lo = *reinterpret_cast<const half8*>(p.pre + bp * p.npad + 2 * ch0);
+            const half8 hi = *reinterpret_cast<const half8*>(p.pre + bp * p.npad + 2 * ch0 + 8);
+            f8 = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            m8 = half8{lo[4], lo[5], lo[6], lo[7], hi[4], hi[5], hi[6], hi[7]};
         }
         float wy[4], wx[4];
 #pragma unroll
@@ -582,8 +559,8 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
                 of[i] = _Float16(df);
                 om[i] = _Float16(dm);
             }
-            *reinterpret_cast<half8*>(dp + ch0)        = of;
-            *reinterpret_cast<half8*>(dp + half + ch0) = om;
+            *reinterpret_cast<half8*>(dp + 2 * ch0)     = half8{of[0], of[1], of[2], of[3], om[0], om[1], om[2], om[3]};
+            *reinterpret_cast<half8*>(dp + 2 * ch0 + 8) = half8{of[4], of[5], of[6], of[7], om[4], om[5], om[6], om[7]};
         }
     }
 }
@@ -626,11 +603,10 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(const BiasGradParams p)
     __syncthreads();
     if ((int)threadIdx.x < p.npad)
     {
-        const int n = threadIdx.x, half = p.npad / 2;
-        const int o = n < half ? n : n - half;
+        const int n = threadIdx.x, o = preact_channel(n);
         if (o < p.cout)
         {
-            float* dst = n < half ? p.d_bias_f : p.d_bias_m;
+            float* dst = preact_is_mask(n) ? p.d_bias_m : p.d_bias_f;
             if (dst) atomicAdd(dst + o, s_sum[n] * p.scale_inv);
         }
     }
@@ -640,13 +616,12 @@ __global__ __launch_bounds__(256) void bias_grad_kernel(const BiasGradParams p)
 struct BwdWeightParams
 {
     int H, W, Hb, Wb;
-    int c_feat, cb_store;
+    int c_feat, below_stride;
     int tiles_x, tiles;  // tiles of one image
     int batch;           // images, one after the other in every array
     const float* feat;
-    const float* feat_below;
-    const _Float16* act_below;
-    const _Float16* dpre;  // [H][W][NPAD]
+    const _Float16* below;  // rows of the level below, [Hb][Wb][below_stride]
+    const _Float16* dpre;   // [H][W][NPAD]
     float* part;           // [gridDim.x][9][NPAD][CIN]
     // bias gradients = sums of dpre over the pixels, taken from the transposed tile while it is in LDS
     float* bias_part;      // [gridDim.x][NPAD] or nullptr
@@ -715,11 +690,10 @@ __device__ __forceinline__ void lds_read_pixel_windows(const _Float16* tile, int
 }
 
 // THREADS: 256, or 512 for the largest shape, whose 9 x NPAD x CIN sums are 288 registers per lane of four wavefronts.
-// CI: image channels the kernel has room for (4, 8 or 16; C <= CI)
-template <int CIN, int NPAD, bool BIAS, int THREADS, int CI>
+// CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
+template <int CIN, int NPAD, bool BIAS, int THREADS, int CI, bool FOUR>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightParams p)
 {
-    constexpr int IQ = CI / 4;  // 16-byte items that carry the image of a pixel of the level below
     constexpr int ROW    = CIN + kLdsChanPad;   // halves per pixel of the input patch
     constexpr int DS     = NPAD + kLdsChanPad;  // halves per pixel of the gradient tile
     constexpr int GROUPS = CIN / 8;
@@ -744,7 +718,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     _Float16* s_below = s_patch + kConvPatchH * kConvPatchW * ROW;      // [kBelowH * kBelowW][ROW]
     _Float16* s_d     = s_below + kBelowH * kBelowW * ROW;              // [kConvTileH * kConvTileW][DS]
     const bool has_below = p.Hb > 0;
-    const int C          = p.c_feat;
+    const int C          = FOUR ? 4 : p.c_feat;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lk = (lane >> 4) * 8;
 
@@ -773,8 +747,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     // flight together), and written to LDS one tile later, so that the loads of tile t + 1 travel while tile t is
     // upsampled and multiplied ----
     constexpr int kFeatItems  = (kConvPatchH * kConvPatchW + THREADS - 1) / THREADS;
-    constexpr int kMaxPerPix  = IQ + CIN / 8;  // image below (four channels per item) + groups of 8 block outputs
-    constexpr int kBelowItems = (kBelowH * kBelowW * kMaxPerPix + THREADS - 1) / THREADS;
+    constexpr int kBelowItems = (kBelowH * kBelowW * GROUPS + THREADS - 1) / THREADS;
     constexpr int kDpreGroups = NPAD / 8;  // 16-byte groups of a pixel's gradient row
     constexpr int kDpreItems  = (kConvTileH * kConvTileW * kDpreGroups + THREADS - 1) / THREADS;
     struct TileLoads
@@ -783,23 +756,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         uint4 below[kBelowItems];
         half8 dpre[kDpreItems];
     };
-    const int act_groups = p.cb_store / 8;
-    const int per_pixel  = IQ + act_groups;
+    const int below_groups = p.below_stride / 8;  // groups of eight that a row of the level below has
     // the images of the batch are walked as one run of tiles: a workgroup keeps its sums from one image to the next
     // (image after image, every image paid for a set of partial sums of its own and for a last round of its own)
-    const float *feat = p.feat, *feat_below = p.feat_below;
-    const _Float16 *act_below = p.act_below, *dpre = p.dpre;
+    const float* feat = p.feat;
+    const _Float16 *below = p.below, *dpre = p.dpre;
     auto of_image = [&](int& tile)
     {
         const int image = p.batch > 1 ? tile / p.tiles : 0;
         tile -= image * p.tiles;
         feat = p.feat + (size_t)image * C * p.H * p.W;
         dpre = p.dpre + (size_t)image * p.H * p.W * NPAD;
-        if (has_below)
-        {
-            feat_below = p.feat_below + (size_t)image * C * p.Hb * p.Wb;
-            act_below  = p.act_below + (size_t)image * p.Hb * p.Wb * p.cb_store;
-        }
+        if (has_below) below = p.below + (size_t)image * p.Hb * p.Wb * p.below_stride;
     };
     auto issue_loads = [&](int tile, TileLoads& r)
     {
@@ -820,26 +788,17 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         }
         if (has_below)
         {
-            const size_t pb = (size_t)p.Hb * p.Wb;
 #pragma unroll
             for (int k = 0; k < kBelowItems; ++k)
             {
                 const int item = threadIdx.x + THREADS * k;
-                r.below[k]     = make_uint4(0u, 0u, 0u, 0u);
-                if (item < kBelowH * kBelowW * per_pixel)
+                const int g = item % GROUPS, bp = item / GROUPS;
+                const int rr = bp / kBelowW, c0 = bp - rr * kBelowW;
+                r.below[k] = make_uint4(0u, 0u, 0u, 0u);
+                if (bp < kBelowH * kBelowW && g < below_groups)
                 {
-                    const int q = item % per_pixel, bp = item / per_pixel;
-                    const int rr = bp / kBelowW, c0 = bp - rr * kBelowW;
                     const int yy = min(max(by0 + rr, 0), p.Hb - 1), xx = min(max(bx0 + c0, 0), p.Wb - 1);
-                    if (q < IQ)
-                    {
-                        float f[4];
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) f[c] = 4 * q + c < C ? feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
-                        r.below[k] = make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
-                    }
-                    else
-                        r.below[k] = *reinterpret_cast<const uint4*>(act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ));
+                    r.below[k]   = *reinterpret_cast<const uint4*>(below + ((size_t)yy * p.Wb + xx) * p.below_stride + 8 * g);
                 }
             }
         }
@@ -860,7 +819,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     auto put_image = [&](int item, const float (&v)[CI])
     {
         _Float16* row = s_patch + (size_t)item * ROW;
-        if (CI == 4 && has_below && C == 4)
+        if (FOUR && has_below)
             *reinterpret_cast<half4*>(row) = half4{_Float16(v[0]), _Float16(v[1]), _Float16(v[2]), _Float16(v[3])};
         else if (has_below)
         {
@@ -881,37 +840,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             }
         }
     };
-    // four channels 4 qi .. 4 qi + 3 of the image of the level below into positions C + 4 qi .. of a below-patch pixel
-    auto put_below_image = [&](int bp, int qi, const float (&v)[4])
-    {
-        _Float16* row = s_below + (size_t)bp * ROW;
-        if (CI == 4 && C == 4)
-            *reinterpret_cast<half4*>(row + 4) = half4{_Float16(v[0]), _Float16(v[1]), _Float16(v[2]), _Float16(v[3])};
-        else
-        {
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (4 * qi + c < C) row[C + 4 * qi + c] = _Float16(v[c]);
-        }
-        if (qi == 0)
-            for (int c = 2 * C + p.cb_store; c < CIN; ++c) row[c] = _Float16(0.f);
-    };
-    // eight block outputs of the level below (item q >= IQ) into positions 2 C + 8 (q - IQ) .. of a below-patch pixel
-    auto put_below_act = [&](int bp, int q, const uint4& v)
-    {
-        _Float16* row = s_below + (size_t)bp * ROW;
-        const int pos = 2 * C + 8 * (q - IQ);
-        if (C == 4)
-            *reinterpret_cast<uint4*>(row + pos) = v;
-        else
-        {
-            // (positions that are not a multiple of 8: element by element; outputs past the padded input are padding)
-            const half8 a = __builtin_bit_cast(half8, v);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (pos + i < CIN) row[pos + i] = a[i];
-        }
-    };
     auto commit_loads = [&](const TileLoads& r)
     {
 #pragma unroll
@@ -926,18 +854,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             for (int k = 0; k < kBelowItems; ++k)
             {
                 const int item = threadIdx.x + THREADS * k;
-                if (item < kBelowH * kBelowW * per_pixel)
-                {
-                    const int q = item % per_pixel, bp = item / per_pixel;
-                    if (q < IQ)
-                    {
-                        const float f[4] = {__uint_as_float(r.below[k].x), __uint_as_float(r.below[k].y), __uint_as_float(r.below[k].z),
-                                            __uint_as_float(r.below[k].w)};
-                        put_below_image(bp, q, f);
-                    }
-                    else
-                        put_below_act(bp, q, r.below[k]);
-                }
+                if (item < kBelowH * kBelowW * GROUPS) *reinterpret_cast<uint4*>(s_below + (item / GROUPS) * ROW + 8 * (item % GROUPS)) = r.below[k];
             }
         }
 #pragma unroll
@@ -967,23 +884,17 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         }
         if (has_below)
         {
-            const size_t pb = (size_t)p.Hb * p.Wb;
-            for (int item = threadIdx.x; item < kBelowH * kBelowW * per_pixel; item += THREADS)
+            for (int item = threadIdx.x; item < kBelowH * kBelowW * GROUPS; item += THREADS)
             {
-                const int q = item % per_pixel, bp = item / per_pixel;
+                const int g = item % GROUPS, bp = item / GROUPS;
                 const int r = bp / kBelowW, c0 = bp - r * kBelowW;
-                const int yy = min(max(by0 + r, 0), p.Hb - 1), xx = min(max(bx0 + c0, 0), p.Wb - 1);
-                if (q < IQ)
+                uint4 v = make_uint4(0u, 0u, 0u, 0u);
+                if (g < below_groups)
                 {
-                    float v[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) v[c] = 4 * q + c < C ? feat_below[(size_t)(4 * q + c) * pb + (size_t)yy * p.Wb + xx] : 0.f;
-                    put_below_image(bp, q, v);
+                    const int yy = min(max(by0 + r, 0), p.Hb - 1), xx = min(max(bx0 + c0, 0), p.Wb - 1);
+                    v            = *reinterpret_cast<const uint4*>(below + ((size_t)yy * p.Wb + xx) * p.below_stride + 8 * g);
                 }
-                else
-                {
-                    put_below_act(bp, q, *reinterpret_cast<const uint4*>(act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (q - IQ)));
-                }
+                *reinterpret_cast<uint4*>(s_below + bp * ROW + 8 * g) = v;
             }
         }
         for (int item = threadIdx.x; item < kConvTileH * kConvTileW * kDpreGroups; item += THREADS)
@@ -1030,47 +941,26 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         if (has_below)
         {
             __syncthreads();
-            // ---- stage 2: bilinear 2x upsampling from the below patch into channels [C, CIN) of the patch, in packed
-            // fp16 exactly as the forward kernel does it (the weights are products of 0, 1/4, 3/4 and 1) ----
-            for (int item = threadIdx.x; item < kConvPatchH * kConvPatchW * GROUPS; item += THREADS)
+            // ---- stage 2: bilinear 2x upsampling from the below patch into channels [C, CIN) of the patch, exactly as the
+            // forward kernel does it: 2 x 2 pixels between four neighbours at a time ----
+            const bool interior = x0 > 0 && y0 > 0 && x0 + kConvTileW < p.W && y0 + kConvTileH < p.H;
+            constexpr int kQuadsX = kConvPatchW / 2, kQuads = kQuadsX * (kConvPatchH / 2);
+            for (int item = threadIdx.x; item < kQuads * GROUPS; item += THREADS)
             {
-                const int g = item % GROUPS, pp = item / GROUPS;
-                const int py = pp / kConvPatchW, px = pp - py * kConvPatchW;
-                const int y = y0 + py - 1, x = x0 + px - 1;
-                half8 h;
+                const int g = item % GROUPS, quad = item / GROUPS;
+                if (8 * g + 8 <= C) continue;
+                const int j = quad / kQuadsX, i = quad - j * kQuadsX;
+                const _Float16* src = s_below + (j * kBelowW + i) * ROW + 8 * g;
+                half8 v[4];
+                upsample_quad(*reinterpret_cast<const half8*>(src), *reinterpret_cast<const half8*>(src + ROW),
+                              *reinterpret_cast<const half8*>(src + kBelowW * ROW), *reinterpret_cast<const half8*>(src + (kBelowW + 1) * ROW), v);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) h[i] = _Float16(0.f);
-                if (y >= 0 && y < p.H && x >= 0 && x < p.W)
+                for (int n = 0; n < 4; ++n)
                 {
-                    int ya, yb, xa, xb;
-                    float ly, lx;
-                    up2_source(y, p.Hb, ya, yb, ly);
-                    up2_source(x, p.Wb, xa, xb, lx);
-                    const _Float16 w00 = _Float16((1.f - ly) * (1.f - lx)), w01 = _Float16((1.f - ly) * lx);
-                    const _Float16 w10 = _Float16(ly * (1.f - lx)), w11 = _Float16(ly * lx);
-                    const half8 a = *reinterpret_cast<const half8*>(s_below + ((ya - by0) * kBelowW + (xa - bx0)) * ROW + 8 * g);
-                    const half8 b = *reinterpret_cast<const half8*>(s_below + ((ya - by0) * kBelowW + (xb - bx0)) * ROW + 8 * g);
-                    const half8 c = *reinterpret_cast<const half8*>(s_below + ((yb - by0) * kBelowW + (xa - bx0)) * ROW + 8 * g);
-                    const half8 d = *reinterpret_cast<const half8*>(s_below + ((yb - by0) * kBelowW + (xb - bx0)) * ROW + 8 * g);
-                    const half8 W00 = {w00, w00, w00, w00, w00, w00, w00, w00}, W01 = {w01, w01, w01, w01, w01, w01, w01, w01};
-                    const half8 W10 = {w10, w10, w10, w10, w10, w10, w10, w10}, W11 = {w11, w11, w11, w11, w11, w11, w11, w11};
-                    h = __builtin_elementwise_fma(d, W11, __builtin_elementwise_fma(c, W10, __builtin_elementwise_fma(b, W01, a * W00)));
+                    const int py = 2 * j + (n >> 1), px = 2 * i + (n & 1);
+                    if (!interior && !((unsigned)(y0 + py - 1) < (unsigned)p.H && (unsigned)(x0 + px - 1) < (unsigned)p.W)) v[n] = half8{};
+                    put_upsampled<FOUR>(s_patch + (py * kConvPatchW + px) * ROW, g, C, v[n]);
                 }
-                _Float16* dst = s_patch + (size_t)pp * ROW + 8 * g;
-                if (8 * g < C)
-                {
-                    // [0, C) holds this level's image
-                    if (CI == 4 && C == 4)
-                        *reinterpret_cast<half4*>(dst + 4) = half4{h[4], h[5], h[6], h[7]};
-                    else
-                    {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            if (8 * g + i >= C) dst[i] = h[i];
-                    }
-                }
-                else
-                    *reinterpret_cast<half8*>(dst) = h;
             }
         }
         __syncthreads();
@@ -1213,10 +1103,10 @@ __global__ __launch_bounds__(256) void reduce_weight_grad_kernel(const ReduceTab
     if ((int)blockIdx.x >= wblocks)
     {
         // one workgroup per pre-activation channel
-        const int n = blockIdx.x - wblocks, half = npad / 2;
+        const int n = blockIdx.x - wblocks;
         if (n >= npad || !l.bias_part) return;
-        const int o = n < half ? n : n - half;
-        float* dst  = n < half ? l.d_bf : l.d_bm;
+        const int o = preact_channel(n);
+        float* dst  = preact_is_mask(n) ? l.d_bm : l.d_bf;
         if (o >= cout || !dst) return;
         const float s = block_column_sum(l.bias_part, l.groups, npad, n);
         if (threadIdx.x == 0) dst[o] = s * scale_inv;
@@ -1225,10 +1115,9 @@ __global__ __launch_bounds__(256) void reduce_weight_grad_kernel(const ReduceTab
     const int i     = blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
     const int c = i % cin_pad, n = (i / cin_pad) % npad, tap = i / (cin_pad * npad);
-    const int half = npad / 2;
-    const int o    = n < half ? n : n - half;
+    const int o = preact_channel(n);
     if (o >= cout || c >= cin_real) return;
-    float* dst = n < half ? d_wf : d_wm;
+    float* dst = preact_is_mask(n) ? d_wm : d_wf;
     if (!dst) return;
     float s = 0.f;
 #pragma unroll
@@ -1272,27 +1161,27 @@ hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int ci
     return hipErrorInvalidValue;
 }
 
-template <int CIN, int NPAD, bool BIAS, int CI>
+template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
 hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, hipStream_t stream)
 {
     constexpr int THREADS = wgrad_threads(CIN, NPAD);
     const size_t lds = ((size_t)(kConvPatchH * kConvPatchW + kBelowH * kBelowW) * (CIN + kLdsChanPad) +
                         (size_t)kConvTileH * kConvTileW * (NPAD + kLdsChanPad)) *
                        sizeof(_Float16);  // up to 133 KB
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI>), dim3(groups), dim3(THREADS), lds, stream, p);
+    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>), dim3(groups), dim3(THREADS), lds, stream, p);
     return hipGetLastError();
 }
 
-template <int CI>
+template <int CI, bool FOUR>
 hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, int cin_pad, int npad, int groups, hipStream_t stream)
 {
 #define TRIPS_BW(CIN_, NPAD_)                                                                  \
     if (cin_pad == CIN_ && npad == NPAD_)                                                      \
-        return p.bias_part ? launch_bwd_weight<CIN_, NPAD_, true, CI>(p, groups, stream) \
-                                          : launch_bwd_weight<CIN_, NPAD_, false, CI>(p, groups, stream);
+        return p.bias_part ? launch_bwd_weight<CIN_, NPAD_, true, CI, FOUR>(p, groups, stream) \
+                                          : launch_bwd_weight<CIN_, NPAD_, false, CI, FOUR>(p, groups, stream);
     TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 96) TRIPS_BW(32, 128)
     TRIPS_BW(64, 32) TRIPS_BW(64, 64) TRIPS_BW(64, 96) TRIPS_BW(64, 128)
 #undef TRIPS_BW
@@ -1301,9 +1190,10 @@ hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, int cin_pad, int npa
 
 hipError_t dispatch_bwd_weight(const BwdWeightParams& p, int cin_pad, int npad, int groups, hipStream_t stream)
 {
-    if (p.c_feat <= 4) return dispatch_bwd_weight_ci<4>(p, cin_pad, npad, groups, stream);
-    if (p.c_feat <= 8) return dispatch_bwd_weight_ci<8>(p, cin_pad, npad, groups, stream);
-    return dispatch_bwd_weight_ci<16>(p, cin_pad, npad, groups, stream);
+    if (p.c_feat == 4) return dispatch_bwd_weight_ci<4, true>(p, cin_pad, npad, groups, stream);
+    if (p.c_feat < 4) return dispatch_bwd_weight_ci<4, false>(p, cin_pad, npad, groups, stream);
+    if (p.c_feat <= 8) return dispatch_bwd_weight_ci<8, false>(p, cin_pad, npad, groups, stream);
+    return dispatch_bwd_weight_ci<16, false>(p, cin_pad, npad, groups, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -1352,10 +1242,10 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     const int K           = d.num_output_channels;
     const int ci          = C <= 4 ? 4 : C <= 8 ? 8 : 16;  // image channels the kernels are built with room for
 
-    auto act_ptr = [&](int level)
+    auto rows_ptr = [&](int level)
     {
         const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<const _Float16*>(sv + l.saved_act_off);
+        return reinterpret_cast<const _Float16*>(sv + l.saved_rows_off);
     };
     auto pre_ptr = [&](int level)
     {
@@ -1405,7 +1295,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         const size_t plane  = (size_t)lv.H * lv.W;
         FinalBwdParams p;
         std::memset(&p, 0, sizeof(p));
-        p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cact_store = lv.cout_store, p.cout = K, p.npad = lv.npad;
+        p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cout = K, p.npad = lv.npad;
         p.scale    = grad_scale;
         p.feat     = inputs[0];
         p.pre      = pre_ptr(0);
@@ -1418,37 +1308,37 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         p.part     = reinterpret_cast<float*>(ws + np.final_part_off);
         const bool wgrad = grads->final_weight || grads->final_bias;
         const int chunks = wgrad ? np.final_groups : p.chunks * p.batch;
-        switch (lv.cout_store)
+        switch (lv.npad)
         {
-#define TRIPS_FW_CI(CS_, CI_)                                                                                     \
-    if (wgrad)                                                                                                    \
-        hipLaunchKernelGGL((final_backward_kernel<CS_, true, CI_>), dim3(chunks), dim3(256), 0, stream, p);       \
-    else                                                                                                          \
-        hipLaunchKernelGGL((final_backward_kernel<CS_, false, CI_>), dim3(chunks), dim3(256), 0, stream, p);
-#define TRIPS_FW(CS_)                \
-    case CS_:                        \
+#define TRIPS_FW_CI(NPAD_, CI_)                                                                               \
+    if (wgrad)                                                                                                \
+        hipLaunchKernelGGL((final_backward_kernel<NPAD_, true, CI_>), dim3(chunks), dim3(256), 0, stream, p); \
+    else                                                                                                      \
+        hipLaunchKernelGGL((final_backward_kernel<NPAD_, false, CI_>), dim3(chunks), dim3(256), 0, stream, p);
+#define TRIPS_FW(NPAD_)              \
+    case NPAD_:                      \
         if (ci == 4)                 \
         {                            \
-        TRIPS_FW_CI(CS_, 4)      \
+            TRIPS_FW_CI(NPAD_, 4)    \
         }                            \
         else if (ci == 8)            \
         {                            \
-        TRIPS_FW_CI(CS_, 8)      \
+            TRIPS_FW_CI(NPAD_, 8)    \
         }                            \
         else                         \
         {                            \
-        TRIPS_FW_CI(CS_, 16)     \
+            TRIPS_FW_CI(NPAD_, 16)   \
         }                            \
         break;
-            TRIPS_FW(8) TRIPS_FW(16) TRIPS_FW(24) TRIPS_FW(32) TRIPS_FW(40) TRIPS_FW(48) TRIPS_FW(56) TRIPS_FW(64)
+            TRIPS_FW(32) TRIPS_FW(64) TRIPS_FW(96) TRIPS_FW(128)
 #undef TRIPS_FW
 #undef TRIPS_FW_CI
-            default: return set_error(TRIPS_ERR_UNSUPPORTED, "block output stride %d", lv.cout_store);
+            default: return set_error(TRIPS_ERR_UNSUPPORTED, "%d pre-activations", lv.npad);
         }
         if (grads->final_weight || grads->final_bias)
         {
             hipLaunchKernelGGL(final_reduce_kernel, dim3(K * (C + lv.cout) + K), dim3(256), 0, stream,
-                               reinterpret_cast<const float*>(ws + np.final_part_off), np.final_groups, ci + lv.cout_store, ci, C,
+                               reinterpret_cast<const float*>(ws + np.final_part_off), np.final_groups, ci + lv.npad / 2, ci, C,
                                lv.cout, K, grads->final_weight, grads->final_bias);
         }
     }
@@ -1488,9 +1378,8 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             if (below)
             {
                 const LevelPlan& lb = np.lv[i + 1];
-                wp.Hb = lb.H, wp.Wb = lb.W, wp.cb_store = lb.cout_store;
-                wp.feat_below = inputs[i + 1];
-                wp.act_below  = act_ptr(i + 1);
+                wp.Hb = lb.H, wp.Wb = lb.W, wp.below_stride = lb.row_stride;
+                wp.below = rows_ptr(i + 1);
             }
             if (want_w)
             {

@@ -24,6 +24,10 @@ constexpr int kFinalPartFloats     = 4 * (kUnetMaxImageChannels + 64) + 4;  // i
 constexpr int kMaxGridImages = 32768;  // images of a batch that one launch takes (the y and z dimensions of a grid end at 65535)
 constexpr int kLdsChanPad  = 8;  // halves added to every LDS row so that 16 lanes reading 16 bytes hit 64 distinct banks
 
+// position n of a pixel's pre-activations (see LevelPlan): its channel, and whether it is the mask's
+__host__ __device__ __forceinline__ int preact_channel(int n) { return (n >> 3) * 4 + (n & 3); }
+__host__ __device__ __forceinline__ bool preact_is_mask(int n) { return (n & 4) != 0; }
+
 // source row / column and weight of torch's bilinear upsampling with scale_factor 2, align_corners = false
 // (area_pixel_compute_source_index: src = max(0, (dst + 0.5) * 0.5 - 0.5))
 __device__ __forceinline__ void up2_source(int dst, int in_size, int& i0, int& i1, float& lambda)
@@ -36,6 +40,39 @@ __device__ __forceinline__ void up2_source(int dst, int in_size, int& i0, int& i
     lambda    = src - float(i0);
 }
 
+// The 2 x 2 pixels that bilinear 2x upsampling (align_corners = false) makes between four neighbouring pixels of the
+// coarser level, v[0..3] = (upper left, upper right, lower left, lower right), eight channels in packed fp16: the
+// weights are 3/4 and 1/4 towards the nearer pixel, along x, then along y. At the image's border the coarser pixels
+// are the clamped ones, which gives torch's values there too.
+__device__ __forceinline__ void upsample_quad(half8 a, half8 b, half8 c, half8 d, half8 (&v)[4])
+{
+    const half8 w1 = {_Float16(0.25f), _Float16(0.25f), _Float16(0.25f), _Float16(0.25f), _Float16(0.25f), _Float16(0.25f), _Float16(0.25f), _Float16(0.25f)};
+    const half8 w3 = {_Float16(0.75f), _Float16(0.75f), _Float16(0.75f), _Float16(0.75f), _Float16(0.75f), _Float16(0.75f), _Float16(0.75f), _Float16(0.75f)};
+    const half8 dt = b - a, db = d - c;
+    const half8 tl = __builtin_elementwise_fma(dt, w1, a), tr = __builtin_elementwise_fma(dt, w3, a);
+    const half8 bl = __builtin_elementwise_fma(db, w1, c), br = __builtin_elementwise_fma(db, w3, c);
+    const half8 dl = bl - tl, dr = br - tr;
+    v[0] = __builtin_elementwise_fma(dl, w1, tl), v[1] = __builtin_elementwise_fma(dr, w1, tr);
+    v[2] = __builtin_elementwise_fma(dl, w3, tl), v[3] = __builtin_elementwise_fma(dr, w3, tr);
+}
+
+// Eight upsampled channels (group g of a patch row) into the row, whose positions [0, C) are the level's own image.
+// FOUR: C is exactly 4.
+template <bool FOUR>
+__device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8 v)
+{
+    _Float16* dst = row + 8 * g;
+    if (FOUR ? g > 0 : 8 * g >= C)
+        *reinterpret_cast<half8*>(dst) = v;
+    else if (FOUR)
+        *reinterpret_cast<half4*>(dst + 4) = half4{v[4], v[5], v[6], v[7]};
+    else
+    {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (8 * g + i >= C) dst[i] = v[i];
+    }
+}
 
 // The 9-tap implicit-GEMM core shared by the forward convolution and the data gradient. A operands are 16-byte LDS
 // reads from a (8+2) x (32+2) pixel patch with KIN channels innermost (row stride KIN + 8 halves). B operands (packed
@@ -200,11 +237,16 @@ constexpr int wgrad_row_split(int cin, int npad) { return (wgrad_threads(cin, np
 // ---- host-side plan of a network: per level the padded GEMM sizes and where its buffers live ----
 inline int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
+// Rows of a level: [B][H][W][row_stride] fp16, what the next finer block reads of this one. Positions [0, C) are zero,
+// [C, 2C) the level's image, [2C, 2C + cout) the block's outputs: the positions that these channels have in the finer
+// block's input, whose first C are its own image. row_stride = 2C + cout rounded up to 8, the rest zero.
+// Pre-activations and their gradients: [B][H][W][npad] fp16, the features and the masks of four channels side by side:
+// position 8 (ch / 4) + 4 (mask) + ch % 4, so that one 16-byte access serves the gate of four channels.
 struct LevelPlan
 {
-    int H, W, cin_real, cin_pad, cout, npad, cout_store;
-    size_t wpack_off, bias_off, act_off;  // bytes into the forward workspace
-    size_t saved_act_off, saved_pre_off;  // bytes into the saved state (training)
+    int H, W, cin_real, cin_pad, cout, npad, row_stride;
+    size_t wpack_off, bias_off, rows_off;  // bytes into the forward workspace
+    size_t saved_rows_off, saved_pre_off;  // bytes into the saved state (training)
     // bytes into the backward workspace
     size_t wt_off;      // packed transposed weights [9][cin_pad][npad] fp16
     size_t dpre_off;    // gradient of the pre-activations [B][H][W][npad] fp16
@@ -219,6 +261,7 @@ struct NetPlan
 {
     LevelPlan lv[TRIPS_UNET_MAX_LEVELS];
     size_t bytes;           // forward workspace
+    size_t fin_off;         // forward workspace: packed weights of the 1x1 output convolution
     size_t saved_bytes;     // saved state
     size_t backward_bytes;  // backward workspace
     size_t final_part_off;  // backward workspace: per-workgroup sums of the 1x1 convolution's weight and bias gradients
@@ -278,18 +321,20 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         lv.cin_pad    = lv.cin_real <= 32 ? 32 : 64;
         lv.cout       = d.filters[i] - ((i == 0 && L > 1) ? C : 2 * C);
         lv.npad       = 2 * round_up(lv.cout, 16);
-        lv.cout_store = round_up(lv.cout, 8);
+        lv.row_stride = round_up(2 * C + lv.cout, 8);
         lv.wpack_off  = o;
         o += align256((size_t)9 * lv.npad * lv.cin_pad * sizeof(_Float16));
         lv.bias_off = o;
         o += align256((size_t)lv.npad * sizeof(float));
     }
+    np.fin_off = o;
+    o += align256((size_t)(np.lv[0].npad / 32 + 1) * 64 * sizeof(_Float16));
     for (int i = 0; i < L; ++i)
     {
-        // (the finest block's output never leaves its kernel: the 1x1 convolution that reads it runs there, and the
-        // backward recomputes it from the saved pre-activations)
-        np.lv[i].act_off = o;
-        if (i > 0) o += align256((size_t)d.batch * np.lv[i].H * np.lv[i].W * np.lv[i].cout_store * sizeof(_Float16));
+        // (the rows of the finest level leave their kernel only where the 1x1 convolution is one of its own; the
+        // backward takes that block's output from the saved pre-activations)
+        np.lv[i].rows_off = o;
+        if (i > 0 || np.lv[0].npad > 64) o += align256((size_t)d.batch * np.lv[i].H * np.lv[i].W * np.lv[i].row_stride * sizeof(_Float16));
     }
     np.bytes = o;
     size_t sv = 0, bw = 0;
@@ -297,8 +342,8 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
     {
         LevelPlan& lv       = np.lv[i];
         const size_t pixels = (size_t)d.batch * lv.H * lv.W;
-        lv.saved_act_off    = sv;
-        if (i > 0) sv += align256(pixels * lv.cout_store * sizeof(_Float16));
+        lv.saved_rows_off   = sv;
+        if (i > 0) sv += align256(pixels * lv.row_stride * sizeof(_Float16));
         lv.saved_pre_off = sv;
         sv += align256(pixels * lv.npad * sizeof(_Float16));
         lv.wt_off = bw;

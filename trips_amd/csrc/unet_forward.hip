@@ -4,14 +4,16 @@
 //                           src/lib/models/Networks.h:751-787, 999-1098
 //                           and, in the finest block's epilogue, the `final` 1x1 Sequential of
 //                           MultiScaleUnet2dDecOnlySmallFixedImpl, Networks.h:1129-1131
+//   final_conv1x1_kernel     the same 1x1 for nets whose finest block has more outputs than one workgroup takes
 //
 // The reference runs, per level, upsample -> cat -> two 3x3 convolutions -> elu / sigmoid -> multiply -> cat as
 // separate libtorch ops on NCHW tensors, materialising every intermediate. Here one kernel per level does all of
 // it as an implicit GEMM: M = 256 output pixels of an 8 x 32 patch, N = feature and mask outputs side by side,
 // K = 9 taps x input channels. The input patch (with its one-pixel halo) is assembled in LDS, channels innermost:
 // channels [0, C) come straight from this level's splat image, the others are the bilinear 2x upsampling of the
-// level below (its splat image, then its convolution outputs), computed while loading, so neither the upsampled
-// tensor nor the concatenations ever exist in memory. Activations between levels are fp16, channels innermost.
+// level below (its splat image, then its convolution outputs), computed on the way in, so neither the upsampled
+// tensor nor the concatenations ever exist in memory. Activations between levels are fp16, channels innermost, and
+// carry the level's image with them (the row format is described at LevelPlan).
 // MFMA: v_mfma_f32_16x16x32_f16; lane l holds, of A, row l % 16 and the 8 consecutive K values (l / 16) * 8 ..,
 // of B the same for column l % 16, and of the 16 x 16 result rows (l / 16) * 4 .. + 3 of column l % 16.
 #include <hip/hip_fp16.h>
@@ -30,24 +32,24 @@ struct ConvParams
     int H, W;            // this level
     int Hb, Wb;          // level below (0 x 0 for the start block)
     int c_feat;          // channels of the splat images (C)
-    int cb_store;        // halves per pixel of act_below (multiple of 8; channels past the real ones hold zero)
     int cout;            // real outputs of each of the two convolutions
-    int cout_store;      // halves per pixel of `out` (multiple of 8)
-    const float* feat;        // [C][H][W]
-    const float* feat_below;  // [C][Hb][Wb]
-    const _Float16* act_below;  // [Hb][Wb][cb_store]
-    const _Float16* wpack;    // [9][NPAD][CIN]
-    const float* bias;        // [NPAD]: feature biases, then mask biases, each padded to NPAD / 2
-    _Float16* out;            // [H][W][cout_store], or nullptr when only the fused 1x1 consumes the block's output
-    _Float16* pre;            // [H][W][NPAD] pre-activations (feature | mask) for the backward, or nullptr
-    // the finest block also applies the net's 1x1 output convolution to x_0 = cat(image, block output)
-    const float* final_w;     // [final_cout][C + cout] or nullptr
-    const float* final_b;     // [final_cout]
-    float* final_out;         // [final_cout][H][W]
+    int npad;            // halves per pixel of `pre`
+    int tiles_x, tiles, batch;  // tiles of a row and of one image, images
+    const float* feat;   // this level's image: element (pixel, channel) at pixel * feat_ps + channel * feat_cs
+    int feat_ps;
+    size_t feat_cs;
+    const _Float16* below;    // rows of the level below, [Hb][Wb][below_stride], or nullptr
+    int below_stride;
+    const _Float16* wfrag;    // weights as MFMA fragments: [pair][tap][CIN / 32][feature, mask][lane][8]
+    const float* bias;        // [pair][feature, mask][16]
+    _Float16* out;            // this level's rows, [H][W][out_stride], or nullptr when only the fused 1x1 reads them
+    int out_stride;
+    _Float16* pre;            // [H][W][npad] pre-activations for the backward (see LevelPlan), or nullptr
+    // the net's 1x1 output convolution on x_0 = cat(image, block output), fused into the finest block, or nullptr
+    const _Float16* fin_frag;  // [pair, then the image][lane % 4 = output][lane / 16][4]: see pack_conv_weights_kernel
+    const float* final_b;      // [final_cout]
+    float* final_out;          // [final_cout][H][W]
     int final_cout;
-    // the images of a batch are the grid's z dimension: the first one's number, elements from one image to the next
-    int first_image;
-    size_t feat_stride, feat_below_stride, act_below_stride, out_stride, pre_stride, final_stride;
 };
 
 // A loaded value that is only needed under a condition is otherwise loaded under that condition by the compiler, in a
@@ -56,503 +58,457 @@ struct ConvParams
 __device__ __forceinline__ void loaded(float& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void loaded(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
-// CI: image channels the kernel has room for (4, 8 or 16; C <= CI)
-template <int CIN, int NPAD, int THREADS, int CI>
-__global__ __launch_bounds__(THREADS) void gated_conv3x3_kernel(ConvParams p)
+// One workgroup walks tiles of 8 x 32 pixels and computes PAIRS pairs of (16 feature, 16 mask) outputs of each. Its
+// wavefronts split the pairs and the tile: a wavefront owns one pair for a strip of 16 pixels x MB rows, so that its A
+// operands (LDS) are shared by the three vertical taps and a lane ends up with four features and the masks of the same
+// four channels of a pixel: the gate, the stores and the 1x1 of the finest level need no LDS and no further exchange.
+// What bounds it: vector instructions (loads, upsampling, the gate's two exponentials), then the latency of the phases
+// between two barriers; the matrix cores are busy for a fifth of the time. Hence: what a tile's threads share is worked
+// out once per workgroup or on the scalar unit, the loads of the next tile travel during this one's products, and the
+// upsampling makes 2 x 2 pixels from one set of four neighbours (382 instead of 710 vector instructions per wavefront
+// and 256-pixel tile at the finest level of the 16/32/64/64 net). 1920 x 1080, that net, per level, against one tile
+// per workgroup with LDS-staged epilogues: 106 -> 74, 61 -> 59, 38 -> 35, 14 -> 13 us.
+// BREGS: the pair's weights (9 taps x 64 inputs: 144 registers) stay in registers for all tiles of the workgroup;
+// with 32 inputs they are staged in LDS once (held in registers they leave room for half the wavefronts: 121 us at the
+// finest level, where six wavefronts per SIMD take 74 and four 83).
+// CI: image channels the kernel has room for (4, 8 or 16); FOUR: C is exactly 4, the splat's usual descriptor width
+template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, bool BREGS, int WAVES_PER_EU>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void gated_conv3x3_kernel(const ConvParams p)
 {
-    // All images of a batch are one launch: the coarse levels of a 512 x 512 crop are 4 to 64 tiles, and image after
-    // image they took the latency of a tile each (four crops, five levels of 32: 256 us in 20 launches).
-    {
-        const size_t b = p.first_image + blockIdx.z;
-        p.feat += b * p.feat_stride, p.feat_below += b * p.feat_below_stride, p.act_below += b * p.act_below_stride;
-        p.out = p.out ? p.out + b * p.out_stride : nullptr, p.pre = p.pre ? p.pre + b * p.pre_stride : nullptr;
-        p.final_out = p.final_out ? p.final_out + b * p.final_stride : nullptr;
-    }
-    constexpr int IQ = CI / 4;  // 16-byte items that carry the image of a pixel of the level below
-    constexpr int MB = 16 / (THREADS / 64);  // 16-pixel row blocks of a wavefront: two rows of the tile, or one
-    constexpr int ROW  = CIN + kLdsChanPad;  // halves per patch pixel in LDS
-    constexpr int NB   = NPAD / 16;          // 16-column blocks; the first half are feature outputs
-    constexpr int HB   = NB / 2;
-    extern __shared__ _Float16 smem[];
-    _Float16* s_patch = smem;  // [kConvPatchH * kConvPatchW][ROW]
+    constexpr int KB      = CIN / 32;
+    constexpr int ROW     = CIN + kLdsChanPad;  // halves per patch pixel in LDS
+    constexpr int GROUPS  = CIN / 8;
+    constexpr int MB      = 16 * PAIRS / (THREADS / 64);  // rows of a wavefront's strip
+    static_assert(MB <= 4, "the 1x1 of the finest level keeps four rows in one accumulator");
+    constexpr int kPatch  = kConvPatchH * kConvPatchW;
+    constexpr int kQuads  = (kConvPatchH / 2) * (kConvPatchW / 2);
+    constexpr int QITEMS  = (kQuads * GROUPS + THREADS - 1) / THREADS;
+    // (8 and 16 image channels leave no registers for the loads of the next tile)
+    constexpr bool kPrefetch = CI == 4 || (CIN == 32 && CI == 8);
+    constexpr int FITEMS     = (kPatch + THREADS - 1) / THREADS;
+    __shared__ __align__(16) _Float16 s_patch[kPatch * ROW];
+    __shared__ __align__(16) _Float16 s_w[BREGS ? 8 : PAIRS * 9 * KB * 2 * 512];
+    __shared__ float4 s_fin[PAIRS == 2 ? 4 * 64 : 1];
 
-    const int x0 = blockIdx.x * kConvTileW, y0 = blockIdx.y * kConvTileH;
-    const bool has_below = p.Hb > 0;
-    ConvTapStage<CIN, NPAD, THREADS> taps;
-    conv_tap_fetch(taps, p.wpack, 0);  // in flight while the patch is assembled
-    // weights and biases of the 1x1 output convolution, rounded to fp16 like every other operand
-    constexpr int kFwBias = 4 * (CI + 64);  // [final_cout <= 4][C + cout <= CI + 64] weights, then the biases
-    __shared__ float s_fw[kFwBias + 4];
+    const int lane = (int)threadIdx.x & 63;
+    // (a wavefront's number is the same for its lanes: kept on the scalar unit)
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lrow = lane & 15, lq = lane >> 4;
+    const int C    = FOUR ? 4 : p.c_feat;
+    const int pair = PAIRS == 1 ? 0 : wave & 1;
+    const int strip = PAIRS == 1 ? wave : wave >> 1;
+    const int r0 = (strip >> 1) * MB, c0 = (strip & 1) * 16;  // the strip's first row and column of the tile
+    const int gp = blockIdx.y * PAIRS + pair;                 // this wavefront's pair of the level
+    const int tiles = p.tiles * p.batch;
 
-    // ---- stage 1: everything the patch needs from memory, all loads of a thread in flight together ----
-    // (a) this level's image -> channels [0, C) of the patch; (b) the level below, x_{i+1} = cat(image, activations),
-    // as a (TILE/2 + 2)^2 patch in the same row format, channel k of the concatenated input at row position k.
-    // Every load below is unconditional, at an address clamped into its array, and what a thread does not need is
-    // replaced by zero afterwards: a load inside a branch is waited for before the branch is left, and the eight or
-    // nine round trips to memory of a thread then ran one after the other (72 % of a tile's life at the finest level).
-    constexpr int GROUPS = CIN / 8;
-    _Float16* s_below    = s_patch + kConvPatchH * kConvPatchW * ROW;  // [kBelowH * kBelowW][ROW]
-    const int by0 = y0 / 2 - 1, bx0 = x0 / 2 - 1;
-    const int C   = p.c_feat;
-    constexpr int kFeatItems  = (kConvPatchH * kConvPatchW + THREADS - 1) / THREADS;
-    constexpr int kMaxPerPix  = IQ + CIN / 8;  // image below (four channels per item) + groups of 8 block outputs
-    constexpr int kBelowItems = (kBelowH * kBelowW * kMaxPerPix + THREADS - 1) / THREADS;
-    float feat_v[kFeatItems][CI];
-    bool feat_in[kFeatItems];
-    uint4 below_v[kBelowItems];
-    float below_f[kBelowItems][4];
-    bool below_have[kBelowItems], below_img[kBelowItems];
-    const int act_groups = has_below ? p.cb_store / 8 : 0;
-    const int per_pixel  = IQ + act_groups;  // items 0 .. IQ - 1 of a pixel: the image below; others: 8 activations each
-    // item / per_pixel without an integer division: items stay below 2^11 and per_pixel below 2^5, so the quotient of
-    // item + 1/2 is at least 1/64 away from every integer, far more than the rounding of the product
-    const float inv_per_pixel = 1.f / float(per_pixel);
-    auto pixel_of_item        = [&](int item) { return (int)((float(item) + 0.5f) * inv_per_pixel); };
-    // the 1x1's weights and biases: requested here, stored to LDS with the patch
-    constexpr int kFwItems = (kFwBias + THREADS - 1) / THREADS;
-    float fw_v[kFwItems], fb_v = 0.f;
-    const int fw_n = p.final_out ? p.final_cout * (p.c_feat + p.cout) : 0;
+    // ---- what stays for all tiles: weights, biases, the 1x1's weights ----
+    const half8* wsrc = reinterpret_cast<const half8*>(p.wfrag) + (size_t)gp * (9 * KB * 2 * 64) + lane;
+    half8 w[BREGS ? 9 : 1][KB][2];
+    if (BREGS)
+    {
+#pragma unroll
+        for (int t = 0; t < (BREGS ? 9 : 1); ++t)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[t][kb][h] = wsrc[((t * KB + kb) * 2 + h) * 64];
+    }
+    else
+    {
+        const half8* src = reinterpret_cast<const half8*>(p.wfrag) + (size_t)blockIdx.y * PAIRS * (9 * KB * 2 * 64);
+        for (int i = threadIdx.x; i < PAIRS * 9 * KB * 2 * 64; i += THREADS) reinterpret_cast<half8*>(s_w)[i] = src[i];
+    }
+    const float4 bias_f = *reinterpret_cast<const float4*>(p.bias + gp * 32 + lq * 4);
+    const float4 bias_m = *reinterpret_cast<const float4*>(p.bias + gp * 32 + 16 + lq * 4);
+    // A operand of the 1x1: rows 4 m + o of block m's product hold output o, so that the products of a strip's MB rows
+    // add up in one accumulator whose lane group m holds the outputs of row m
+    half4 fw = half4{}, fimg = half4{};
     if (p.final_out)
     {
-#pragma unroll
-        for (int k = 0; k < kFwItems; ++k) fw_v[k] = p.final_w[min((int)threadIdx.x + THREADS * k, fw_n - 1)];
-        fb_v = p.final_b[min((int)threadIdx.x, p.final_cout - 1)];
+        fw   = *reinterpret_cast<const half4*>(p.fin_frag + (gp * 16 + (lrow & 3) * 4 + lq) * 4);
+        fimg = *reinterpret_cast<const half4*>(p.fin_frag + ((p.npad / 32) * 16 + (lrow & 3) * 4 + lq) * 4);
     }
+    // channels that nothing ever writes: of the start block all but the image's, of the others the groups that the
+    // rows of the level below do not have
+    const int below_groups = p.below_stride / 8;
+    for (int i = threadIdx.x; i < kPatch * GROUPS; i += THREADS)
+        if (i % GROUPS >= below_groups) *reinterpret_cast<half8*>(s_patch + (i / GROUPS) * ROW + 8 * (i % GROUPS)) = half8{};
+
+    // ---- this thread's share of the loads of a tile ----
+    struct Loads
     {
-        const size_t plane = (size_t)p.H * p.W;
+        float f[FITEMS][CI];   // pixels of the image patch
+        uint4 q[QITEMS][4];    // eight channels of 2 x 2 pixels of the level below: they make 2 x 2 pixels of the patch
+    };
+    struct Tile
+    {
+        int image, x0, y0;
+    };
+    auto decode = [&](int t)
+    {
+        Tile r;
+        r.image      = t / p.tiles;
+        const int i  = t - r.image * p.tiles;
+        const int ty = i / p.tiles_x;
+        r.x0         = (i - ty * p.tiles_x) * kConvTileW;
+        r.y0         = ty * kConvTileH;
+        return r;
+    };
+    auto issue = [&](const Tile& t, int tid, Loads& r)
+    {
+        // (addresses: what a tile shares is added up on the scalar unit, a thread's own part fits 32 bits)
+        const float* img = p.feat + (size_t)t.image * p.H * p.W * C + ((size_t)t.y0 * p.W + t.x0) * p.feat_ps;
 #pragma unroll
-        for (int k = 0; k < kFeatItems; ++k)
+        for (int k = 0; k < FITEMS; ++k)
         {
-            const int item = (int)threadIdx.x + THREADS * k;
-            const int py = item / kConvPatchW, px = item - py * kConvPatchW;
-            const int y = y0 + py - 1, x = x0 + px - 1;
-            const bool in = item < kConvPatchH * kConvPatchW && y >= 0 && y < p.H && x >= 0 && x < p.W;
-            const float* src = p.feat + (size_t)min(max(y, 0), p.H - 1) * p.W + min(max(x, 0), p.W - 1);
-            feat_in[k] = in;
+            const int item = min(tid + THREADS * k, kPatch - 1);
+            const int y = t.y0 + item / kConvPatchW - 1, x = t.x0 + item % kConvPatchW - 1;
+            const int off = ((min(max(y, 0), p.H - 1) - t.y0) * p.W + min(max(x, 0), p.W - 1) - t.x0) * p.feat_ps;
 #pragma unroll
-            for (int c = 0; c < CI; ++c) feat_v[k][c] = src[(c < C ? c : 0) * plane];
+            for (int c = 0; c < CI; ++c) r.f[k][c] = (img + (c < C ? c : 0) * p.feat_cs)[off];
         }
-    }
-    if (has_below)
-    {
-        const size_t pb = (size_t)p.Hb * p.Wb;
-#pragma unroll
-        for (int k = 0; k < kBelowItems; ++k)
+        if (below_groups > 0)
         {
-            const int item = (int)threadIdx.x + THREADS * k;
-            // (kBelowItems is sized for the widest level below; a round in which no thread has an item is skipped as a
-            // whole: the finest level of the usual plan has 432 items for its 512 threads)
-            if (THREADS * k >= kBelowH * kBelowW * per_pixel) break;
-            const bool have = item < kBelowH * kBelowW * per_pixel;
-            const int it    = have ? item : 0;
-            const int bp = pixel_of_item(it), q = it - bp * per_pixel;
-            const int r = bp / kBelowW, c0 = bp - r * kBelowW;
-            const int yy = min(max(by0 + r, 0), p.Hb - 1), xx = min(max(bx0 + c0, 0), p.Wb - 1);
-            const bool img = q < IQ;
-            // an image item: four planes of the image below; any other item reads plane 0 four times and drops it
-            const float* src = p.feat_below + (size_t)yy * p.Wb + xx;
+            const int y00 = max(t.y0 / 2 - 1, 0);
+            const _Float16* src = p.below + ((size_t)t.image * p.Hb + y00) * p.Wb * p.below_stride;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) below_f[k][c] = src[(size_t)(img && 4 * q + c < C ? 4 * q + c : 0) * pb];
-            // an item of block outputs: eight of them; an image item reads the pixel's first eight and drops them
-            below_v[k]    = *reinterpret_cast<const uint4*>(p.act_below + ((size_t)yy * p.Wb + xx) * p.cb_store + 8 * (img ? 0 : q - IQ));
-            below_have[k] = have;
-            below_img[k]  = img;
-        }
-    }
-    // ---- all loads are on their way: from here on their values are used ----
-    if (p.final_out)
-    {
-#pragma unroll
-        for (int k = 0; k < kFwItems; ++k) loaded(fw_v[k]);
-        loaded(fb_v);
-    }
-#pragma unroll
-    for (int k = 0; k < kFeatItems; ++k)
-#pragma unroll
-        for (int c = 0; c < CI; ++c)
-        {
-            loaded(feat_v[k][c]);
-            if (!(feat_in[k] && c < C)) feat_v[k][c] = 0.f;
-        }
-    if (has_below)
-    {
-#pragma unroll
-        for (int k = 0; k < kBelowItems; ++k)
-        {
-            if (THREADS * k >= kBelowH * kBelowW * per_pixel) break;
-            const int item = (int)threadIdx.x + THREADS * k;
-            const int it   = below_have[k] ? item : 0;
-            const int q    = it - pixel_of_item(it) * per_pixel;
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
+            for (int k = 0; k < QITEMS; ++k)
             {
-                loaded(below_f[k][c]);
-                if (!(below_img[k] && 4 * q + c < C)) below_f[k][c] = 0.f;
-            }
-            loaded(below_v[k]);
-            if (below_img[k])
-                below_v[k] = make_uint4(__float_as_uint(below_f[k][0]), __float_as_uint(below_f[k][1]), __float_as_uint(below_f[k][2]),
-                                        __float_as_uint(below_f[k][3]));
-            if (!below_have[k]) below_v[k] = make_uint4(0u, 0u, 0u, 0u);
-        }
-    }
-    if (p.final_out)
-    {
-#pragma unroll
-        for (int k = 0; k < kFwItems; ++k)
-            if ((int)threadIdx.x + THREADS * k < fw_n) s_fw[(int)threadIdx.x + THREADS * k] = float(_Float16(fw_v[k]));
-        if ((int)threadIdx.x < p.final_cout) s_fw[kFwBias + (int)threadIdx.x] = fb_v;
-    }
-#pragma unroll
-    for (int k = 0; k < kFeatItems; ++k)
-    {
-        const int item = (int)threadIdx.x + THREADS * k;
-        if (item < kConvPatchH * kConvPatchW)
-        {
-            _Float16* row = s_patch + (size_t)item * ROW;
-            if (CI == 4 && C == 4)  // one 8-byte LDS store instead of four 2-byte ones
-                *reinterpret_cast<half4*>(row) =
-                    half4{_Float16(feat_v[k][0]), _Float16(feat_v[k][1]), _Float16(feat_v[k][2]), _Float16(feat_v[k][3])};
-            else
-            {
-#pragma unroll
-                for (int c = 0; c < CI; ++c)  // (a run-time bound would put the register array into scratch memory)
-                    if (c < C) row[c] = _Float16(feat_v[k][c]);
-            }
-            if (!has_below)
-            {
-                // start block: the image is the whole input
-                for (int c = C; c < CIN; ++c) row[c] = _Float16(0.f);
+                const int item = tid + THREADS * k;
+                const int g = item % GROUPS, quad = min(item / GROUPS, kQuads - 1);
+                const int j = quad / (kConvPatchW / 2), i = quad - j * (kConvPatchW / 2);
+                const int ya = min(max(t.y0 / 2 - 1 + j, 0), p.Hb - 1) - y00, yb = min(t.y0 / 2 + j, p.Hb - 1) - y00;
+                const int xa = min(max(t.x0 / 2 - 1 + i, 0), p.Wb - 1), xb = min(t.x0 / 2 + i, p.Wb - 1);
+                const _Float16* s = src + 8 * min(g, below_groups - 1);
+                const int ra = ya * p.Wb, rb = yb * p.Wb;
+                r.q[k][0] = *reinterpret_cast<const uint4*>(s + (ra + xa) * p.below_stride);
+                r.q[k][1] = *reinterpret_cast<const uint4*>(s + (ra + xb) * p.below_stride);
+                r.q[k][2] = *reinterpret_cast<const uint4*>(s + (rb + xa) * p.below_stride);
+                r.q[k][3] = *reinterpret_cast<const uint4*>(s + (rb + xb) * p.below_stride);
             }
         }
-    }
-    if (has_below)
+    };
+    // ... and from the registers into the patch: the 2x upsampling on the way
+    auto commit = [&](const Tile& t, int tid, Loads& r)
     {
+        const bool interior = t.y0 > 0 && t.x0 > 0 && t.y0 + kConvTileH < p.H && t.x0 + kConvTileW < p.W;
 #pragma unroll
-        for (int k = 0; k < kBelowItems; ++k)
+        for (int k = 0; k < FITEMS; ++k)
         {
-            const int item = (int)threadIdx.x + THREADS * k;
-            if (THREADS * k >= kBelowH * kBelowW * per_pixel) break;
-            if (item < kBelowH * kBelowW * per_pixel)
+            const int item = tid + THREADS * k;
+            if (item < kPatch)
             {
-                const int bp = pixel_of_item(item), q = item - bp * per_pixel;
-                _Float16* row = s_below + (size_t)bp * ROW;
-                if (q < IQ)
-                {
-                    const float f[4] = {__uint_as_float(below_v[k].x), __uint_as_float(below_v[k].y), __uint_as_float(below_v[k].z),
-                                        __uint_as_float(below_v[k].w)};
-                    if (CI == 4 && C == 4)
-                        *reinterpret_cast<half4*>(row + 4) = half4{_Float16(f[0]), _Float16(f[1]), _Float16(f[2]), _Float16(f[3])};
-                    else
-                    {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c)
-                            if (4 * q + c < C) row[C + 4 * q + c] = _Float16(f[c]);
-                    }
-                    if (q == 0)
-                        for (int c = 2 * C + p.cb_store; c < CIN; ++c) row[c] = _Float16(0.f);  // padding channels
-                }
+                const int y = t.y0 + item / kConvPatchW - 1, x = t.x0 + item % kConvPatchW - 1;
+                const bool in = interior || ((unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W);
+                _Float16* row = s_patch + item * ROW;
+                if (FOUR)
+                    *reinterpret_cast<half4*>(row) =
+                        in ? half4{_Float16(r.f[k][0]), _Float16(r.f[k][1]), _Float16(r.f[k][2]), _Float16(r.f[k][3])} : half4{};
                 else
                 {
-                    const int pos = 2 * C + 8 * (q - IQ);
-                    if (C == 4)
-                        *reinterpret_cast<uint4*>(row + pos) = below_v[k];
-                    else
-                    {
-                        const half8 a = __builtin_bit_cast(half8, below_v[k]);
-                        for (int i = 0; i < 8; ++i)
-                            if (pos + i < CIN) row[pos + i] = a[i];
-                    }
+#pragma unroll
+                    for (int c = 0; c < CI; ++c)  // (a run-time bound would put the register array into scratch memory)
+                        if (c < C) row[c] = in ? _Float16(r.f[k][c]) : _Float16(0.f);
                 }
             }
         }
+        if (below_groups > 0)
+        {
+#pragma unroll
+            for (int k = 0; k < QITEMS; ++k)
+            {
+                const int item = tid + THREADS * k;
+                const int g = item % GROUPS, quad = item / GROUPS;
+                if (quad >= kQuads || g >= below_groups || 8 * g + 8 <= C) continue;
+                const int j = quad / (kConvPatchW / 2), i = quad - j * (kConvPatchW / 2);
+                half8 v[4];
+                upsample_quad(__builtin_bit_cast(half8, r.q[k][0]), __builtin_bit_cast(half8, r.q[k][1]), __builtin_bit_cast(half8, r.q[k][2]),
+                              __builtin_bit_cast(half8, r.q[k][3]), v);
+#pragma unroll
+                for (int n = 0; n < 4; ++n)
+                {
+                    const int py = 2 * j + (n >> 1), px = 2 * i + (n & 1);
+                    if (!interior && !((unsigned)(t.y0 + py - 1) < (unsigned)p.H && (unsigned)(t.x0 + px - 1) < (unsigned)p.W)) v[n] = half8{};
+                    put_upsampled<FOUR>(s_patch + (py * kConvPatchW + px) * ROW, g, C, v[n]);
+                }
+            }
+        }
+    };
+
+    // consecutive tiles share their halos: they go to one XCD (workgroups are dealt to the eight of them in turn)
+    const int xcds = min(8, (int)gridDim.x), xcd = (int)blockIdx.x % xcds;
+    const int share = (tiles + xcds - 1) / xcds, in_xcd = ((int)gridDim.x - xcd + xcds - 1) / xcds;
+    const int last = min(tiles, (xcd + 1) * share);
+    int at = xcd * share + (int)blockIdx.x / xcds;
+
+    Loads cur;
+    if (kPrefetch && at < last) issue(decode(at), (int)threadIdx.x, cur);
+    for (; at < last; at += in_xcd)
+    {
+        const Tile t = decode(at);
+        // The thread's number is made anew for every tile: what follows from it (addresses of loads, of the patch, of the
+        // staged weights and the weights themselves) would otherwise be kept in registers across the loop, which has
+        // none to spare.
+        int tid = (int)threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, lrow = lane & 15, lq = lane >> 4;
+        __syncthreads();  // the previous tile's patch has been read (and the fills above are done)
+        if (!kPrefetch) issue(t, tid, cur);
+        commit(t, tid, cur);
         __syncthreads();
-        // ---- stage 2: bilinear 2x upsampling from the below patch into channels [C, CIN) of the patch ----
-        // A thread takes a pixel of the patch and walks its groups of 8 channels: the pixel's position, sources and
-        // weights are worked out once (with an item per (pixel, group) that arithmetic was most of the stage).
-        for (int pp = (int)threadIdx.x; pp < kConvPatchH * kConvPatchW; pp += THREADS)
+        if (kPrefetch && at + in_xcd < last) issue(decode(at + in_xcd), tid, cur);  // travels during the taps and the epilogue
+
+        floatx4 acc[MB][2];
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
         {
-            const int py = pp / kConvPatchW, px = pp - py * kConvPatchW;
-            const int y = y0 + py - 1, x = x0 + px - 1;
-            const bool inside = y >= 0 && y < p.H && x >= 0 && x < p.W;
-            // The interpolation runs in packed fp16: the weights are products of 0, 1/4, 3/4 and 1 (exact in fp16), the
-            // operands are fp16 already and the result is stored as fp16; three fused multiply-adds per pair of channels
-            // instead of eight conversions and four fp32 operations per channel.
-            int ya = by0, yb = by0, xa = bx0, xb = bx0;
-            float ly = 0.f, lx = 0.f;
-            if (inside)
-            {
-                up2_source(y, p.Hb, ya, yb, ly);
-                up2_source(x, p.Wb, xa, xb, lx);
-            }
-            const _Float16 w00 = _Float16((1.f - ly) * (1.f - lx)), w01 = _Float16((1.f - ly) * lx);
-            const _Float16 w10 = _Float16(ly * (1.f - lx)), w11 = _Float16(ly * lx);
-            const half8 W00 = {w00, w00, w00, w00, w00, w00, w00, w00}, W01 = {w01, w01, w01, w01, w01, w01, w01, w01};
-            const half8 W10 = {w10, w10, w10, w10, w10, w10, w10, w10}, W11 = {w11, w11, w11, w11, w11, w11, w11, w11};
-            const _Float16* sa = s_below + ((ya - by0) * kBelowW + (xa - bx0)) * ROW;
-            const _Float16* sb = s_below + ((ya - by0) * kBelowW + (xb - bx0)) * ROW;
-            const _Float16* sc = s_below + ((yb - by0) * kBelowW + (xa - bx0)) * ROW;
-            const _Float16* sd = s_below + ((yb - by0) * kBelowW + (xb - bx0)) * ROW;
-            _Float16* drow     = s_patch + (size_t)pp * ROW;
+            acc[m][0] = floatx4{bias_f.x, bias_f.y, bias_f.z, bias_f.w};
+            acc[m][1] = floatx4{bias_m.x, bias_m.y, bias_m.z, bias_m.w};
+        }
+        const half8* wlds  = reinterpret_cast<const half8*>(s_w) + pair * (9 * KB * 2 * 64) + lane;
+        const _Float16* a0 = s_patch + (r0 * kConvPatchW + c0 + lrow) * ROW + lq * 8;
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g)
-            {
-                half8 h;
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) h[i] = _Float16(0.f);
-                if (inside)
+            for (int dx = 0; dx < 3; ++dx)
+            {
+                half8 b[3][2];
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) b[dy][h] = BREGS ? w[BREGS ? 3 * dy + dx : 0][kb][h] : wlds[(((3 * dy + dx) * KB + kb) * 2 + h) * 64];
+#pragma unroll
+                for (int r = 0; r < MB + 2; ++r)
                 {
-                    const half8 a = *reinterpret_cast<const half8*>(sa + 8 * g);
-                    const half8 b = *reinterpret_cast<const half8*>(sb + 8 * g);
-                    const half8 c = *reinterpret_cast<const half8*>(sc + 8 * g);
-                    const half8 d = *reinterpret_cast<const half8*>(sd + 8 * g);
-                    h = __builtin_elementwise_fma(d, W11, __builtin_elementwise_fma(c, W10, __builtin_elementwise_fma(b, W01, a * W00)));
-                }
-                _Float16* dst = drow + 8 * g;
-                if (8 * g < C)
-                {
-                    // [0, C) holds this level's image
-                    if (CI == 4 && C == 4)
-                        *reinterpret_cast<half4*>(dst + 4) = half4{h[4], h[5], h[6], h[7]};
-                    else
+                    const half8 a = *reinterpret_cast<const half8*>(a0 + (r * kConvPatchW + dx) * ROW + kb * 32);
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy)
                     {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-                            if (8 * g + i >= C) dst[i] = h[i];
+                        const int m = r - dy;
+                        if (m < 0 || m >= MB) continue;
+                        acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][0], a, acc[m][0], 0, 0, 0);
+                        acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][1], a, acc[m][1], 0, 0, 0);
                     }
                 }
-                else
-                    *reinterpret_cast<half8*>(dst) = h;
             }
-        }
-    }
 
-    __syncthreads();  // patch complete; the patch of the level below is no longer needed
-    // the staged taps of the weights, in place of the patch of the level below
-    _Float16* s_taps = s_patch + kConvPatchH * kConvPatchW * ROW;
-    conv_tap_stage(taps, s_taps);
-    __syncthreads();
-    floatx4 acc[MB][NB];
-    conv_taps_mfma<CIN, NPAD, true, THREADS>(s_patch, s_taps, p.wpack, taps, acc);  // a lane: four channels of one pixel
-    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
-    const int lrow = lane & 15, lk = (lane >> 4) * 8;
-
-    // ---- epilogue: elu(feature) * sigmoid(mask) in fp16, staged in LDS (the patch is no longer needed) and
-    // written channels innermost with full-line stores; the pre-activations too when the backward needs them ----
-    constexpr int IPAD = CI > kLdsChanPad ? CI : kLdsChanPad;  // padding columns of a staged row: room for the image
-    constexpr int AS = NPAD / 2 + IPAD, PS = NPAD + kLdsChanPad;
-    _Float16* s_act = smem;                                      // [256][AS]
-    _Float16* s_pre = smem + kConvTileH * kConvTileW * AS;       // [256][PS]
-    float my_feat[CI];  // this thread's pixel of the image, as the convolution saw it (fp16)
+        // ---- epilogue: elu(feature) * sigmoid(mask); a lane: four channels of one pixel per row of the strip ----
+        const int x = t.x0 + c0 + lrow, ch0 = gp * 16 + lq * 4;
+        const size_t tile_pix = (size_t)t.image * p.H * p.W + (size_t)t.y0 * p.W + t.x0;
+        _Float16* pre_tile    = p.pre ? p.pre + tile_pix * p.npad : nullptr;
+        _Float16* out_tile    = p.out ? p.out + tile_pix * p.out_stride : nullptr;
+        floatx4 fin = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < CI; ++c) my_feat[c] = 0.f;
-    const bool owns_pixel = THREADS == kConvTileH * kConvTileW || (int)threadIdx.x < kConvTileH * kConvTileW;  // one thread per pixel
-    if (p.final_out && owns_pixel)
-    {
-        const _Float16* row = s_patch + (size_t)(((int)threadIdx.x / kConvTileW + 1) * kConvPatchW + (int)threadIdx.x % kConvTileW + 1) * ROW;
-#pragma unroll
-        for (int c = 0; c < CI; ++c)
-            if (c < C) my_feat[c] = float(row[c]);
-    }
-    __syncthreads();  // every wavefront is done reading the patch
-#pragma unroll
-    for (int m = 0; m < MB; ++m)
-    {
-        const int tp = (MB == 4 ? 2 * wave + (m >> 1) : wave) * kConvTileW + (m & 1) * 16 + lrow;  // this lane's pixel of the block
-#pragma unroll
-        for (int j = 0; j < HB; ++j)
+        for (int m = 0; m < MB; ++m)
         {
-            const int ch0   = 16 * j + (lane >> 4) * 4;  // this lane's four channels
-            const float4 bf = *reinterpret_cast<const float4*>(p.bias + ch0), bm = *reinterpret_cast<const float4*>(p.bias + NPAD / 2 + ch0);
-            const float f[4] = {acc[m][j][0] + bf.x, acc[m][j][1] + bf.y, acc[m][j][2] + bf.z, acc[m][j][3] + bf.w};
-            // (both 0 for padding channels)
-            const float g[4] = {acc[m][HB + j][0] + bm.x, acc[m][HB + j][1] + bm.y, acc[m][HB + j][2] + bm.z, acc[m][HB + j][3] + bm.w};
-            if (p.pre)
+            const int y       = t.y0 + r0 + m;
+            const bool inside = y < p.H && x < p.W;
+            const int pix     = (r0 + m) * p.W + c0 + lrow;  // from the tile's first
+            const floatx4 f = acc[m][0], g = acc[m][1];
+            if (p.pre && inside)
             {
-                *reinterpret_cast<half4*>(s_pre + tp * PS + ch0)            = half4{_Float16(f[0]), _Float16(f[1]), _Float16(f[2]), _Float16(f[3])};
-                *reinterpret_cast<half4*>(s_pre + tp * PS + NPAD / 2 + ch0) = half4{_Float16(g[0]), _Float16(g[1]), _Float16(g[2]), _Float16(g[3])};
+                const half8 v = half8{_Float16(f[0]), _Float16(f[1]), _Float16(f[2]), _Float16(f[3]),
+                                      _Float16(g[0]), _Float16(g[1]), _Float16(g[2]), _Float16(g[3])};
+                __builtin_nontemporal_store(v, reinterpret_cast<half8*>(pre_tile + pix * p.npad + 2 * ch0));
             }
-            half4 out;
+            half4 o;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
             {
                 const float e = f[i] > 0.f ? f[i] : (__expf(f[i]) - 1.f);
                 // v_rcp_f32 is good to 1 ulp of fp32 and the product is rounded to fp16 next: no IEEE division needed
                 const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-g[i]));
-                out[i]         = ch0 + i < p.cout ? _Float16(e * sg) : _Float16(0.f);
+                o[i]           = _Float16(e * sg);  // (0 for padding channels: their weights and biases are 0)
             }
-            *reinterpret_cast<half4*>(s_act + tp * AS + ch0) = out;
-        }
-    }
-    __syncthreads();
-    if (p.out) store_tile_nhwc<THREADS>(s_act, AS, p.cout_store / 8, p.out, p.cout_store, x0, y0, p.W, p.H);
-    if (p.pre) store_tile_nhwc<THREADS, true>(s_pre, PS, NPAD / 8, p.pre, NPAD, x0, y0, p.W, p.H);
-    if (p.final_out)
-    {
-        // `final` of the net (Networks.h:1129-1131) on the matrix cores: per 16 pixels one MFMA per 32 input channels,
-        // A = the staged tile rows (block outputs, then the image in the row's padding columns), B = the 1x1 weights,
-        // rounded to fp16 like every other operand, outputs in the first columns.
-        constexpr int KF  = NPAD / 2 + IPAD;  // block outputs (padded) | image | zeros
-        constexpr int KFB = (KF + 31) / 32;
-        const int cin     = C + p.cout;
-        // the image joins the staged rows (columns NPAD/2 .. NPAD/2 + IPAD - 1; nobody has read them yet)
-        if (owns_pixel)
-        {
-            _Float16* row = s_act + (size_t)(int)threadIdx.x * AS + NPAD / 2;
-#pragma unroll
-            for (int c = 0; c < IPAD; ++c) row[c] = (c < CI && c < C) ? _Float16(my_feat[c < CI ? c : 0]) : _Float16(0.f);
-        }
-        half8 bfin[KFB];
-#pragma unroll
-        for (int kb = 0; kb < KFB; ++kb)
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
+            // the image of the pixel, as the convolution saw it: channels lq * 4 .. + 3
+            const _Float16* mine = s_patch + ((r0 + m + 1) * kConvPatchW + c0 + lrow + 1) * ROW;
+            if (p.out && inside)
             {
-                const int k = kb * 32 + lk + i;  // position in a staged row
-                float w     = 0.f;
-                if (lrow < p.final_cout)
+                _Float16* row = out_tile + pix * p.out_stride;
+                const int pos = 2 * C + ch0;
+                if (pos + 4 <= p.out_stride)
                 {
-                    if (k < p.cout)
-                        w = s_fw[lrow * cin + C + k];
-                    else if (k >= NPAD / 2 && k < NPAD / 2 + C)
-                        w = s_fw[lrow * cin + (k - NPAD / 2)];
-                }
-                bfin[kb][i] = _Float16(w);  // exact: the table holds fp16 values
-            }
-        __syncthreads();  // image columns in place
-        const size_t plane = (size_t)p.H * p.W;
-        const float fb     = lrow < p.final_cout ? s_fw[kFwBias + lrow] : 0.f;
-#pragma unroll
-        for (int m = 0; m < MB; ++m)
-        {
-            const int tp0 = (MB == 4 ? 2 * wave + (m >> 1) : wave) * kConvTileW + (m & 1) * 16;  // first pixel of this 16-pixel block
-            floatx4 o     = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < KFB; ++kb)
-            {
-                half8 a;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) a[i] = _Float16(0.f);
-                if (kb * 32 + lk < KF) a = *reinterpret_cast<const half8*>(s_act + (size_t)(tp0 + lrow) * AS + kb * 32 + lk);
-                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bfin[kb], o, 0, 0, 0);
-            }
-            // lane: output channel lrow, pixels tp0 + (lane / 16) * 4 .. + 3
-            if (lrow < p.final_cout)
-            {
-                const int tp = tp0 + (lane >> 4) * 4;
-                const int y = y0 + tp / kConvTileW, x = x0 + tp % kConvTileW;
-                float* dst = p.final_out + lrow * plane + (size_t)y * p.W + x;
-                if (y < p.H)
-                {
-                    if (x + 3 < p.W && (reinterpret_cast<uintptr_t>(dst) & 15) == 0)
-                        *reinterpret_cast<float4*>(dst) = make_float4(o[0] + fb, o[1] + fb, o[2] + fb, o[3] + fb);
+                    if (FOUR || (C & 1) == 0)
+                        *reinterpret_cast<half4*>(row + pos) = o;
                     else
                     {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (x + i < p.W) dst[i] = o[i] + fb;
+                        typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                        *reinterpret_cast<half2v*>(row + pos)     = half2v{o[0], o[1]};
+                        *reinterpret_cast<half2v*>(row + pos + 2) = half2v{o[2], o[3]};
                     }
                 }
+                else
+                {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (pos + i < p.out_stride) row[pos + i] = o[i];
+                }
+                if (gp == 0 && FOUR)
+                {
+                    if (lq == 0)
+                    {
+                        const half4 im                 = *reinterpret_cast<const half4*>(mine);
+                        *reinterpret_cast<half8*>(row) = half8{_Float16(0.f), _Float16(0.f), _Float16(0.f), _Float16(0.f), im[0], im[1], im[2], im[3]};
+                    }
+                }
+                else if (gp == 0)
+                {
+                    // the row's other positions: [0, C) zero, [C, 2C) the image, what the outputs do not reach zero
+                    for (int c = lq; c < C; c += 4) row[c] = _Float16(0.f), row[C + c] = mine[c];
+                    for (int c = 2 * C + p.npad / 2 + lq; c < p.out_stride; c += 4) row[c] = _Float16(0.f);
+                }
+            }
+            if (p.final_out)
+            {
+                const half4 im  = *reinterpret_cast<const half4*>(mine + (CI == 4 ? 0 : lq * 4));
+                const half4 sel = (lrow >> 2) == m ? fw : half4{}, sim = (lrow >> 2) == m ? fimg : half4{};
+                fin             = __builtin_amdgcn_mfma_f32_16x16x16f16(sel, o, fin, 0, 0, 0);
+                if (pair == 0) fin = __builtin_amdgcn_mfma_f32_16x16x16f16(sim, im, fin, 0, 0, 0);
+            }
+        }
+        if (p.final_out)
+        {
+            // lane group m: the outputs of row m, pixel lrow; with two pairs the wavefront of the second one hands over
+            // its share of the sums
+            if (PAIRS == 2)
+            {
+                if (pair == 1) s_fin[strip * 64 + lane] = make_float4(fin[0], fin[1], fin[2], fin[3]);
+                __syncthreads();
+            }
+            const int y = t.y0 + r0 + lq;
+            if (pair == 0 && lq < MB && y < p.H && x < p.W)
+            {
+                if (PAIRS == 2)
+                {
+                    const float4 o = s_fin[strip * 64 + lane];
+                    fin[0] += o.x, fin[1] += o.y, fin[2] += o.z, fin[3] += o.w;
+                }
+                const size_t plane = (size_t)p.H * p.W;
+                float* dst         = p.final_out + (size_t)t.image * p.final_cout * plane + (size_t)y * p.W + x;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k < p.final_cout) dst[k * plane] = fin[k] + p.final_b[k];
             }
         }
     }
 }
 
-// wpack[tap][n][c]: n < NPAD/2 feature output n, else mask output n - NPAD/2; zero outside the real ranges.
-// All levels in one launch, the level is blockIdx.y (a launch per level costs more than the work itself).
+// The 1x1 output convolution on rows of the finest level, for nets whose finest block has more than 32 outputs (their
+// pairs are split over workgroups, none of which holds a whole pixel). A thread per pixel; bound by its row's bytes.
+__global__ __launch_bounds__(256) void final_conv1x1_kernel(const _Float16* __restrict__ rows, int stride, int c_feat, int cin,
+                                                            const float* __restrict__ weight, const float* __restrict__ bias, int cout,
+                                                            size_t plane, size_t pixels, float* __restrict__ out)
+{
+    __shared__ float s_w[4 * (kUnetMaxImageChannels + 64)];
+    for (int i = threadIdx.x; i < cout * cin; i += 256) s_w[i] = float(_Float16(weight[i]));  // fp16 like every other operand
+    __syncthreads();
+    for (size_t pix = (size_t)blockIdx.x * 256 + threadIdx.x; pix < pixels; pix += (size_t)gridDim.x * 256)
+    {
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        const _Float16* row = rows + pix * stride;
+        for (int g = 0; g < stride / 8; ++g)
+        {
+            const half8 v = *reinterpret_cast<const half8*>(row + 8 * g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+            {
+                const int c = 8 * g + i - c_feat;  // channel of x_0: the image at positions [C, 2C), then the block outputs
+                if (c < 0 || c >= cin) continue;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k < cout) a[k] = __builtin_fmaf(s_w[k * cin + c], float(v[i]), a[k]);
+            }
+        }
+        const size_t b = pix / plane;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k < cout) out[b * cout * plane + k * plane + (pix - b * plane)] = a[k] + bias[k];
+    }
+}
+
+// Weights of all levels in one launch, the level is blockIdx.y (a launch per level costs more than the work itself):
+// MFMA fragments in the order a wavefront reads them, [pair][tap][cin / 32][feature, mask][lane][8]: output pair * 16 +
+// lane % 16, input channel 32 kb + (lane / 16) * 8 + i; zero outside the real ranges. Behind them the biases,
+// [pair][feature, mask][16]. The finest level's workgroups also pack the 1x1's weights:
+// [pair, then the image][output o < 4][quarter q][i]: channel 16 pair + 4 q + i of the block (of the image).
 struct PackLevel
 {
     const float *wf, *bf, *wm, *bm;
     int cout, cin_real, cin_pad, npad;
-    _Float16* wpack;
+    _Float16* wfrag;
     float* bias;
 };
 struct PackTable
 {
     PackLevel lv[TRIPS_UNET_MAX_LEVELS];
+    const float* final_w;
+    _Float16* fin_frag;
+    int c_feat, final_cout;
 };
 __global__ __launch_bounds__(256) void pack_conv_weights_kernel(const PackTable t)
 {
     const PackLevel& l = t.lv[blockIdx.y];
-    const float* __restrict__ wf = l.wf;
-    const float* __restrict__ bf = l.bf;
-    const float* __restrict__ wm = l.wm;
-    const float* __restrict__ bm = l.bm;
-    const int cout = l.cout, cin_real = l.cin_real, cin_pad = l.cin_pad, npad = l.npad;
-    _Float16* __restrict__ wpack = l.wpack;
-    float* __restrict__ bias     = l.bias;
-    const int total = 9 * npad * cin_pad;
+    const int cout = l.cout, cin_real = l.cin_real, npad = l.npad, kbs = l.cin_pad / 32;
+    const int total = 9 * npad * l.cin_pad;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256)
     {
-        const int c = i % cin_pad, n = (i / cin_pad) % npad, tap = i / (cin_pad * npad);
-        const int half = npad / 2;
-        const int o    = n < half ? n : n - half;
-        float v        = 0.f;
-        if (o < cout && c < cin_real) v = (n < half ? wf : wm)[((size_t)o * cin_real + c) * 9 + tap];
-        wpack[i] = _Float16(v);
+        const int e = i & 7, lane = (i >> 3) & 63, h = (i >> 9) & 1;
+        const int rest = i >> 10, kb = rest % kbs, tap = (rest / kbs) % 9, pair = rest / (kbs * 9);
+        const int o = pair * 16 + (lane & 15), c = kb * 32 + (lane >> 4) * 8 + e;
+        float v = 0.f;
+        if (o < cout && c < cin_real) v = (h ? l.wm : l.wf)[((size_t)o * cin_real + c) * 9 + tap];
+        l.wfrag[i] = _Float16(v);
     }
     for (int n = blockIdx.x * 256 + threadIdx.x; n < npad; n += gridDim.x * 256)
     {
-        const int half = npad / 2;
-        const int o    = n < half ? n : n - half;
-        bias[n]        = o < cout ? (n < half ? bf : bm)[o] : 0.f;
+        const int o = (n >> 5) * 16 + (n & 15);
+        l.bias[n]   = o < cout ? ((n & 16) ? l.bm : l.bf)[o] : 0.f;
+    }
+    if (blockIdx.y == 0)
+    {
+        const int pairs = npad / 32, cin = t.c_feat + cout;
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < (pairs + 1) * 64; i += gridDim.x * 256)
+        {
+            const int pair = i >> 6, o = (i >> 4) & 3, k = i & 15;
+            const int c = pair < pairs ? (pair * 16 + k < cout ? t.c_feat + pair * 16 + k : -1) : (k < t.c_feat ? k : -1);
+            t.fin_frag[i] = _Float16(o < t.final_cout && c >= 0 ? t.final_w[o * cin + c] : 0.f);
+        }
     }
 }
 
 // ---------------------------------------------------------------------------------------------------------
 namespace
 {
-template <int CIN, int NPAD, int CI>
-hipError_t launch_conv(const ConvParams& p, int batch, hipStream_t stream)
+template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, bool BREGS, int WAVES_PER_EU>
+hipError_t launch_conv(const ConvParams& p, int splits, hipStream_t stream)
 {
-    constexpr int ROW  = CIN + kLdsChanPad;
-    constexpr int IPAD = CI > kLdsChanPad ? CI : kLdsChanPad;
-    // the patch, then the patch of the level below or (later) the staged taps of the weights, whichever is larger
-    const size_t lds_in  = (size_t)(kConvPatchH * kConvPatchW * ROW + std::max(kBelowH * kBelowW * ROW, ConvTapStage<CIN, NPAD, 512>::LDS_HALVES)) * sizeof(_Float16);
-    const size_t lds_out = (size_t)kConvTileH * kConvTileW * ((NPAD / 2 + IPAD) + (p.pre ? NPAD + kLdsChanPad : 0)) * sizeof(_Float16);
-    const size_t lds     = std::max(lds_in, lds_out);  // up to 104 KB when the largest block saves its pre-activations
-    // eight wavefronts per tile (one row each): the phases around the tap loop run at the latency of their loads and LDS
-    // round trips, and twice the wavefronts per tile hide twice as much of it
-    constexpr int THREADS = 512;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gated_conv3x3_kernel<CIN, NPAD, THREADS, CI>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    for (int b = 0; b < batch; b += kMaxGridImages)
-    {
-        ConvParams q = p;
-        q.first_image = b;
-        dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH, std::min(batch - b, kMaxGridImages));
-        hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, NPAD, THREADS, CI>), grid, dim3(THREADS), lds, stream, q);
-    }
+    const long long tiles = (long long)p.tiles * p.batch;
+    // as many workgroups as are resident at once
+    const int resident = std::max(1, 256 * (4 * WAVES_PER_EU / (THREADS / 64)) / splits);
+    const dim3 grid((unsigned)std::min<long long>(tiles, resident), splits);
+    hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, PAIRS, CI, FOUR, THREADS, BREGS, WAVES_PER_EU>), grid, dim3(THREADS), 0, stream, p);
     return hipGetLastError();
 }
 
-template <int CI>
-hipError_t dispatch_conv_ci(const ConvParams& p, int batch, int cin_pad, int npad, hipStream_t stream)
+template <int CI, bool FOUR>
+hipError_t dispatch_conv_ci(const ConvParams& p, int cin_pad, hipStream_t stream)
 {
-    if (cin_pad == 32)
-    {
-        if (npad == 32) return launch_conv<32, 32, CI>(p, batch, stream);
-        if (npad == 64) return launch_conv<32, 64, CI>(p, batch, stream);
-        if (npad == 96) return launch_conv<32, 96, CI>(p, batch, stream);
-        if (npad == 128) return launch_conv<32, 128, CI>(p, batch, stream);
-    }
-    else
-    {
-        if (npad == 32) return launch_conv<64, 32, CI>(p, batch, stream);
-        if (npad == 64) return launch_conv<64, 64, CI>(p, batch, stream);
-        if (npad == 96) return launch_conv<64, 96, CI>(p, batch, stream);
-        if (npad == 128) return launch_conv<64, 128, CI>(p, batch, stream);
-    }
-    return hipErrorInvalidValue;
+    // Two pairs of outputs per workgroup where there are enough tiles to fill the chip's 256 CUs that way (the patch is
+    // then assembled half as often); an odd number of pairs and the coarse levels take one: with a few tiles the level
+    // lasts as long as one tile's chain of products, which two pairs double (64 -> 128, 3 tiles: 16 -> 10 us).
+    const int pairs = p.npad / 32;
+    const bool two  = pairs % 2 == 0 && ((p.final_out && pairs == 2) || (long long)p.tiles * p.batch * (pairs / 2) >= 256);
+    if (cin_pad == 32) return two ? launch_conv<32, 2, CI, FOUR, 512, false, 4>(p, pairs / 2, stream) : launch_conv<32, 1, CI, FOUR, 512, false, (FOUR ? 6 : 4)>(p, pairs, stream);
+    return two ? launch_conv<64, 2, CI, FOUR, 512, true, 2>(p, pairs / 2, stream) : launch_conv<64, 1, CI, FOUR, 512, true, 2>(p, pairs, stream);
 }
 
-// (the kernel is built for 4, 8 and 16 image channels; fewer use the next size up)
-hipError_t dispatch_conv(const ConvParams& p, int batch, int cin_pad, int npad, hipStream_t stream)
+// (the kernel is built for exactly 4 image channels and with room for 4, 8 and 16; other counts use the next size up)
+hipError_t dispatch_conv(const ConvParams& p, int cin_pad, hipStream_t stream)
 {
-    if (p.c_feat <= 4) return dispatch_conv_ci<4>(p, batch, cin_pad, npad, stream);
-    if (p.c_feat <= 8) return dispatch_conv_ci<8>(p, batch, cin_pad, npad, stream);
-    return dispatch_conv_ci<16>(p, batch, cin_pad, npad, stream);
+    if (p.c_feat == 4) return dispatch_conv_ci<4, true>(p, cin_pad, stream);
+    if (p.c_feat < 4) return dispatch_conv_ci<4, false>(p, cin_pad, stream);
+    if (p.c_feat <= 8) return dispatch_conv_ci<8, false>(p, cin_pad, stream);
+    return dispatch_conv_ci<16, false>(p, cin_pad, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -590,9 +546,14 @@ int trips_unet_flops(const TripsUnetDesc* desc, double* flops)
     return TRIPS_OK;
 }
 
-int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeights* weights,
-                       const float* const inputs[TRIPS_UNET_MAX_LEVELS], float* output, void* saved, void* workspace,
-                       size_t workspace_bytes, void* stream_)
+}  // extern "C"
+
+namespace
+{
+// hwc: inputs[i] is [batch, level_h, level_w, C] (the splat's eval layout) instead of [batch, C, level_h, level_w]
+int unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeights* weights,
+                 const float* const inputs[TRIPS_UNET_MAX_LEVELS], bool hwc, float* output, void* saved, void* workspace,
+                 size_t workspace_bytes, void* stream_)
 {
     if (!ctx) return set_error(TRIPS_ERR_INVALID_ARG, "ctx is NULL");
     if (int e = check_unet_desc(desc)) return e;
@@ -615,12 +576,8 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
     char* ws           = reinterpret_cast<char*>(workspace);
     char* sv           = reinterpret_cast<char*>(saved);
     Profiler* prof     = ctx->prof.enabled ? &ctx->prof : nullptr;
-    // block outputs live in the saved state when there is one (the backward reads them), else in the workspace
-    auto act_ptr = [&](int level)
-    {
-        const LevelPlan& l = np.lv[level];
-        return reinterpret_cast<_Float16*>(sv ? sv + l.saved_act_off : ws + l.act_off);
-    };
+    // the rows of a level live in the saved state when there is one (the backward reads them), else in the workspace
+    auto rows_ptr = [&](int level) { return reinterpret_cast<_Float16*>(sv && level > 0 ? sv + np.lv[level].saved_rows_off : ws + np.lv[level].rows_off); };
 
     if (!d.weights_packed)
     {
@@ -635,6 +592,10 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
                                  reinterpret_cast<float*>(ws + lv.bias_off)};
             most     = std::max(most, 9 * lv.npad * lv.cin_pad);
         }
+        pt.final_w    = weights->final_weight;
+        pt.fin_frag   = reinterpret_cast<_Float16*>(ws + np.fin_off);
+        pt.c_feat     = C;
+        pt.final_cout = d.num_output_channels;
         hipLaunchKernelGGL(pack_conv_weights_kernel, dim3((most + 255) / 256, L), dim3(256), 0, stream, pt);
     }
     static const char* const kLevelNames[TRIPS_UNET_MAX_LEVELS] = {"unet_conv_l0", "unet_conv_l1", "unet_conv_l2", "unet_conv_l3",
@@ -643,46 +604,63 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
     {
         const LevelPlan& lv = np.lv[i];
         ProfScope ps(prof, kLevelNames[i], stream);
+        const bool fused_final = i == 0 && lv.npad <= 64;
         ConvParams p;
         std::memset(&p, 0, sizeof(p));
-        p.H           = lv.H;
-        p.W           = lv.W;
-        p.c_feat      = C;
-        p.cout        = lv.cout;
-        p.cout_store  = lv.cout_store;
-        p.feat        = inputs[i];
-        p.feat_stride = (size_t)C * lv.H * lv.W;
-        p.wpack       = reinterpret_cast<const _Float16*>(ws + lv.wpack_off);
-        p.bias        = reinterpret_cast<const float*>(ws + lv.bias_off);
-        // (nobody reads the finest block's output again: its 1x1 runs in the same kernel, and the backward takes
+        p.H       = lv.H;
+        p.W       = lv.W;
+        p.c_feat  = C;
+        p.cout    = lv.cout;
+        p.npad    = lv.npad;
+        p.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
+        p.tiles   = p.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
+        p.batch   = d.batch;
+        p.feat    = inputs[i];
+        p.feat_ps = hwc ? C : 1;
+        p.feat_cs = hwc ? 1 : (size_t)lv.H * lv.W;
+        p.wfrag   = reinterpret_cast<const _Float16*>(ws + lv.wpack_off);
+        p.bias    = reinterpret_cast<const float*>(ws + lv.bias_off);
+        // (nobody reads the finest block's output again when its 1x1 runs in the same kernel, and the backward takes
         // it from the pre-activations)
-        p.out        = i == 0 ? nullptr : act_ptr(i);
-        p.out_stride = (size_t)lv.H * lv.W * lv.cout_store;
+        p.out        = fused_final ? nullptr : rows_ptr(i);
+        p.out_stride = lv.row_stride;
         p.pre        = sv ? reinterpret_cast<_Float16*>(sv + lv.saved_pre_off) : nullptr;
-        p.pre_stride = (size_t)lv.H * lv.W * lv.npad;
         if (i < L - 1)
         {
-            const LevelPlan& lb = np.lv[i + 1];
-            p.Hb                = lb.H;
-            p.Wb                = lb.W;
-            p.cb_store          = lb.cout_store;
-            p.feat_below        = inputs[i + 1];
-            p.feat_below_stride = (size_t)C * lb.H * lb.W;
-            p.act_below         = act_ptr(i + 1);
-            p.act_below_stride  = (size_t)lb.H * lb.W * lb.cout_store;
+            p.Hb           = np.lv[i + 1].H;
+            p.Wb           = np.lv[i + 1].W;
+            p.below        = rows_ptr(i + 1);
+            p.below_stride = np.lv[i + 1].row_stride;
         }
-        if (i == 0)
+        if (fused_final)
         {
-            p.final_w      = weights->final_weight;
-            p.final_b      = weights->final_bias;
-            p.final_out    = output;
-            p.final_stride = (size_t)d.num_output_channels * lv.H * lv.W;
-            p.final_cout   = d.num_output_channels;
+            p.fin_frag   = reinterpret_cast<const _Float16*>(ws + np.fin_off);
+            p.final_b    = weights->final_bias;
+            p.final_out  = output;
+            p.final_cout = d.num_output_channels;
         }
-        hipError_t e = dispatch_conv(p, d.batch, lv.cin_pad, lv.npad, stream);
+        hipError_t e = dispatch_conv(p, lv.cin_pad, stream);
+        if (e == hipSuccess && i == 0 && !fused_final)
+        {
+            const size_t plane = (size_t)lv.H * lv.W;
+            hipLaunchKernelGGL(final_conv1x1_kernel, dim3((unsigned)std::min<size_t>((d.batch * plane + 255) / 256, 8192)), dim3(256), 0, stream,
+                               p.out, p.out_stride, C, C + lv.cout, weights->final_weight, weights->final_bias, d.num_output_channels, plane,
+                               d.batch * plane, output);
+            e = hipGetLastError();
+        }
         if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "gated conv launch (level %d): %s", i, hipGetErrorString(e));
     }
     return TRIPS_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeights* weights,
+                       const float* const inputs[TRIPS_UNET_MAX_LEVELS], float* output, void* saved, void* workspace,
+                       size_t workspace_bytes, void* stream)
+{
+    return unet_forward(ctx, desc, weights, inputs, false, output, saved, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"
