@@ -87,6 +87,12 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
                        const float* const inputs[TRIPS_UNET_MAX_LEVELS], float* output, void* saved, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/* The inference forward for a pyramid in the splat's eval layout (TRIPS_LAYOUT_HWC): inputs[i] is
+ * [batch, level_h[i], level_w[i], C]; otherwise trips_unet_forward with saved = NULL. */
+int trips_unet_forward_hwc(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeights* weights,
+                           const float* const inputs[TRIPS_UNET_MAX_LEVELS], float* output, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
 /* Backward of the forward that wrote `saved` (same desc, weights and inputs). d_output: [batch, out, H, W] fp32.
  * Intermediate gradients are fp16: they are carried multiplied by grad_scale (a power of two such as 65536 keeps
  * dL/doutput ~ 1e-7 of a mean loss over millions of pixels in range) and every fp32 result is divided by it again.

@@ -42,3 +42,17 @@ def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
         got, want = got.cpu().numpy(), want.numpy()
         scale = np.abs(want).max()
         assert np.abs(got - want).max() < GRAD_TOL * scale, f"{name}: {np.abs(got - want).max() / scale:.3e}"
+
+
+@pytest.mark.parametrize("filters,w,h,cin,batch", [
+    ([16, 32], 37, 29, 4, 2), ([24, 32], 40, 24, 3, 1), ([32, 48], 33, 17, 8, 1), ([48, 64], 32, 8, 16, 1), ([16, 32], 1, 1, 4, 1),
+])
+def test_channels_last_pyramids_are_read_in_place(filters, w, h, cin, batch):
+    """Views of [B, H, W, C] images (what the splat's eval mode returns) give the bits of their contiguous copies."""
+    net = _net(filters, 2, seed=70 + cin, cin=cin).cuda()
+    inputs = [t.cuda() for t in _pyramid(w, h, 2, cin, batch=batch, seed=71)]
+    with torch.no_grad():
+        want = net.forward(inputs)
+        got = net.forward([t.permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2) for t in inputs])
+        mixed = net.forward([inputs[0], inputs[1].permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2)])
+    assert torch.equal(got, want) and torch.equal(mixed, want)

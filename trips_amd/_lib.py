@@ -21,7 +21,7 @@ SYMBOLS = [
 ]
 # every symbol include/trips_unet.h declares
 UNET_SYMBOLS = ["trips_unet_workspace_size", "trips_unet_saved_size", "trips_unet_backward_workspace_size",
-                "trips_unet_forward", "trips_unet_backward", "trips_unet_flops"]
+                "trips_unet_forward", "trips_unet_forward_hwc", "trips_unet_backward", "trips_unet_flops"]
 
 
 class TripsError(RuntimeError):
@@ -71,6 +71,8 @@ def load():
     lib.trips_unet_backward_workspace_size.argtypes = [C.POINTER(abi.TripsUnetDesc), C.POINTER(C.c_size_t)]
     lib.trips_unet_forward.argtypes = [vp, C.POINTER(abi.TripsUnetDesc), C.POINTER(abi.TripsUnetWeights),
                                        C.POINTER(vp), vp, vp, vp, C.c_size_t, vp]
+    lib.trips_unet_forward_hwc.argtypes = [vp, C.POINTER(abi.TripsUnetDesc), C.POINTER(abi.TripsUnetWeights),
+                                           C.POINTER(vp), vp, vp, C.c_size_t, vp]
     lib.trips_unet_backward.argtypes = [vp, C.POINTER(abi.TripsUnetDesc), C.POINTER(abi.TripsUnetWeights),
                                         C.POINTER(vp), vp, vp, C.c_float, C.POINTER(abi.TripsUnetGrads), vp,
                                         C.c_size_t, vp]

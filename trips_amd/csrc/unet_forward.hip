@@ -663,4 +663,11 @@ int trips_unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnet
     return unet_forward(ctx, desc, weights, inputs, false, output, saved, workspace, workspace_bytes, stream);
 }
 
+int trips_unet_forward_hwc(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeights* weights,
+                           const float* const inputs[TRIPS_UNET_MAX_LEVELS], float* output, void* workspace, size_t workspace_bytes,
+                           void* stream)
+{
+    return unet_forward(ctx, desc, weights, inputs, true, output, nullptr, workspace, workspace_bytes, stream);
+}
+
 }  // extern "C"

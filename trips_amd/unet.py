@@ -184,7 +184,7 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             ptrs[i] = t.data_ptr()
         return ptrs
 
-    def _run_forward(self, ins, params, saved):
+    def _run_forward(self, ins, params, saved, hwc=False):
         dev = ins[0].device
         ctx = get_context(dev.index or 0)
         d = self.desc(ins)
@@ -198,8 +198,12 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             d.weights_packed = 1
         self._packed_key = key if saved is None else None
         out = torch.empty((d.batch, d.num_output_channels, d.level_h[0], d.level_w[0]), dtype=torch.float32, device=dev)
-        _lib.check(ctx.lib.trips_unet_forward(ctx.ctx, C.byref(d), C.byref(w), self._input_ptrs(ins), _ptr(out),
-                                              _ptr(saved), _ptr(ws), nbytes, _stream_ptr(dev)))
+        if hwc:
+            _lib.check(ctx.lib.trips_unet_forward_hwc(ctx.ctx, C.byref(d), C.byref(w), self._input_ptrs(ins), _ptr(out),
+                                                      _ptr(ws), nbytes, _stream_ptr(dev)))
+        else:
+            _lib.check(ctx.lib.trips_unet_forward(ctx.ctx, C.byref(d), C.byref(w), self._input_ptrs(ins), _ptr(out),
+                                                  _ptr(saved), _ptr(ws), nbytes, _stream_ptr(dev)))
         return out
 
     def _run_backward(self, ins, params, saved, d_out):
@@ -233,17 +237,20 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
         if dev.type != "cuda":
             raise RuntimeError("MultiScaleUnet2dDecOnlySmallFixed needs GPU tensors: there is no CPU implementation")
         L = p.num_layers
-        ins = []
         for i in range(L):
             t = inputs[i]
             if t.dtype != torch.float32 or t.shape[1] != p.num_input_channels:
                 raise ValueError(f"inputs[{i}]: expected float32 [B, {p.num_input_channels}, H, W]")
-            ins.append(t.contiguous())
         params = [q.to(dev, torch.float32).contiguous() for q in self.ordered_parameters()]
+        ins = inputs[:L]
         needs_grad = torch.is_grad_enabled() and (any(t.requires_grad for t in ins) or any(q.requires_grad for q in params))
         if needs_grad:
-            return _UnetFunction.apply(self, L, *ins, *params)
-        return self._run_forward([t.detach() for t in ins], [q.detach() for q in params], None)
+            return _UnetFunction.apply(self, L, *(t.contiguous() for t in ins), *params)
+        # the splat's eval mode hands over views of [B, H, W, C] images: the kernels read those as they are
+        hwc = all(t.permute(0, 2, 3, 1).is_contiguous() for t in ins)
+        if not hwc:
+            ins = [t.contiguous() for t in ins]
+        return self._run_forward([t.detach() for t in ins], [q.detach() for q in params], None, hwc)
 
     def flops(self, inputs):
         d = self.desc(inputs)
