@@ -13,6 +13,43 @@ from . import abi
 from .renderer import get_context
 
 
+_NO_BOUNDS = (0.0, abi.FLT_MAX)
+
+
+def _options(group):
+    """The options of a parameter group in the order of the fields of TripsAdamTensor from `lr` on."""
+    beta1, beta2 = group["betas"]
+    return (group["lr"], beta1, beta2, group["eps"], group["relative_weight_decay"], group["absolute_weight_decay"],
+            group["weight_clipping_magnitude"])
+
+
+def _lr_bounds(group, step):
+    """AdaBound bounds, MyAdam.cu:213-221"""
+    beta2 = group["betas"][1]
+    return 0.1 - 0.1 / ((1 - beta2) * float(step) + 1), 0.1 + 0.1 / ((1 - beta2) * float(step))
+
+
+def _check_param(p, grad):
+    if grad is not None and grad.is_sparse:
+        raise RuntimeError("Adam does not support sparse gradients")
+    if p.dtype not in (torch.float32, torch.float64):
+        raise RuntimeError("MyAdam supports float32 and float64 parameters")
+    if not p.is_contiguous():
+        raise RuntimeError("MyAdam needs contiguous parameters")
+
+
+def _tensor_desc(p, g, st, options, bounds):
+    """One TripsAdamTensor; `st` None: the state is packed elsewhere. (Filled by position: a keyword or an assignment per
+    field took as long as everything else of a step over the net's small tensors.)"""
+    dtype = abi.TRIPS_DTYPE_F64 if p.dtype is torch.float64 else abi.TRIPS_DTYPE_F32
+    if st is None:
+        return abi.TripsAdamTensor(p.data_ptr(), g.data_ptr(), None, None, None, p.numel(), dtype, *options, *bounds, 1.0, 0)
+    steps = st["param_steps"]
+    return abi.TripsAdamTensor(p.data_ptr(), g.data_ptr(), st["first_moments"].data_ptr(), st["second_moments"].data_ptr(),
+                               steps.data_ptr(), p.numel(), dtype, *options, *bounds, 1.0,
+                               abi.TRIPS_STEPS_I32 if steps.dtype is torch.int32 else abi.TRIPS_STEPS_I64)
+
+
 class MyAdam(torch.optim.Optimizer):
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), eps=1e-8, relative_weight_decay=0.0,
                  absolute_weight_decay=0.0, weight_clipping_magnitude=0.0, adabound=False,
@@ -54,42 +91,18 @@ class MyAdam(torch.optim.Optimizer):
                 loss = closure()
         descs, keep, device = [], [], None
         for group in self.param_groups:
-            beta1, beta2 = group["betas"]
+            options = _options(group)
             for p in group["params"]:
-                if p.grad is None:
+                g = p.grad
+                if g is None:
                     continue
-                if p.grad.is_sparse:
-                    raise RuntimeError("Adam does not support sparse gradients")
-                if p.dtype not in (torch.float32, torch.float64):
-                    raise RuntimeError("MyAdam supports float32 and float64 parameters")
-                if not p.is_contiguous():
-                    raise RuntimeError("MyAdam needs contiguous parameters")
+                _check_param(p, g)
                 st = self._state_for(p)
                 st["current_step"] += 1
-                lower, upper = 0.0, abi.FLT_MAX
-                if group["adabound"]:
-                    # AdaBound bounds, MyAdam.cu:213-221
-                    lower = 0.1 - 0.1 / ((1 - beta2) * float(st["current_step"]) + 1)
-                    upper = 0.1 + 0.1 / ((1 - beta2) * float(st["current_step"]))
-                g = p.grad.contiguous()
+                g = g.contiguous()
                 keep.append(g)
-                t = abi.TripsAdamTensor()
-                t.weights = p.data_ptr()
-                t.grads = g.data_ptr()
-                t.first_moment = st["first_moments"].data_ptr()
-                t.second_moment = st["second_moments"].data_ptr()
-                t.steps = st["param_steps"].data_ptr()
-                t.steps_dtype = abi.TRIPS_STEPS_I32 if st["param_steps"].dtype == torch.int32 else abi.TRIPS_STEPS_I64
-                t.n = p.numel()
-                t.dtype = abi.TRIPS_DTYPE_F64 if p.dtype == torch.float64 else abi.TRIPS_DTYPE_F32
-                t.lr = group["lr"]
-                t.beta1, t.beta2, t.eps = beta1, beta2, group["eps"]
-                t.relative_weight_decay = group["relative_weight_decay"]
-                t.absolute_weight_decay = group["absolute_weight_decay"]
-                t.weight_clipping_magnitude = group["weight_clipping_magnitude"]
-                t.lower_lr_bound, t.upper_lr_bound = lower, upper
-                t.loss_scale = 1.0
-                descs.append(t)
+                bounds = _lr_bounds(group, st["current_step"]) if group["adabound"] else _NO_BOUNDS
+                descs.append(_tensor_desc(p, g, st, options, bounds))
                 device = p.device
         if descs:
             get_context(device).adam_step(descs)
@@ -186,56 +199,33 @@ class MyAdamPoints(MyAdam):
         packed_descs = [None] * 4
         any_packed_grad = any(p.grad is not None for p in self._packed)
         for group in self.param_groups:
-            beta1, beta2 = group["betas"]
+            options = _options(group)
             for p in group["params"]:
                 slot = packed_ids.get(id(p))
-                if p.grad is None and (slot is None or not any_packed_grad):
+                g = p.grad
+                if g is None and (slot is None or not any_packed_grad):
                     continue
-                if p.grad is not None and p.grad.is_sparse:
-                    raise RuntimeError("Adam does not support sparse gradients")
-                if p.dtype not in (torch.float32, torch.float64):
-                    raise RuntimeError("MyAdam supports float32 and float64 parameters")
-                if not p.is_contiguous():
-                    raise RuntimeError("MyAdam needs contiguous parameters")
+                _check_param(p, g)
                 if slot is None:
                     st = self._state_for(p)
                 else:
                     st = self.state[p]
                     st.setdefault("current_step", 0)
-                lower, upper = 0.0, abi.FLT_MAX
-                if p.grad is not None:
+                if g is not None:
                     st["current_step"] += 1
-                    g = p.grad.contiguous()
+                    g = g.contiguous()
                 else:
                     # a point parameter without a gradient in this step: zeros leave it and its state as they are
                     g = self._zero_grads.get(id(p))
                     if g is None or g.shape != p.shape:
                         g = self._zero_grads[id(p)] = torch.zeros_like(p)
-                if group["adabound"] and st["current_step"] > 0:
-                    lower = 0.1 - 0.1 / ((1 - beta2) * float(st["current_step"]) + 1)
-                    upper = 0.1 + 0.1 / ((1 - beta2) * float(st["current_step"]))
+                bounds = _lr_bounds(group, st["current_step"]) if group["adabound"] and st["current_step"] > 0 else _NO_BOUNDS
                 keep.append(g)
-                t = abi.TripsAdamTensor()
-                t.weights = p.data_ptr()
-                t.grads = g.data_ptr()
-                t.n = p.numel()
-                t.dtype = abi.TRIPS_DTYPE_F64 if p.dtype == torch.float64 else abi.TRIPS_DTYPE_F32
-                t.lr = group["lr"]
-                t.beta1, t.beta2, t.eps = beta1, beta2, group["eps"]
-                t.relative_weight_decay = group["relative_weight_decay"]
-                t.absolute_weight_decay = group["absolute_weight_decay"]
-                t.weight_clipping_magnitude = group["weight_clipping_magnitude"]
-                t.lower_lr_bound, t.upper_lr_bound = lower, upper
-                t.loss_scale = 1.0
                 device = p.device
                 if slot is None:
-                    t.first_moment = st["first_moments"].data_ptr()
-                    t.second_moment = st["second_moments"].data_ptr()
-                    t.steps = st["param_steps"].data_ptr()
-                    t.steps_dtype = abi.TRIPS_STEPS_I32 if st["param_steps"].dtype == torch.int32 else abi.TRIPS_STEPS_I64
-                    descs.append(t)
+                    descs.append(_tensor_desc(p, g, st, options, bounds))
                 else:
-                    packed_descs[slot] = t
+                    packed_descs[slot] = _tensor_desc(p, g, None, options, bounds)
         if any_packed_grad:
             n, c = self._geometry()
             dev = self._packed[0].device

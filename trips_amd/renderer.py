@@ -21,11 +21,13 @@ from . import _lib, abi
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    """Device pointer of a tensor as ctypes takes it for a void*."""
+    return None if t is None else t.data_ptr()
 
 
 def _stream_ptr(device):
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """hipStream_t of torch's current stream on `device` (a torch.device with an index)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 class SplatContext:
@@ -37,6 +39,7 @@ class SplatContext:
             raise RuntimeError("trips_amd needs a GPU: the splat path has no CPU implementation")
         self.device = torch.device("cuda", device if isinstance(device, int) else torch.device(device).index or 0)
         self.ctx = C.c_void_p()
+        self._sizes = {}
         _lib.check(self.lib.trips_ctx_create(C.byref(self.ctx), self.device.index))
 
     def __del__(self):
@@ -56,6 +59,17 @@ class SplatContext:
         b = C.c_size_t(0)
         _lib.check(self.lib.trips_splat_saved_size(C.byref(desc), C.byref(b)))
         return int(b.value)
+
+    def sizes(self, desc):
+        """(workspace, saved state) in bytes. Kept per descriptor value: a training or viewing loop asks with the same one
+        every step, and answering takes the library longer than looking it up."""
+        key = bytes(desc)
+        got = self._sizes.get(key)
+        if got is None:
+            if len(self._sizes) >= 64:
+                self._sizes.clear()
+            got = self._sizes[key] = (self.workspace_size(desc), self.saved_size(desc))
+        return got
 
     def alloc_bytes(self, n):
         # torch's allocator returns 512-byte aligned blocks; the ABI asks for 256
@@ -275,7 +289,7 @@ class PointRendererCache:
     def build(self, ctx, desc, train, dropout):
         key = (desc.num_channels, desc.num_points, desc.num_layers, desc.num_views, desc.views[0].h, desc.views[0].w,
                desc.list_depth, int(train))
-        need = ctx.workspace_size(desc)
+        need = ctx.sizes(desc)[0]
         if key != self.cache_size or self.workspace is None or self.workspace.numel() < need:
             self.workspace = ctx.alloc_bytes(need)
             self.cache_size = key
@@ -324,8 +338,8 @@ class PointRender(torch.autograd.Function):
     backward returns the 8 gradients in that order plus None for info."""
 
     @staticmethod
-    def forward(ctx, texture, background_color, points, pose_tangents, intrinsics, confidence, dynamic_refinement,
-                layer_value_of_point, info):
+    def render(texture, background_color, points, intrinsics, confidence, dynamic_refinement, layer_value_of_point, info):
+        """The forward itself: (images, desc, the tensors it read, saved state)."""
         sc = info.scene
         sctx = get_context(texture.device)
         desc = _desc_from_info(info, texture)
@@ -346,8 +360,28 @@ class PointRender(torch.autograd.Function):
                        dropout=cache.dropout_points, displacement=displacement)
         tin = SplatContext.make_in(**tensors)
         images = sctx.alloc_images(desc)
-        saved = sctx.alloc_bytes(sctx.saved_size(desc)) if info.train else None
+        saved = sctx.alloc_bytes(sctx.sizes(desc)[1]) if info.train else None
         sctx.forward(desc, tin, images, saved, cache.workspace)
+        return images, desc, tensors, saved
+
+    @staticmethod
+    def outputs(images, info):
+        """What the operator returns for the rendered images (output arity of PointRenderer.cu:482-505,1183-1190)."""
+        if not info.train:
+            images = [im.permute(0, 3, 1, 2) for im in images]  # PointRenderer.cu:747-749
+        extra = []
+        for flag in (info.params.add_depth_to_network, info.params.output_background_mask):
+            if flag:
+                extra += [torch.zeros((im.shape[0], 1, im.shape[2], im.shape[3]), dtype=torch.float32, device=im.device)
+                          for im in images]
+        return tuple(images) + tuple(extra)
+
+    @staticmethod
+    def forward(ctx, texture, background_color, points, pose_tangents, intrinsics, confidence, dynamic_refinement,
+                layer_value_of_point, info):
+        images, desc, tensors, saved = PointRender.render(texture, background_color, points, intrinsics, confidence,
+                                                          dynamic_refinement, layer_value_of_point, info)
+        ctx.set_materialize_grads(False)  # (a layer that nobody consumed: None instead of a tensor of zeros)
         ctx.render_info = info
         ctx.desc = desc
         ctx.tensors = tensors
@@ -357,15 +391,8 @@ class PointRender(torch.autograd.Function):
         ctx.saved_state = saved
         ctx.shapes = dict(points=points.shape, layer=layer_value_of_point.shape, confidence=confidence.shape,
                           pose=pose_tangents.shape)
-        ctx.image_shapes = [tuple(im.shape) for im in images]
-        if not info.train:
-            images = [im.permute(0, 3, 1, 2) for im in images]  # PointRenderer.cu:747-749
-        extra = []
-        for flag in (info.params.add_depth_to_network, info.params.output_background_mask):
-            if flag:
-                extra += [torch.zeros((im.shape[0], 1, im.shape[2], im.shape[3]), dtype=torch.float32, device=im.device)
-                          for im in images]
-        return tuple(images) + tuple(extra)
+        ctx.image_shapes = [im.shape for im in images]
+        return PointRender.outputs(images, info)
 
     @staticmethod
     def backward(ctx, *grad_output):
@@ -389,9 +416,12 @@ class PointRender(torch.autograd.Function):
             d_pose=torch.empty((desc.num_images, 6), dtype=torch.float64, device=dev) if need[3] else None,
             d_intrinsics=torch.empty_like(t["intrinsics"]) if need[4] else None,
         )
-        # a layer nobody consumed (a net with fewer levels than the pyramid) arrives without a gradient
-        gi = [g.contiguous() if g is not None else torch.zeros(shape, dtype=torch.float32, device=dev)
-              for g, shape in zip(grad_output[:desc.num_layers], ctx.image_shapes)]
+        # a layer nobody consumed (a net with fewer levels than the pyramid) arrives without a gradient: all of them read
+        # one run of zeros
+        gi = list(grad_output[:desc.num_layers])
+        absent = [shape.numel() for g, shape in zip(gi, ctx.image_shapes) if g is None]
+        zeros = torch.zeros(max(absent), dtype=torch.float32, device=dev) if absent else None
+        gi = [zeros if g is None else g.contiguous() for g in gi]
         tin = SplatContext.make_in(**t)
         sctx.backward(desc, tin, ctx.saved_state, gi, grads, info.cache.workspace if info.cache else None,
                       overwrite_point_grads=True, clear_block_sums=True)
@@ -405,10 +435,16 @@ class PointRender(torch.autograd.Function):
 def BlendPointCloud(info: NeuralRenderInfo):
     """Render the scene into a batch of image pyramids (RenderInfo.cpp:27-40)."""
     sc = info.scene
-    return list(PointRender.apply(sc.texture.texture, sc.texture.background_color, sc.point_cloud_cuda.t_position,
-                                  sc.poses.tangent_poses, sc.intrinsics.intrinsics,
-                                  sc.texture.confidence_value_of_point, sc.dynamic_refinement_t,
-                                  sc.point_cloud_cuda.t_point_size, info))
+    inputs = (sc.texture.texture, sc.texture.background_color, sc.point_cloud_cuda.t_position, sc.poses.tangent_poses,
+              sc.intrinsics.intrinsics, sc.texture.confidence_value_of_point, sc.dynamic_refinement_t,
+              sc.point_cloud_cuda.t_point_size)
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
+        return list(PointRender.apply(*inputs, info))
+    # no graph to record (a viewer's frame): the render without the autograd function around it
+    texture, background, points, _, intrinsics, confidence, refinement, layer = inputs
+    with torch.no_grad():
+        images, _, _, _ = PointRender.render(texture, background, points, intrinsics, confidence, refinement, layer, info)
+        return list(PointRender.outputs(images, info))
 
 
 # ---- minimal scene containers with the reference's member names ----

@@ -76,17 +76,19 @@ class _UnetFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx_, net, n_levels, *tensors):
+        # (autograd hands over the inputs themselves: detached where they are kept past this call)
         ins = [t.detach() for t in tensors[:n_levels]]
         params = [t.detach() for t in tensors[n_levels:]]
-        saved = net._alloc("saved", net._size("trips_unet_saved_size", ins), ins[0].device)
-        out = net._run_forward(ins, params, saved)
-        ctx_.net, ctx_.ins, ctx_.params, ctx_.saved = net, ins, params, saved
+        d = net.desc(ins)
+        saved = net._alloc("saved", net._sizes(d)[1], ins[0].device)
+        out = net._run_forward(d, ins, params, saved)
+        ctx_.net, ctx_.desc, ctx_.ins, ctx_.params, ctx_.saved = net, d, ins, params, saved
         return out
 
     @staticmethod
     def backward(ctx_, d_out):
         net = ctx_.net
-        d_ins, d_params = net._run_backward(ctx_.ins, ctx_.params, ctx_.saved, d_out.contiguous().float())
+        d_ins, d_params = net._run_backward(ctx_.desc, ctx_.ins, ctx_.params, ctx_.saved, d_out.contiguous().float())
         return (None, None, *d_ins, *d_params)
 
 
@@ -110,6 +112,7 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             self.add_module(f"up{i + 1}", UpsampleDecOnlySmallBlockFixed(F[i + 1], out))
         self.final = torch.nn.Sequential(torch.nn.Conv2d(F[0], p.num_output_channels, 1), torch.nn.Identity())
         self._buffers_dev = {}
+        self._sizes_of = {}
         # A viewer sets this: the weights then count as unchanged from one no-grad forward to the next (they are packed
         # to fp16 once, not per frame). Whoever changes them in place afterwards (load_state_dict, an optimiser step)
         # calls invalidate_packed_weights().
@@ -130,11 +133,19 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
 
     def ordered_parameters(self):
         """Parameters in the order of the C structs: per level feature weight, bias, mask weight, bias; then final."""
-        out = []
-        for i in range(self.params.num_layers):
-            b = self.block(i)
-            out += [b.feature_conv.weight, b.feature_conv.bias, b.mask_conv.weight, b.mask_conv.bias]
-        return out + [self.final_conv.weight, self.final_conv.bias]
+        # (through the modules' own tables: an attribute of a module is looked up in three of them, and a small frame
+        # spent a quarter of its time on that)
+        mods, L, out = self._modules, self.params.num_layers, []
+        for i in range(L):
+            blk = mods["start"]._modules["conv"] if i == L - 1 else mods[f"up{i + 1}"]._modules["convolution"]
+            for branch in ("feature_transform", "mask_transform"):
+                conv = blk._modules[branch]._modules["0"]
+                out.append(conv.weight)
+                out.append(conv.bias)
+        conv = mods["final"]._modules["0"]
+        out.append(conv.weight)
+        out.append(conv.bias)
+        return out
 
     def he_normal_(self, generator=None):
         """He-normal weights, zero biases (the initialisation the benchmark configuration names)."""
@@ -153,11 +164,20 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
                                   batch=int(inputs[0].shape[0]))
 
     # ---- plumbing ----
-    def _size(self, fn, inputs):
-        d = self.desc(inputs)
-        n = C.c_size_t(0)
-        _lib.check(getattr(_lib.load(), fn)(C.byref(d), C.byref(n)))
-        return int(n.value)
+    def _sizes(self, d):
+        """(forward workspace, saved state, backward workspace) in bytes, kept per descriptor value."""
+        key = bytes(d)
+        got = self._sizes_of.get(key)
+        if got is None:
+            lib, got = _lib.load(), []
+            for fn in (lib.trips_unet_workspace_size, lib.trips_unet_saved_size, lib.trips_unet_backward_workspace_size):
+                n = C.c_size_t(0)
+                _lib.check(fn(C.byref(d), C.byref(n)))
+                got.append(int(n.value))
+            if len(self._sizes_of) >= 64:
+                self._sizes_of.clear()
+            self._sizes_of[key] = got
+        return got
 
     def _alloc(self, key, nbytes, dev):
         if key == "saved":  # one per forward: a later forward must not overwrite what an earlier graph still needs
@@ -171,11 +191,11 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
     def _weights_struct(self, params):
         w = abi.TripsUnetWeights()
         L = self.params.num_layers
-        for i in range(L):
-            w.feature_weight[i], w.feature_bias[i] = params[4 * i].data_ptr(), params[4 * i + 1].data_ptr()
-            w.mask_weight[i], w.mask_bias[i] = params[4 * i + 2].data_ptr(), params[4 * i + 3].data_ptr()
-        w.final_weight, w.final_bias = params[4 * L].data_ptr(), params[4 * L + 1].data_ptr()
-        return w
+        ptrs = [q.data_ptr() for q in params]
+        w.feature_weight[:L], w.feature_bias[:L] = ptrs[0:4 * L:4], ptrs[1:4 * L:4]
+        w.mask_weight[:L], w.mask_bias[:L] = ptrs[2:4 * L:4], ptrs[3:4 * L:4]
+        w.final_weight, w.final_bias = ptrs[4 * L], ptrs[4 * L + 1]
+        return w, tuple(ptrs)
 
     @staticmethod
     def _input_ptrs(ins):
@@ -184,18 +204,17 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             ptrs[i] = t.data_ptr()
         return ptrs
 
-    def _run_forward(self, ins, params, saved, hwc=False):
+    def _run_forward(self, d, ins, params, saved, hwc=False):
         dev = ins[0].device
         ctx = get_context(dev.index or 0)
-        d = self.desc(ins)
-        w = self._weights_struct(params)
-        nbytes = self._size("trips_unet_workspace_size", ins)
+        w, ptrs = self._weights_struct(params)
+        nbytes = self._sizes(d)[0]
         ws = self._alloc("forward", nbytes, dev)
         # the packed weights in the workspace stay valid while the weights do (reuse_packed_weights), for the same
         # buffer and level sizes
-        key = (ws.data_ptr(), bytes(d), tuple(q.data_ptr() for q in params))
+        key = (ws.data_ptr(), bytes(d), ptrs)
         if self.reuse_packed_weights and saved is None and self._packed_key == key:
-            d.weights_packed = 1
+            d.weights_packed = 1  # (this call's own descriptor)
         self._packed_key = key if saved is None else None
         out = torch.empty((d.batch, d.num_output_channels, d.level_h[0], d.level_w[0]), dtype=torch.float32, device=dev)
         if hwc:
@@ -206,22 +225,21 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
                                                   _ptr(saved), _ptr(ws), nbytes, _stream_ptr(dev)))
         return out
 
-    def _run_backward(self, ins, params, saved, d_out):
+    def _run_backward(self, d, ins, params, saved, d_out):
         dev = ins[0].device
         ctx = get_context(dev.index or 0)
-        d = self.desc(ins)
-        w = self._weights_struct(params)
-        nbytes = self._size("trips_unet_backward_workspace_size", ins)
+        w, _ = self._weights_struct(params)
+        nbytes = self._sizes(d)[2]
         ws = self._alloc("backward", nbytes, dev)
         L = self.params.num_layers
         g = abi.TripsUnetGrads()
         d_params = [torch.empty_like(t) for t in params]
         d_ins = [torch.empty_like(t) for t in ins]
-        for i in range(L):
-            g.feature_weight[i], g.feature_bias[i] = d_params[4 * i].data_ptr(), d_params[4 * i + 1].data_ptr()
-            g.mask_weight[i], g.mask_bias[i] = d_params[4 * i + 2].data_ptr(), d_params[4 * i + 3].data_ptr()
-            g.inputs[i] = d_ins[i].data_ptr()
-        g.final_weight, g.final_bias = d_params[4 * L].data_ptr(), d_params[4 * L + 1].data_ptr()
+        ptrs = [t.data_ptr() for t in d_params]
+        g.feature_weight[:L], g.feature_bias[:L] = ptrs[0:4 * L:4], ptrs[1:4 * L:4]
+        g.mask_weight[:L], g.mask_bias[:L] = ptrs[2:4 * L:4], ptrs[3:4 * L:4]
+        g.final_weight, g.final_bias = ptrs[4 * L], ptrs[4 * L + 1]
+        g.inputs[:L] = [t.data_ptr() for t in d_ins]
         _lib.check(ctx.lib.trips_unet_backward(ctx.ctx, C.byref(d), C.byref(w), self._input_ptrs(ins), _ptr(saved),
                                                _ptr(d_out), C.c_float(self.grad_scale), C.byref(g), _ptr(ws), nbytes,
                                                _stream_ptr(dev)))
@@ -241,7 +259,8 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             t = inputs[i]
             if t.dtype != torch.float32 or t.shape[1] != p.num_input_channels:
                 raise ValueError(f"inputs[{i}]: expected float32 [B, {p.num_input_channels}, H, W]")
-        params = [q.to(dev, torch.float32).contiguous() for q in self.ordered_parameters()]
+        params = [q if q.dtype is torch.float32 and q.device == dev and q.is_contiguous() else q.to(dev, torch.float32).contiguous()
+                  for q in self.ordered_parameters()]
         ins = inputs[:L]
         needs_grad = torch.is_grad_enabled() and (any(t.requires_grad for t in ins) or any(q.requires_grad for q in params))
         if needs_grad:
@@ -250,7 +269,7 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
         hwc = all(t.permute(0, 2, 3, 1).is_contiguous() for t in ins)
         if not hwc:
             ins = [t.contiguous() for t in ins]
-        return self._run_forward([t.detach() for t in ins], [q.detach() for q in params], None, hwc)
+        return self._run_forward(self.desc(ins), ins, params, None, hwc)
 
     def flops(self, inputs):
         d = self.desc(inputs)
