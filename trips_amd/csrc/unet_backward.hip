@@ -621,10 +621,11 @@ struct BwdWeightParams
     int batch;           // images, one after the other in every array
     const float* feat;
     const _Float16* below;  // rows of the level below, [Hb][Wb][below_stride]
-    const _Float16* dpre;   // [H][W][NPAD]
-    float* part;           // [gridDim.x][9][NPAD][CIN]
+    int npad;               // pre-activations of a pixel, of which a workgroup takes NPAD (the grid's y dimension the others)
+    const _Float16* dpre;   // [H][W][npad]
+    float* part;           // [gridDim.x][9][npad][CIN]
     // bias gradients = sums of dpre over the pixels, taken from the transposed tile while it is in LDS
-    float* bias_part;      // [gridDim.x][NPAD] or nullptr
+    float* bias_part;      // [gridDim.x][npad] or nullptr
 };
 
 // Pixel-major tiles and the transposing LDS read. Both operands of the weight-gradient GEMM are needed with eight
@@ -689,7 +690,6 @@ __device__ __forceinline__ void lds_read_pixel_windows(const _Float16* tile, int
     w[2] = out.h;
 }
 
-// THREADS: 256, or 512 for the largest shape, whose 9 x NPAD x CIN sums are 288 registers per lane of four wavefronts.
 // CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
 template <int CIN, int NPAD, bool BIAS, int THREADS, int CI, bool FOUR>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightParams p)
@@ -759,14 +759,15 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     const int below_groups = p.below_stride / 8;  // groups of eight that a row of the level below has
     // the images of the batch are walked as one run of tiles: a workgroup keeps its sums from one image to the next
     // (image after image, every image paid for a set of partial sums of its own and for a last round of its own)
+    const int n0      = (int)blockIdx.y * NPAD;  // this workgroup's first pre-activation
     const float* feat = p.feat;
-    const _Float16 *below = p.below, *dpre = p.dpre;
+    const _Float16 *below = p.below, *dpre = p.dpre + n0;
     auto of_image = [&](int& tile)
     {
         const int image = p.batch > 1 ? tile / p.tiles : 0;
         tile -= image * p.tiles;
         feat = p.feat + (size_t)image * C * p.H * p.W;
-        dpre = p.dpre + (size_t)image * p.H * p.W * NPAD;
+        dpre = p.dpre + (size_t)image * p.H * p.W * p.npad + n0;
         if (has_below) below = p.below + (size_t)image * p.Hb * p.Wb * p.below_stride;
     };
     auto issue_loads = [&](int tile, TileLoads& r)
@@ -811,7 +812,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
 #pragma unroll
             for (int i = 0; i < 8; ++i) r.dpre[k][i] = _Float16(0.f);
             if (tp < kConvTileH * kConvTileW && y < p.H && x < p.W)
-                r.dpre[k] = *reinterpret_cast<const half8*>(dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
+                r.dpre[k] = *reinterpret_cast<const half8*>(dpre + ((size_t)y * p.W + x) * p.npad + 8 * g);
         }
     };
     // this level's image into channels [0, C) of a patch pixel (the channels [C, 8) follow from the upsampling, or are
@@ -866,49 +867,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         }
     };
 
-    // the same without registers in between, for the shapes that have none to spare
-    auto stream_stage1 = [&](int x0, int y0, int by0, int bx0)
-    {
-        {
-            const size_t plane = (size_t)p.H * p.W;
-            for (int item = threadIdx.x; item < kConvPatchH * kConvPatchW; item += THREADS)
-            {
-                const int py = item / kConvPatchW, px = item - py * kConvPatchW;
-                const int y = y0 + py - 1, x = x0 + px - 1;
-                const bool in = y >= 0 && y < p.H && x >= 0 && x < p.W;
-                float v[CI];
-#pragma unroll
-                for (int c = 0; c < CI; ++c) v[c] = (in && c < C) ? feat[c * plane + (size_t)y * p.W + x] : 0.f;
-                put_image(item, v);
-            }
-        }
-        if (has_below)
-        {
-            for (int item = threadIdx.x; item < kBelowH * kBelowW * GROUPS; item += THREADS)
-            {
-                const int g = item % GROUPS, bp = item / GROUPS;
-                const int r = bp / kBelowW, c0 = bp - r * kBelowW;
-                uint4 v = make_uint4(0u, 0u, 0u, 0u);
-                if (g < below_groups)
-                {
-                    const int yy = min(max(by0 + r, 0), p.Hb - 1), xx = min(max(bx0 + c0, 0), p.Wb - 1);
-                    v            = *reinterpret_cast<const uint4*>(below + ((size_t)yy * p.Wb + xx) * p.below_stride + 8 * g);
-                }
-                *reinterpret_cast<uint4*>(s_below + bp * ROW + 8 * g) = v;
-            }
-        }
-        for (int item = threadIdx.x; item < kConvTileH * kConvTileW * kDpreGroups; item += THREADS)
-        {
-            const int g = item % kDpreGroups, tp = item / kDpreGroups;
-            const int y = y0 + tp / kConvTileW, x = x0 + tp % kConvTileW;
-            half8 v;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = _Float16(0.f);
-            if (y < p.H && x < p.W) v = *reinterpret_cast<const half8*>(dpre + ((size_t)y * p.W + x) * NPAD + 8 * g);
-            *reinterpret_cast<half8*>(s_d + (size_t)tp * DS + 8 * g) = v;
-        }
-    };
-
     // start block: the channels beyond the image's groups of eight of a patch pixel are never written and stay zero
     constexpr int kImageGroups = (CI + 7) / 8;
     if (!has_below)
@@ -920,24 +878,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
             *reinterpret_cast<half8*>(s_patch + (size_t)(i / (GROUPS - kImageGroups)) * ROW + 8 * (kImageGroups + i % (GROUPS - kImageGroups))) = z;
         }
 
-    // with 64 input channels and more than 64 pre-activations the accumulators leave no registers for a tile in flight
-    constexpr bool kPrefetch = !(CIN == 64 && NPAD > 64);
     TileLoads cur;
     const int tiles = p.tiles * p.batch;
-    if (kPrefetch && (int)blockIdx.x < tiles) issue_loads(blockIdx.x, cur);
+    if ((int)blockIdx.x < tiles) issue_loads(blockIdx.x, cur);
     for (int tile0 = blockIdx.x; tile0 < tiles; tile0 += gridDim.x)
     {
         int tile = tile0;
         of_image(tile);
         const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
         const int x0 = tx * kConvTileW, y0 = ty * kConvTileH;
-        const int by0 = y0 / 2 - 1, bx0 = x0 / 2 - 1;
         __syncthreads();  // the previous tile's operands have been consumed (and the zero fill is done)
-        if (!kPrefetch)
-            stream_stage1(x0, y0, by0, bx0);
-        else
-            commit_loads(cur);
-        if (kPrefetch && tile0 + (int)gridDim.x < tiles) issue_loads(tile0 + gridDim.x, cur);  // travels during stage 2 and the taps
+        commit_loads(cur);
+        if (tile0 + (int)gridDim.x < tiles) issue_loads(tile0 + gridDim.x, cur);  // travels during stage 2 and the taps
         if (has_below)
         {
             __syncthreads();
@@ -1027,13 +979,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     if (BIAS && cb0 == 0 && (lane & 15) == 0)
     {
         // column 0 of the row sums: this lane holds rows (lane / 16) * 4 .. + 3 of every block
-        float* dst = p.bias_part + (size_t)set * NPAD;
+        float* dst = p.bias_part + (size_t)set * p.npad + n0;
 #pragma unroll
         for (int n = 0; n < MYNB; ++n)
 #pragma unroll
             for (int i = 0; i < 4; ++i) dst[(nb0 + n) * 16 + (lane >> 4) * 4 + i] = bias_acc[n][i];
     }
-    float* part = p.part + (size_t)set * 9 * NPAD * CIN;
+    float* part = p.part + ((size_t)set * 9 * p.npad + n0) * CIN;
     const int lrow = lane & 15;
     // (the input channels are the rows of the MFMA result: a lane holds four neighbouring ones of output lrow)
 #pragma unroll
@@ -1042,7 +994,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         for (int n = 0; n < MYNB; ++n)
 #pragma unroll
             for (int c = 0; c < MYCB; ++c)
-                *reinterpret_cast<float4*>(part + ((size_t)tap * NPAD + (nb0 + n) * 16 + lrow) * CIN + (cb0 + c) * 16 + (lane >> 4) * 4) =
+                *reinterpret_cast<float4*>(part + ((size_t)tap * p.npad + (nb0 + n) * 16 + lrow) * CIN + (cb0 + c) * 16 + (lane >> 4) * 4) =
                     make_float4(acc[tap][n][c][0], acc[tap][n][c][1], acc[tap][n][c][2], acc[tap][n][c][3]);
 }
 
@@ -1162,28 +1114,30 @@ hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int ci
 }
 
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
-hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, hipStream_t stream)
+hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, hipStream_t stream)
 {
     constexpr int THREADS = wgrad_threads(CIN, NPAD);
     const size_t lds = ((size_t)(kConvPatchH * kConvPatchW + kBelowH * kBelowW) * (CIN + kLdsChanPad) +
                         (size_t)kConvTileH * kConvTileW * (NPAD + kLdsChanPad)) *
-                       sizeof(_Float16);  // up to 133 KB
+                       sizeof(_Float16);  // up to 101 KB
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>), dim3(groups), dim3(THREADS), lds, stream, p);
+    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>), dim3(groups, splits), dim3(THREADS), lds, stream, p);
     return hipGetLastError();
 }
 
 template <int CI, bool FOUR>
 hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, int cin_pad, int npad, int groups, hipStream_t stream)
 {
-#define TRIPS_BW(CIN_, NPAD_)                                                                  \
-    if (cin_pad == CIN_ && npad == NPAD_)                                                      \
-        return p.bias_part ? launch_bwd_weight<CIN_, NPAD_, true, CI, FOUR>(p, groups, stream) \
-                                          : launch_bwd_weight<CIN_, NPAD_, false, CI, FOUR>(p, groups, stream);
-    TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 96) TRIPS_BW(32, 128)
-    TRIPS_BW(64, 32) TRIPS_BW(64, 64) TRIPS_BW(64, 96) TRIPS_BW(64, 128)
+    // 64 pre-activations to a workgroup at most (more would leave it no registers for a tile in flight: 64 x 128 in one
+    // workgroup spilled and took four times as long per tile as 64 x 64); the others are workgroups of their own
+    const int nt = wgrad_tile(npad);
+#define TRIPS_BW(CIN_, NT_)                                                                    \
+    if (cin_pad == CIN_ && nt == NT_)                                                          \
+        return p.bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(p, groups, npad / NT_, stream) \
+                           : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(p, groups, npad / NT_, stream);
+    TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
 #undef TRIPS_BW
     return hipErrorInvalidValue;
 }
@@ -1372,6 +1326,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
             wp.batch   = d.batch;
             wp.feat    = inputs[i];
+            wp.npad    = lv.npad;
             wp.dpre    = dpre_ptr(i);
             wp.part    = reinterpret_cast<float*>(ws + lv.part_off);
             if (bp.d_bias_f || bp.d_bias_m) wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off);

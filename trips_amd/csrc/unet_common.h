@@ -226,7 +226,8 @@ __device__ __forceinline__ void store_tile_nhwc(const _Float16* s_tile, int lds_
 // Work split of the weight-gradient kernel for a (padded input channels, padded pre-activations) shape: threads per
 // workgroup; how many ways the wavefronts split the 16-channel input blocks, the 16-channel pre-activation blocks and,
 // where there are more wavefronts than blocks, the rows of a tile.
-constexpr int wgrad_threads(int cin, int npad) { return (cin == 32 && npad == 96) ? 256 : 512; }
+constexpr int wgrad_threads(int, int) { return 512; }
+constexpr int wgrad_tile(int npad) { return npad % 64 == 0 ? 64 : 32; }  // pre-activations of a workgroup
 constexpr int wgrad_cbw(int cin) { return cin / 16 < 4 ? cin / 16 : 4; }
 constexpr int wgrad_nbw(int cin, int npad)
 {
@@ -354,8 +355,10 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         bw += align256(pixels * lv.cin_pad * sizeof(_Float16));
         const long long tiles = (long long)d.batch * ((lv.W + kConvTileW - 1) / kConvTileW) * ((lv.H + kConvTileH - 1) / kConvTileH);
         // persistent workgroups of the weight-gradient kernel: as many as are resident at once (two per CU for the
-        // smallest shape, else one); every further one would only add a set of partial sums to write and reduce
-        const int resident = (lv.cin_pad * lv.npad <= 1024 ? 2 : 1) * 256;
+        // smallest shape, else one; those that share the pre-activations of a tile between them count together); every
+        // further one would only add a set of partial sums to write and reduce (32 x 64 with two per CU: 64 instead of
+        // 70 us at 1245 x 825, and 7 us more for the sums)
+        const int resident = 256 * (lv.cin_pad == 32 && wgrad_tile(lv.npad) == 32 ? 2 : 1) / (lv.npad / wgrad_tile(lv.npad));
         lv.groups          = tiles < resident ? (int)tiles : resident;
         lv.part_off     = bw;
         bw += align256((size_t)lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
