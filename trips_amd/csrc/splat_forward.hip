@@ -321,7 +321,6 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     {
         p.chunk_valid[blockIdx.x]                = next - begin;
         p.chunk_valid[p.bin_groups + blockIdx.x] = s_flags;
-        p.chunk_valid[2 * p.bin_groups + blockIdx.x] = 0;
         p.chunk_valid[3 * p.bin_groups + blockIdx.x] = next_pair;
     }
 }
@@ -335,142 +334,127 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 //   * slices of split tiles: a tile with more than kSliceEntries bin entries (hundreds of points per pixel, e.g.
 //     tight clusters) would keep a single workgroup busy for milliseconds; it is cut into slices of kSliceEntries
 //     entries, each a workgroup of its own. slice_start[t] = number of slices of split tiles before tile t.
-// The workgroups after the first clear `clear_n` 16-byte words at `clear` (the per-cell counters of the list
-// kernels), which saves a launch of its own.
+// Its time is a chain of barriers and round trips, so every thread takes its share of the tiles at once (all loads in
+// flight together) and the scans over chunks and tiles share their barriers.
+// The workgroups after the first clear the per-cell counters `counts` and `run` of the tiles that may be split: the
+// slices add to them. Those of any other tile are written, not added to, where its keys are placed (clearing all of
+// them was 22 MB at 1920 x 1080 and eight layers: with that and a scan of 1024 tiles at a time, 13.8 us there; now 6).
+constexpr int kPlanPer = (kMaxBins + 1023) / 1024;  // tiles of a thread
 __global__ __launch_bounds__(1024) void scan_plan_kernel(const int32_t* __restrict__ bin_count, int32_t* __restrict__ bin_start,
                                                          int32_t* __restrict__ slice_start, int NB, long long capacity,
                                                          int32_t* __restrict__ chunk_valid, int G, ViewHeader* header,
                                                          ViewHeader* status, int first_view, int32_t* __restrict__ long_count,
-                                                         uint4* __restrict__ clear, long long clear_n, int32_t* __restrict__ saved_chunk_valid)
+                                                         int32_t* __restrict__ counts, int32_t* __restrict__ run,
+                                                         int32_t* __restrict__ saved_chunk_valid)
 {
     if (blockIdx.x > 0)
     {
-        for (long long i = (long long)(blockIdx.x - 1) * 1024 + threadIdx.x; i < clear_n; i += (long long)(gridDim.x - 1) * 1024)
-            clear[i] = make_uint4(0u, 0u, 0u, 0u);
+        // (a superset of the tiles that are split: entries past the capacity may leave a tile whole)
+        static_assert(kTilePixels == 1024, "a thread per cell");
+        for (int t = blockIdx.x - 1; t < NB; t += gridDim.x - 1)
+            if (bin_count[t] > kSliceEntries)
+            {
+                counts[(size_t)t * kTilePixels + threadIdx.x] = 0;
+                run[(size_t)t * kTilePixels + threadIdx.x]    = 0;
+            }
         return;
     }
-    __shared__ int s_wave[2][16];
-    __shared__ int s_carry[2];
-    __shared__ unsigned long long s_valid_total, s_same_total;
-    __shared__ int s_flags;
-    __shared__ int s_over_total;
-    if (threadIdx.x == 0)
-    {
-        s_over_total = 0;
-        s_carry[0] = s_carry[1] = 0;
-        s_valid_total = s_same_total = 0;
-        s_flags                 = 0;
-        *long_count             = 0;
-    }
-    __syncthreads();
+    __shared__ int s_over[16], s_tiles[16], s_slices[16], s_valid[16], s_flag[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per  = (NB + 1023) / 1024;
+    const int t0   = (int)threadIdx.x * per;
+    int v[kPlanPer];
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j) v[j] = j < per && t0 + j < NB ? bin_count[t0 + j] : 0;
+    const bool chunk = (int)threadIdx.x < G;  // (G <= 1024)
+    const int valid = chunk ? chunk_valid[threadIdx.x] : 0;
+    const int flags = chunk ? chunk_valid[G + threadIdx.x] : 0;
+    const int over  = chunk ? chunk_valid[3 * G + threadIdx.x] : 0;
+
+    auto wave_scan = [&](int x)
     {
-        // sums over the chunks: per wavefront first, then one LDS atomic per wavefront and sum
-        unsigned long long v = 0, st = 0;
-        int f = 0;
-        for (int g = threadIdx.x; g < G; g += 1024)
+        for (int o = 1; o < 64; o <<= 1)
         {
-            v += (unsigned long long)(unsigned)chunk_valid[g];
-            f |= chunk_valid[G + g];
-            st += (unsigned long long)(unsigned)chunk_valid[2 * G + g];
+            const int t = __shfl_up(x, o);
+            if (lane >= o) x += t;
         }
-        // number of every chunk's first overflow row: exclusive prefix of the chunks' row counts (G <= 1024)
+        return x;
+    };
+    // sum over the wavefronts before this one, and over all of them
+    auto wave_prefix = [&](const int* waves, int& all)
+    {
+        int before = 0;
+        all        = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w)
         {
-            const int mine = (int)threadIdx.x < G ? chunk_valid[3 * G + threadIdx.x] : 0;
-            int inc        = mine;
-            for (int o = 1; o < 64; o <<= 1)
-            {
-                const int t = __shfl_up(inc, o);
-                if (lane >= o) inc += t;
-            }
-            if (lane == 63) s_wave[0][wave] = inc;
-            __syncthreads();
-            int prefix = inc - mine;
-            for (int w = 0; w < wave; ++w) prefix += s_wave[0][w];
-            if ((int)threadIdx.x < G) chunk_valid[4 * G + threadIdx.x] = prefix;
-            if ((int)threadIdx.x == G - 1) s_over_total = prefix + mine;
-            if (saved_chunk_valid && (int)threadIdx.x < G) saved_chunk_valid[threadIdx.x] = chunk_valid[threadIdx.x];
-            if (saved_chunk_valid && (int)threadIdx.x < kRetainedParts) saved_chunk_valid[G + threadIdx.x] = 0;  // (the blend adds)
-            __syncthreads();
+            const int x = waves[w];
+            before += w < wave ? x : 0;
+            all += x;
         }
-        for (int o = 32; o > 0; o >>= 1)
+        return before;
+    };
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j) sum += v[j];
+    const int inc_tiles = wave_scan(sum), inc_over = wave_scan(over), inc_valid = wave_scan(valid);
+    const int wave_flags = (__ballot(flags & 1) ? 1 : 0) | (__ballot(flags & 2) ? 2 : 0);
+    if (lane == 63) s_tiles[wave] = inc_tiles, s_over[wave] = inc_over, s_valid[wave] = inc_valid, s_flag[wave] = wave_flags;
+    __syncthreads();
+    int total, total_over, total_valid, total_slices;
+    int first = wave_prefix(s_tiles, total) + inc_tiles - sum;  // first slot of the thread's first tile
+    // number of every chunk's first overflow row
+    const int first_over = wave_prefix(s_over, total_over) + inc_over - over;
+    if (chunk) chunk_valid[4 * G + threadIdx.x] = first_over;
+    if (saved_chunk_valid && chunk) saved_chunk_valid[threadIdx.x] = valid;
+    if (saved_chunk_valid && (int)threadIdx.x < kRetainedParts) saved_chunk_valid[G + threadIdx.x] = 0;  // (the blend adds)
+    // slices of the tiles' entries that fit the capacity
+    int sl[kPlanPer], slices = 0;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j)
+    {
+        sl[j] = 0;
+        if (j < per && t0 + j < NB)
         {
-            v += __shfl_xor(v, o);
-            st += __shfl_xor(st, o);
-            f |= __shfl_xor(f, o);
+            bin_start[t0 + j]    = first;
+            const long long last = min((long long)first + v[j], capacity);
+            const long long n    = max(last - (long long)first, 0ll);
+            sl[j]                = n > kSliceEntries ? (int)((n + kSliceEntries - 1) / kSliceEntries) : 0;
         }
-        if (lane == 0)
-        {
-            if (v) atomicAdd(&s_valid_total, v);
-            if (st) atomicAdd(&s_same_total, st);
-            if (f) atomicOr(&s_flags, f);
-        }
+        first += v[j];
+        slices += sl[j];
     }
-    for (int base = 0; base < NB; base += 1024)
+    const int inc_slices = wave_scan(slices);
+    if (lane == 63) s_slices[wave] = inc_slices;
+    __syncthreads();
+    int first_slice = wave_prefix(s_slices, total_slices) + inc_slices - slices;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j)
     {
-        const int idx = base + threadIdx.x;
-        const int v   = idx < NB ? bin_count[idx] : 0;
-        int inc       = v;
-        for (int o = 1; o < 64; o <<= 1)
-        {
-            int t = __shfl_up(inc, o);
-            if (lane >= o) inc += t;
-        }
-        if (lane == 63) s_wave[0][wave] = inc;
-        __syncthreads();
-        int wave_prefix = 0;
-        for (int w = 0; w < wave; ++w) wave_prefix += s_wave[0][w];
-        const int carry = s_carry[0];
-        const int ex    = carry + wave_prefix + inc - v;  // first slot of the tile
-        if (idx < NB) bin_start[idx] = ex;
-        // slices of the tile's entries that fit the capacity
-        int sl = 0;
-        if (idx < NB)
-        {
-            const long long first = ex;
-            long long last        = (long long)ex + v;
-            if (last > capacity) last = capacity;
-            const long long n = last > first ? last - first : 0;
-            sl                = n > kSliceEntries ? (int)((n + kSliceEntries - 1) / kSliceEntries) : 0;
-        }
-        int inc2 = sl;
-        for (int o = 1; o < 64; o <<= 1)
-        {
-            int t = __shfl_up(inc2, o);
-            if (lane >= o) inc2 += t;
-        }
-        if (lane == 63) s_wave[1][wave] = inc2;
-        __syncthreads();
-        int wave_prefix2 = 0;
-        for (int w = 0; w < wave; ++w) wave_prefix2 += s_wave[1][w];
-        const int carry2 = s_carry[1];
-        if (idx < NB) slice_start[idx] = carry2 + wave_prefix2 + inc2 - sl;
-        __syncthreads();
-        if (threadIdx.x == 1023)
-        {
-            s_carry[0] = carry + wave_prefix + inc;
-            s_carry[1] = carry2 + wave_prefix2 + inc2;
-        }
-        __syncthreads();
+        if (j < per && t0 + j < NB) slice_start[t0 + j] = first_slice;
+        first_slice += sl[j];
     }
     if (threadIdx.x == 0)
     {
-        bin_start[NB]   = s_carry[0];
-        slice_start[NB] = s_carry[1];
-        const unsigned long long bad = (unsigned long long)((s_flags >> 1) & 1);
-        header->n_valid      = s_valid_total;
-        header->n_entries    = (unsigned long long)(unsigned)s_carry[0];
-        header->overflow     = 0;
-        header->retained     = 0;
-        header->not_identity = (unsigned long long)(s_flags & 1);
-        header->bad_index    = 0;
-        header->same_tile_as_previous = s_same_total;
-        header->overflow_rows         = (unsigned long long)(unsigned)s_over_total;
+        wave_prefix(s_valid, total_valid);
+        int any_flags = 0;
+        for (int w = 0; w < 16; ++w) any_flags |= s_flag[w];
+        *long_count     = 0;
+        bin_start[NB]   = total;
+        slice_start[NB] = total_slices;
+        const unsigned long long bad = (unsigned long long)((any_flags >> 1) & 1);
+        header->n_valid       = (unsigned long long)(unsigned)total_valid;
+        header->n_entries     = (unsigned long long)(unsigned)total;
+        header->overflow      = 0;
+        header->retained      = 0;
+        header->not_identity  = (unsigned long long)(any_flags & 1);
+        header->bad_index     = 0;
+        header->overflow_rows = (unsigned long long)(unsigned)total_over;
         if (first_view)
         {
             status->n_valid = status->n_entries = status->overflow = status->retained = status->not_identity = 0;
             status->bad_index                                                       = bad;
-            status->same_tile_as_previous = status->overflow_rows = 0;
+            status->overflow_rows                                                   = 0;
         }
         else if (bad)
             status->bad_index = 1;  // (the views of a call run one after the other on the stream)
@@ -1508,11 +1492,9 @@ hipError_t launch_forward_view(const ForwardParams& p, int channels, bool train,
     {
         ProfScope ps(prof, "bin_scan", stream);
         hipLaunchKernelGGL(bin_column_scan_kernel, dim3((NB + kScanCols - 1) / kScanCols), dim3(256), 0, stream, p.bin_hist, p.bin_count, NB, G);
-        // counts and run are neighbours in the workspace: cleared together, by the workgroups behind the scanning one
-        const long long quads = 2ll * NB * kTilePixels / 4;
-        hipLaunchKernelGGL(scan_plan_kernel, dim3(1 + (unsigned)std::min<long long>((quads + 1023) / 1024, 1024)), dim3(1024), 0, stream,
-                           p.bin_count, p.bin_start, p.slice_start, NB, p.capacity, p.chunk_valid, G, p.header, p.status, first_view ? 1 : 0,
-                           p.long_count, reinterpret_cast<uint4*>(p.counts), quads, p.saved_chunk_valid);
+        hipLaunchKernelGGL(scan_plan_kernel, dim3(1 + std::min(NB, 255)), dim3(1024), 0, stream, p.bin_count, p.bin_start,
+                           p.slice_start, NB, p.capacity, p.chunk_valid, G, p.header, p.status, first_view ? 1 : 0, p.long_count,
+                           p.counts, p.run, p.saved_chunk_valid);
     }
     {
         ProfScope ps(prof, "bin_scatter", stream);

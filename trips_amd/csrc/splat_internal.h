@@ -233,10 +233,6 @@ struct ViewHeader
     unsigned long long retained;    // R: sum of the retained entries (filled by the counters query)
     unsigned long long not_identity;  // some point's descriptor column differs from its own index
     unsigned long long bad_index;   // some point's descriptor column lies outside [0, num_texels): the point was skipped
-    // valid points whose finest-layer tile is also that of the point before them in memory: near n_valid for a cloud
-    // stored along a space-filling curve, near zero for one in random order (the backward chooses its exchange layout
-    // by it)
-    unsigned long long same_tile_as_previous;
     // rows of the backward's overflow table that the view's points own: sum over the valid points of max(layers - 2, 0)
     unsigned long long overflow_rows;
 };

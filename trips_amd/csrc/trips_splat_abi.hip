@@ -244,7 +244,7 @@ WorkspaceLayout workspace_layout(const TripsSplatDesc& d, const PyramidGeom& g)
     o += align256(N * kPointRecordFloats * sizeof(float));
     w.counts = o;
     o += align256(P * sizeof(int32_t));
-    w.run = o;  // directly behind counts: one fill clears both
+    w.run = o;
     o += align256(P * sizeof(int32_t));
     w.cursor = o;
     o += align256(P * sizeof(int32_t));
