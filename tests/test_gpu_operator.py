@@ -250,3 +250,15 @@ def test_backward_refuses_inputs_modified_in_place_after_the_forward():
         ns.point_cloud_cuda.t_position.add_(0.0)
     with pytest.raises(RuntimeError, match="modified in place"):
         sum(o.sum() for o in outs).backward()
+
+
+def test_forward_mode_is_refused_without_a_graph_as_well():
+    import torch.autograd.forward_ad as fwad
+    from trips_amd.renderer import BlendPointCloud, NeuralScene
+    sc = scenes.tiny(n=200, w=32, h=24, f=30.0, num_layers=2, list_depth=16, seed=43)
+    ns = NeuralScene.from_arrays(sc)
+    info = _info(sc, ns, train=False)
+    with torch.no_grad(), fwad.dual_level():
+        ns.texture.texture = fwad.make_dual(ns.texture.texture, torch.ones_like(ns.texture.texture))
+        with pytest.raises(NotImplementedError):
+            BlendPointCloud(info)
