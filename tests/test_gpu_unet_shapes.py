@@ -56,3 +56,17 @@ def test_channels_last_pyramids_are_read_in_place(filters, w, h, cin, batch):
         got = net.forward([t.permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2) for t in inputs])
         mixed = net.forward([inputs[0], inputs[1].permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2)])
     assert torch.equal(got, want) and torch.equal(mixed, want)
+
+
+def test_upsampling_of_neighbours_far_apart():
+    """Images near the ends of fp16's range with changing signs: their bilinear mixes stay inside it, so the net's output
+    is the restatement's (a difference of two neighbours would not be: it is an infinity in fp16). Weights of 1e-4 keep
+    the convolutions' sums, up to 72 x 6e4 x 1e-4, in range as well; the bar is that of the other forward tests."""
+    net = _net([16, 32], 2, seed=80)
+    with torch.no_grad():
+        for m in net.modules():
+            if isinstance(m, torch.nn.Conv2d) and m.kernel_size == (3, 3):
+                m.weight.mul_(1e-4 / m.weight.abs().max())
+    g = torch.Generator().manual_seed(81)
+    inputs = [torch.sign(torch.rand(t.shape, generator=g) - 0.5) * (4e4 + 2e4 * t) for t in _pyramid(45, 37, 2, 4, batch=1, seed=82)]
+    _compare(net, inputs)

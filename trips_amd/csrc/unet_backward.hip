@@ -905,7 +905,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
                 const _Float16* src = s_below + (j * kBelowW + i) * ROW + 8 * g;
                 half8 v[4];
                 upsample_quad(*reinterpret_cast<const half8*>(src), *reinterpret_cast<const half8*>(src + ROW),
-                              *reinterpret_cast<const half8*>(src + kBelowW * ROW), *reinterpret_cast<const half8*>(src + (kBelowW + 1) * ROW), v);
+                              *reinterpret_cast<const half8*>(src + kBelowW * ROW), *reinterpret_cast<const half8*>(src + (kBelowW + 1) * ROW),
+                              y0 + j == 0, x0 + i == 0, v);
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
                 {

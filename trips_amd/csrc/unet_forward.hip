@@ -223,7 +223,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
                 const int j = quad / (kConvPatchW / 2), i = quad - j * (kConvPatchW / 2);
                 half8 v[4];
                 upsample_quad(__builtin_bit_cast(half8, r.q[k][0]), __builtin_bit_cast(half8, r.q[k][1]), __builtin_bit_cast(half8, r.q[k][2]),
-                              __builtin_bit_cast(half8, r.q[k][3]), v);
+                              __builtin_bit_cast(half8, r.q[k][3]), t.y0 + j == 0, t.x0 + i == 0, v);
 #pragma unroll
                 for (int n = 0; n < 4; ++n)
                 {
