@@ -76,27 +76,39 @@ struct PointProjection
     float d_softplus;  // softplus'(raw size), training mode
 };
 
-// What the projection reads of a point in point order (fetched one step ahead of its use).
+// What the projection kernel reads of a point (fetched one step ahead of its use; the descriptor column, which the
+// descriptor's loads need, two steps).
+template <int CPAD>
 struct PointInputs
 {
     int tex;  // descriptor column
     float4 pos;
-    float raw_size;
+    float raw_size, dropout;
+    float conf, d[CPAD];
 };
 
-__device__ __forceinline__ PointInputs load_point(const ForwardParams& p, int pid)
+template <int C, bool TRAIN, int CPAD>
+__device__ __forceinline__ void load_point(const ForwardParams& p, int pid, int tex, PointInputs<CPAD>& in)
 {
-    PointInputs in;
-    in.tex      = p.index[pid];
+    in.tex      = tex;
     in.pos      = p.position[pid];
     in.raw_size = p.point_size[pid];
-    return in;
+    in.dropout  = TRAIN && p.dropout ? p.dropout[pid] : 0.f;
+    in.conf     = 0.f;
+#pragma unroll
+    for (int c = 0; c < CPAD; ++c) in.d[c] = 0.f;
+    if ((unsigned)tex < (unsigned)p.num_texels)
+    {
+        in.conf = p.confidence[tex];
+#pragma unroll
+        for (int c = 0; c < C; ++c) in.d[c] = p.texture[(size_t)c * p.num_texels + tex];
+    }
 }
 
 // `s_hist`: LDS counters, one per tile; every layer the point is written to adds one to the tile of the footprint's
 // first pixel (px, py). (The footprint (px..px+1, py..py+1) lies inside the image because px < w-1 and py < h-1.)
-template <bool TRAIN>
-__device__ __forceinline__ PointProjection project_point(const ForwardParams& p, const Camera& cam, int pid, const PointInputs& in,
+template <bool TRAIN, int CPAD>
+__device__ __forceinline__ PointProjection project_point(const ForwardParams& p, const Camera& cam, int pid, const PointInputs<CPAD>& in,
                                                          int* s_hist, bool& not_identity, bool& bad_index)
 {
     PointProjection o;
@@ -120,12 +132,9 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
     }
     if (p.viewer_only && !skip)
     {
-        if (p.confidence[o.tex] < p.stability_cutoff_value) skip = true;
+        if (in.conf < p.stability_cutoff_value) skip = true;
     }
-    if (TRAIN && p.dropout)
-    {
-        if (p.dropout[pid] == 1.f) skip = true;
-    }
+    if (TRAIN && in.dropout == 1.f) skip = true;
     if (skip) return o;
     float4 pos = in.pos;
     if (p.displacement)
@@ -225,27 +234,24 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     int next       = begin;  // workgroup-uniform: compact number of the chunk's next valid point
     int next_pair  = 0;      // workgroup-uniform: overflow rows of the chunk's points so far
     int step       = 0;
-    // the loads of the next step's points are in flight while this step's are projected
-    PointInputs nxt;
-    nxt.tex = 0, nxt.pos = make_float4(0.f, 0.f, 0.f, 0.f), nxt.raw_size = 0.f;
-    if (begin + (int)threadIdx.x < end) nxt = load_point(p, begin + (int)threadIdx.x);
+    // The loads of the next step's points, their descriptors and dropout flags among them (whether a point is visible or
+    // not), are in flight while this step's are projected. (With the dropout flag and the descriptor requested in the
+    // step itself, its waits were a part of every step: 9M points with dropout 225 us, now 197; 6M without 152, now 150,
+    // which its vector instructions, 100 us, and the 520 MB that it moves, 105 us at a copy's rate, bound together.)
+    PointInputs<CPAD> nxt;
+    int next_tex = 0;  // descriptor column of the step after `nxt`'s
+    if (begin + (int)threadIdx.x < end)
+    {
+        const int tex = p.index[begin + (int)threadIdx.x];
+        if (begin + (int)threadIdx.x + kBinThreads < end) next_tex = p.index[begin + (int)threadIdx.x + kBinThreads];
+        load_point<C, TRAIN>(p, begin + (int)threadIdx.x, tex, nxt);
+    }
     for (int base = begin; base < end; base += kBinThreads, step ^= 1)
     {
-        const int pid        = base + threadIdx.x;
-        const PointInputs in = nxt;
-        if (pid + kBinThreads < end) nxt = load_point(p, pid + kBinThreads);
-        // the descriptor of the point is requested before it is known whether the point is visible: the loads then run
-        // beside the projection instead of after it
-        float conf = 0.f;
-        float d[CPAD];
-#pragma unroll
-        for (int c = 0; c < CPAD; ++c) d[c] = 0.f;
-        if (pid < end && (unsigned)in.tex < (unsigned)p.num_texels)
-        {
-            conf = p.confidence[in.tex];
-#pragma unroll
-            for (int c = 0; c < C; ++c) d[c] = p.texture[(size_t)c * p.num_texels + in.tex];
-        }
+        const int pid              = base + threadIdx.x;
+        const PointInputs<CPAD> in = nxt;
+        if (pid + kBinThreads < end) load_point<C, TRAIN>(p, pid + kBinThreads, next_tex, nxt);
+        if (pid + 2 * kBinThreads < end) next_tex = p.index[pid + 2 * kBinThreads];
         PointProjection o;
         o.valid  = false;
         o.layers = 0;
@@ -292,9 +298,9 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 
         // record for the blend (and the pixel pass of the backward)
         float4 recv[NREC];
-        recv[0] = make_float4(o.ipx, o.ipy, encode_size_field(o.size_px, L), conf);
+        recv[0] = make_float4(o.ipx, o.ipy, encode_size_field(o.size_px, L), in.conf);
 #pragma unroll
-        for (int q = 0; q < CPAD / 4; ++q) recv[1 + q] = make_float4(d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]);
+        for (int q = 0; q < CPAD / 4; ++q) recv[1 + q] = make_float4(in.d[4 * q], in.d[4 * q + 1], in.d[4 * q + 2], in.d[4 * q + 3]);
         float4* rec = reinterpret_cast<float4*>(p.rec + (size_t)cid * p.rec_floats);
 #pragma unroll
         for (int q = 0; q < NREC; ++q) __builtin_nontemporal_store(vf4{recv[q].x, recv[q].y, recv[q].z, recv[q].w}, reinterpret_cast<vf4*>(rec) + q);
