@@ -22,6 +22,14 @@ pytestmark = pytest.mark.gpu
     ([32, 24], 544, 272, 4, 1),     # enough tiles for two pairs per workgroup at both levels
     ([48, 64], 544, 272, 4, 1),     # ... at the coarser level only (the finest has three pairs)
     ([64, 64], 544, 136, 6, 2),     # ... at the finest, where the pairs are split over workgroups
+    # the data gradient's strips, of 15 coarser columns and 4 n - 1 coarser rows:
+    ([16, 32], 30, 6, 4, 1),        # one strip, filled exactly
+    ([32, 32], 31, 7, 3, 2),        # a column and a row more, odd sizes, outputs that start at position 6
+    ([16, 48], 60, 14, 6, 1),       # two strips; 64 inputs
+    ([32, 48], 29, 5, 16, 1),       # sixteen image channels
+    ([16, 32], 302, 166, 4, 4),     # strips of several steps, two workgroups per CU, the last strip a short one
+    ([32, 32], 301, 203, 8, 3),     # ... one workgroup per CU, odd sizes
+    ([16, 48], 301, 95, 2, 5),
 ])
 def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
     from tests.ref_unet import unet_forward

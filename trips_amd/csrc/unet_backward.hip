@@ -6,6 +6,7 @@
 //                             the gradient of the finest block's pre-activations; its weight and bias gradients
 //   conv_bwd_data_kernel      gradient of a block's input: the forward's implicit GEMM with flipped, transposed
 //                             weights (M = 256 pixels, N = input channels, K = 9 taps x pre-activations)
+//   conv_bwd_data_up_kernel   these two in one, for blocks of few enough channels
 //   up2_adjoint_gate_kernel   adjoint of the bilinear 2x upsampling (a gather over <= 4 x 4 finer pixels), then
 //                             dL/d in[i+1] and the gate of the coarser block
 //   conv_bwd_weight_kernel    weight gradients: GEMM with the pixels as the reduction dimension. Both operands are
@@ -566,6 +567,336 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// conv_bwd_data_kernel and up2_adjoint_gate_kernel in one, for blocks with a level below: the gradient of the block's
+// input, 2 to 4 bytes written and read again per byte of result, never leaves the chip.
+//
+// A workgroup walks down a strip of 15 columns of the coarser level, eight rows of the finer one at a time. Per step: the
+// data gradient of 8 x 32 pixels (30 columns of its own and one at each side, which the neighbour works out too) goes
+// into a ring of ten rows in LDS, rounded to fp16 as it was in memory; four rows of the coarser level then gather their
+// 4 x 4 finer pixels from it, in the order of up2_adjoint_gate_kernel, and leave gated. The patch of pre-activation
+// gradients is a ring of ten rows too, and the eight rows of the next step travel in registers during the products.
+// A wavefront owns 4 x 16 pixels and half of the outputs and keeps the weights of those in registers for the whole strip:
+// an operand read from the patch then serves up to three taps, and the sums run in the order of conv_taps_mfma.
+//
+// Bound by the steps' latencies (two barriers each) at one or two workgroups per CU, no longer by memory. 1920 x 1080,
+// 32 pre-activations x 32 inputs: 90 + 85 us as two kernels, 125 us as one; 1245 x 825 and the levels below it, 64 x 32: 119 + 60
+// us, 164 us. 64 x 64 stays as two (960 x 540: 54 + 22 us against 83 us: its weights take 144 registers of a lane, and
+// nothing is left to hide the loads with). The gather as matrix products from a ring with the pixels innermost took
+// 358 us where this takes 164.
+struct BwdDataUpParams
+{
+    BwdDataParams fine;   // d_in is not used
+    UpAdjointParams up;   // d_in, first_image are not used
+    int steps;            // of a workgroup: 8 * steps rows of the finer level, of which it owns 8 * steps - 2
+};
+// The weights with which rows (columns) 2 v - 1 .. 2 v + 2 of the finer level read row v of the coarser one: up2_weight for
+// all four, 0 only for rows outside the image.
+__device__ __forceinline__ void up2_adjoint_weights(int v, int fine_size, int coarse_size, float (&w)[4])
+{
+    w[0] = v > 0 ? 0.25f : 0.f;
+    w[1] = v > 0 ? 0.75f : 1.f;
+    w[2] = 2 * v + 1 >= fine_size ? 0.f : v + 1 < coarse_size ? 0.75f : 1.f;
+    w[3] = v + 1 < coarse_size ? 0.25f : 0.f;
+}
+constexpr int kStripFine   = kConvTileW - 2;  // columns of the finer level that a strip owns
+constexpr int kStripCoarse = kStripFine / 2;
+constexpr int kRingRows    = kConvTileH + 2;
+constexpr int strip_lds_bytes(int kc, int nn, int ci)
+{
+    return kConvPatchH * kConvPatchW * (kc + kLdsChanPad) * 2 + kRingRows * kConvTileW * (nn + kLdsChanPad) * 2 + kConvTileH * kConvTileW * ci * 4;
+}
+// Workgroups of a CU: two where LDS and registers (the weights take 36 (kc / 32) (nn / 32) of a lane) hold them.
+constexpr int strip_resident(int kc, int nn, int ci) { return 2 * strip_lds_bytes(kc, nn, ci) <= 160 * 1024 && kc * nn <= 32 * 32 ? 2 : 1; }
+
+// ALIGNED: 2 C is a multiple of 8, so that a group of eight block outputs is one aligned read (both forms in one kernel
+// took 40 registers more).
+template <int KC, int NN, int CI, bool ALIGNED>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_resident(KC, NN, CI)))) void conv_bwd_data_up_kernel(BwdDataUpParams q)
+{
+    constexpr int THREADS = 512;
+    constexpr int ROW = KC + kLdsChanPad, OS = NN + kLdsChanPad;
+    constexpr int GROUPS = KC / 8, KB = KC / 32, NBW = NN / 32;
+    constexpr int kPixels = kConvTileH * kConvTileW;
+    const int H = q.fine.H, W = q.fine.W, C = q.fine.c_feat, Hb = q.up.Hb, Wb = q.up.Wb, npad_b = q.up.npad;
+    const size_t image  = (size_t)q.fine.first_image + blockIdx.z;
+    const size_t plane  = (size_t)H * W, plane_b = (size_t)Hb * Wb;
+    const _Float16* dpre  = q.fine.dpre + image * plane * KC;
+    float* d_feat         = q.fine.d_feat + image * plane * C;
+    const _Float16* pre_b = q.up.pre + image * plane_b * npad_b;
+    _Float16* dpre_b      = q.up.dpre + image * plane_b * npad_b;
+    float* d_feat_b       = q.up.d_feat + image * plane_b * C;
+    const float scale_inv = q.fine.scale_inv;
+
+    extern __shared__ _Float16 smem[];
+    _Float16* s_patch = smem;                                       // [10 rows][34][ROW]
+    _Float16* s_ring  = s_patch + kConvPatchH * kConvPatchW * ROW;  // [10 rows][32][OS]
+    float* s_img      = reinterpret_cast<float*>(s_ring + kRingRows * kConvTileW * OS);  // [CI][8 x 32]
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lrow = lane & 15, lk = (lane >> 4) * 8;
+    const int wr = (wave & 1) * 4, wc = ((wave >> 1) & 1) * 16, wn = (wave >> 2) * NBW;  // this wavefront's rows, columns, output blocks
+    const int rows_own = 4 * q.steps - 1;                      // rows of the coarser level
+    const int Y0 = blockIdx.y * rows_own, Y1 = min(Y0 + rows_own, Hb);
+    const int yf = 2 * Y0 - 1, xf = blockIdx.x * kStripFine - 1;  // the strip's first computed pixel
+    const int steps = (2 * (Y1 - Y0) + 2 + kConvTileH - 1) / kConvTileH;
+
+    half8 b[9][KB][NBW];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+                b[tap][kb][n] = *reinterpret_cast<const half8*>(q.fine.wt + ((size_t)tap * NN + (wn + n) * 16 + lrow) * KC + kb * 32 + lk);
+
+    // This thread's number, worked out anew where it is called: what follows from it (positions, LDS addresses, weights of
+    // the upsampling) would otherwise be kept in registers over the whole strip, beside the convolution's weights.
+    auto thread = [&]()
+    {
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        return t;
+    };
+    // A row of the patch per wavefront, 16 bytes of a lane at a time; rows are those of the finer level from yf - 1 on.
+    // (Unconditional loads, at positions clamped into the image: a load under a condition is waited for where the condition
+    // ends.)
+    constexpr int kRowItems = kConvPatchW * GROUPS;
+    constexpr int kNext     = (kRowItems + 63) / 64;
+    uint4 next[kNext];
+    auto fetch_row = [&](int row)
+    {
+        const int tl = thread() & 63;
+        const _Float16* src = dpre + (size_t)min(max(yf - 1 + row, 0), H - 1) * W * KC;
+#pragma unroll
+        for (int j = 0; j < kNext; ++j)
+        {
+            const int x = min(max(xf - 1 + (tl + 64 * j) / GROUPS, 0), W - 1);
+            next[j]     = *reinterpret_cast<const uint4*>(src + x * KC + 8 * (tl % GROUPS));
+        }
+    };
+    auto put_row = [&](int row, int slot)
+    {
+        const int tl = thread() & 63;
+        const int y  = yf - 1 + row;
+        _Float16* dst = s_patch + (slot * kConvPatchW + tl / GROUPS) * ROW + 8 * (tl % GROUPS);
+#pragma unroll
+        for (int j = 0; j < kNext; ++j)
+        {
+            const int px = (tl + 64 * j) / GROUPS, x = xf - 1 + px;
+            const bool in = y >= 0 && y < H && x >= 0 && x < W;
+            const uint4 v = make_uint4(in ? next[j].x : 0u, in ? next[j].y : 0u, in ? next[j].z : 0u, in ? next[j].w : 0u);
+            if (kRowItems % 64 == 0 || px < kConvPatchW) *reinterpret_cast<uint4*>(dst + j * (64 / GROUPS) * ROW) = v;
+        }
+    };
+    if (wave < 2)
+    {
+        fetch_row(wave);
+        put_row(wave, wave);
+    }
+    fetch_row(wave + 2);
+    put_row(wave + 2, wave + 2);
+
+    // the items of the adjoint: a pixel of the coarser level and eight positions (see up2_adjoint_gate_kernel)
+    const int g0 = C / 8, ig = (2 * C - 1) / 8 - g0 + 1;
+    const int groups = ig + npad_b / 16;
+    const int items  = 4 * kStripCoarse * groups;
+    struct Item
+    {
+        int q, c, cx;
+    };
+    auto item_of = [&](int item)
+    {
+        const int bp = item / groups;
+        return Item{item - bp * groups, bp / kStripCoarse, bp % kStripCoarse};
+    };
+    auto load_pre = [&](const Item& it, int Yk, half8& lo, half8& hi)
+    {
+        const int Y = min(max(Yk + it.c, 0), Hb - 1), X = min((int)blockIdx.x * kStripCoarse + it.cx, Wb - 1);
+        const _Float16* src = pre_b + ((size_t)Y * Wb + X) * npad_b + 16 * max(it.q - ig, 0);
+        lo = *reinterpret_cast<const half8*>(src);
+        hi = *reinterpret_cast<const half8*>(src + 8);
+    };
+    const Item first_item = item_of(threadIdx.x);
+    const int packed      = first_item.q | first_item.c << 8 | first_item.cx << 16;
+    auto mine             = [&]()
+    {
+        int t = packed;
+        asm volatile("" : "+v"(t));
+        return Item{t & 255, t >> 8 & 255, t >> 16};
+    };
+    __syncthreads();
+
+    int slot = 0;  // of the step's first row, in both rings
+    for (int k = 0; k < steps; ++k)
+    {
+        const int yk = yf + kConvTileH * k;  // the step's first row of the finer level
+        const int Yk = Y0 - 1 + 4 * k;       // ... and of the coarser one (k = 0: the strip above owns that row)
+        const bool more = k + 1 < steps;
+        // in flight during the products: the next step's rows
+        if (more) fetch_row(kConvTileH * (k + 1) + 2 + wave);
+        half8 lo, hi;
+        float old[kPixels * CI / THREADS];
+        auto load_rest = [&]()
+        {
+            load_pre(mine(), Yk, lo, hi);
+            const int tid_load = thread();
+#pragma unroll
+            for (int j = 0; j < kPixels * CI / THREADS; ++j)
+            {
+                const int v = tid_load + THREADS * j, px = v % kPixels;
+                const int y = min(max(yk + px / kConvTileW, 0), H - 1), x = min(max(xf + px % kConvTileW, 0), W - 1);
+                old[j] = d_feat[min(v / kPixels, C - 1) * plane + (size_t)y * W + x];
+            }
+        };
+        // (before the products where there are registers for it: nothing else hides this latency with one workgroup per CU)
+        constexpr bool kEarly = strip_resident(KC, NN, CI) == 1;
+        if (kEarly) load_rest();
+        floatx4 acc[4][NBW];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+        // step t: column dx = t % 3 of patch row pr = t / 3; its operands are requested two steps ahead (and no further:
+        // the registers would not do)
+        half8 a3[3][KB];
+        auto operands = [&](int t)
+        {
+            const int pr  = t / 3, dx = t - 3 * pr;
+            const int at  = slot + wr + pr < kConvPatchH ? slot + wr + pr : slot + wr + pr - kConvPatchH;
+            const _Float16* src = s_patch + (at * kConvPatchW + wc + lrow + dx) * ROW + lk;
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) a3[t % 3][kb] = *reinterpret_cast<const half8*>(src + kb * 32);
+        };
+        operands(0);
+        operands(1);
+#pragma unroll
+        for (int t = 0; t < 18; ++t)
+        {
+            const int pr = t / 3, dx = t - 3 * pr;
+            if (t + 2 < 18) operands(t + 2);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy)
+                    if (pr - dy >= 0 && pr - dy < 4)
+#pragma unroll
+                        for (int n = 0; n < NBW; ++n)
+                            acc[pr - dy][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy * 3 + dx][kb][n], a3[t % 3][kb], acc[pr - dy][n], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!kEarly)
+        {
+            __builtin_amdgcn_sched_barrier(0);  // (not before the products: their registers are all taken)
+            load_rest();
+        }
+        // a lane: outputs 16 n + 4 (lane / 16) .. + 3 of the pixel in column lane % 16
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const int at = slot + wr + r < kRingRows ? slot + wr + r : slot + wr + r - kRingRows;
+            const int y = yk + wr + r, x = xf + wc + lrow;
+            const bool in = y >= 0 && y < H && x >= 0 && x < W;
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+            {
+                const int c0 = (wn + n) * 16 + (lane >> 4) * 4;
+                if (!in) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+                *reinterpret_cast<half4*>(s_ring + (at * kConvTileW + wc + lrow) * OS + c0) =
+                    half4{_Float16(acc[r][n][0]), _Float16(acc[r][n][1]), _Float16(acc[r][n][2]), _Float16(acc[r][n][3])};
+                if (n == 0 && c0 < CI)
+                {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s_img[(c0 + i) * kPixels + (wr + r) * kConvTileW + wc + lrow] = acc[r][0][i];
+                }
+            }
+        }
+        __syncthreads();  // the step's rows are in the ring; nobody reads the patch any more
+        if (more) put_row(kConvTileH * (k + 1) + 2 + wave, slot + wave < kConvPatchH ? slot + wave : slot + wave - kConvPatchH);  // (rows 2 .. 9 of the next step: the slots of rows 0 .. 7 of this one)
+
+        // the finer level's own image
+        const int tid_store = thread();
+#pragma unroll
+        for (int j = 0; j < kPixels * CI / THREADS; ++j)
+        {
+            const int v = tid_store + THREADS * j, px = v % kPixels, c = v / kPixels;
+            const int y = yk + px / kConvTileW, col = px % kConvTileW, x = xf + col;
+            if (c < C && y >= 2 * Y0 && y < min(2 * Y1, H) && col >= 1 && col <= kStripFine && x < W)
+                d_feat[c * plane + (size_t)y * W + x] = old[j] + s_img[v] * scale_inv;
+        }
+
+        for (int item = threadIdx.x; item < items; item += THREADS)
+        {
+            const Item it = item < THREADS ? mine() : item_of(item);
+            const int Y = Yk + it.c, X = (int)blockIdx.x * kStripCoarse + it.cx;
+            if (Y < Y0 || Y >= Y1 || X >= Wb) continue;
+            if (item >= THREADS) load_pre(it, Yk, lo, hi);
+            const int ch0 = 8 * (it.q - ig);
+            const int pos = it.q < ig ? 8 * (g0 + it.q) : 2 * C + ch0;  // first of the eight positions
+            float wy[4], wx[4], a[8];
+            up2_adjoint_weights(Y, H, Hb, wy);
+            up2_adjoint_weights(X, W, Wb, wx);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[i] = 0.f;
+            if (pos < NN)  // (a row ends with eight unused halves: the last group may reach into them, past the block's outputs)
+            {
+#pragma unroll
+                for (int ky = 0; ky < 4; ++ky)
+                {
+                    // rows 2 c - 2 + ky of the step, those before it from the step before
+                    int at = slot + 8 + 2 * it.c + ky;
+                    at -= at >= 2 * kRingRows ? 2 * kRingRows : at >= kRingRows ? kRingRows : 0;
+                    const _Float16* src = s_ring + (at * kConvTileW + 2 * it.cx) * OS + pos;
+                    __builtin_amdgcn_sched_barrier(0);  // one row's reads at a time: sixteen in flight cost 64 registers
+#pragma unroll
+                    for (int kx = 0; kx < 4; ++kx)
+                    {
+                        half8 v;
+                        if (ALIGNED)
+                            v = *reinterpret_cast<const half8*>(src + kx * OS);
+                        else
+                        {
+                            // (2 C is even: words of four bytes)
+                            const unsigned* w4 = reinterpret_cast<const unsigned*>(src + kx * OS);
+                            v = __builtin_bit_cast(half8, make_uint4(w4[0], w4[1], w4[2], w4[3]));
+                        }
+                        const float w = wy[ky] * wx[kx];  // (0 for pixels outside the image only: the ring holds zeros there)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) a[i] = __builtin_fmaf(w, float(v[i]), a[i]);
+                    }
+                }
+            }
+            const size_t bp = (size_t)Y * Wb + X;
+            if (it.q < ig)
+            {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                {
+                    const int c = pos + i - C;
+                    if (c >= 0 && c < C) d_feat_b[(size_t)c * plane_b + bp] = a[i] * scale_inv;
+                }
+            }
+            else
+            {
+                half8 of, om;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                {
+                    float df, dm;
+                    gate_backward(ch0 + i < q.up.cout ? a[i] : 0.f, float(i < 4 ? lo[i & 3] : hi[i & 3]), float(i < 4 ? lo[4 + (i & 3)] : hi[4 + (i & 3)]), df, dm);
+                    of[i] = _Float16(df);
+                    om[i] = _Float16(dm);
+                }
+                _Float16* dp = dpre_b + bp * npad_b + 2 * ch0;
+                *reinterpret_cast<half8*>(dp)     = half8{of[0], of[1], of[2], of[3], om[0], om[1], om[2], om[3]};
+                *reinterpret_cast<half8*>(dp + 8) = half8{of[4], of[5], of[6], of[7], om[4], om[5], om[6], om[7]};
+            }
+        }
+        slot = slot + kConvTileH < kRingRows ? slot + kConvTileH : slot + kConvTileH - kRingRows;
+        __syncthreads();  // the next step's patch is in place; nobody reads the ring any more
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------
 struct BiasGradParams
 {
     size_t pixels;
@@ -1114,6 +1445,50 @@ hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int ci
     return hipErrorInvalidValue;
 }
 
+template <int KC, int NN, int CI, bool ALIGNED>
+hipError_t launch_bwd_data_up(const BwdDataUpParams& p, int batch, hipStream_t stream)
+{
+    constexpr int lds = strip_lds_bytes(KC, NN, CI);
+    static_assert(lds <= 160 * 1024, "the rings do not fit");
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_data_up_kernel<KC, NN, CI, ALIGNED>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+    const int strips = (p.up.Wb + kStripCoarse - 1) / kStripCoarse;
+    for (int b = 0; b < batch; b += kMaxGridImages)
+    {
+        BwdDataUpParams q      = p;
+        q.fine.first_image     = b;
+        const int images       = std::min(batch - b, kMaxGridImages);
+        // the shortest strips whose workgroups are all resident at once (a step more costs each a row that it shares with
+        // the strip above; a second round of workgroups costs a whole strip)
+        const long long resident = 256 * strip_resident(KC, NN, CI);
+        const int most           = (p.up.Hb + 1 + 3) / 4;  // steps of a strip of the whole height
+        auto segments            = [&](int steps) { return (p.up.Hb + 4 * steps - 2) / (4 * steps - 1); };
+        q.steps                  = 1;
+        while (q.steps < most && (long long)strips * images * segments(q.steps) > resident) ++q.steps;
+        hipLaunchKernelGGL((conv_bwd_data_up_kernel<KC, NN, CI, ALIGNED>), dim3(strips, segments(q.steps), images), dim3(512), lds, stream, q);
+    }
+    return hipGetLastError();
+}
+
+hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, int cin_pad, hipStream_t stream)
+{
+    const bool aligned = p.fine.c_feat % 4 == 0;
+#define TRIPS_BDU_CI(KC_, NN_, CI_) \
+    return aligned ? launch_bwd_data_up<KC_, NN_, CI_, true>(p, batch, stream) : launch_bwd_data_up<KC_, NN_, CI_, false>(p, batch, stream)
+#define TRIPS_BDU(KC_, NN_)                                     \
+    if (npad == KC_ && cin_pad == NN_)                          \
+    {                                                           \
+        if (p.fine.c_feat <= 4) TRIPS_BDU_CI(KC_, NN_, 4);      \
+        if (p.fine.c_feat <= 8) TRIPS_BDU_CI(KC_, NN_, 8);      \
+        TRIPS_BDU_CI(KC_, NN_, 16);                             \
+    }
+    TRIPS_BDU(32, 32) TRIPS_BDU(64, 32) TRIPS_BDU(32, 64)
+#undef TRIPS_BDU
+#undef TRIPS_BDU_CI
+    return hipErrorInvalidValue;
+}
+
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
 hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, hipStream_t stream)
 {
@@ -1352,8 +1727,12 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             dp.wt        = reinterpret_cast<const _Float16*>(ws + lv.wt_off);
             dp.d_feat    = grads->inputs[i];
             dp.d_in      = below ? din_ptr(i) : nullptr;
-            hipError_t e = dispatch_bwd_data(dp, d.batch, lv.npad, lv.cin_pad, stream);
-            if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
+            const bool fused = bwd_data_up_fits(lv.npad, lv.cin_pad, below);
+            if (!fused)
+            {
+                hipError_t e = dispatch_bwd_data(dp, d.batch, lv.npad, lv.cin_pad, stream);
+                if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
+            }
             if (below)
             {
                 const LevelPlan& lb = np.lv[i + 1];
@@ -1368,8 +1747,16 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
                 up.pre       = pre_ptr(i + 1);
                 up.d_feat    = grads->inputs[i + 1];
                 up.dpre      = dpre_ptr(i + 1);
+                if (fused)
+                {
+                    BwdDataUpParams du;
+                    du.fine      = dp;
+                    du.up        = up;
+                    hipError_t e = dispatch_bwd_data_up(du, d.batch, lv.npad, lv.cin_pad, stream);
+                    if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
+                }
                 const size_t items = (size_t)lb.H * lb.W * ((2 * C - 1) / 8 - C / 8 + 1 + lb.npad / 16);
-                for (up.first_image = 0; up.first_image < d.batch; up.first_image += kMaxGridImages)
+                for (up.first_image = fused ? d.batch : 0; up.first_image < d.batch; up.first_image += kMaxGridImages)
                 {
                     const dim3 blocks((unsigned)std::min<size_t>((items + 255) / 256, 1u << 20), std::min(d.batch - up.first_image, kMaxGridImages));
                     switch ((2 * C) & 7)

@@ -269,12 +269,17 @@ struct LevelPlan
     // bytes into the backward workspace
     size_t wt_off;      // packed transposed weights [9][cin_pad][npad] fp16
     size_t dpre_off;    // gradient of the pre-activations [B][H][W][npad] fp16
-    size_t din_off;     // gradient of the block input [B][H][W][cin_pad] fp16
+    size_t din_off;     // gradient of the block input [B][H][W][cin_pad] fp16, where it leaves its kernel
     size_t part_off;    // partial weight gradients [groups][9][npad][cin_pad] fp32
     size_t sliced_off;  // partial sums of the partials [16][9][npad][cin_pad] fp32
     size_t bias_part_off;  // per-workgroup sums of the pre-activation gradients [groups][npad] fp32
     int groups;         // persistent workgroups of the weight-gradient kernel, for all images of the batch
 };
+
+// Whether the data gradient of a block and the adjoint of the upsampling below it run as one kernel
+// (conv_bwd_data_up_kernel): where there is a level below and the weights of a wavefront's outputs leave it registers to
+// work with (64 x 32: 164 us instead of 179; 64 x 64: 83 us instead of 76).
+inline bool bwd_data_up_fits(int npad, int cin_pad, bool below) { return below && npad <= 64 && npad * cin_pad <= 64 * 32; }
 
 struct NetPlan
 {
@@ -370,7 +375,7 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         lv.dpre_off = bw;
         bw += align256(pixels * lv.npad * sizeof(_Float16));
         lv.din_off = bw;
-        bw += align256(pixels * lv.cin_pad * sizeof(_Float16));
+        if (i < L - 1 && !bwd_data_up_fits(lv.npad, lv.cin_pad, true)) bw += align256(pixels * lv.cin_pad * sizeof(_Float16));
         const long long tiles = (long long)d.batch * ((lv.W + kConvTileW - 1) / kConvTileW) * ((lv.H + kConvTileH - 1) / kConvTileH);
         // persistent workgroups of the weight-gradient kernel: as many as are resident at once (two per CU for the
         // smallest shape, else one; those that share the pre-activations of a tile between them count together); every
