@@ -30,6 +30,7 @@ pytestmark = pytest.mark.gpu
     ([16, 32], 302, 166, 4, 4),     # strips of several steps, two workgroups per CU, the last strip a short one
     ([32, 32], 301, 203, 8, 3),     # ... one workgroup per CU, odd sizes
     ([16, 48], 301, 95, 2, 5),
+    ([32, 48], 290, 131, 4, 3),     # 64 pre-activations x 64 inputs
 ])
 def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
     from tests.ref_unet import unet_forward

@@ -578,11 +578,10 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
 // A wavefront owns 4 x 16 pixels and half of the outputs and keeps the weights of those in registers for the whole strip:
 // an operand read from the patch then serves up to three taps, and the sums run in the order of conv_taps_mfma.
 //
-// Bound by the steps' latencies (two barriers each) at one or two workgroups per CU, no longer by memory. 1920 x 1080,
-// 32 pre-activations x 32 inputs: 90 + 85 us as two kernels, 125 us as one; 1245 x 825 and the levels below it, 64 x 32: 119 + 60
-// us, 164 us. 64 x 64 stays as two (960 x 540: 54 + 22 us against 83 us: its weights take 144 registers of a lane, and
-// nothing is left to hide the loads with). The gather as matrix products from a ring with the pixels innermost took
-// 358 us where this takes 164.
+// Bound by the steps' latencies (two barriers each) at one or two workgroups per CU, no longer by memory. As two kernels
+// and as one: 1920 x 1080, 32 pre-activations x 32 inputs: 90 + 68 and 125 us; 960 x 540, 64 x 64: 54 + 36 and 83 us;
+// 1245 x 825 and the levels below it, 64 x 32: 119 + 60 and 164 us. The gather as matrix products from a ring with the
+// pixels innermost took 358 us where this takes 164.
 struct BwdDataUpParams
 {
     BwdDataParams fine;   // d_in is not used
@@ -749,7 +748,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
             }
         };
         // (before the products where there are registers for it: nothing else hides this latency with one workgroup per CU)
-        constexpr bool kEarly = strip_resident(KC, NN, CI) == 1;
+        constexpr bool kEarly = strip_resident(KC, NN, CI) == 1 && KC * NN <= 64 * 32;
         if (kEarly) load_rest();
         floatx4 acc[4][NBW];
 #pragma unroll
@@ -1483,7 +1482,7 @@ hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, i
         if (p.fine.c_feat <= 8) TRIPS_BDU_CI(KC_, NN_, 8);      \
         TRIPS_BDU_CI(KC_, NN_, 16);                             \
     }
-    TRIPS_BDU(32, 32) TRIPS_BDU(64, 32) TRIPS_BDU(32, 64)
+    TRIPS_BDU(32, 32) TRIPS_BDU(64, 32) TRIPS_BDU(32, 64) TRIPS_BDU(64, 64)
 #undef TRIPS_BDU
 #undef TRIPS_BDU_CI
     return hipErrorInvalidValue;

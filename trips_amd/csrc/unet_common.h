@@ -277,9 +277,9 @@ struct LevelPlan
 };
 
 // Whether the data gradient of a block and the adjoint of the upsampling below it run as one kernel
-// (conv_bwd_data_up_kernel): where there is a level below and the weights of a wavefront's outputs leave it registers to
-// work with (64 x 32: 164 us instead of 179; 64 x 64: 83 us instead of 76).
-inline bool bwd_data_up_fits(int npad, int cin_pad, bool below) { return below && npad <= 64 && npad * cin_pad <= 64 * 32; }
+// (conv_bwd_data_up_kernel): where there is a level below and the weights of a wavefront's outputs fit its registers
+// (64 x 64 takes 144 of a lane's 256; 96 would take 216).
+inline bool bwd_data_up_fits(int npad, int cin_pad, bool below) { return below && npad <= 64 && cin_pad <= 64; }
 
 struct NetPlan
 {
