@@ -31,18 +31,18 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "d9c026c0d3e07d77b1959417be03cf789c9f51952ba1a1782b13b9803885a19b"
+PMC_SOURCES_SHA256 = "9ce256d47d0461803c4a2d1dff7e97db55acd3262ae72a0e5edf88d805124ed1"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129117, 244115),
-    "bin_scatter": (96028, 166743),
-    "tile_count": (13152, 2296),
-    "tile_scatter": (26691, 108508),
-    "cell_sort": (35350, 42126),
-    "blend": (317781, 195746),
-    "backward_prologue": (55, 265170),
-    "backward_tiles": (426000, 121572),
-    "backward_points": (297376, 234503),
-    "adam_fused": (383789, 498420),
+    "project_bin": (129115, 237081),
+    "bin_scatter": (95997, 167514),
+    "tile_count": (13148, 2296),
+    "tile_scatter": (26680, 105764),
+    "cell_sort": (35343, 42137),
+    "blend": (317900, 195584),
+    "backward_prologue": (55, 265128),
+    "backward_tiles": (425427, 121570),
+    "backward_points": (297409, 234503),
+    "adam_fused": (383788, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
                         "splat_internal.h", "trips_math.h", "row16.h")
