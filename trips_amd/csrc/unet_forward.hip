@@ -120,8 +120,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
     }
     const float4 bias_f = *reinterpret_cast<const float4*>(p.bias + gp * 32 + lq * 4);
     const float4 bias_m = *reinterpret_cast<const float4*>(p.bias + gp * 32 + 16 + lq * 4);
-    // A operand of the 1x1: rows 4 m + o of block m's product hold output o, so that the products of a strip's MB rows
-    // add up in one accumulator whose lane group m holds the outputs of row m
+    // A operand of the 1x1: every lane group's rows hold the four outputs, of which group m keeps those of the strip's row m
+    // (the same number of selects as zero weights for the other rows, through which an infinite operand of one row would
+    // make all of them not a number)
     half4 fw = half4{}, fimg = half4{};
     if (p.final_out)
     {
@@ -361,9 +362,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
             if (p.final_out)
             {
                 const half4 im  = *reinterpret_cast<const half4*>(mine + (CI == 4 ? 0 : lq * 4));
-                const half4 sel = (lrow >> 2) == m ? fw : half4{}, sim = (lrow >> 2) == m ? fimg : half4{};
-                fin             = __builtin_amdgcn_mfma_f32_16x16x16f16(sel, o, fin, 0, 0, 0);
-                if (pair == 0) fin = __builtin_amdgcn_mfma_f32_16x16x16f16(sim, im, fin, 0, 0, 0);
+                floatx4 row     = __builtin_amdgcn_mfma_f32_16x16x16f16(fw, o, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                if (pair == 0) row = __builtin_amdgcn_mfma_f32_16x16x16f16(fimg, im, row, 0, 0, 0);
+                fin = lq == m ? row : fin;
             }
         }
         if (p.final_out)
