@@ -49,3 +49,30 @@ def test_an_output_past_the_range_stays_at_its_pixel(filters, cin):
     for (b, y, x) in ((0, 5, 20), (1, 18, 41), (1, 31, 66)):
         inputs[0][b, 0, y, x] = 5e4
     _held_to_restatement(net, inputs, 3 * 3)
+
+
+def _gates_that_take_infinities(net):
+    """Every sum of an infinite channel 0 is -inf in the features (elu: -1) and +inf in the masks (sigmoid: 1)."""
+    with torch.no_grad():
+        for i in range(net.params.num_layers):
+            b, C = net.block(i), net.params.num_input_channels
+            for c in (0, C) if i < net.params.num_layers - 1 else (0,):
+                b.feature_conv.weight[:, c] = -b.feature_conv.weight[:, c].abs() - 1e-3
+                b.mask_conv.weight[:, c] = b.mask_conv.weight[:, c].abs() + 1e-3
+
+
+@pytest.mark.parametrize("level,filters,cin", [
+    (0, [16, 32], 4), (0, [32, 32], 4), (0, [16, 48], 4), (0, [16, 32], 3), (0, [32, 48], 8), (0, [48, 64], 4),
+    # the coarser level's rows end with positions that no output has: 12 outputs behind 8 positions of image
+    (1, [16, 20], 4), (1, [16, 40], 4), (1, [48, 28], 4),
+])
+def test_padding_channels_take_no_part(level, filters, cin):
+    """An infinite image channel that the gates turn into finite outputs: of the padding channels, whose weights are zero,
+    nothing comes out either."""
+    net = _net(filters, 2, seed=100 + cin, cin=cin)
+    _gates_that_take_infinities(net)
+    inputs = _pyramid(70, 38, 2, cin, batch=2, seed=101)
+    for (b, y, x) in ((0, 5, 8), (1, 9, 17), (1, 15, 32)):
+        inputs[level][b, 0, y, x] = 1e5  # (infinite as an operand)
+    # the infinite image reaches the output through the 1x1, at its own pixel
+    _held_to_restatement(net, inputs, 3 * 3 if level == 0 else 0)

@@ -319,7 +319,17 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
                 const float e = f[i] > 0.f ? f[i] : (__expf(f[i]) - 1.f);
                 // v_rcp_f32 is good to 1 ulp of fp32 and the product is rounded to fp16 next: no IEEE division needed
                 const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-g[i]));
-                o[i]           = _Float16(e * sg);  // (0 for padding channels: their weights and biases are 0)
+                o[i]           = _Float16(e * sg);
+            }
+            // padding channels: of an infinite operand their zero weights make not a number, not zero
+            if (p.cout & 15)
+            {
+                if (p.cout & 3)
+                {
+#pragma unroll
+                    for (int i = 1; i < 4; ++i) o[i] = ch0 + i < p.cout ? o[i] : _Float16(0.f);
+                }
+                if (ch0 >= p.cout) o = half4{};
             }
             // the image of the pixel, as the convolution saw it: channels lq * 4 .. + 3
             const _Float16* mine = s_patch + ((r0 + m + 1) * kConvPatchW + c0 + lrow + 1) * ROW;
