@@ -16,7 +16,7 @@ from tests.test_gpu_unet import _net, _pyramid
 pytestmark = pytest.mark.gpu
 
 
-def _held_to_restatement(net, inputs, min_nonfinite):
+def _held_to_restatement(net, inputs, min_nonfinite, nan=False):
     from tests.ref_unet import unet_forward
     with torch.no_grad(), torch.backends.mkldnn.flags(enabled=False):
         want = unet_forward(copy.deepcopy(net), inputs)
@@ -25,6 +25,7 @@ def _held_to_restatement(net, inputs, min_nonfinite):
     assert int((~finite).sum()) >= min_nonfinite and int(finite.sum()) > finite.numel() // 2
     wrong = (torch.isfinite(got) != finite).nonzero().tolist()
     assert not wrong, f"{len(wrong)} outputs, the first at {wrong[:6]}"
+    assert not nan or torch.equal(got.isnan(), want.isnan())
     scale = want[finite].abs().max()
     assert (got[finite] - want[finite]).abs().max() < 2e-3 * scale
 
@@ -76,3 +77,19 @@ def test_padding_channels_take_no_part(level, filters, cin):
         inputs[level][b, 0, y, x] = 1e5  # (infinite as an operand)
     # the infinite image reaches the output through the 1x1, at its own pixel
     _held_to_restatement(net, inputs, 3 * 3 if level == 0 else 0)
+
+
+@pytest.mark.parametrize("level,filters,cin", [
+    (0, [16, 32], 4), (0, [32, 32], 4), (0, [16, 32], 3), (0, [12, 20], 1), (0, [32, 48], 8), (0, [48, 64], 16), (0, [48, 64], 4),
+    # behind the image, a row of the patch holds the upsampled one
+    (1, [16, 20], 3), (1, [24, 20], 6), (1, [32, 36], 8), (1, [40, 56], 12), (1, [48, 64], 16),
+])
+def test_the_output_convolution_reads_the_image_alone(level, filters, cin):
+    """The 1x1's products over the image: an infinite channel gives what its weight makes of it, and of what lies beside the
+    image in the same row nothing comes out."""
+    net = _net(filters, 2, seed=110 + cin, cin=cin)
+    _gates_that_take_infinities(net)
+    inputs = _pyramid(70, 38, 2, cin, batch=2, seed=111)
+    for (b, y, x) in ((0, 5, 8), (1, 9, 17), (1, 15, 32)):
+        inputs[level][b, 0, y, x] = 1e5
+    _held_to_restatement(net, inputs, 3 * 3 if level == 0 else 0, nan=True)

@@ -130,10 +130,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
         fimg = *reinterpret_cast<const half4*>(p.fin_frag + ((p.npad / 32) * 16 + (lrow & 3) * 4 + lq) * 4);
     }
     // channels that nothing ever writes: of the start block all but the image's, of the others the groups that the
-    // rows of the level below do not have
+    // rows of the level below do not have; and the padding of the patch's rows
     const int below_groups = p.below_stride / 8;
-    for (int i = threadIdx.x; i < kPatch * GROUPS; i += THREADS)
-        if (i % GROUPS >= below_groups) *reinterpret_cast<half8*>(s_patch + (i / GROUPS) * ROW + 8 * (i % GROUPS)) = half8{};
+    for (int i = threadIdx.x; i < kPatch * (GROUPS + 1); i += THREADS)
+        if (i % (GROUPS + 1) >= below_groups) *reinterpret_cast<half8*>(s_patch + (i / (GROUPS + 1)) * ROW + 8 * (i % (GROUPS + 1))) = half8{};
 
     // ---- this thread's share of the loads of a tile ----
     struct Loads
@@ -371,7 +371,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
             }
             if (p.final_out)
             {
-                const half4 im  = *reinterpret_cast<const half4*>(mine + (CI == 4 ? 0 : lq * 4));
+                // (of the 16 positions that a product takes, those past the image are zero: for four channels read from the
+                // row's padding, else cleared)
+                half4 im = *reinterpret_cast<const half4*>(mine + (FOUR ? (lq == 0 ? 0 : CIN) : CI == 4 ? 0 : lq * 4));
+                if (!FOUR)
+                {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) im[i] = lq * 4 + i < C ? im[i] : _Float16(0.f);
+                }
                 floatx4 row     = __builtin_amdgcn_mfma_f32_16x16x16f16(fw, o, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                 if (pair == 0) row = __builtin_amdgcn_mfma_f32_16x16x16f16(fimg, im, row, 0, 0, 0);
                 fin = lq == m ? row : fin;
