@@ -262,3 +262,22 @@ def test_forward_mode_is_refused_without_a_graph_as_well():
         ns.texture.texture = fwad.make_dual(ns.texture.texture, torch.ones_like(ns.texture.texture))
         with pytest.raises(NotImplementedError):
             BlendPointCloud(info)
+
+
+def test_a_trace_without_a_graph_renders():
+    """torch.jit.trace of the operator without gradients: the traced program renders what it is given."""
+    from trips_amd.renderer import BlendPointCloud, NeuralScene
+    sc = scenes.tiny(n=200, w=32, h=24, f=30.0, num_layers=2, list_depth=16, seed=44)
+    ns = NeuralScene.from_arrays(sc)
+    info = _info(sc, ns, train=False)
+    texture = ns.texture.texture.detach().clone()
+
+    def render(t):
+        ns.texture.texture = t
+        return tuple(BlendPointCloud(info))
+
+    with torch.no_grad():
+        traced = torch.jit.trace(render, (texture,), check_trace=False)
+        want = render(2 * texture)
+        got = traced(2 * texture)
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and float(want[0].abs().max()) > 0

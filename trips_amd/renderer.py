@@ -439,9 +439,10 @@ def BlendPointCloud(info: NeuralRenderInfo):
     inputs = (sc.texture.texture, sc.texture.background_color, sc.point_cloud_cuda.t_position, sc.poses.tangent_poses,
               sc.intrinsics.intrinsics, sc.texture.confidence_value_of_point, sc.dynamic_refinement_t,
               sc.point_cloud_cuda.t_point_size)
-    # (what the function refuses, forward-mode duals and functional transforms, it refuses without a graph as well)
+    # (what the function refuses, forward-mode duals and functional transforms, it refuses without a graph as well; a
+    # trace records the function's call, of the render by itself it would keep nothing but the empty images)
     if (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs)) or \
-            forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active():
+            forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or torch.jit.is_tracing():
         return list(PointRender.apply(*inputs, info))
     # no graph to record (a viewer's frame): the render without the autograd function around it
     texture, background, points, _, intrinsics, confidence, refinement, layer = inputs
