@@ -1,6 +1,5 @@
-"""The net's kernels at the edges of their dispatch, against the plain-torch restatement: finest blocks whose 1x1 runs
-as a kernel of its own, workgroups of one and of two output pairs on either side of the line between them, sizes at the
-edges of the 8 x 32 tiles. Bars of tests/test_gpu_unet.py: 2e-3 of the largest output against the restatement that
+"""The net's kernels at the edges of their dispatch, against the plain-torch restatement: workgroups of one to four output
+pairs on either side of the lines between them, sizes at the edges of the 8 x 32 tiles. Bars of tests/test_gpu_unet.py: 2e-3 of the largest output against the restatement that
 rounds where the device rounds (summation order, fast exp), 2e-2 of each gradient's largest element (fp16 operands)."""
 import copy
 
@@ -14,14 +13,22 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("filters,w,h,cin,batch", [
-    ([48, 64], 33, 9, 4, 1),        # 44 outputs at the finest level: three pairs, each in a workgroup of its own
+    ([48, 64], 33, 9, 4, 1),        # 44 outputs at the finest level: three pairs, 64 inputs
     ([64, 64], 31, 7, 3, 2),        # 61: four pairs, the last one nearly empty; an odd number of image channels
+    ([64, 32], 35, 12, 4, 2),       # ... on 32 inputs
+    ([60, 64], 40, 11, 16, 1),      # three pairs, sixteen image channels
     ([64, 32], 64, 16, 8, 1),       # whole tiles
     ([36, 24], 65, 17, 2, 3),       # 34: the third pair holds two outputs
     ([32, 36], 40, 40, 4, 1),       # 28 outputs on 36 inputs: the block's own 1x1 with two pairs and 64 channels
     ([32, 24], 544, 272, 4, 1),     # enough tiles for two pairs per workgroup at both levels
     ([48, 64], 544, 272, 4, 1),     # ... at the coarser level only (the finest has three pairs)
-    ([64, 64], 544, 136, 6, 2),     # ... at the finest, where the pairs are split over workgroups
+    ([64, 64], 544, 136, 6, 2),
+    # three and four pairs at the coarser levels, either side of the 512 tiles from which they share a workgroup:
+    ([16, 48], 129, 65, 4, 35),     # 3 x 5 tiles x 35 images
+    ([16, 48, 52], 126, 64, 4, 63), # 2 x 4 x 63: not enough
+    ([16, 50, 52], 130, 64, 4, 45), # 3 x 4 x 45, 64 inputs
+    ([16, 60, 56], 130, 64, 2, 45), # four pairs
+    ([16, 62, 30], 130, 66, 1, 35), # ... on 32 inputs
     # the data gradient's strips, of 15 coarser columns and 4 n - 1 coarser rows:
     ([16, 32], 30, 6, 4, 1),        # one strip, filled exactly
     ([32, 32], 31, 7, 3, 2),        # a column and a row more, odd sizes, outputs that start at position 6
@@ -34,8 +41,9 @@ pytestmark = pytest.mark.gpu
 ])
 def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
     from tests.ref_unet import unet_forward
-    net = _net(filters, 2, seed=60 + w + cin, cin=cin)
-    inputs = _pyramid(w, h, 2, cin, batch=batch, seed=61)
+    levels = len(filters)
+    net = _net(filters, levels, seed=60 + w + cin, cin=cin)
+    inputs = _pyramid(w, h, levels, cin, batch=batch, seed=61)
     _compare(copy.deepcopy(net), inputs)
     g = torch.Generator().manual_seed(62)
     upstream = torch.randn((batch, 3, h, w), generator=g) * 1e-3
@@ -45,7 +53,7 @@ def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
     net = net.cuda()
     ins = [t.cuda().requires_grad_(True) for t in inputs]
     (net.forward(ins) * upstream.cuda()).sum().backward()
-    pairs = [(f"d inputs[{i}]", ins[i].grad, ins_ref[i].grad) for i in range(2)]
+    pairs = [(f"d inputs[{i}]", ins[i].grad, ins_ref[i].grad) for i in range(levels)]
     pairs += [(n, p.grad, q.grad) for (n, p), (_, q) in zip(net.named_parameters(), ref.named_parameters())]
     for name, got, want in pairs:
         got, want = got.cpu().numpy(), want.numpy()

@@ -355,10 +355,9 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
     o += align256((size_t)(np.lv[0].npad / 32 + 1) * 64 * sizeof(_Float16));
     for (int i = 0; i < L; ++i)
     {
-        // (the rows of the finest level leave their kernel only where the 1x1 convolution is one of its own; the
-        // backward takes that block's output from the saved pre-activations)
+        // (the rows of the finest level do not leave their kernel)
         np.lv[i].rows_off = o;
-        if (i > 0 || np.lv[0].npad > 64) o += align256((size_t)d.batch * np.lv[i].H * np.lv[i].W * np.lv[i].row_stride * sizeof(_Float16));
+        if (i > 0) o += align256((size_t)d.batch * np.lv[i].H * np.lv[i].W * np.lv[i].row_stride * sizeof(_Float16));
     }
     np.bytes = o;
     size_t sv = 0, bw = 0;

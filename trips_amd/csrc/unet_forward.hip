@@ -4,7 +4,6 @@
 //                           src/lib/models/Networks.h:751-787, 999-1098
 //                           and, in the finest block's epilogue, the `final` 1x1 Sequential of
 //                           MultiScaleUnet2dDecOnlySmallFixedImpl, Networks.h:1129-1131
-//   final_conv1x1_kernel     the same 1x1 for nets whose finest block has more outputs than one workgroup takes
 //
 // The reference runs, per level, upsample -> cat -> two 3x3 convolutions -> elu / sigmoid -> multiply -> cat as
 // separate libtorch ops on NCHW tensors, materialising every intermediate. Here one kernel per level does all of
@@ -59,7 +58,7 @@ __device__ __forceinline__ void loaded(float& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void loaded(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
 // One workgroup walks tiles of 8 x 32 pixels and computes PAIRS pairs of (16 feature, 16 mask) outputs of each. Its
-// wavefronts split the pairs and the tile: a wavefront owns one pair for a strip of 16 pixels x MB rows, so that its A
+// wavefronts split the pairs and the tile: a wavefront owns one pair for STRIPS strips of 16 pixels x MB rows, so that its A
 // operands (LDS) are shared by the three vertical taps and a lane ends up with four features and the masks of the same
 // four channels of a pixel: the gate, the stores and the 1x1 of the finest level need no LDS and no further exchange.
 // What bounds it: vector instructions (loads, upsampling, the gate's two exponentials), then the latency of the phases
@@ -68,55 +67,62 @@ __device__ __forceinline__ void loaded(uint4& v) { asm volatile("" : "+v"(v.x), 
 // upsampling makes 2 x 2 pixels from one set of four neighbours (382 instead of 710 vector instructions per wavefront
 // and 256-pixel tile at the finest level of the 16/32/64/64 net). 1920 x 1080, that net, per level, against one tile
 // per workgroup with LDS-staged epilogues: 106 -> 74, 61 -> 59, 38 -> 35, 14 -> 13 us.
-// BREGS: the pair's weights (9 taps x 64 inputs: 144 registers) stay in registers for all tiles of the workgroup;
-// with 32 inputs they are staged in LDS once (held in registers they leave room for half the wavefronts: 121 us at the
-// finest level, where six wavefronts per SIMD take 74 and four 83).
+// KREG: the pair's weights of so many blocks of 32 inputs (9 taps: 72 registers each) stay in registers for all tiles of
+// the workgroup, the others are staged in LDS once. With 32 inputs all are (held in registers they leave room for half the
+// wavefronts: 121 us at the finest level, where six wavefronts per SIMD take 74 and four 83); with 64 none, but for three
+// pairs, where half of them in LDS let twelve wavefronts share the SIMDs evenly: 252 us for 64 -> 96 at 1920 x 1080, 364
+// with six wavefronts and all weights in registers.
 // CI: image channels the kernel has room for (4, 8 or 16); FOUR: C is exactly 4, the splat's usual descriptor width
-template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, bool BREGS, int WAVES_PER_EU>
+template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, int KREG, int WAVES_PER_EU>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void gated_conv3x3_kernel(const ConvParams p)
 {
     constexpr int KB      = CIN / 32;
     constexpr int ROW     = CIN + kLdsChanPad;  // halves per patch pixel in LDS
     constexpr int GROUPS  = CIN / 8;
-    constexpr int MB      = 16 * PAIRS / (THREADS / 64);  // rows of a wavefront's strip
-    static_assert(MB <= 4, "the 1x1 of the finest level keeps four rows in one accumulator");
+    constexpr int WAVES   = THREADS / 64;
+    constexpr int MB      = std::min(16 * PAIRS / WAVES, 4);  // rows of a strip (the 1x1 keeps them in one accumulator)
+    constexpr int STRIPS  = 16 * PAIRS / WAVES / MB;          // strips of a wavefront, one after the other
+    static_assert(WAVES % PAIRS == 0 && WAVES * MB * STRIPS == 16 * PAIRS, "the strips of a tile");
+    static_assert(PAIRS > 2 || STRIPS == 1, "the sums of the 1x1 are handed over once per tile");
     constexpr int kPatch  = kConvPatchH * kConvPatchW;
     constexpr int kQuads  = (kConvPatchH / 2) * (kConvPatchW / 2);
     constexpr int QITEMS  = (kQuads * GROUPS + THREADS - 1) / THREADS;
-    // (8 and 16 image channels leave no registers for the loads of the next tile)
-    constexpr bool kPrefetch = CI == 4 || (CIN == 32 && CI == 8);
+    // (8 and 16 image channels, and 64 inputs with three and more pairs, leave no registers for the loads of the next tile:
+    // 64 -> 96 at 1920 x 1080, 273 us with them and 18 registers spilled, 252 without)
+    constexpr bool kPrefetch = (CI == 4 && (CIN == 32 || PAIRS <= 2)) || (CIN == 32 && CI == 8);
     constexpr int FITEMS     = (kPatch + THREADS - 1) / THREADS;
+    constexpr int KLDS       = KB - KREG;  // 32-input blocks whose weights sit in LDS
     __shared__ __align__(16) _Float16 s_patch[kPatch * ROW];
-    __shared__ __align__(16) _Float16 s_w[BREGS ? 8 : PAIRS * 9 * KB * 2 * 512];
-    __shared__ float4 s_fin[PAIRS == 2 ? 4 * 64 : 1];
+    __shared__ __align__(16) _Float16 s_w[KLDS == 0 ? 8 : PAIRS * 9 * KLDS * 2 * 512];
+    __shared__ float4 s_fin[PAIRS == 1 ? 1 : (PAIRS == 2 ? 1 : PAIRS) * 4 * 64];
 
     const int lane = (int)threadIdx.x & 63;
     // (a wavefront's number is the same for its lanes: kept on the scalar unit)
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lrow = lane & 15, lq = lane >> 4;
     const int C    = FOUR ? 4 : p.c_feat;
-    const int pair = PAIRS == 1 ? 0 : wave & 1;
-    const int strip = PAIRS == 1 ? wave : wave >> 1;
-    const int r0 = (strip >> 1) * MB, c0 = (strip & 1) * 16;  // the strip's first row and column of the tile
-    const int gp = blockIdx.y * PAIRS + pair;                 // this wavefront's pair of the level
+    const int pair = PAIRS == 1 ? 0 : PAIRS == 2 ? wave & 1 : wave % PAIRS;
+    const int gp   = blockIdx.y * PAIRS + pair;  // this wavefront's pair of the level
+    const int first_strip = PAIRS == 1 ? wave : wave / PAIRS;
     const int tiles = p.tiles * p.batch;
 
     // ---- what stays for all tiles: weights, biases, the 1x1's weights ----
     const half8* wsrc = reinterpret_cast<const half8*>(p.wfrag) + (size_t)gp * (9 * KB * 2 * 64) + lane;
-    half8 w[BREGS ? 9 : 1][KB][2];
-    if (BREGS)
+    half8 w[KREG > 0 ? 9 : 1][KREG > 0 ? KREG : 1][2];
+    if (KREG > 0)
     {
 #pragma unroll
-        for (int t = 0; t < (BREGS ? 9 : 1); ++t)
+        for (int t = 0; t < (KREG > 0 ? 9 : 1); ++t)
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
+            for (int kb = 0; kb < KREG; ++kb)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) w[t][kb][h] = wsrc[((t * KB + kb) * 2 + h) * 64];
     }
-    else
+    if (KLDS > 0)
     {
         const half8* src = reinterpret_cast<const half8*>(p.wfrag) + (size_t)blockIdx.y * PAIRS * (9 * KB * 2 * 64);
-        for (int i = threadIdx.x; i < PAIRS * 9 * KB * 2 * 64; i += THREADS) reinterpret_cast<half8*>(s_w)[i] = src[i];
+        for (int i = threadIdx.x; i < PAIRS * 9 * KLDS * 2 * 64; i += THREADS)
+            reinterpret_cast<half8*>(s_w)[i] = src[KREG == 0 ? i : (i / (KLDS * 2 * 64)) * (KB * 2 * 64) + KREG * 2 * 64 + i % (KLDS * 2 * 64)];
     }
     const float4 bias_f = *reinterpret_cast<const float4*>(p.bias + gp * 32 + lq * 4);
     const float4 bias_m = *reinterpret_cast<const float4*>(p.bias + gp * 32 + 16 + lq * 4);
@@ -259,188 +265,191 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
         __syncthreads();
         if (kPrefetch && at + in_xcd < last) issue(decode(at + in_xcd), tid, cur);  // travels during the taps and the epilogue
 
-        floatx4 acc[MB][2];
-#pragma unroll
-        for (int m = 0; m < MB; ++m)
+        int strip = first_strip;
+        do  // (a loop with STRIPS = 1 cost the kernel of the finest level 12 spilled registers and a fifth of its time)
         {
-            acc[m][0] = floatx4{bias_f.x, bias_f.y, bias_f.z, bias_f.w};
-            acc[m][1] = floatx4{bias_m.x, bias_m.y, bias_m.z, bias_m.w};
-        }
-        const half8* wlds  = reinterpret_cast<const half8*>(s_w) + pair * (9 * KB * 2 * 64) + lane;
-        const _Float16* a0 = s_patch + (r0 * kConvPatchW + c0 + lrow) * ROW + lq * 8;
+            const int r0 = (strip >> 1) * MB, c0 = (strip & 1) * 16;  // the strip's first row and column of the tile
+            floatx4 acc[MB][2];
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx)
+            for (int m = 0; m < MB; ++m)
             {
-                half8 b[3][2];
+                acc[m][0] = floatx4{bias_f.x, bias_f.y, bias_f.z, bias_f.w};
+                acc[m][1] = floatx4{bias_m.x, bias_m.y, bias_m.z, bias_m.w};
+            }
+            const half8* wlds  = reinterpret_cast<const half8*>(s_w) + pair * (9 * KLDS * 2 * 64) + lane;
+            const _Float16* a0 = s_patch + (r0 * kConvPatchW + c0 + lrow) * ROW + lq * 8;
 #pragma unroll
-                for (int dy = 0; dy < 3; ++dy)
+            for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) b[dy][h] = BREGS ? w[BREGS ? 3 * dy + dx : 0][kb][h] : wlds[(((3 * dy + dx) * KB + kb) * 2 + h) * 64];
-#pragma unroll
-                for (int r = 0; r < MB + 2; ++r)
+                for (int dx = 0; dx < 3; ++dx)
                 {
-                    const half8 a = *reinterpret_cast<const half8*>(a0 + (r * kConvPatchW + dx) * ROW + kb * 32);
+                    half8 b[3][2];
 #pragma unroll
                     for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) b[dy][h] = kb < KREG ? w[KREG > 0 ? 3 * dy + dx : 0][kb < KREG ? kb : 0][h] : wlds[(((3 * dy + dx) * KLDS + kb - KREG) * 2 + h) * 64];
+#pragma unroll
+                    for (int r = 0; r < MB + 2; ++r)
                     {
-                        const int m = r - dy;
-                        if (m < 0 || m >= MB) continue;
-                        acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][0], a, acc[m][0], 0, 0, 0);
-                        acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][1], a, acc[m][1], 0, 0, 0);
+                        const half8 a = *reinterpret_cast<const half8*>(a0 + (r * kConvPatchW + dx) * ROW + kb * 32);
+#pragma unroll
+                        for (int dy = 0; dy < 3; ++dy)
+                        {
+                            const int m = r - dy;
+                            if (m < 0 || m >= MB) continue;
+                            acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][0], a, acc[m][0], 0, 0, 0);
+                            acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy][1], a, acc[m][1], 0, 0, 0);
+                        }
                     }
                 }
-            }
 
-        // ---- epilogue: elu(feature) * sigmoid(mask); a lane: four channels of one pixel per row of the strip ----
-        const int x = t.x0 + c0 + lrow, ch0 = gp * 16 + lq * 4;
-        const size_t tile_pix = (size_t)t.image * p.H * p.W + (size_t)t.y0 * p.W + t.x0;
-        _Float16* pre_tile    = p.pre ? p.pre + tile_pix * p.npad : nullptr;
-        _Float16* out_tile    = p.out ? p.out + tile_pix * p.out_stride : nullptr;
-        floatx4 fin = floatx4{0.f, 0.f, 0.f, 0.f};
+            // ---- epilogue: elu(feature) * sigmoid(mask); a lane: four channels of one pixel per row of the strip ----
+            const int x = t.x0 + c0 + lrow, ch0 = gp * 16 + lq * 4;
+            const size_t tile_pix = (size_t)t.image * p.H * p.W + (size_t)t.y0 * p.W + t.x0;
+            _Float16* pre_tile    = p.pre ? p.pre + tile_pix * p.npad : nullptr;
+            _Float16* out_tile    = p.out ? p.out + tile_pix * p.out_stride : nullptr;
+            floatx4 fin = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int m = 0; m < MB; ++m)
-        {
-            const int y       = t.y0 + r0 + m;
-            const bool inside = y < p.H && x < p.W;
-            const int pix     = (r0 + m) * p.W + c0 + lrow;  // from the tile's first
-            const floatx4 f = acc[m][0], g = acc[m][1];
-            if (p.pre && inside)
+            for (int m = 0; m < MB; ++m)
             {
-                const half8 v = half8{_Float16(f[0]), _Float16(f[1]), _Float16(f[2]), _Float16(f[3]),
-                                      _Float16(g[0]), _Float16(g[1]), _Float16(g[2]), _Float16(g[3])};
-                __builtin_nontemporal_store(v, reinterpret_cast<half8*>(pre_tile + pix * p.npad + 2 * ch0));
-            }
-            half4 o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-            {
-                const float e = f[i] > 0.f ? f[i] : (__expf(f[i]) - 1.f);
-                // v_rcp_f32 is good to 1 ulp of fp32 and the product is rounded to fp16 next: no IEEE division needed
-                const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-g[i]));
-                o[i]           = _Float16(e * sg);
-            }
-            // padding channels: of an infinite operand their zero weights make not a number, not zero
-            if (p.cout & 15)
-            {
-                if (p.cout & 3)
+                const int y       = t.y0 + r0 + m;
+                const bool inside = y < p.H && x < p.W;
+                const int pix     = (r0 + m) * p.W + c0 + lrow;  // from the tile's first
+                const floatx4 f = acc[m][0], g = acc[m][1];
+                if (p.pre && inside)
                 {
-#pragma unroll
-                    for (int i = 1; i < 4; ++i) o[i] = ch0 + i < p.cout ? o[i] : _Float16(0.f);
+                    const half8 v = half8{_Float16(f[0]), _Float16(f[1]), _Float16(f[2]), _Float16(f[3]),
+                                          _Float16(g[0]), _Float16(g[1]), _Float16(g[2]), _Float16(g[3])};
+                    __builtin_nontemporal_store(v, reinterpret_cast<half8*>(pre_tile + pix * p.npad + 2 * ch0));
                 }
-                if (ch0 >= p.cout) o = half4{};
-            }
-            // the image of the pixel, as the convolution saw it: channels lq * 4 .. + 3
-            const _Float16* mine = s_patch + ((r0 + m + 1) * kConvPatchW + c0 + lrow + 1) * ROW;
-            if (p.out && inside)
-            {
-                _Float16* row = out_tile + pix * p.out_stride;
-                const int pos = 2 * C + ch0;
-                if (pos + 4 <= p.out_stride)
+                half4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
                 {
-                    if (FOUR || (C & 1) == 0)
-                        *reinterpret_cast<half4*>(row + pos) = o;
+                    const float e = f[i] > 0.f ? f[i] : (__expf(f[i]) - 1.f);
+                    // v_rcp_f32 is good to 1 ulp of fp32 and the product is rounded to fp16 next: no IEEE division needed
+                    const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-g[i]));
+                    o[i]           = _Float16(e * sg);
+                }
+                // padding channels: of an infinite operand their zero weights make not a number, not zero
+                if (p.cout & 15)
+                {
+                    if (p.cout & 3)
+                    {
+#pragma unroll
+                        for (int i = 1; i < 4; ++i) o[i] = ch0 + i < p.cout ? o[i] : _Float16(0.f);
+                    }
+                    if (ch0 >= p.cout) o = half4{};
+                }
+                // the image of the pixel, as the convolution saw it: channels lq * 4 .. + 3
+                const _Float16* mine = s_patch + ((r0 + m + 1) * kConvPatchW + c0 + lrow + 1) * ROW;
+                if (p.out && inside)
+                {
+                    _Float16* row = out_tile + pix * p.out_stride;
+                    const int pos = 2 * C + ch0;
+                    if (pos + 4 <= p.out_stride)
+                    {
+                        if (FOUR || (C & 1) == 0)
+                            *reinterpret_cast<half4*>(row + pos) = o;
+                        else
+                        {
+                            typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                            *reinterpret_cast<half2v*>(row + pos)     = half2v{o[0], o[1]};
+                            *reinterpret_cast<half2v*>(row + pos + 2) = half2v{o[2], o[3]};
+                        }
+                    }
                     else
                     {
-                        typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-                        *reinterpret_cast<half2v*>(row + pos)     = half2v{o[0], o[1]};
-                        *reinterpret_cast<half2v*>(row + pos + 2) = half2v{o[2], o[3]};
-                    }
-                }
-                else
-                {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (pos + i < p.out_stride) row[pos + i] = o[i];
-                }
-                if (gp == 0 && FOUR)
-                {
-                    if (lq == 0)
+                        for (int i = 0; i < 4; ++i)
+                            if (pos + i < p.out_stride) row[pos + i] = o[i];
+                    }
+                    if (gp == 0 && FOUR)
                     {
-                        const half4 im                 = *reinterpret_cast<const half4*>(mine);
-                        *reinterpret_cast<half8*>(row) = half8{_Float16(0.f), _Float16(0.f), _Float16(0.f), _Float16(0.f), im[0], im[1], im[2], im[3]};
+                        if (lq == 0)
+                        {
+                            const half4 im                 = *reinterpret_cast<const half4*>(mine);
+                            *reinterpret_cast<half8*>(row) = half8{_Float16(0.f), _Float16(0.f), _Float16(0.f), _Float16(0.f), im[0], im[1], im[2], im[3]};
+                        }
+                    }
+                    else if (gp == 0)
+                    {
+                        // the row's other positions: [0, C) zero, [C, 2C) the image, what the outputs do not reach zero
+                        for (int c = lq; c < C; c += 4) row[c] = _Float16(0.f), row[C + c] = mine[c];
+                        for (int c = 2 * C + p.npad / 2 + lq; c < p.out_stride; c += 4) row[c] = _Float16(0.f);
                     }
                 }
-                else if (gp == 0)
+                if (p.final_out)
                 {
-                    // the row's other positions: [0, C) zero, [C, 2C) the image, what the outputs do not reach zero
-                    for (int c = lq; c < C; c += 4) row[c] = _Float16(0.f), row[C + c] = mine[c];
-                    for (int c = 2 * C + p.npad / 2 + lq; c < p.out_stride; c += 4) row[c] = _Float16(0.f);
+                    // (of the 16 positions that a product takes, those past the image are zero: for four channels read from the
+                    // row's padding, else cleared)
+                    half4 im = *reinterpret_cast<const half4*>(mine + (FOUR ? (lq == 0 ? 0 : CIN) : CI == 4 ? 0 : lq * 4));
+                    if (!FOUR)
+                    {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) im[i] = lq * 4 + i < C ? im[i] : _Float16(0.f);
+                    }
+                    floatx4 row     = __builtin_amdgcn_mfma_f32_16x16x16f16(fw, o, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    if (pair == 0) row = __builtin_amdgcn_mfma_f32_16x16x16f16(fimg, im, row, 0, 0, 0);
+                    fin = lq == m ? row : fin;
                 }
             }
             if (p.final_out)
             {
-                // (of the 16 positions that a product takes, those past the image are zero: for four channels read from the
-                // row's padding, else cleared)
-                half4 im = *reinterpret_cast<const half4*>(mine + (FOUR ? (lq == 0 ? 0 : CIN) : CI == 4 ? 0 : lq * 4));
-                if (!FOUR)
+                // lane group m: the outputs of row m, pixel lrow; with two pairs the wavefront of the second one hands over
+                // its share of the sums, with more all of them do
+                if constexpr (PAIRS > 2)
                 {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) im[i] = lq * 4 + i < C ? im[i] : _Float16(0.f);
+                    s_fin[(pair * 4 + strip) * 64 + lane] = make_float4(fin[0], fin[1], fin[2], fin[3]);
+                    continue;
                 }
-                floatx4 row     = __builtin_amdgcn_mfma_f32_16x16x16f16(fw, o, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                if (pair == 0) row = __builtin_amdgcn_mfma_f32_16x16x16f16(fimg, im, row, 0, 0, 0);
-                fin = lq == m ? row : fin;
-            }
-        }
-        if (p.final_out)
-        {
-            // lane group m: the outputs of row m, pixel lrow; with two pairs the wavefront of the second one hands over
-            // its share of the sums
-            if (PAIRS == 2)
-            {
-                if (pair == 1) s_fin[strip * 64 + lane] = make_float4(fin[0], fin[1], fin[2], fin[3]);
-                __syncthreads();
-            }
-            const int y = t.y0 + r0 + lq;
-            if (pair == 0 && lq < MB && y < p.H && x < p.W)
-            {
                 if (PAIRS == 2)
                 {
-                    const float4 o = s_fin[strip * 64 + lane];
-                    fin[0] += o.x, fin[1] += o.y, fin[2] += o.z, fin[3] += o.w;
+                    if (pair == 1) s_fin[strip * 64 + lane] = make_float4(fin[0], fin[1], fin[2], fin[3]);
+                    __syncthreads();
                 }
-                const size_t plane = (size_t)p.H * p.W;
-                float* dst         = p.final_out + (size_t)t.image * p.final_cout * plane + (size_t)y * p.W + x;
+                const int y = t.y0 + r0 + lq;
+                if (pair == 0 && lq < MB && y < p.H && x < p.W)
+                {
+                    if (PAIRS == 2)
+                    {
+                        const float4 o = s_fin[strip * 64 + lane];
+                        fin[0] += o.x, fin[1] += o.y, fin[2] += o.z, fin[3] += o.w;
+                    }
+                    const size_t plane = (size_t)p.H * p.W;
+                    float* dst         = p.final_out + (size_t)t.image * p.final_cout * plane + (size_t)y * p.W + x;
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k < p.final_cout) dst[k * plane] = fin[k] + p.final_b[k];
+                    for (int k = 0; k < 4; ++k)
+                        if (k < p.final_cout) dst[k * plane] = fin[k] + p.final_b[k];
+                }
             }
-        }
-    }
-}
-
-// The 1x1 output convolution on rows of the finest level, for nets whose finest block has more than 32 outputs (their
-// pairs are split over workgroups, none of which holds a whole pixel). A thread per pixel; bound by its row's bytes.
-__global__ __launch_bounds__(256) void final_conv1x1_kernel(const _Float16* __restrict__ rows, int stride, int c_feat, int cin,
-                                                            const float* __restrict__ weight, const float* __restrict__ bias, int cout,
-                                                            size_t plane, size_t pixels, float* __restrict__ out)
-{
-    __shared__ float s_w[4 * (kUnetMaxImageChannels + 64)];
-    for (int i = threadIdx.x; i < cout * cin; i += 256) s_w[i] = float(_Float16(weight[i]));  // fp16 like every other operand
-    __syncthreads();
-    for (size_t pix = (size_t)blockIdx.x * 256 + threadIdx.x; pix < pixels; pix += (size_t)gridDim.x * 256)
-    {
-        float a[4] = {0.f, 0.f, 0.f, 0.f};
-        const _Float16* row = rows + pix * stride;
-        for (int g = 0; g < stride / 8; ++g)
-        {
-            const half8 v = *reinterpret_cast<const half8*>(row + 8 * g);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
+        } while (STRIPS > 1 && (strip += WAVES / PAIRS) < 16 / MB);
+        if constexpr (PAIRS > 2)
+            if (p.final_out)
             {
-                const int c = 8 * g + i - c_feat;  // channel of x_0: the image at positions [C, 2C), then the block outputs
-                if (c < 0 || c >= cin) continue;
+                __syncthreads();
+                if (tid < kConvTileH * kConvTileW)
+                {
+                    float4 sum = s_fin[tid];
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k < cout) a[k] = __builtin_fmaf(s_w[k * cin + c], float(v[i]), a[k]);
+                    for (int j = 1; j < PAIRS; ++j)
+                    {
+                        const float4 o = s_fin[j * (4 * 64) + tid];
+                        sum.x += o.x, sum.y += o.y, sum.z += o.z, sum.w += o.w;
+                    }
+                    const int of = tid >> 6;  // the pixel's strip: of four rows, whatever the number of pairs
+                    const int y = t.y0 + (of >> 1) * 4 + lq, x = t.x0 + (of & 1) * 16 + lrow;
+                    if (y < p.H && x < p.W)
+                    {
+                        const size_t plane = (size_t)p.H * p.W;
+                        float* dst         = p.final_out + (size_t)t.image * p.final_cout * plane + (size_t)y * p.W + x;
+                        const float f[4]   = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if (k < p.final_cout) dst[k * plane] = f[k] + p.final_b[k];
+                    }
+                }
             }
-        }
-        const size_t b = pix / plane;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k < cout) out[b * cout * plane + k * plane + (pix - b * plane)] = a[k] + bias[k];
     }
 }
 
@@ -497,14 +506,14 @@ __global__ __launch_bounds__(256) void pack_conv_weights_kernel(const PackTable 
 // ---------------------------------------------------------------------------------------------------------
 namespace
 {
-template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, bool BREGS, int WAVES_PER_EU>
+template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, int KREG, int WAVES_PER_EU>
 hipError_t launch_conv(const ConvParams& p, int splits, hipStream_t stream)
 {
     const long long tiles = (long long)p.tiles * p.batch;
     // as many workgroups as are resident at once
     const int resident = std::max(1, 256 * (4 * WAVES_PER_EU / (THREADS / 64)) / splits);
     const dim3 grid((unsigned)std::min<long long>(tiles, resident), splits);
-    hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, PAIRS, CI, FOUR, THREADS, BREGS, WAVES_PER_EU>), grid, dim3(THREADS), 0, stream, p);
+    hipLaunchKernelGGL((gated_conv3x3_kernel<CIN, PAIRS, CI, FOUR, THREADS, KREG, WAVES_PER_EU>), grid, dim3(THREADS), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -514,10 +523,20 @@ hipError_t dispatch_conv_ci(const ConvParams& p, int cin_pad, hipStream_t stream
     // Two pairs of outputs per workgroup where there are enough tiles to fill the chip's 256 CUs that way (the patch is
     // then assembled half as often); an odd number of pairs and the coarse levels take one: with a few tiles the level
     // lasts as long as one tile's chain of products, which two pairs double (64 -> 128, 3 tiles: 16 -> 10 us).
-    const int pairs = p.npad / 32;
-    const bool two  = pairs % 2 == 0 && ((p.final_out && pairs == 2) || (long long)p.tiles * p.batch * (pairs / 2) >= 256);
-    if (cin_pad == 32) return two ? launch_conv<32, 2, CI, FOUR, 512, false, 4>(p, pairs / 2, stream) : launch_conv<32, 1, CI, FOUR, 512, false, (FOUR ? 6 : 4)>(p, pairs, stream);
-    return two ? launch_conv<64, 2, CI, FOUR, 512, true, 2>(p, pairs / 2, stream) : launch_conv<64, 1, CI, FOUR, 512, true, 2>(p, pairs, stream);
+    // Three and four pairs go together where every CU has tiles to walk: with 2040 tiles 125 -> 68 us (64 -> 96) and
+    // 111 -> 97 us (64 -> 128), with 300 tiles 26 and 27 -> 31 us. The finest level takes all of them in any case: its 1x1
+    // needs a whole pixel, and as a kernel of its own, behind rows written for it, it and the patches assembled three and
+    // four times took 665 us instead of 252 (1920 x 1080, 64 -> 96) and 717 instead of 370 (64 -> 128).
+    const int pairs       = p.npad / 32;
+    const long long tiles = (long long)p.tiles * p.batch;
+    if (pairs > 2 && (p.final_out || tiles >= 512))
+    {
+        if (pairs == 3) return cin_pad == 32 ? launch_conv<32, 3, CI, FOUR, 768, 0, 3>(p, 1, stream) : launch_conv<64, 3, CI, FOUR, 768, 1, 3>(p, 1, stream);
+        return cin_pad == 32 ? launch_conv<32, 4, CI, FOUR, 1024, 0, 4>(p, 1, stream) : launch_conv<64, 4, CI, FOUR, 512, 2, 2>(p, 1, stream);
+    }
+    const bool two = pairs % 2 == 0 && (p.final_out || tiles * (pairs / 2) >= 256);
+    if (cin_pad == 32) return two ? launch_conv<32, 2, CI, FOUR, 512, 0, 4>(p, pairs / 2, stream) : launch_conv<32, 1, CI, FOUR, 512, 0, (FOUR ? 6 : 4)>(p, pairs, stream);
+    return two ? launch_conv<64, 2, CI, FOUR, 512, 2, 2>(p, pairs / 2, stream) : launch_conv<64, 1, CI, FOUR, 512, 2, 2>(p, pairs, stream);
 }
 
 // (the kernel is built for exactly 4 image channels and with room for 4, 8 and 16; other counts use the next size up)
@@ -622,7 +641,6 @@ int unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeight
     {
         const LevelPlan& lv = np.lv[i];
         ProfScope ps(prof, kLevelNames[i], stream);
-        const bool fused_final = i == 0 && lv.npad <= 64;
         ConvParams p;
         std::memset(&p, 0, sizeof(p));
         p.H       = lv.H;
@@ -638,9 +656,9 @@ int unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeight
         p.feat_cs = hwc ? 1 : (size_t)lv.H * lv.W;
         p.wfrag   = reinterpret_cast<const _Float16*>(ws + lv.wpack_off);
         p.bias    = reinterpret_cast<const float*>(ws + lv.bias_off);
-        // (nobody reads the finest block's output again when its 1x1 runs in the same kernel, and the backward takes
-        // it from the pre-activations)
-        p.out        = fused_final ? nullptr : rows_ptr(i);
+        // (nobody reads the finest block's output again: its 1x1 runs in the same kernel, and the backward takes it from
+        // the pre-activations)
+        p.out        = i > 0 ? rows_ptr(i) : nullptr;
         p.out_stride = lv.row_stride;
         p.pre        = sv ? reinterpret_cast<_Float16*>(sv + lv.saved_pre_off) : nullptr;
         if (i < L - 1)
@@ -650,7 +668,7 @@ int unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeight
             p.below        = rows_ptr(i + 1);
             p.below_stride = np.lv[i + 1].row_stride;
         }
-        if (fused_final)
+        if (i == 0)
         {
             p.fin_frag   = reinterpret_cast<const _Float16*>(ws + np.fin_off);
             p.final_b    = weights->final_bias;
@@ -658,14 +676,6 @@ int unet_forward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUnetWeight
             p.final_cout = d.num_output_channels;
         }
         hipError_t e = dispatch_conv(p, lv.cin_pad, stream);
-        if (e == hipSuccess && i == 0 && !fused_final)
-        {
-            const size_t plane = (size_t)lv.H * lv.W;
-            hipLaunchKernelGGL(final_conv1x1_kernel, dim3((unsigned)std::min<size_t>((d.batch * plane + 255) / 256, 8192)), dim3(256), 0, stream,
-                               p.out, p.out_stride, C, C + lv.cout, weights->final_weight, weights->final_bias, d.num_output_channels, plane,
-                               d.batch * plane, output);
-            e = hipGetLastError();
-        }
         if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "gated conv launch (level %d): %s", i, hipGetErrorString(e));
     }
     return TRIPS_OK;
