@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
     ([60, 64], 40, 11, 16, 1),      # three pairs, sixteen image channels
     ([64, 32], 64, 16, 8, 1),       # whole tiles
     ([36, 24], 65, 17, 2, 3),       # 34: the third pair holds two outputs
+    ([32, 16], 160, 120, 4, 1),     # 75 and 24 tiles: a workgroup each, dealt to the eight XCDs
     ([32, 36], 40, 40, 4, 1),       # 28 outputs on 36 inputs: the block's own 1x1 with two pairs and 64 channels
     ([32, 24], 544, 272, 4, 1),     # enough tiles for two pairs per workgroup at both levels
     ([48, 64], 544, 272, 4, 1),     # ... at the coarser level only (the finest has three pairs)

@@ -242,11 +242,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
         }
     };
 
-    // consecutive tiles share their halos: they go to one XCD (workgroups are dealt to the eight of them in turn)
-    const int xcds = min(8, (int)gridDim.x), xcd = (int)blockIdx.x % xcds;
-    const int share = (tiles + xcds - 1) / xcds, in_xcd = ((int)gridDim.x - xcd + xcds - 1) / xcds;
-    const int last = min(tiles, (xcd + 1) * share);
-    int at = xcd * share + (int)blockIdx.x / xcds;
+    // Consecutive tiles share their halos: they go to one XCD (workgroups are dealt to the eight of them in turn). The XCDs'
+    // shares differ by one tile at most, the first ones' being the larger as are their numbers of workgroups: with as many
+    // workgroups as tiles each has one. (With shares rounded up, a workgroup of some XCD took a second tile: 75 tiles of
+    // 32 -> 32, 11.0 instead of 8.2 us, of 64 -> 64 at 160 x 120, 19.5 instead of 13.1.)
+    const int xcd  = (int)blockIdx.x & 7, in_xcd = ((int)gridDim.x - xcd + 7) >> 3;
+    const int last = (xcd + 1) * (tiles >> 3) + min(xcd + 1, tiles & 7);
+    int at         = xcd * (tiles >> 3) + min(xcd, tiles & 7) + ((int)blockIdx.x >> 3);
 
     Loads cur;
     if (kPrefetch && at < last) issue(decode(at), (int)threadIdx.x, cur);
