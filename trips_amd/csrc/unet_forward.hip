@@ -90,6 +90,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
     // (8 and 16 image channels, and 64 inputs with three and more pairs, leave no registers for the loads of the next tile:
     // 64 -> 96 at 1920 x 1080, 273 us with them and 18 registers spilled, 252 without)
     constexpr bool kPrefetch = (CI == 4 && (CIN == 32 || PAIRS <= 2)) || (CIN == 32 && CI == 8);
+    // ... and beside weights in registers none for them over the end of a tile either
+    constexpr bool kAhead = kPrefetch || KREG == 0;
     constexpr int FITEMS     = (kPatch + THREADS - 1) / THREADS;
     constexpr int KLDS       = KB - KREG;  // 32-input blocks whose weights sit in LDS
     __shared__ __align__(16) _Float16 s_patch[kPatch * ROW];
@@ -106,41 +108,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
     const int first_strip = PAIRS == 1 ? wave : wave / PAIRS;
     const int tiles = p.tiles * p.batch;
 
-    // ---- what stays for all tiles: weights, biases, the 1x1's weights ----
-    const half8* wsrc = reinterpret_cast<const half8*>(p.wfrag) + (size_t)gp * (9 * KB * 2 * 64) + lane;
-    half8 w[KREG > 0 ? 9 : 1][KREG > 0 ? KREG : 1][2];
-    if (KREG > 0)
-    {
-#pragma unroll
-        for (int t = 0; t < (KREG > 0 ? 9 : 1); ++t)
-#pragma unroll
-            for (int kb = 0; kb < KREG; ++kb)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) w[t][kb][h] = wsrc[((t * KB + kb) * 2 + h) * 64];
-    }
-    if (KLDS > 0)
-    {
-        const half8* src = reinterpret_cast<const half8*>(p.wfrag) + (size_t)blockIdx.y * PAIRS * (9 * KB * 2 * 64);
-        for (int i = threadIdx.x; i < PAIRS * 9 * KLDS * 2 * 64; i += THREADS)
-            reinterpret_cast<half8*>(s_w)[i] = src[KREG == 0 ? i : (i / (KLDS * 2 * 64)) * (KB * 2 * 64) + KREG * 2 * 64 + i % (KLDS * 2 * 64)];
-    }
-    const float4 bias_f = *reinterpret_cast<const float4*>(p.bias + gp * 32 + lq * 4);
-    const float4 bias_m = *reinterpret_cast<const float4*>(p.bias + gp * 32 + 16 + lq * 4);
-    // A operand of the 1x1: every lane group's rows hold the four outputs, of which group m keeps those of the strip's row m
-    // (the same number of selects as zero weights for the other rows, through which an infinite operand of one row would
-    // make all of them not a number)
-    half4 fw = half4{}, fimg = half4{};
-    if (p.final_out)
-    {
-        fw   = *reinterpret_cast<const half4*>(p.fin_frag + (gp * 16 + (lrow & 3) * 4 + lq) * 4);
-        fimg = *reinterpret_cast<const half4*>(p.fin_frag + ((p.npad / 32) * 16 + (lrow & 3) * 4 + lq) * 4);
-    }
-    // channels that nothing ever writes: of the start block all but the image's, of the others the groups that the
-    // rows of the level below do not have; and the padding of the patch's rows
     const int below_groups = p.below_stride / 8;
-    for (int i = threadIdx.x; i < kPatch * (GROUPS + 1); i += THREADS)
-        if (i % (GROUPS + 1) >= below_groups) *reinterpret_cast<half8*>(s_patch + (i / (GROUPS + 1)) * ROW + 8 * (i % (GROUPS + 1))) = half8{};
-
     // ---- this thread's share of the loads of a tile ----
     struct Loads
     {
@@ -195,6 +163,65 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
             }
         }
     };
+    // Consecutive tiles share their halos: they go to one XCD (workgroups are dealt to the eight of them in turn). The XCDs'
+    // shares differ by one tile at most, the first ones' being the larger as are their numbers of workgroups: with as many
+    // workgroups as tiles each has one. (With shares rounded up, a workgroup of some XCD took a second tile: 75 tiles of
+    // 32 -> 32, 11.0 instead of 8.2 us, of 64 -> 64 at 160 x 120, 19.5 instead of 13.1.)
+    const int xcd  = (int)blockIdx.x & 7, in_xcd = ((int)gridDim.x - xcd + 7) >> 3;
+    const int last = (xcd + 1) * (tiles >> 3) + min(xcd + 1, tiles & 7);
+    int at         = xcd * (tiles >> 3) + min(xcd, tiles & 7) + ((int)blockIdx.x >> 3);
+
+    // The first tile's loads travel while weights are staged and the patch is cleared, and the weights on their way to LDS
+    // are all requested together: a level of few tiles lasts as long as this and one tile (finest level of 160 x 120,
+    // 32 -> 64: 10.7 -> 9.8 us, start block of eight image channels: 9.5 -> 8.8).
+    Loads cur;
+    if (kAhead && KREG == 0 && at < last) issue(decode(at), (int)threadIdx.x, cur);
+
+    // ---- what stays for all tiles: weights, biases, the 1x1's weights ----
+    const half8* wsrc = reinterpret_cast<const half8*>(p.wfrag) + (size_t)gp * (9 * KB * 2 * 64) + lane;
+    half8 w[KREG > 0 ? 9 : 1][KREG > 0 ? KREG : 1][2];
+    if (KREG > 0)
+    {
+#pragma unroll
+        for (int t = 0; t < (KREG > 0 ? 9 : 1); ++t)
+#pragma unroll
+            for (int kb = 0; kb < KREG; ++kb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[t][kb][h] = wsrc[((t * KB + kb) * 2 + h) * 64];
+    }
+    constexpr int kRun = KLDS > 0 ? KLDS * 2 * 64 : 1;  // 16-byte words of a tap
+    constexpr int kStaged = PAIRS * 9 * KLDS * 2 * 64, WITEMS = (kStaged + THREADS - 1) / THREADS;
+    half8 staged[WITEMS > 0 ? WITEMS : 1];
+    {
+        const half8* src = reinterpret_cast<const half8*>(p.wfrag) + (size_t)blockIdx.y * PAIRS * (9 * KB * 2 * 64);
+#pragma unroll
+        for (int k = 0; k < WITEMS; ++k)
+        {
+            const int i = min((int)threadIdx.x + THREADS * k, kStaged - 1);
+            staged[k]   = src[KREG == 0 ? i : i / kRun * (KB * 2 * 64) + KREG * 2 * 64 + i % kRun];
+        }
+    }
+    const float4 bias_f = *reinterpret_cast<const float4*>(p.bias + gp * 32 + lq * 4);
+    const float4 bias_m = *reinterpret_cast<const float4*>(p.bias + gp * 32 + 16 + lq * 4);
+    // A operand of the 1x1: every lane group's rows hold the four outputs, of which group m keeps those of the strip's row m
+    // (the same number of selects as zero weights for the other rows, through which an infinite operand of one row would
+    // make all of them not a number)
+    half4 fw = half4{}, fimg = half4{};
+    if (p.final_out)
+    {
+        fw   = *reinterpret_cast<const half4*>(p.fin_frag + (gp * 16 + (lrow & 3) * 4 + lq) * 4);
+        fimg = *reinterpret_cast<const half4*>(p.fin_frag + ((p.npad / 32) * 16 + (lrow & 3) * 4 + lq) * 4);
+    }
+    if (kAhead && KREG > 0 && at < last) issue(decode(at), (int)threadIdx.x, cur);
+    // channels that nothing ever writes: of the start block all but the image's, of the others the groups that the
+    // rows of the level below do not have; and the padding of the patch's rows
+    for (int i = threadIdx.x; i < kPatch * (GROUPS + 1); i += THREADS)
+        if (i % (GROUPS + 1) >= below_groups) *reinterpret_cast<half8*>(s_patch + (i / (GROUPS + 1)) * ROW + 8 * (i % (GROUPS + 1))) = half8{};
+
+#pragma unroll
+    for (int k = 0; k < WITEMS; ++k)
+        if (kStaged % THREADS == 0 || (int)threadIdx.x + THREADS * k < kStaged) reinterpret_cast<half8*>(s_w)[threadIdx.x + THREADS * k] = staged[k];
+
     // ... and from the registers into the patch: the 2x upsampling on the way
     auto commit = [&](const Tile& t, int tid, Loads& r)
     {
@@ -242,16 +269,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
         }
     };
 
-    // Consecutive tiles share their halos: they go to one XCD (workgroups are dealt to the eight of them in turn). The XCDs'
-    // shares differ by one tile at most, the first ones' being the larger as are their numbers of workgroups: with as many
-    // workgroups as tiles each has one. (With shares rounded up, a workgroup of some XCD took a second tile: 75 tiles of
-    // 32 -> 32, 11.0 instead of 8.2 us, of 64 -> 64 at 160 x 120, 19.5 instead of 13.1.)
-    const int xcd  = (int)blockIdx.x & 7, in_xcd = ((int)gridDim.x - xcd + 7) >> 3;
-    const int last = (xcd + 1) * (tiles >> 3) + min(xcd + 1, tiles & 7);
-    int at         = xcd * (tiles >> 3) + min(xcd, tiles & 7) + ((int)blockIdx.x >> 3);
-
-    Loads cur;
-    if (kPrefetch && at < last) issue(decode(at), (int)threadIdx.x, cur);
     for (; at < last; at += in_xcd)
     {
         const Tile t = decode(at);
@@ -261,8 +278,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
         const int lane = tid & 63, lrow = lane & 15, lq = lane >> 4;
+        if (!kAhead) issue(t, tid, cur);
         __syncthreads();  // the previous tile's patch has been read (and the fills above are done)
-        if (!kPrefetch) issue(t, tid, cur);
         commit(t, tid, cur);
         __syncthreads();
         if (kPrefetch && at + in_xcd < last) issue(decode(at + in_xcd), tid, cur);  // travels during the taps and the epilogue
@@ -426,6 +443,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_P
                 }
             }
         } while (STRIPS > 1 && (strip += WAVES / PAIRS) < 16 / MB);
+        if (kAhead && !kPrefetch && at + in_xcd < last) issue(decode(at + in_xcd), tid, cur);
         if constexpr (PAIRS > 2)
             if (p.final_out)
             {
