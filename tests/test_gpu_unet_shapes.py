@@ -24,6 +24,10 @@ pytestmark = pytest.mark.gpu
     ([32, 24], 544, 272, 4, 1),     # enough tiles for two pairs per workgroup at both levels
     ([48, 64], 544, 272, 4, 1),     # ... at the coarser level only (the finest has three pairs)
     ([64, 64], 544, 136, 6, 2),
+    # image channels that end inside a group of eight, with upsampled ones behind them
+    ([24, 32, 32], 70, 41, 5, 2),
+    ([24, 48, 40], 70, 41, 7, 2),
+    ([40, 60, 56], 45, 50, 12, 1),
     # three and four pairs at the coarser levels, either side of the 512 tiles from which they share a workgroup:
     ([16, 48], 129, 65, 4, 35),     # 3 x 5 tiles x 35 images
     ([16, 48, 52], 126, 64, 4, 63), # 2 x 4 x 63: not enough
