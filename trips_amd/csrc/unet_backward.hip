@@ -1155,8 +1155,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
         else if (has_below)
         {
 #pragma unroll
-            for (int c = 0; c < CI; ++c)  // a run-time bound would put the register array into scratch memory
-                if (c < C) row[c] = _Float16(v[c]);
+            for (int g4 = 0; g4 < CI / 4; ++g4)  // (run-time bounds would put the register array into scratch memory)
+            {
+                if (4 * g4 + 4 <= C)
+                    *reinterpret_cast<half4*>(row + 4 * g4) =
+                        half4{_Float16(v[4 * g4]), _Float16(v[4 * g4 + 1]), _Float16(v[4 * g4 + 2]), _Float16(v[4 * g4 + 3])};
+                else
+                {
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        if (4 * g4 + i < C) row[4 * g4 + i] = _Float16(v[4 * g4 + i]);
+                }
+            }
         }
         else
         {

@@ -86,9 +86,15 @@ __device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8
         *reinterpret_cast<half4*>(dst + 4) = half4{v[4], v[5], v[6], v[7]};
     else
     {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (8 * g + i >= C) dst[i] = v[i];
+        // (the words of the image are there already)
+        const uint4 have = *reinterpret_cast<const uint4*>(dst), up = __builtin_bit_cast(uint4, v);
+        auto word = [C](int k, unsigned a, unsigned b)
+        {
+            const int n         = (C & 7) - 2 * k;  // halves of the word that are the image's
+            const unsigned mask = n >= 2 ? 0xffffffffu : n == 1 ? 0xffffu : 0u;
+            return (a & mask) | (b & ~mask);
+        };
+        *reinterpret_cast<uint4*>(dst) = make_uint4(word(0, have.x, up.x), word(1, have.y, up.y), word(2, have.z, up.z), word(3, have.w, up.w));
     }
 }
 
