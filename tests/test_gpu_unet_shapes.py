@@ -43,6 +43,9 @@ pytestmark = pytest.mark.gpu
     ([32, 32], 301, 203, 8, 3),     # ... one workgroup per CU, odd sizes
     ([16, 48], 301, 95, 2, 5),
     ([32, 48], 290, 131, 4, 3),     # 64 pre-activations x 64 inputs
+    # the weight gradient takes 128 pre-activations on 32 inputs in one workgroup from 512 tiles on
+    ([64, 32], 290, 131, 4, 3),     # 10 x 17 x 3: two short of it
+    ([62, 30], 290, 129, 3, 4),
 ])
 def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
     from tests.ref_unet import unet_forward

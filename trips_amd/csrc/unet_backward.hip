@@ -1513,26 +1513,23 @@ hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, h
 }
 
 template <int CI, bool FOUR>
-hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, int cin_pad, int npad, int groups, hipStream_t stream)
+hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, const LevelPlan& lv, hipStream_t stream)
 {
-    // 64 pre-activations to a workgroup at most (more would leave it no registers for a tile in flight: 64 x 128 in one
-    // workgroup spilled and took four times as long per tile as 64 x 64); the others are workgroups of their own
-    const int nt = wgrad_tile(npad);
 #define TRIPS_BW(CIN_, NT_)                                                                    \
-    if (cin_pad == CIN_ && nt == NT_)                                                          \
-        return p.bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(p, groups, npad / NT_, stream) \
-                           : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(p, groups, npad / NT_, stream);
-    TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
+    if (lv.cin_pad == CIN_ && lv.wgrad_tile == NT_)                                            \
+        return p.bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(p, lv.groups, lv.npad / NT_, stream) \
+                           : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(p, lv.groups, lv.npad / NT_, stream);
+    TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 128) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
 #undef TRIPS_BW
     return hipErrorInvalidValue;
 }
 
-hipError_t dispatch_bwd_weight(const BwdWeightParams& p, int cin_pad, int npad, int groups, hipStream_t stream)
+hipError_t dispatch_bwd_weight(const BwdWeightParams& p, const LevelPlan& lv, hipStream_t stream)
 {
-    if (p.c_feat == 4) return dispatch_bwd_weight_ci<4, true>(p, cin_pad, npad, groups, stream);
-    if (p.c_feat < 4) return dispatch_bwd_weight_ci<4, false>(p, cin_pad, npad, groups, stream);
-    if (p.c_feat <= 8) return dispatch_bwd_weight_ci<8, false>(p, cin_pad, npad, groups, stream);
-    return dispatch_bwd_weight_ci<16, false>(p, cin_pad, npad, groups, stream);
+    if (p.c_feat == 4) return dispatch_bwd_weight_ci<4, true>(p, lv, stream);
+    if (p.c_feat < 4) return dispatch_bwd_weight_ci<4, false>(p, lv, stream);
+    if (p.c_feat <= 8) return dispatch_bwd_weight_ci<8, false>(p, lv, stream);
+    return dispatch_bwd_weight_ci<16, false>(p, lv, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -1723,7 +1720,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             }
             if (want_w)
             {
-                hipError_t e = dispatch_bwd_weight(wp, lv.cin_pad, lv.npad, lv.groups, stream);
+                hipError_t e = dispatch_bwd_weight(wp, lv, stream);
                 if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
             }
         }

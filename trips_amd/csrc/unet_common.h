@@ -251,7 +251,10 @@ __device__ __forceinline__ void store_tile_nhwc(const _Float16* s_tile, int lds_
 // workgroup; how many ways the wavefronts split the 16-channel input blocks, the 16-channel pre-activation blocks and,
 // where there are more wavefronts than blocks, the rows of a tile.
 constexpr int wgrad_threads(int, int) { return 512; }
-constexpr int wgrad_tile(int npad) { return npad % 64 == 0 ? 64 : 32; }  // pre-activations of a workgroup
+// Pre-activations of a workgroup: 64 at most, so that a tile in flight has registers beside the sums (64 inputs x 128 in one
+// workgroup spilled and took four times as long per tile as 64 x 64). 32 x 128 fits, and where every workgroup has tiles to
+// walk it saves assembling the patch twice: 1920 x 1080, 272 -> 206 us; with 300 tiles 21 -> 23, with 30 9 -> 13.
+constexpr int wgrad_tile(int cin, int npad, long long tiles) { return npad == 128 && cin == 32 && tiles >= 512 ? 128 : npad % 64 == 0 ? 64 : 32; }
 constexpr int wgrad_cbw(int cin) { return cin / 16 < 4 ? cin / 16 : 4; }
 constexpr int wgrad_nbw(int cin, int npad)
 {
@@ -279,6 +282,7 @@ struct LevelPlan
     size_t part_off;    // partial weight gradients [groups][9][npad][cin_pad] fp32
     size_t sliced_off;  // partial sums of the partials [16][9][npad][cin_pad] fp32
     size_t bias_part_off;  // per-workgroup sums of the pre-activation gradients [groups][npad] fp32
+    int wgrad_tile;     // pre-activations of a workgroup of the weight-gradient kernel
     int groups;         // persistent workgroups of the weight-gradient kernel, for all images of the batch
 };
 
@@ -386,7 +390,8 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         // smallest shape, else one; those that share the pre-activations of a tile between them count together); every
         // further one would only add a set of partial sums to write and reduce (32 x 64 with two per CU: 64 instead of
         // 70 us at 1245 x 825, and 7 us more for the sums)
-        const int resident = 256 * (lv.cin_pad == 32 && wgrad_tile(lv.npad) == 32 ? 2 : 1) / (lv.npad / wgrad_tile(lv.npad));
+        lv.wgrad_tile      = wgrad_tile(lv.cin_pad, lv.npad, tiles);
+        const int resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1) / (lv.npad / lv.wgrad_tile);
         lv.groups          = tiles < resident ? (int)tiles : resident;
         lv.part_off     = bw;
         bw += align256((size_t)lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
