@@ -66,6 +66,25 @@ def test_unet_ctypes_mirrors_and_host_checks(tmp_path):
     assert lib.trips_unet_workspace_size(C.byref(d), C.byref(b)) == abi.TRIPS_ERR_UNSUPPORTED
 
 
+def test_unet_module_does_not_carry_buffer_sizes():
+    """What the library answers for its buffers is asked again in a process that loads a pickled module; a module pickled
+    before sizes were kept at all has no attribute for them."""
+    import pickle
+
+    from trips_amd import unet
+    net = unet.MultiScaleUnet2dDecOnlySmallFixed(unet.MultiScaleUnet2dParams(num_layers=2, num_input_layers=2, filters_network=[16, 32]))
+    assert not [k for k in net.__dict__ if "size" in k]
+    before = pickle.dumps(net.__dict__)
+    d = abi.make_unet_desc([16, 32], abi.layer_sizes(97, 45, 2))
+    lib, want = _lib.load(), []
+    for fn in (lib.trips_unet_workspace_size, lib.trips_unet_saved_size, lib.trips_unet_backward_workspace_size):
+        b = C.c_size_t(0)
+        assert fn(C.byref(d), C.byref(b)) == 0
+        want.append(b.value)
+    assert unet._buffer_sizes(bytes(d)) == tuple(want)
+    assert pickle.dumps(net.__dict__) == before
+
+
 def test_ctypes_mirrors_have_c_sizes(tmp_path):
     prog = tmp_path / "sizes.c"
     prog.write_text('#include <stdio.h>\n#include "trips_splat.h"\nint main(){printf("%zu %zu %zu %zu %zu %zu %zu\\n",'

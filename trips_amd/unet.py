@@ -10,6 +10,7 @@ forward() runs the HIP kernels (fp16 operands on the matrix cores, fp32 accumula
 records one graph node whose backward is the device backward. There is no CPU path.
 """
 import ctypes as C
+import functools
 import math
 from dataclasses import dataclass, field
 from typing import List
@@ -71,6 +72,18 @@ class UpsampleDecOnlySmallBlockFixed(torch.nn.Module):
         self.convolution = GatedBlock(in_channels, conv_out_channels)
 
 
+@functools.lru_cache(maxsize=64)
+def _buffer_sizes(desc):
+    """(forward workspace, saved state, backward workspace) in bytes for the bytes of a TripsUnetDesc. (Kept by the process and
+    not by the module: a pickled module would carry the sizes of one library into another.)"""
+    d, lib, got = abi.TripsUnetDesc.from_buffer_copy(desc), _lib.load(), []
+    for fn in (lib.trips_unet_workspace_size, lib.trips_unet_saved_size, lib.trips_unet_backward_workspace_size):
+        n = C.c_size_t(0)
+        _lib.check(fn(C.byref(d), C.byref(n)))
+        got.append(int(n.value))
+    return tuple(got)
+
+
 class _UnetFunction(torch.autograd.Function):
     """One graph node for the whole net: inputs (pyramid levels) and parameters in, image out."""
 
@@ -80,7 +93,7 @@ class _UnetFunction(torch.autograd.Function):
         ins = [t.detach() for t in tensors[:n_levels]]
         params = [t.detach() for t in tensors[n_levels:]]
         d = net.desc(ins)
-        saved = net._alloc("saved", net._sizes(d)[1], ins[0].device)
+        saved = net._alloc("saved", _buffer_sizes(bytes(d))[1], ins[0].device)
         out = net._run_forward(d, ins, params, saved)
         ctx_.net, ctx_.desc, ctx_.ins, ctx_.params, ctx_.saved = net, d, ins, params, saved
         return out
@@ -112,7 +125,6 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
             self.add_module(f"up{i + 1}", UpsampleDecOnlySmallBlockFixed(F[i + 1], out))
         self.final = torch.nn.Sequential(torch.nn.Conv2d(F[0], p.num_output_channels, 1), torch.nn.Identity())
         self._buffers_dev = {}
-        self._sizes_of = {}
         # A viewer sets this: the weights then count as unchanged from one no-grad forward to the next (they are packed
         # to fp16 once, not per frame). Whoever changes them in place afterwards (load_state_dict, an optimiser step)
         # calls invalidate_packed_weights().
@@ -164,21 +176,6 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
                                   batch=int(inputs[0].shape[0]))
 
     # ---- plumbing ----
-    def _sizes(self, d):
-        """(forward workspace, saved state, backward workspace) in bytes, kept per descriptor value."""
-        key = bytes(d)
-        got = self._sizes_of.get(key)
-        if got is None:
-            lib, got = _lib.load(), []
-            for fn in (lib.trips_unet_workspace_size, lib.trips_unet_saved_size, lib.trips_unet_backward_workspace_size):
-                n = C.c_size_t(0)
-                _lib.check(fn(C.byref(d), C.byref(n)))
-                got.append(int(n.value))
-            if len(self._sizes_of) >= 64:
-                self._sizes_of.clear()
-            self._sizes_of[key] = got
-        return got
-
     def _alloc(self, key, nbytes, dev):
         if key == "saved":  # one per forward: a later forward must not overwrite what an earlier graph still needs
             return get_context(dev.index or 0).alloc_bytes(nbytes)
@@ -208,7 +205,7 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
         dev = ins[0].device
         ctx = get_context(dev.index or 0)
         w, ptrs = self._weights_struct(params)
-        nbytes = self._sizes(d)[0]
+        nbytes = _buffer_sizes(bytes(d))[0]
         ws = self._alloc("forward", nbytes, dev)
         # the packed weights in the workspace stay valid while the weights do (reuse_packed_weights), for the same
         # buffer and level sizes
@@ -229,7 +226,7 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
         dev = ins[0].device
         ctx = get_context(dev.index or 0)
         w, _ = self._weights_struct(params)
-        nbytes = self._sizes(d)[2]
+        nbytes = _buffer_sizes(bytes(d))[2]
         ws = self._alloc("backward", nbytes, dev)
         L = self.params.num_layers
         g = abi.TripsUnetGrads()
