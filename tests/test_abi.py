@@ -143,6 +143,29 @@ def test_size_queries_and_layer_sizes_host_only():
     assert b.value == 2 * a.value
 
 
+def test_sizes_are_kept_by_the_fields_they_depend_on(monkeypatch):
+    """Another image, camera or crop of a loop is answered without the library; whatever changes a size is not."""
+    from trips_amd.renderer import SplatContext
+    ctx = SplatContext.__new__(SplatContext)
+    ctx.lib, ctx._sizes = _lib.load(), {}
+    asked = []
+    real = SplatContext.workspace_size
+    monkeypatch.setattr(SplatContext, "workspace_size", lambda self, d: asked.append(1) or real(self, d))
+
+    def desc(views=1, w=64, h=48, train=True, crop=(1.0, 1.0, 0.0, 0.0, 0.0), image=0, camera=0, **kw):
+        kw = dict(dict(num_points=5000, num_texels=5000, num_channels=4, num_layers=4, list_depth=16, num_images=9, num_cameras=9), **kw)
+        return abi.make_desc(views=[dict(w=w, h=h, image_index=image, camera_index=camera, crop_transform=crop)] * views, train=train, **kw)
+
+    first = ctx.sizes(desc())
+    for step in range(1, 9):
+        assert ctx.sizes(desc(crop=(1.0 + step, 1.0, 0.5 * step, 0.0, 0.0), image=step, camera=step, dist_cutoff=step)) == first
+    assert len(asked) == 1
+    for kw in (dict(num_points=6000), dict(num_channels=8), dict(num_layers=3), dict(list_depth=8), dict(views=2), dict(w=65), dict(h=47),
+               dict(train=False), dict(floor_layer_sizes=True, w=63), dict(w=63), dict(max_list_entries=100)):
+        d = desc(**kw)
+        assert ctx.sizes(d) == (real(ctx, d), ctx.saved_size(d) if d.train else 0), kw
+
+
 @pytest.mark.parametrize("field,value,code", [
     ("abi_version", 99, abi.TRIPS_ERR_INVALID_ARG),
     ("num_layers", 0, abi.TRIPS_ERR_INVALID_ARG),

@@ -62,14 +62,16 @@ class SplatContext:
         return int(b.value)
 
     def sizes(self, desc):
-        """(workspace, saved state) in bytes. Kept per descriptor value: a training or viewing loop asks with the same one
-        every step, and answering takes the library longer than looking it up."""
-        key = bytes(desc)
+        """(workspace, saved state) in bytes, the latter 0 for a descriptor of eval mode. Kept by the fields that they depend
+        on: a training loop takes another image and another crop every step, at one size."""
+        view = desc.views[0]
+        key = (desc.num_points, desc.num_channels, desc.num_layers, desc.list_depth, desc.num_views, desc.train,
+               desc.floor_layer_sizes, desc.max_list_entries, view.w, view.h)
         got = self._sizes.get(key)
         if got is None:
             if len(self._sizes) >= 64:
                 self._sizes.clear()
-            got = self._sizes[key] = (self.workspace_size(desc), self.saved_size(desc))
+            got = self._sizes[key] = (self.workspace_size(desc), self.saved_size(desc) if desc.train else 0)
         return got
 
     def alloc_bytes(self, n):
