@@ -325,9 +325,9 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     for (int i = threadIdx.x; i < NB; i += kBinThreads) row[i] = s_hist[i];
     if (threadIdx.x == 0)
     {
-        p.chunk_valid[blockIdx.x]                = next - begin;
-        p.chunk_valid[p.bin_groups + blockIdx.x] = s_flags;
-        p.chunk_valid[3 * p.bin_groups + blockIdx.x] = next_pair;
+        p.chunk_valid[blockIdx.x]                    = next - begin;
+        p.chunk_valid[p.bin_groups + blockIdx.x]     = s_flags;
+        p.chunk_valid[2 * p.bin_groups + blockIdx.x] = next_pair;
     }
 }
 
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(1024) void scan_plan_kernel(const int32_t* __restri
     const bool chunk = (int)threadIdx.x < G;  // (G <= 1024)
     const int valid = chunk ? chunk_valid[threadIdx.x] : 0;
     const int flags = chunk ? chunk_valid[G + threadIdx.x] : 0;
-    const int over  = chunk ? chunk_valid[3 * G + threadIdx.x] : 0;
+    const int over  = chunk ? chunk_valid[2 * G + threadIdx.x] : 0;
 
     auto wave_scan = [&](int x)
     {
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(1024) void scan_plan_kernel(const int32_t* __restri
     int first = wave_prefix(s_tiles, total) + inc_tiles - sum;  // first slot of the thread's first tile
     // number of every chunk's first overflow row
     const int first_over = wave_prefix(s_over, total_over) + inc_over - over;
-    if (chunk) chunk_valid[4 * G + threadIdx.x] = first_over;
+    if (chunk) chunk_valid[3 * G + threadIdx.x] = first_over;
     if (saved_chunk_valid && chunk) saved_chunk_valid[threadIdx.x] = valid;
     if (saved_chunk_valid && (int)threadIdx.x < kRetainedParts) saved_chunk_valid[G + threadIdx.x] = 0;  // (the blend adds)
     // slices of the tiles' entries that fit the capacity
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     int begin, end;
     chunk_point_range(p, begin, end);
     const int n      = p.chunk_valid[blockIdx.x];
-    const int pair_base = p.chunk_valid[4 * p.bin_groups + blockIdx.x];
+    const int pair_base = p.chunk_valid[3 * p.bin_groups + blockIdx.x];
     unsigned dropped = 0;
     constexpr int U  = 2;  // records of a thread in flight together
     for (int cid0 = begin + (int)threadIdx.x; cid0 < begin + n; cid0 += U * kBinThreads)

@@ -289,12 +289,15 @@ struct BackwardWorkspaceLayout
 
 struct WorkspaceLayout
 {
-    size_t chunk_valid;   // int32 [5 G]  per chunk of the binning kernels: valid points, flags, (unused), overflow rows of the
+    size_t chunk_valid;   // int32 [4 G]  per chunk of the binning kernels: valid points, flags, overflow rows of the
                           //              backward, and (from the scan) the number of the chunk's first overflow row
     size_t prec;         // float4 [N]         point records, when there is no saved state to hold them
-    size_t counts;       // int32 [Pi]   list length per cell (the points whose 2 x 2 footprint starts at that pixel)
+    size_t counts;       // int32 [Pi]   list length per cell (the points whose 2 x 2 footprint starts at that pixel): added up
+                         //              by the slices of tiles with more than kSliceEntries bin entries, whose counters are
+                         //              cleared per view, and written by one workgroup for every other tile
     size_t cursor;       // int32 [Pi]   first key of each cell's list (-1 - first candidate row for a long list)
-    size_t run;          // int32 [Pi]   keys of a cell already claimed by slices of a split tile (zeroed per view)
+    size_t run;          // int32 [Pi]   keys of a cell already claimed by slices of a split tile (cleared per view for tiles with
+                         //              more than kSliceEntries bin entries; undefined for every other tile)
     size_t slice_start;  // int32 [NB+1] exclusive scan of the slices of split tiles (0 for a tile that is not split)
     size_t long_count;   // int32 [1]    segments of long lists handed out so far
     size_t long_items;   // int2  [max_long_items] {first key, number of keys} of each segment of a long list

@@ -239,7 +239,7 @@ WorkspaceLayout workspace_layout(const TripsSplatDesc& d, const PyramidGeom& g)
     o += align256(sizeof(ViewHeader));
     o += align256(N * (size_t)record_floats(d.num_channels) * sizeof(float));
     w.chunk_valid = o;
-    o += align256((size_t)kBinGroups * (kBinThreads / 64) * sizeof(int32_t));
+    o += align256((size_t)kBinGroups * 4 * sizeof(int32_t));
     w.prec = o;
     o += align256(N * kPointRecordFloats * sizeof(float));
     w.counts = o;

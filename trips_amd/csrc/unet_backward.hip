@@ -309,6 +309,142 @@ __global__ __launch_bounds__(256) void final_reduce_kernel(const float* __restri
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// The 9-tap implicit-GEMM core of the data gradient. A operands are 16-byte LDS reads from a (8+2) x (32+2) pixel patch with
+// KIN channels innermost (row stride KIN + 8 halves). B operands (packed weights [tap][NOUT][KIN]) reach the matrix cores
+// through LDS as well: with every wavefront loading its own fragments from memory, each of a tile's wavefronts pulled the
+// level's whole weight set out of the L2 again, and that traffic, not the MFMAs, set the length of the tap loop. The rows
+// have the patch's bank-conflict-free layout. A tap's MFMAs take far less time than a round trip to the L2, so as many taps
+// as the LDS has room for are staged together: all nine (requested when the kernel starts; the tap loop then has neither
+// loads nor barriers), or three (the next three travel in registers while these are multiplied; two barriers per three
+// taps), or one (two buffers, one barrier per tap).
+// Each of the workgroup's eight wavefronts owns one row of the 8 x 32 output tile = two 16-pixel row blocks; acc[m][n] is
+// the 16 x 16 block of pixels m, outputs 16n .. 16n+15.
+constexpr int kTapThreads  = 512;
+constexpr int kTapLdsBytes = 28 * 1024;  // LDS that the staged taps of a workgroup may take
+template <int KIN, int NOUT>
+struct ConvTapStage
+{
+    static constexpr int NB    = NOUT / 16;
+    static constexpr int KB    = KIN / 32;
+    static constexpr int ROW   = KIN + kLdsChanPad;   // halves per output row of a tap in LDS
+    static constexpr int ITEMS = NOUT * KIN / 8;      // 16-byte words per tap
+    static constexpr int MB    = 16 / (kTapThreads / 64);  // 16-pixel row blocks of a wavefront
+    static constexpr int BUF   = NOUT * ROW;           // halves per tap in LDS
+    // taps staged together
+    static constexpr int T = 9 * BUF * 2 <= kTapLdsBytes ? 9 : 3 * BUF * 2 <= kTapLdsBytes ? 3 : 1;
+    static constexpr int STAGE_ITEMS = T * ITEMS;      // 16-byte words per stage
+    static constexpr int PER   = (STAGE_ITEMS + kTapThreads - 1) / kTapThreads;  // per thread
+    static constexpr int LDS_HALVES = (T == 1 ? 2 : T) * BUF;  // what the kernel provides at s_taps
+    half8 r[PER];
+};
+
+// this thread's share of taps `tap` .. `tap` + T - 1 from memory into registers (the packed weights are dense:
+// [tap][NOUT][KIN])
+template <int KIN, int NOUT>
+__device__ __forceinline__ void conv_tap_fetch(ConvTapStage<KIN, NOUT>& st, const _Float16* __restrict__ wpack, int tap)
+{
+    using S = ConvTapStage<KIN, NOUT>;
+    const half8* src = reinterpret_cast<const half8*>(wpack + (size_t)tap * NOUT * KIN);
+#pragma unroll
+    for (int j = 0; j < S::PER; ++j)
+    {
+        const int item = threadIdx.x + kTapThreads * j;
+        if (S::STAGE_ITEMS % kTapThreads == 0 || item < S::STAGE_ITEMS) st.r[j] = src[item];
+    }
+}
+
+// ... and from the registers into the tap buffers at s_tap (T of them, one after the other)
+template <int KIN, int NOUT>
+__device__ __forceinline__ void conv_tap_stage(const ConvTapStage<KIN, NOUT>& st, _Float16* s_tap)
+{
+    using S = ConvTapStage<KIN, NOUT>;
+#pragma unroll
+    for (int j = 0; j < S::PER; ++j)
+    {
+        const int item = threadIdx.x + kTapThreads * j;
+        if (S::STAGE_ITEMS % kTapThreads == 0 || item < S::STAGE_ITEMS)
+        {
+            const int t = item / S::ITEMS, w = item - t * S::ITEMS;
+            *reinterpret_cast<half8*>(s_tap + t * S::BUF + (w / (KIN / 8)) * S::ROW + (w % (KIN / 8)) * 8) = st.r[j];
+        }
+    }
+}
+
+// Precondition: the first T taps sit at s_taps (conv_tap_fetch(.., 0) + conv_tap_stage) and a barrier has passed since.
+// Every thread of the workgroup must call this (it contains barriers unless all nine taps are staged).
+// Result layout: lane l holds, of the 16 x 16 block acc[m][n], outputs 16n + (l / 16) * 4 .. + 3 of pixel l % 16, four
+// neighbouring channels of one pixel, which an epilogue can store as one 8-byte word (the weights are the MFMA's A operand).
+template <int KIN, int NOUT>
+__device__ __forceinline__ void conv_taps_mfma(const _Float16* s_patch, _Float16* s_taps, const _Float16* __restrict__ wpack,
+                                               ConvTapStage<KIN, NOUT>& st,
+                                               floatx4 (&acc)[ConvTapStage<KIN, NOUT>::MB][NOUT / 16])
+{
+    using S = ConvTapStage<KIN, NOUT>;
+    constexpr int MB = S::MB;
+    constexpr int ROW = KIN + kLdsChanPad;
+    constexpr int NB  = S::NB;
+    constexpr int KB  = S::KB;
+    constexpr int T   = S::T;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lrow = lane & 15, lk = (lane >> 4) * 8;
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+    {
+        const int dy = tap / 3, dx = tap - dy * 3;  // patch coordinates already include the halo
+        // the next stage's weights: requested before this stage's first tap is multiplied
+        if (T < 9 && tap % T == 0 && tap + T < 9) conv_tap_fetch(st, wpack, tap + T);
+        const _Float16* sb = s_taps + (T == 1 ? tap & 1 : tap % T) * S::BUF;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+        {
+            half8 bfrag[NB];
+#pragma unroll
+            for (int n = 0; n < NB; ++n) bfrag[n] = *reinterpret_cast<const half8*>(sb + (n * 16 + lrow) * S::ROW + kb * 32 + lk);
+#pragma unroll
+            for (int m = 0; m < MB; ++m)
+            {
+                const int r = wave, cb = m * 16;
+                const half8 a = *reinterpret_cast<const half8*>(s_patch + ((r + dy) * kConvPatchW + cb + lrow + dx) * ROW + kb * 32 + lk);
+#pragma unroll
+                for (int n = 0; n < NB; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bfrag[n], a, acc[m][n], 0, 0, 0);
+            }
+        }
+        if (T == 1)
+        {
+            if (tap + 1 < 9) conv_tap_stage(st, s_taps + ((tap + 1) & 1) * S::BUF);
+            __syncthreads();  // the next tap is in place; nobody reads this tap's buffer any more
+        }
+        else if (T < 9 && tap % T == T - 1 && tap + 1 < 9)
+        {
+            __syncthreads();  // nobody reads this stage's taps any more
+            conv_tap_stage(st, s_taps);
+            __syncthreads();  // the next stage is in place
+        }
+    }
+    if (T != 1) __syncthreads();  // (as after the last tap of the one-tap form: patch and taps may be overwritten now)
+}
+
+// Copies `groups` x 8 halves per pixel of an 8 x 32 tile staged in LDS ([256][lds_stride]) to a channels-innermost
+// image ([H][W][dst_stride]) with 16-byte stores: consecutive lanes write consecutive 16 bytes, so a tile row leaves
+// as whole lines (2-byte stores straight from the MFMA result layout cost twice the memory requests).
+__device__ __forceinline__ void store_tile_nhwc(const _Float16* s_tile, int lds_stride, int groups, _Float16* dst,
+                                                int dst_stride, int x0, int y0, int W, int H)
+{
+    for (int item = threadIdx.x; item < kConvTileH * kConvTileW * groups; item += kTapThreads)
+    {
+        const int g = item % groups, tp = item / groups;
+        const int y = y0 + tp / kConvTileW, x = x0 + tp % kConvTileW;
+        if (y < H && x < W)
+            *reinterpret_cast<half8*>(dst + ((size_t)y * W + x) * dst_stride + 8 * g) =
+                *reinterpret_cast<const half8*>(s_tile + (size_t)tp * lds_stride + 8 * g);
+    }
+}
+
 struct BwdDataParams
 {
     int H, W, c_feat;
@@ -321,8 +457,8 @@ struct BwdDataParams
 };
 
 // CI = image channels the kernel has room for (4, 8 or 16): positions [0, C) of the block input are the level's image.
-template <int KC, int NN, int THREADS, int CI>
-__global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
+template <int KC, int NN, int CI>
+__global__ __launch_bounds__(kTapThreads) void conv_bwd_data_kernel(BwdDataParams p)
 {
     {
         const size_t pixels = (size_t)(p.first_image + blockIdx.z) * p.H * p.W;
@@ -330,14 +466,14 @@ __global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
         p.d_feat += pixels * p.c_feat;
         p.d_in = p.d_in ? p.d_in + pixels * NN : nullptr;
     }
-    constexpr int MB = 16 / (THREADS / 64);  // 16-pixel row blocks of a wavefront: two rows of the tile, or one
+    constexpr int THREADS = kTapThreads, MB = ConvTapStage<KC, NN>::MB;
     constexpr int ROW    = KC + kLdsChanPad;
     constexpr int GROUPS = KC / 8;
     constexpr int NB     = NN / 16;
     extern __shared__ _Float16 smem[];
     _Float16* s_patch = smem;
     const int x0 = blockIdx.x * kConvTileW, y0 = blockIdx.y * kConvTileH;
-    ConvTapStage<KC, NN, THREADS> taps;
+    ConvTapStage<KC, NN> taps;
     conv_tap_fetch(taps, p.wt, 0);  // in flight while the patch is loaded
     _Float16* s_taps = s_patch + kConvPatchH * kConvPatchW * ROW;  // the staged taps of the weights
     // the patch of pre-activation gradients, four 16-byte loads of a thread in flight together
@@ -376,7 +512,7 @@ __global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
     conv_tap_stage(taps, s_taps);
     __syncthreads();
     floatx4 acc[MB][NB];
-    conv_taps_mfma<KC, NN, true, THREADS>(s_patch, s_taps, p.wt, taps, acc);  // a lane: four channels of one pixel
+    conv_taps_mfma<KC, NN>(s_patch, s_taps, p.wt, taps, acc);  // a lane: four channels of one pixel
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lrow = lane & 15;
     // ---- epilogue: the tile staged in LDS (the patch is no longer needed) and written channels innermost with
@@ -388,7 +524,7 @@ __global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
 #pragma unroll
     for (int m = 0; m < MB; ++m)
     {
-        const int tp = (MB == 4 ? 2 * wave + (m >> 1) : wave) * kConvTileW + (m & 1) * 16 + lrow;  // this lane's pixel of the block
+        const int tp = wave * kConvTileW + m * 16 + lrow;  // this lane's pixel of the block
 #pragma unroll
         for (int n = 0; n < NB; ++n)
         {
@@ -403,7 +539,7 @@ __global__ __launch_bounds__(THREADS) void conv_bwd_data_kernel(BwdDataParams p)
         }
     }
     __syncthreads();
-    if (p.d_in) store_tile_nhwc<THREADS>(s_out, OS, NN / 8, p.d_in, NN, x0, y0, p.W, p.H);
+    if (p.d_in) store_tile_nhwc(s_out, OS, NN / 8, p.d_in, NN, x0, y0, p.W, p.H);
     {
         const size_t plane = (size_t)p.H * p.W;
         const int y = y0 + threadIdx.x / kConvTileW, x = x0 + threadIdx.x % kConvTileW;
@@ -1020,9 +1156,33 @@ __device__ __forceinline__ void lds_read_pixel_windows(const _Float16* tile, int
     w[2] = out.h;
 }
 
+// Eight upsampled channels (group g of a patch row) into the row, whose positions [0, C) are the level's own image.
+// FOUR: C is exactly 4.
+template <bool FOUR>
+__device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8 v)
+{
+    _Float16* dst = row + 8 * g;
+    if (FOUR ? g > 0 : 8 * g >= C)
+        *reinterpret_cast<half8*>(dst) = v;
+    else if (FOUR)
+        *reinterpret_cast<half4*>(dst + 4) = half4{v[4], v[5], v[6], v[7]};
+    else
+    {
+        // (the words of the image are there already)
+        const uint4 have = *reinterpret_cast<const uint4*>(dst), up = __builtin_bit_cast(uint4, v);
+        auto word = [C](int k, unsigned a, unsigned b)
+        {
+            const int n         = (C & 7) - 2 * k;  // halves of the word that are the image's
+            const unsigned mask = n >= 2 ? 0xffffffffu : n == 1 ? 0xffffu : 0u;
+            return (a & mask) | (b & ~mask);
+        };
+        *reinterpret_cast<uint4*>(dst) = make_uint4(word(0, have.x, up.x), word(1, have.y, up.y), word(2, have.z, up.z), word(3, have.w, up.w));
+    }
+}
+
 // CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
-template <int CIN, int NPAD, bool BIAS, int THREADS, int CI, bool FOUR>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightParams p)
+template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
+__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightParams p)
 {
     constexpr int ROW    = CIN + kLdsChanPad;   // halves per pixel of the input patch
     constexpr int DS     = NPAD + kLdsChanPad;  // halves per pixel of the gradient tile
@@ -1035,10 +1195,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(CIN == 
     constexpr int CBW    = CB < 4 ? CB : 4;
     // (More wavefronts than 16 x 16 blocks to deal out: the wavefronts also split the rows of a tile, RW ways; the
     // shares are added up through LDS at the end.)
+    constexpr int THREADS = kWgradThreads;
     constexpr int WAVES  = THREADS / 64;
     constexpr int NBW    = wgrad_nbw(CIN, NPAD);
     constexpr int RW     = wgrad_row_split(CIN, NPAD);
-    static_assert(THREADS == wgrad_threads(CIN, NPAD) && CBW == wgrad_cbw(CIN), "work split");
+    static_assert(CBW == wgrad_cbw(CIN), "work split");
     constexpr int MYCB   = CB / CBW;
     constexpr int MYNB   = NB / NBW;
     constexpr int MYROWS = kConvTileH / RW;
@@ -1425,11 +1586,10 @@ template <int KC, int NN, int CI>
 hipError_t launch_bwd_data(const BwdDataParams& p, int batch, hipStream_t stream)
 {
     // the patch and the staged taps of the weights
-    const size_t lds_in  = ((size_t)kConvPatchH * kConvPatchW * (KC + kLdsChanPad) + ConvTapStage<KC, NN, 512>::LDS_HALVES) * sizeof(_Float16);
+    const size_t lds_in  = ((size_t)kConvPatchH * kConvPatchW * (KC + kLdsChanPad) + ConvTapStage<KC, NN>::LDS_HALVES) * sizeof(_Float16);
     const size_t lds_out = (size_t)kConvTileH * kConvTileW * ((NN + kLdsChanPad) * sizeof(_Float16) + CI * sizeof(float));
     const size_t lds     = std::max(lds_in, lds_out);
-    constexpr int THREADS = 512;  // eight wavefronts per tile, as in the forward convolution
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_data_kernel<KC, NN, THREADS, CI>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_data_kernel<KC, NN, CI>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     for (int b = 0; b < batch; b += kMaxGridImages)
@@ -1437,7 +1597,7 @@ hipError_t launch_bwd_data(const BwdDataParams& p, int batch, hipStream_t stream
         BwdDataParams q = p;
         q.first_image   = b;
         dim3 grid((p.W + kConvTileW - 1) / kConvTileW, (p.H + kConvTileH - 1) / kConvTileH, std::min(batch - b, kMaxGridImages));
-        hipLaunchKernelGGL((conv_bwd_data_kernel<KC, NN, THREADS, CI>), grid, dim3(THREADS), lds, stream, q);
+        hipLaunchKernelGGL((conv_bwd_data_kernel<KC, NN, CI>), grid, dim3(kTapThreads), lds, stream, q);
     }
     return hipGetLastError();
 }
@@ -1448,8 +1608,8 @@ hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int ci
     if (npad == KC_ && cin_pad == NN_)                                                       \
         return p.c_feat <= 4 ? launch_bwd_data<KC_, NN_, 4>(p, batch, stream)                       \
                              : p.c_feat <= 8 ? launch_bwd_data<KC_, NN_, 8>(p, batch, stream) : launch_bwd_data<KC_, NN_, 16>(p, batch, stream);
-    TRIPS_BD(32, 32) TRIPS_BD(64, 32) TRIPS_BD(96, 32) TRIPS_BD(128, 32)
-    TRIPS_BD(32, 64) TRIPS_BD(64, 64) TRIPS_BD(96, 64) TRIPS_BD(128, 64)
+    // (start blocks have at most 16 inputs; up to 64 pre-activations the others are conv_bwd_data_up_kernel's)
+    TRIPS_BD(32, 32) TRIPS_BD(64, 32) TRIPS_BD(96, 32) TRIPS_BD(128, 32) TRIPS_BD(96, 64) TRIPS_BD(128, 64)
 #undef TRIPS_BD
     return hipErrorInvalidValue;
 }
@@ -1501,14 +1661,13 @@ hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, i
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
 hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, hipStream_t stream)
 {
-    constexpr int THREADS = wgrad_threads(CIN, NPAD);
     const size_t lds = ((size_t)(kConvPatchH * kConvPatchW + kBelowH * kBelowW) * (CIN + kLdsChanPad) +
                         (size_t)kConvTileH * kConvTileW * (NPAD + kLdsChanPad)) *
                        sizeof(_Float16);  // up to 101 KB
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, THREADS, CI, FOUR>), dim3(groups, splits), dim3(THREADS), lds, stream, p);
+    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>), dim3(groups, splits), dim3(kWgradThreads), lds, stream, p);
     return hipGetLastError();
 }
 
@@ -1761,16 +1920,19 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
                     hipError_t e = dispatch_bwd_data_up(du, d.batch, lv.npad, lv.cin_pad, stream);
                     if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "data gradient launch (level %d): %s", i, hipGetErrorString(e));
                 }
-                const size_t items = (size_t)lb.H * lb.W * ((2 * C - 1) / 8 - C / 8 + 1 + lb.npad / 16);
-                for (up.first_image = fused ? d.batch : 0; up.first_image < d.batch; up.first_image += kMaxGridImages)
+                else
                 {
-                    const dim3 blocks((unsigned)std::min<size_t>((items + 255) / 256, 1u << 20), std::min(d.batch - up.first_image, kMaxGridImages));
-                    switch ((2 * C) & 7)
+                    const size_t items = (size_t)lb.H * lb.W * ((2 * C - 1) / 8 - C / 8 + 1 + lb.npad / 16);
+                    for (up.first_image = 0; up.first_image < d.batch; up.first_image += kMaxGridImages)
                     {
-                        case 0: hipLaunchKernelGGL(up2_adjoint_gate_kernel<0>, blocks, dim3(256), 0, stream, up); break;
-                        case 2: hipLaunchKernelGGL(up2_adjoint_gate_kernel<2>, blocks, dim3(256), 0, stream, up); break;
-                        case 4: hipLaunchKernelGGL(up2_adjoint_gate_kernel<4>, blocks, dim3(256), 0, stream, up); break;
-                        default: hipLaunchKernelGGL(up2_adjoint_gate_kernel<6>, blocks, dim3(256), 0, stream, up); break;
+                        const dim3 blocks((unsigned)std::min<size_t>((items + 255) / 256, 1u << 20), std::min(d.batch - up.first_image, kMaxGridImages));
+                        switch ((2 * C) & 7)
+                        {
+                            case 0: hipLaunchKernelGGL(up2_adjoint_gate_kernel<0>, blocks, dim3(256), 0, stream, up); break;
+                            case 2: hipLaunchKernelGGL(up2_adjoint_gate_kernel<2>, blocks, dim3(256), 0, stream, up); break;
+                            case 4: hipLaunchKernelGGL(up2_adjoint_gate_kernel<4>, blocks, dim3(256), 0, stream, up); break;
+                            default: hipLaunchKernelGGL(up2_adjoint_gate_kernel<6>, blocks, dim3(256), 0, stream, up); break;
+                        }
                     }
                 }
             }

@@ -43,8 +43,8 @@ __device__ __forceinline__ void up2_source(int dst, int in_size, int& i0, int& i
 // The 2 x 2 pixels that bilinear 2x upsampling (align_corners = false) makes between four neighbouring pixels of the
 // coarser level, v[0..3] = (upper left, upper right, lower left, lower right), eight channels in packed fp16. The
 // weights (products of 1/4 and 3/4) are exact, and a sum of products stays in fp16's range wherever its result does;
-// the separable form, along x, then along y, needs differences of neighbours, which need not (and 12 instead of 16
-// packed operations buy nothing here: see gated_conv3x3_kernel).
+// the separable form, along x, then along y, needs differences of neighbours, which need not (its 12 packed operations
+// instead of 16 made no difference in time).
 // `top` / `left`: the lower / right pixels are the image's first row / column, whose source is that of the coarser level
 // alone.
 __device__ __forceinline__ void upsample_quad(half8 a, half8 b, half8 c, half8 d, bool top, bool left, half8 (&v)[4])
@@ -74,183 +74,10 @@ __device__ __forceinline__ void upsample_quad(half8 a, half8 b, half8 c, half8 d
     }
 }
 
-// Eight upsampled channels (group g of a patch row) into the row, whose positions [0, C) are the level's own image.
-// FOUR: C is exactly 4.
-template <bool FOUR>
-__device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8 v)
-{
-    _Float16* dst = row + 8 * g;
-    if (FOUR ? g > 0 : 8 * g >= C)
-        *reinterpret_cast<half8*>(dst) = v;
-    else if (FOUR)
-        *reinterpret_cast<half4*>(dst + 4) = half4{v[4], v[5], v[6], v[7]};
-    else
-    {
-        // (the words of the image are there already)
-        const uint4 have = *reinterpret_cast<const uint4*>(dst), up = __builtin_bit_cast(uint4, v);
-        auto word = [C](int k, unsigned a, unsigned b)
-        {
-            const int n         = (C & 7) - 2 * k;  // halves of the word that are the image's
-            const unsigned mask = n >= 2 ? 0xffffffffu : n == 1 ? 0xffffu : 0u;
-            return (a & mask) | (b & ~mask);
-        };
-        *reinterpret_cast<uint4*>(dst) = make_uint4(word(0, have.x, up.x), word(1, have.y, up.y), word(2, have.z, up.z), word(3, have.w, up.w));
-    }
-}
-
-// The 9-tap implicit-GEMM core shared by the forward convolution and the data gradient. A operands are 16-byte LDS
-// reads from a (8+2) x (32+2) pixel patch with KIN channels innermost (row stride KIN + 8 halves). B operands (packed
-// weights [tap][NOUT][KIN]) reach the matrix cores through LDS as well: with every wavefront loading its own
-// fragments from memory, each of a tile's four wavefronts pulled the level's whole weight set (18 - 147 KB) out of
-// the L2 again, 0.6 GB per launch at the two finest levels, and that traffic, not the MFMAs, set the length of the
-// tap loop. Now the workgroup copies the weights into LDS and every wavefront reads its fragments from there: a
-// quarter of the L2 traffic, the same bank-conflict-free row layout as the patch. A tap's MFMAs take far less time
-// than a round trip to the L2, so as many taps as the LDS has room for are staged together: all nine (requested when
-// the kernel starts; the tap loop then has neither loads nor barriers), or three (the next three travel in
-// registers while these are multiplied; two barriers per three taps), or one (two buffers, one barrier per tap).
-// A wavefront owns two rows of the 8 x 32 output tile = four 16-pixel row blocks; acc[m][n] is the 16 x 16 block of
-// pixels m, outputs 16n .. 16n+15.
-// THREADS = threads of the workgroup: 256 (a wavefront owns two rows of the tile = four 16-pixel row blocks) or 512 (one
-// row = two row blocks).
-constexpr int kTapLdsBytes = 28 * 1024;  // LDS that the staged taps of a workgroup may take
-template <int KIN, int NOUT, int THREADS = 256>
-struct ConvTapStage
-{
-    static constexpr int NB    = NOUT / 16;
-    static constexpr int KB    = KIN / 32;
-    static constexpr int ROW   = KIN + kLdsChanPad;   // halves per output row of a tap in LDS
-    static constexpr int ITEMS = NOUT * KIN / 8;      // 16-byte words per tap
-    static constexpr int MB    = 16 / (THREADS / 64);  // 16-pixel row blocks of a wavefront
-    static constexpr int BUF   = NOUT * ROW;           // halves per tap in LDS
-    // taps staged together
-    static constexpr int T = 9 * BUF * 2 <= kTapLdsBytes ? 9 : 3 * BUF * 2 <= kTapLdsBytes ? 3 : 1;
-    static constexpr int STAGE_ITEMS = T * ITEMS;      // 16-byte words per stage
-    static constexpr int PER   = (STAGE_ITEMS + THREADS - 1) / THREADS;  // per thread
-    static constexpr int LDS_HALVES = (T == 1 ? 2 : T) * BUF;  // what the kernel provides at s_taps
-    half8 r[PER];
-};
-
-// this thread's share of taps `tap` .. `tap` + T - 1 from memory into registers (the packed weights are dense:
-// [tap][NOUT][KIN])
-template <int KIN, int NOUT, int THREADS>
-__device__ __forceinline__ void conv_tap_fetch(ConvTapStage<KIN, NOUT, THREADS>& st, const _Float16* __restrict__ wpack, int tap)
-{
-    using S = ConvTapStage<KIN, NOUT, THREADS>;
-    const half8* src = reinterpret_cast<const half8*>(wpack + (size_t)tap * NOUT * KIN);
-#pragma unroll
-    for (int j = 0; j < S::PER; ++j)
-    {
-        const int item = threadIdx.x + THREADS * j;
-        if (S::STAGE_ITEMS % THREADS == 0 || item < S::STAGE_ITEMS) st.r[j] = src[item];
-    }
-}
-
-// ... and from the registers into the tap buffers at s_tap (T of them, one after the other)
-template <int KIN, int NOUT, int THREADS>
-__device__ __forceinline__ void conv_tap_stage(const ConvTapStage<KIN, NOUT, THREADS>& st, _Float16* s_tap)
-{
-    using S = ConvTapStage<KIN, NOUT, THREADS>;
-#pragma unroll
-    for (int j = 0; j < S::PER; ++j)
-    {
-        const int item = threadIdx.x + THREADS * j;
-        if (S::STAGE_ITEMS % THREADS == 0 || item < S::STAGE_ITEMS)
-        {
-            const int t = item / S::ITEMS, w = item - t * S::ITEMS;
-            *reinterpret_cast<half8*>(s_tap + t * S::BUF + (w / (KIN / 8)) * S::ROW + (w % (KIN / 8)) * 8) = st.r[j];
-        }
-    }
-}
-
-// Precondition: the first T taps sit at s_taps (conv_tap_fetch(.., 0) + conv_tap_stage) and a barrier has passed since.
-// Every thread of the workgroup must call this (it contains barriers unless all nine taps are staged).
-// Result layout: lane l holds, of the 16 x 16 block acc[m][n], pixels (l / 16) * 4 .. + 3 of output 16n + l % 16; with
-// OUTPUTS_IN_ROWS (the operands of the MFMA exchanged) outputs 16n + (l / 16) * 4 .. + 3 of pixel l % 16, four
-// neighbouring channels of one pixel, which an epilogue can store as one 8-byte word.
-template <int KIN, int NOUT, bool OUTPUTS_IN_ROWS = false, int THREADS = 256>
-__device__ __forceinline__ void conv_taps_mfma(const _Float16* s_patch, _Float16* s_taps, const _Float16* __restrict__ wpack,
-                                               ConvTapStage<KIN, NOUT, THREADS>& st,
-                                               floatx4 (&acc)[ConvTapStage<KIN, NOUT, THREADS>::MB][NOUT / 16])
-{
-    using S = ConvTapStage<KIN, NOUT, THREADS>;
-    constexpr int MB = S::MB;
-    constexpr int ROW = KIN + kLdsChanPad;
-    constexpr int NB  = S::NB;
-    constexpr int KB  = S::KB;
-    constexpr int T   = S::T;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lrow = lane & 15, lk = (lane >> 4) * 8;
-#pragma unroll
-    for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int n = 0; n < NB; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tap = 0; tap < 9; ++tap)
-    {
-        const int dy = tap / 3, dx = tap - dy * 3;  // patch coordinates already include the halo
-        // the next stage's weights: requested before this stage's first tap is multiplied
-        if (T < 9 && tap % T == 0 && tap + T < 9) conv_tap_fetch(st, wpack, tap + T);
-        const _Float16* sb = s_taps + (T == 1 ? tap & 1 : tap % T) * S::BUF;
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-        {
-            half8 bfrag[NB];
-#pragma unroll
-            for (int n = 0; n < NB; ++n) bfrag[n] = *reinterpret_cast<const half8*>(sb + (n * 16 + lrow) * S::ROW + kb * 32 + lk);
-#pragma unroll
-            for (int m = 0; m < MB; ++m)
-            {
-                const int r = MB == 4 ? 2 * wave + (m >> 1) : wave, cb = (m & 1) * 16;
-                const half8 a = *reinterpret_cast<const half8*>(s_patch + ((r + dy) * kConvPatchW + cb + lrow + dx) * ROW + kb * 32 + lk);
-#pragma unroll
-                for (int n = 0; n < NB; ++n)
-                    acc[m][n] = OUTPUTS_IN_ROWS ? __builtin_amdgcn_mfma_f32_16x16x32_f16(bfrag[n], a, acc[m][n], 0, 0, 0)
-                                                : __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bfrag[n], acc[m][n], 0, 0, 0);
-            }
-        }
-        if (T == 1)
-        {
-            if (tap + 1 < 9) conv_tap_stage(st, s_taps + ((tap + 1) & 1) * S::BUF);
-            __syncthreads();  // the next tap is in place; nobody reads this tap's buffer any more
-        }
-        else if (T < 9 && tap % T == T - 1 && tap + 1 < 9)
-        {
-            __syncthreads();  // nobody reads this stage's taps any more
-            conv_tap_stage(st, s_taps);
-            __syncthreads();  // the next stage is in place
-        }
-    }
-    if (T != 1) __syncthreads();  // (as after the last tap of the one-tap form: patch and taps may be overwritten now)
-}
-
-// Copies `groups` x 8 halves per pixel of an 8 x 32 tile staged in LDS ([256][lds_stride]) to a channels-innermost
-// image ([H][W][dst_stride]) with 16-byte stores: consecutive lanes write consecutive 16 bytes, so a tile row leaves
-// as whole lines (2-byte stores straight from the MFMA result layout cost twice the memory requests). STREAM: with
-// the non-temporal hint, for data that nothing reads again soon.
-template <int THREADS = 256, bool STREAM = false>
-__device__ __forceinline__ void store_tile_nhwc(const _Float16* s_tile, int lds_stride, int groups, _Float16* dst,
-                                                int dst_stride, int x0, int y0, int W, int H)
-{
-    for (int item = threadIdx.x; item < kConvTileH * kConvTileW * groups; item += THREADS)
-    {
-        const int g = item % groups, tp = item / groups;
-        const int y = y0 + tp / kConvTileW, x = x0 + tp % kConvTileW;
-        if (y < H && x < W)
-        {
-            const half8 v = *reinterpret_cast<const half8*>(s_tile + (size_t)tp * lds_stride + 8 * g);
-            half8* to     = reinterpret_cast<half8*>(dst + ((size_t)y * W + x) * dst_stride + 8 * g);
-            if (STREAM)
-                __builtin_nontemporal_store(v, to);
-            else
-                *to = v;
-        }
-    }
-}
-
-// Work split of the weight-gradient kernel for a (padded input channels, padded pre-activations) shape: threads per
-// workgroup; how many ways the wavefronts split the 16-channel input blocks, the 16-channel pre-activation blocks and,
-// where there are more wavefronts than blocks, the rows of a tile.
-constexpr int wgrad_threads(int, int) { return 512; }
+// Work split of the weight-gradient kernel for a (padded input channels, padded pre-activations) shape: how many ways the
+// wavefronts split the 16-channel input blocks, the 16-channel pre-activation blocks and, where there are more wavefronts
+// than blocks, the rows of a tile.
+constexpr int kWgradThreads = 512;
 // Pre-activations of a workgroup: 64 at most, so that a tile in flight has registers beside the sums (64 inputs x 128 in one
 // workgroup spilled and took four times as long per tile as 64 x 64). 32 x 128 fits, and where every workgroup has tiles to
 // walk it saves assembling the patch twice: 1920 x 1080, 272 -> 206 us; with 300 tiles 21 -> 23, with 30 9 -> 13.
@@ -258,9 +85,9 @@ constexpr int wgrad_tile(int cin, int npad, long long tiles) { return npad == 12
 constexpr int wgrad_cbw(int cin) { return cin / 16 < 4 ? cin / 16 : 4; }
 constexpr int wgrad_nbw(int cin, int npad)
 {
-    return (wgrad_threads(cin, npad) / 64) / wgrad_cbw(cin) < npad / 16 ? (wgrad_threads(cin, npad) / 64) / wgrad_cbw(cin) : npad / 16;
+    return (kWgradThreads / 64) / wgrad_cbw(cin) < npad / 16 ? (kWgradThreads / 64) / wgrad_cbw(cin) : npad / 16;
 }
-constexpr int wgrad_row_split(int cin, int npad) { return (wgrad_threads(cin, npad) / 64) / (wgrad_cbw(cin) * wgrad_nbw(cin, npad)); }
+constexpr int wgrad_row_split(int cin, int npad) { return (kWgradThreads / 64) / (wgrad_cbw(cin) * wgrad_nbw(cin, npad)); }
 
 // ---- host-side plan of a network: per level the padded GEMM sizes and where its buffers live ----
 inline int round_up(int v, int m) { return (v + m - 1) / m * m; }
@@ -402,8 +229,9 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
     }
     {
         const size_t chunks = d.batch * (((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
-        // as many workgroups as are resident at once (three per CU at the kernel's 160 registers) walk the chunks: a
-        // second, partly filled round of one-chunk workgroups cost a third of the kernel's time
+        // as many workgroups as are resident at once walk the chunks (three per CU at the 162 registers of the instance for
+        // 16 image channels; the others, at 109 to 125, would leave room for a fourth): a second, partly filled round of
+        // one-chunk workgroups cost a third of the kernel's time
         np.final_groups     = chunks < 768 ? (int)chunks : 768;
         np.final_part_off   = bw;
         bw += align256((size_t)np.final_groups * kFinalPartFloats * sizeof(float));

@@ -51,12 +51,6 @@ struct ConvParams
     int final_cout;
 };
 
-// A loaded value that is only needed under a condition is otherwise loaded under that condition by the compiler, in a
-// branch that waits for it before it ends. Values passed through here exist where this is called, whatever they are
-// used for later: called for all loads of a stage after the last of them, it keeps them in flight together.
-__device__ __forceinline__ void loaded(float& v) { asm volatile("" : "+v"(v)); }
-__device__ __forceinline__ void loaded(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
-
 // One workgroup walks tiles of 8 x 32 pixels and computes PAIRS pairs of (16 feature, 16 mask) outputs of each. Its
 // wavefronts split the pairs and the tile: a wavefront owns one pair for STRIPS strips of 16 pixels x MB rows, so that its A
 // operands (LDS) are shared by the three vertical taps and a lane ends up with four features and the masks of the same
