@@ -264,6 +264,25 @@ def test_forward_mode_is_refused_without_a_graph_as_well():
             BlendPointCloud(info)
 
 
+@pytest.mark.parametrize("transform", ["vmap", "grad", "jvp", "functionalize"])
+def test_functional_transforms_are_refused_without_a_graph_as_well(transform):
+    from trips_amd.renderer import BlendPointCloud, NeuralScene
+    sc = scenes.tiny(n=200, w=32, h=24, f=30.0, num_layers=2, list_depth=16, seed=43)
+    ns = NeuralScene.from_arrays(sc)
+    info = _info(sc, ns, train=False)
+    texture = ns.texture.texture.detach()
+
+    def render(t):
+        ns.texture.texture = t
+        return tuple(BlendPointCloud(info))
+
+    f = torch.func
+    call = dict(vmap=lambda: f.vmap(render)(texture[None]), grad=lambda: f.grad(lambda t: render(t)[0].sum())(texture),
+                jvp=lambda: f.jvp(render, (texture,), (texture,)), functionalize=lambda: f.functionalize(render)(texture))[transform]
+    with torch.no_grad(), pytest.raises(RuntimeError, match="autograd.Function"):
+        call()
+
+
 def test_a_trace_without_a_graph_renders():
     """torch.jit.trace of the operator without gradients: the traced program renders what it is given."""
     from trips_amd.renderer import BlendPointCloud, NeuralScene

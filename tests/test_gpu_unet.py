@@ -51,7 +51,7 @@ def _compare(net, inputs, tol_rounded=2e-3, tol_fp32=2e-2):
     ([16, 24], 2, 37, 29),               # partial tiles everywhere
     ([20], 1, 40, 24),                   # start block only
     ([32, 64, 64], 3, 70, 50),           # 64 input channels at the finest level, whose kernel also holds the 1x1
-    ([16, 48, 32], 3, 70, 50),           # 40 outputs on 32 inputs: the one shape whose weight gradient runs four wavefronts
+    ([16, 48, 32], 3, 70, 50),           # 40 outputs on 32 inputs: three pairs of sixteen
 ])
 def test_unet_forward_matches_torch(filters, levels, w, h):
     net = _net(filters, levels, seed=levels)

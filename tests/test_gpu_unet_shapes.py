@@ -48,6 +48,10 @@ pytestmark = pytest.mark.gpu
     ([62, 30], 290, 129, 3, 4),
 ])
 def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
+    _held_to_restatement(filters, w, h, cin, batch)
+
+
+def _held_to_restatement(filters, w, h, cin, batch):
     from tests.ref_unet import unet_forward
     levels = len(filters)
     net = _net(filters, levels, seed=60 + w + cin, cin=cin)
@@ -67,6 +71,30 @@ def test_forward_and_gradients_at_dispatch_edges(filters, w, h, cin, batch):
         got, want = got.cpu().numpy(), want.numpy()
         scale = np.abs(want).max()
         assert np.abs(got - want).max() < GRAD_TOL * scale, f"{name}: {np.abs(got - want).max() / scale:.3e}"
+
+
+def _strip_steps(preact, inputs, cin, coarse_w, coarse_h, batch):
+    """Steps of a strip of the data gradient that takes the upsampling's adjoint with it: the fewest with which all strips
+    are resident at once. (Sizes in LDS: the patch, the ring of gradients, the image's share.)"""
+    image = 4 if cin <= 4 else 8 if cin <= 8 else 16
+    lds = 10 * 34 * (preact + 8) * 2 + 10 * 32 * (inputs + 8) * 2 + 8 * 32 * image * 4
+    per_cu = 2 if 2 * lds <= 160 * 1024 and preact * inputs <= 32 * 32 else 1
+    strips, steps = (coarse_w + 14) // 15 * batch, 1
+    while steps < (coarse_h + 4) // 4 and strips * ((coarse_h + 4 * steps - 2) // (4 * steps - 1)) > 256 * per_cu:
+        steps += 1
+    return steps
+
+
+@pytest.mark.parametrize("filters,preact,inputs,w,h,cin,batch", [
+    ([16, 32], 32, 32, 30, 800, 4, 24),  # two workgroups per CU
+    ([32, 32], 64, 32, 29, 799, 4, 15),
+    ([16, 48], 32, 64, 30, 800, 3, 15),  # block outputs that start at position 6
+    ([32, 48], 64, 64, 30, 799, 4, 15),
+])
+def test_gradients_through_strips_of_many_steps(filters, preact, inputs, w, h, cin, batch):
+    """The strips' rings of ten rows go on by eight: their first row is 0, 8, 6, 4, 2 and, in the sixth step, 0 again."""
+    assert _strip_steps(preact, inputs, cin, (w + 1) // 2, (h + 1) // 2, batch) >= 6
+    _held_to_restatement(filters, w, h, cin, batch)
 
 
 @pytest.mark.parametrize("filters,w,h,cin,batch", [
