@@ -31,17 +31,17 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "9ce256d47d0461803c4a2d1dff7e97db55acd3262ae72a0e5edf88d805124ed1"
+PMC_SOURCES_SHA256 = "14f2165ef7675dbf5de03cbc4b7e7224bee2e22f3e62b9af4fbd4273fb754787"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129115, 237081),
-    "bin_scatter": (95997, 167514),
+    "project_bin": (129116, 237345),
+    "bin_scatter": (95985, 166944),
     "tile_count": (13148, 2296),
-    "tile_scatter": (26680, 105764),
-    "cell_sort": (35343, 42137),
-    "blend": (317900, 195584),
-    "backward_prologue": (55, 265128),
-    "backward_tiles": (425427, 121570),
-    "backward_points": (297409, 234503),
+    "tile_scatter": (26677, 105766),
+    "cell_sort": (35344, 42151),
+    "blend": (319572, 195403),
+    "backward_prologue": (55, 265130),
+    "backward_tiles": (425689, 121568),
+    "backward_points": (297354, 234503),
     "adam_fused": (383788, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
