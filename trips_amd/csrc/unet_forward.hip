@@ -58,14 +58,14 @@ struct ConvParams
 // What bounds it: vector instructions (loads, upsampling, the gate's two exponentials), then the latency of the phases
 // between two barriers; the matrix cores are busy for a fifth of the time. Hence: what a tile's threads share is worked
 // out once per workgroup or on the scalar unit, the loads of the next tile travel during this one's products, and the
-// upsampling makes 2 x 2 pixels from one set of four neighbours (382 instead of 710 vector instructions per wavefront
+// upsampling makes 2 x 2 pixels from one set of four neighbours (385 instead of 710 vector instructions per wavefront
 // and 256-pixel tile at the finest level of the 16/32/64/64 net). 1920 x 1080, that net, per level, against one tile
-// per workgroup with LDS-staged epilogues: 106 -> 74, 61 -> 59, 38 -> 35, 14 -> 13 us.
+// per workgroup with LDS-staged epilogues: 100 -> 76, 59 -> 60, 36 -> 34, 13 -> 11 us.
 // KREG: the pair's weights of so many blocks of 32 inputs (9 taps: 72 registers each) stay in registers for all tiles of
 // the workgroup, the others are staged in LDS once. With 32 inputs all are (held in registers they leave room for half the
-// wavefronts: 121 us at the finest level, where six wavefronts per SIMD take 74 and four 83); with 64 none, but for three
-// pairs, where half of them in LDS let twelve wavefronts share the SIMDs evenly: 252 us for 64 -> 96 at 1920 x 1080, 364
-// with six wavefronts and all weights in registers.
+// wavefronts: 121 us at the finest level, where six wavefronts per SIMD, with 4 registers spilled, take 74 and four 83);
+// with 64 none, but for three pairs, where half of them in LDS let twelve wavefronts share the SIMDs evenly: 252 us for
+// 64 -> 96 at 1920 x 1080, 364 with six wavefronts and all weights in registers.
 // CI: image channels the kernel has room for (4, 8 or 16); FOUR: C is exactly 4, the splat's usual descriptor width
 template <int CIN, int PAIRS, int CI, bool FOUR, int THREADS, int KREG, int WAVES_PER_EU>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES_PER_EU))) void gated_conv3x3_kernel(const ConvParams p)
