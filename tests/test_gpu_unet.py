@@ -157,7 +157,7 @@ GRAD_TOL = 2e-2
     ([32, 32, 32, 32, 32], 5, 100, 60, 2, 4),  # shipped filters, odd sizes, two images
     ([16, 24], 2, 37, 29, 1, 4),               # partial tiles
     ([32, 64, 64], 3, 70, 50, 1, 4),           # 64 input channels at the finest level
-    ([16, 48, 32], 3, 70, 50, 2, 4),           # 40 outputs on 32 inputs (the weight gradient's four-wavefront shape)
+    ([16, 48, 32], 3, 70, 50, 2, 4),           # 40 outputs on 32 inputs: three pairs of sixteen
     # fewer than four image channels: the coarser level's outputs then start at a position of the finer block's input
     # that is not a multiple of eight
     ([16, 32, 64, 64], 4, 96, 72, 1, 3),       # 58 outputs below 64 inputs: no spare position
