@@ -56,6 +56,40 @@ def test_fused_adam_matches_oracle(oracle):
             np.testing.assert_allclose(gt["w"].cpu().numpy(), s["w"], rtol=2e-6, atol=1e-7, err_msg=f"tensor {i}")
 
 
+@pytest.mark.parametrize("steps_dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("n", [1, 3, 31, 32, 33, 255, 1024, 4099])
+def test_fused_adam_runs_of_unseen_elements(oracle, n, steps_dtype):
+    """Eight lanes (32 elements) skip or write a line together: elements without gradient keep their bits wherever the runs
+    begin and end, whatever they hold, also under a loss scale that is divided out; the others follow the oracle (tolerances
+    as above)."""
+    from tests.oracle_lib import fill_adam_tensor
+    from trips_amd.renderer import get_context
+    ctx = get_context(0)
+    rng = np.random.default_rng(n)
+    s = _mk(n, rng, lr=1e-2, loss_scale=128.0)
+    s["steps"], s["steps_dtype"] = np.zeros(n, steps_dtype), abi.TRIPS_STEPS_I32 if steps_dtype is np.int32 else abi.TRIPS_STEPS_I64
+    s["steps"][::5] = 7  # counters of a run that differ
+    seen = np.ones(n, bool)
+    for start, length in ((0, 32), (40, 3), (64, 31), (101, 64), (200, 33), (260, 700), (1024, 32), (2000, 2050)):
+        seen[start:start + length] = False
+    s["g"][:] = np.where(seen, rng.normal(0, 100, n), 0)
+    s["w"][~seen] = np.where(rng.random(int((~seen).sum())) < 0.5, np.nan, np.inf)
+    gpu = {k: (torch.as_tensor(v).cuda() if isinstance(v, np.ndarray) else v) for k, v in s.items()}
+    before = {k: s[k].copy() for k in ("w", "m", "v", "steps")}
+    d = abi.TripsAdamTensor()
+    fill_adam_tensor(d, gpu, lambda a: a.data_ptr())
+    ctx.adam_step([d])
+    torch.cuda.synchronize()
+    got = {k: gpu[k].cpu().numpy() for k in before}
+    for k, v in before.items():
+        assert got[k][~seen].tobytes() == v[~seen].tobytes(), k
+    oracle.adam_step([s])
+    np.testing.assert_array_equal(got["steps"], s["steps"])
+    np.testing.assert_allclose(got["m"], s["m"], rtol=1e-6, atol=1e-9)
+    np.testing.assert_allclose(got["v"], s["v"], rtol=1e-6, atol=1e-12)
+    np.testing.assert_allclose(got["w"], s["w"], rtol=2e-6, atol=1e-7)
+
+
 def test_myadam_optimizer_matches_oracle(oracle):
     from trips_amd.adam import MyAdam
     rng = np.random.default_rng(1)

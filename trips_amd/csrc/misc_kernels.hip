@@ -24,65 +24,103 @@ struct AdamTable
     int32_t n;
 };
 
+// What an optimiser step reads and writes passes through once: non-temporal accesses (16 bytes or a scalar each) keep it from
+// displacing, and from waiting for the displacement of, what the caches hold.
+typedef unsigned vu4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ T nt_load(const T* a)
+{
+    if constexpr (sizeof(T) == 16)
+        return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const vu4*>(a)));
+    else
+        return __builtin_nontemporal_load(a);
+}
+template <typename T>
+__device__ __forceinline__ void nt_store(const T& v, T* a)
+{
+    if constexpr (sizeof(T) == 16)
+        __builtin_nontemporal_store(__builtin_bit_cast(vu4, v), reinterpret_cast<vu4*>(a));
+    else
+        __builtin_nontemporal_store(v, a);
+}
+
 struct AdamScalars
 {
     float lr, beta1, beta2, eps, rel_wd, abs_wd, clip, lo, hi, loss_scale;
 };
 
-// beta^t for a step count t: by squaring in double precision, rounded to float once. (The library powf is some 400
-// instructions, and two of them per point were half of the packed kernel's work. The squarings' error doubles per
-// squaring from 2^-53: below a float's for any t < 2^28, and beta^t of a beta < 1 is zero long before that.)
-__device__ __forceinline__ float pow_step(float beta, uint32_t t)
+// beta1^t and beta2^t for a step count t: by squaring in double precision, rounded to float once. (The library powf is some
+// 400 instructions, and two of them per point were half of the packed kernel's work. The squarings' error doubles per
+// squaring from 2^-53: below a float's for any t < 2^28, and beta^t of a beta < 1 is zero long before that.) The loop runs
+// until the largest count of the wavefront is done: its squares are the same for every lane.
+__device__ __forceinline__ void pow_steps(float beta1, float beta2, uint32_t t, float& p1, float& p2)
 {
-    double r = 1.0, b = (double)beta;
-    while (t)
+    double r1 = 1.0, r2 = 1.0, b1 = (double)beta1, b2 = (double)beta2;
+    while (__ballot(t != 0u))
     {
-        if (t & 1u) r *= b;
-        b *= b;
+        const double n1 = r1 * b1, n2 = r2 * b2;
+        const bool bit  = (t & 1u) != 0u;
+        r1 = bit ? n1 : r1;
+        r2 = bit ? n2 : r2;
+        b1 *= b1;
+        b2 *= b2;
         t >>= 1;
     }
-    return (float)r;
+    p1 = (float)r1;
+    p2 = (float)r2;
 }
 
 // learning rate with the bias correction of step `current_step` (MyAdam.cu:66-68)
 __device__ __forceinline__ float adam_corrected_lr(const AdamScalars& h, uint32_t current_step)
 {
+    float p1, p2;
+    pow_steps(h.beta1, h.beta2, current_step, p1, p2);
     float learning_rate = h.lr;
-    learning_rate *= sqrtf(1 - pow_step(h.beta2, current_step)) / (1 - pow_step(h.beta1, current_step));
+    learning_rate *= sqrtf(1 - p2) / (1 - p1);
     return learning_rate;
 }
 
-// `lr_of_step`: the corrected learning rate of step `lr_step`, if the caller has it already (two powf, a square root
-// and a division that elements with equal counters share); lr_step = 0 for none.
-__device__ __forceinline__ bool adam_element(const AdamScalars& h, float gradient_raw, float weight_fp, float& m,
-                                             float& v, long long& step, float& new_weight, uint32_t lr_step = 0,
-                                             float lr_of_step = 0.f)
+// What the elements of a step with one corrected learning rate share.
+struct AdamRate
 {
-    float gradient = gradient_raw;
-    if (h.loss_scale != 1.f) gradient = gradient_raw / h.loss_scale;  // (a division by 1 changes nothing: skipped)
-    if (gradient == 0.f) return false;  // parameter not seen in this step (MyAdam.cu:57-61)
+    float lr, decay, ab;
+};
+__device__ __forceinline__ AdamRate adam_rate(const AdamScalars& h, float learning_rate)
+{
+    const float rel = h.rel_wd * learning_rate;
+    return AdamRate{learning_rate, 1 - rel, h.abs_wd * learning_rate};
+}
+
+// One element with a gradient (after the loss scale): moments and weight.
+__device__ __forceinline__ void adam_update(const AdamScalars& h, const AdamRate& r, float gradient, float& w, float& m, float& v)
+{
     const float gradient_sq   = gradient * gradient;
     const float first_moment  = h.beta1 * m + (1 - h.beta1) * gradient;
     const float second_moment = h.beta2 * v + (1 - h.beta2) * gradient_sq;
     m                         = first_moment;
     v                         = second_moment;
-    step                      = step + 1;
-    const uint32_t current_step = (uint32_t)step;
-    float learning_rate         = lr_of_step;
-    if (current_step != lr_step) learning_rate = adam_corrected_lr(h, current_step);
-    const float effective_learning_rate =
-        fminf(fmaxf(learning_rate / (sqrtf(second_moment) + h.eps), h.lo), h.hi);
-    const float rel            = h.rel_wd * learning_rate;
-    const float ab             = h.abs_wd * learning_rate;
-    const float decayed_weight = (1 - rel) * weight_fp - copysignf(ab, weight_fp);
-    float w                    = decayed_weight - effective_learning_rate * first_moment;
+    const float effective_learning_rate = fminf(fmaxf(r.lr / (sqrtf(second_moment) + h.eps), h.lo), h.hi);
+    const float decayed_weight          = r.decay * w - copysignf(r.ab, w);
+    float nw                            = decayed_weight - effective_learning_rate * first_moment;
     if (h.clip != 0.0f)
     {
         const float lo = -h.clip, hi = h.clip;
-        w = w < lo ? lo : (hi < w ? hi : w);
+        nw = nw < lo ? lo : (hi < nw ? hi : nw);
     }
-    new_weight = w;
-    return true;
+    w = nw;
+}
+
+// The gradients divided by the loss scale. A division by 1 changes nothing: skipped, in a branch of its own (the asm keeps
+// the compiler from working the divisions out in any case and choosing afterwards, a dozen instructions per element).
+template <int E>
+__device__ __forceinline__ void adam_unscale(float loss_scale, float (&g)[E])
+{
+    if (loss_scale != 1.f)
+    {
+        asm volatile("");
+#pragma unroll
+        for (int e = 0; e < E; ++e) g[e] = g[e] / loss_scale;
+    }
 }
 
 // STEP = long long (the reference's state tensor) or int
@@ -102,70 +140,95 @@ __device__ __forceinline__ void adam_block(const AdamTable& tab, int ti)
     {
         float* w       = reinterpret_cast<float*>(T.weights);
         const float* g = reinterpret_cast<const float*>(T.grads);
-        const float4 g4 = *reinterpret_cast<const float4*>(g + i0);
-        if (g4.x == 0.f && g4.y == 0.f && g4.z == 0.f && g4.w == 0.f) return;
-        float4 w4 = *reinterpret_cast<const float4*>(w + i0);
-        float4 m4 = *reinterpret_cast<const float4*>(mo + i0);
-        float4 v4 = *reinterpret_cast<const float4*>(vo + i0);
+        const float4 g4 = nt_load(reinterpret_cast<const float4*>(g + i0));
+        float ge[4]     = {g4.x, g4.y, g4.z, g4.w};
+        adam_unscale(h.loss_scale, ge);
+        // (A parameter not seen in this step stays as it is, MyAdam.cu:57-61.) Eight lanes share the 128-byte lines of every
+        // float array: they skip a line together or write all of it, unseen elements as they were read. (Lane by lane, the
+        // lines of a cloud with culled points leave in pieces, and non-temporal accesses then cost time instead of saving it:
+        // 10M elements with 64-bit counters, 39 % of them without a gradient, 98 us with ordinary accesses, 111 with
+        // non-temporal ones, 80 = 5.5 TB/s with whole lines.)
+        const bool some             = !(ge[0] == 0.f && ge[1] == 0.f && ge[2] == 0.f && ge[3] == 0.f);
+        const unsigned long long by = __ballot(some);
+        if (((by >> (threadIdx.x & 56u)) & 0xFFull) == 0) return;
+        const float4 w4 = nt_load(reinterpret_cast<const float4*>(w + i0));
+        const float4 m4 = nt_load(reinterpret_cast<const float4*>(mo + i0));
+        const float4 v4 = nt_load(reinterpret_cast<const float4*>(vo + i0));
         STEP s[4];
         if (sizeof(STEP) == 8)
         {
-            *reinterpret_cast<longlong2*>(&s[0]) = *reinterpret_cast<const longlong2*>(st + i0);
-            *reinterpret_cast<longlong2*>(&s[2]) = *reinterpret_cast<const longlong2*>(st + i0 + 2);
+            *reinterpret_cast<longlong2*>(&s[0]) = nt_load(reinterpret_cast<const longlong2*>(st + i0));
+            *reinterpret_cast<longlong2*>(&s[2]) = nt_load(reinterpret_cast<const longlong2*>(st + i0 + 2));
         }
         else
-            *reinterpret_cast<int4*>(&s[0]) = *reinterpret_cast<const int4*>(st + i0);
-        long long s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
-        // The four elements are mostly updated together, so their counters agree: the bias correction (two powf, a square
+            *reinterpret_cast<int4*>(&s[0]) = nt_load(reinterpret_cast<const int4*>(st + i0));
+        // The four elements are mostly updated together, so their counters agree: the bias correction (two powers, a square
         // root, a division) of the run's largest counter is computed once and taken by every element whose new counter
         // equals it.
-        const uint32_t top = (uint32_t)max(max(s0, s1), max(s2, s3)) + 1u;
-        const float top_lr = adam_corrected_lr(h, top);
-        float nw;
-        if (adam_element(h, g4.x, w4.x, m4.x, v4.x, s0, nw, top, top_lr)) w4.x = nw;
-        if (adam_element(h, g4.y, w4.y, m4.y, v4.y, s1, nw, top, top_lr)) w4.y = nw;
-        if (adam_element(h, g4.z, w4.z, m4.z, v4.z, s2, nw, top, top_lr)) w4.z = nw;
-        if (adam_element(h, g4.w, w4.w, m4.w, v4.w, s3, nw, top, top_lr)) w4.w = nw;
-        s[0] = (STEP)s0, s[1] = (STEP)s1, s[2] = (STEP)s2, s[3] = (STEP)s3;
-        *reinterpret_cast<float4*>(w + i0)  = w4;
-        *reinterpret_cast<float4*>(mo + i0) = m4;
-        *reinterpret_cast<float4*>(vo + i0) = v4;
+        const uint32_t top   = (uint32_t)max(max(s[0], s[1]), max(s[2], s[3])) + 1u;
+        const AdamRate top_r = adam_rate(h, adam_corrected_lr(h, top));
+        float we[4] = {w4.x, w4.y, w4.z, w4.w}, me[4] = {m4.x, m4.y, m4.z, m4.w}, ve[4] = {v4.x, v4.y, v4.z, v4.w};
+        bool others = false;  // some element with a gradient has another counter
+#pragma unroll
+        for (int k = 0; k < 4; ++k) others = others || (ge[k] != 0.f && (uint32_t)s[k] + 1u != top);
+        const bool any_others = __ballot(others) != 0ull;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            const bool seen = ge[k] != 0.f;
+            AdamRate r      = top_r;
+            if (any_others)  // (skipped by the whole wavefront in the usual case)
+            {
+                asm volatile("");
+                const uint32_t own = (uint32_t)s[k] + 1u;
+                if (seen && own != top) r = adam_rate(h, adam_corrected_lr(h, own));
+            }
+            float nw = we[k], nm = me[k], nv = ve[k];
+            adam_update(h, r, ge[k], nw, nm, nv);
+            we[k] = seen ? nw : we[k];
+            me[k] = seen ? nm : me[k];
+            ve[k] = seen ? nv : ve[k];
+            s[k]  = (STEP)((long long)s[k] + (seen ? 1 : 0));
+        }
+        nt_store(make_float4(we[0], we[1], we[2], we[3]), reinterpret_cast<float4*>(w + i0));
+        nt_store(make_float4(me[0], me[1], me[2], me[3]), reinterpret_cast<float4*>(mo + i0));
+        nt_store(make_float4(ve[0], ve[1], ve[2], ve[3]), reinterpret_cast<float4*>(vo + i0));
         if (sizeof(STEP) == 8)
         {
-            *reinterpret_cast<longlong2*>(st + i0)     = *reinterpret_cast<longlong2*>(&s[0]);
-            *reinterpret_cast<longlong2*>(st + i0 + 2) = *reinterpret_cast<longlong2*>(&s[2]);
+            nt_store(*reinterpret_cast<longlong2*>(&s[0]), reinterpret_cast<longlong2*>(st + i0));
+            nt_store(*reinterpret_cast<longlong2*>(&s[2]), reinterpret_cast<longlong2*>(st + i0 + 2));
         }
         else
-            *reinterpret_cast<int4*>(st + i0) = *reinterpret_cast<int4*>(&s[0]);
+            nt_store(*reinterpret_cast<int4*>(&s[0]), reinterpret_cast<int4*>(st + i0));
         return;
     }
     for (int k = 0; k < 4; ++k)
     {
         const long long i = i0 + k;
         if (i >= T.n) break;
-        float gr, wf;
+        float gr[1], wf;
         if (T.dtype == TRIPS_DTYPE_F64)
         {
-            gr = (float)reinterpret_cast<const double*>(T.grads)[i];
-            wf = (float)reinterpret_cast<double*>(T.weights)[i];
+            gr[0] = (float)reinterpret_cast<const double*>(T.grads)[i];
+            wf    = (float)reinterpret_cast<double*>(T.weights)[i];
         }
         else
         {
-            gr = reinterpret_cast<const float*>(T.grads)[i];
-            wf = reinterpret_cast<float*>(T.weights)[i];
+            gr[0] = reinterpret_cast<const float*>(T.grads)[i];
+            wf    = reinterpret_cast<float*>(T.weights)[i];
         }
-        float m = mo[i], v = vo[i], nw;
-        long long s = st[i];
-        if (adam_element(h, gr, wf, m, v, s, nw))
-        {
-            mo[i] = m;
-            vo[i] = v;
-            st[i] = (STEP)s;
-            if (T.dtype == TRIPS_DTYPE_F64)
-                reinterpret_cast<double*>(T.weights)[i] = nw;
-            else
-                reinterpret_cast<float*>(T.weights)[i] = nw;
-        }
+        adam_unscale(h.loss_scale, gr);
+        if (gr[0] == 0.f) continue;
+        float m = mo[i], v = vo[i];
+        const long long s = (long long)st[i] + 1;
+        adam_update(h, adam_rate(h, adam_corrected_lr(h, (uint32_t)s)), gr[0], wf, m, v);
+        mo[i] = m;
+        vo[i] = v;
+        st[i] = (STEP)s;
+        if (T.dtype == TRIPS_DTYPE_F64)
+            reinterpret_cast<double*>(T.weights)[i] = wf;
+        else
+            reinterpret_cast<float*>(T.weights)[i] = wf;
     }
 }
 
@@ -216,7 +279,12 @@ hipError_t launch_adam(const TripsAdamTensor* tensors, int n_tensors, hipStream_
 // state arrays its state shares every line with its neighbours' and travels anyway; packed, the row of a point that
 // is skipped is never touched. Same arithmetic per element as adam_fused_kernel.
 // One thread per point. The rows of a wavefront's live points pass through LDS so that the accesses to memory stay
-// whole lines: 64 / CHUNKS rows per load instruction, lane = (row, 16-byte chunk).
+// whole lines: 64 / USED rows per load instruction, lane = (row, 16-byte word).
+// What bounds it: memory (6M points of four channels, 39 % of them culled: 1.30 GB in 224 us = 5.8 TB/s; a large copy runs at
+// 6.2). Gradients and rows are read once and rows written whole: non-temporal (278 us without; the weights, of which
+// live points write parts of lines, are not: 266 with). A third of its vector instructions were divisions by a loss scale
+// of one and two loops per bias correction; without them the time of four channels stayed and that of eight, whose rows in
+// LDS leave room for few wavefronts, went from 50 to 45 us at 300k points.
 struct AdamPointsParams
 {
     float *w_pos, *w_size, *w_tex, *w_conf;
@@ -224,30 +292,40 @@ struct AdamPointsParams
     uint4* state;  // [N][CHUNKS]
     long long tex_stride;  // elements between two descriptor rows
     int num_points;
+    int scaled;        // some tensor has a loss scale other than 1
     AdamScalars h[4];  // position, size, descriptors, confidence
 };
 
-template <int C, int CHUNKS>
-__global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams p)
+template <int C, int CHUNKS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void adam_points_kernel(const AdamPointsParams p)
 {
     constexpr int E   = 6 + C;
-    constexpr int LS  = CHUNKS + 1;  // LDS row stride in 16-byte words: an odd multiple spreads the rows over the banks
-    constexpr int RPP = 64 / CHUNKS;  // rows per load instruction
-    static_assert(3 * E <= 4 * CHUNKS, "row too short");
-    __shared__ uint4 s_rows[4][64 * LS];
-    __shared__ unsigned char s_list[4][64];
+    constexpr int USED = (3 * E + 15) / 16 * 4;  // 16-byte words of a row that travel: whole 64-byte pieces
+    constexpr int LS   = USED + 1;   // LDS row stride in 16-byte words: an odd multiple spreads the rows over the banks
+    constexpr int RPP  = 64 / USED;  // rows per load instruction
+    static_assert(USED <= CHUNKS, "row too short");
+    __shared__ uint4 s_rows[WAVES][64 * LS];
+    __shared__ unsigned char s_list[WAVES][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long first = (long long)blockIdx.x * 256 + wave * 64;  // first point of this wavefront
+    const long long first = (long long)blockIdx.x * (64 * WAVES) + wave * 64;  // first point of this wavefront
     const long long point = first + lane;
     const bool in         = point < p.num_points;
     float g[E];
     {
-        const float4 gp = in ? reinterpret_cast<const float4*>(p.g_pos)[point] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 gp = in ? nt_load(reinterpret_cast<const float4*>(p.g_pos) + point) : make_float4(0.f, 0.f, 0.f, 0.f);
         g[0] = gp.x, g[1] = gp.y, g[2] = gp.z, g[3] = gp.w;
-        g[4] = in ? p.g_size[point] : 0.f;
+        g[4] = in ? nt_load(p.g_size + point) : 0.f;
 #pragma unroll
-        for (int c = 0; c < C; ++c) g[5 + c] = in ? p.g_tex[c * p.tex_stride + point] : 0.f;
-        g[5 + C] = in ? p.g_conf[point] : 0.f;
+        for (int c = 0; c < C; ++c) g[5 + c] = in ? nt_load(p.g_tex + c * p.tex_stride + point) : 0.f;
+        g[5 + C] = in ? nt_load(p.g_conf + point) : 0.f;
+    }
+    auto tensor_of = [](int e) constexpr { return e < 4 ? 0 : e == 4 ? 1 : e < 5 + C ? 2 : 3; };
+    if (p.scaled)
+    {
+        asm volatile("");  // (kept out of the way of the usual case, as in adam_unscale)
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (p.h[tensor_of(e)].loss_scale != 1.f) g[e] = g[e] / p.h[tensor_of(e)].loss_scale;
     }
     bool live = false;
 #pragma unroll
@@ -272,7 +350,7 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
         for (int c = 0; c < C; ++c) w[5 + c] = p.w_tex[c * p.tex_stride + point];
         w[5 + C] = p.w_conf[point];
     }
-    const int my_r = lane / CHUNKS, my_c = lane - my_r * CHUNKS;
+    const int my_r = lane / USED, my_c = lane - my_r * USED;
     {
         // every load of the wavefront's rows is issued before the first one is waited for (as a loop that loads and
         // stores pass by pass the round trips to memory ran one after the other)
@@ -288,7 +366,7 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
             if (my_r < RPP && r < nlive)
             {
                 src[it] = s_list[wave][r];
-                v[it]   = p.state[(first + src[it]) * CHUNKS + my_c];
+                v[it]   = nt_load(p.state + (first + src[it]) * CHUNKS + my_c);
             }
         }
 #pragma unroll
@@ -300,9 +378,9 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (live)
     {
-        uint32_t row[4 * CHUNKS];
+        uint32_t row[4 * USED];
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j)
+        for (int j = 0; j < USED; ++j)
         {
             const uint4 t = s_rows[wave][lane * LS + j];
             row[4 * j] = t.x, row[4 * j + 1] = t.y, row[4 * j + 2] = t.z, row[4 * j + 3] = t.w;
@@ -311,38 +389,45 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
         // tensor's largest counter is computed once and taken by every element whose new counter equals it.
         int top[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-        {
-            const int t = e < 4 ? 0 : e == 4 ? 1 : e < 5 + C ? 2 : 3;
-            top[t]      = max(top[t], (int)row[3 * e + 2]);
-        }
+        for (int e = 0; e < E; ++e) top[tensor_of(e)] = max(top[tensor_of(e)], (int)row[3 * e + 2]);
         // (and tensors with the same learning rate and betas whose largest counters agree share it: usually all four)
-        float top_lr[4];
-        top_lr[0] = adam_corrected_lr(p.h[0], (uint32_t)(top[0] + 1));
+        AdamRate top_r[4];
+        const float lr0 = adam_corrected_lr(p.h[0], (uint32_t)(top[0] + 1));
+        top_r[0]        = adam_rate(p.h[0], lr0);
 #pragma unroll
         for (int t = 1; t < 4; ++t)
         {
             const bool same_scalars = p.h[t].lr == p.h[0].lr && p.h[t].beta1 == p.h[0].beta1 && p.h[t].beta2 == p.h[0].beta2;
             const bool shares       = same_scalars && top[t] == top[0];
-            top_lr[t]               = top_lr[0];
+            float lr                = lr0;
             if (__ballot(!shares))  // (skipped by the whole wavefront in the usual case)
             {
-                if (!shares) top_lr[t] = adam_corrected_lr(p.h[t], (uint32_t)(top[t] + 1));
+                if (!shares) lr = adam_corrected_lr(p.h[t], (uint32_t)(top[t] + 1));
             }
+            top_r[t] = adam_rate(p.h[t], lr);
         }
+        bool others = false;  // some element with a gradient has a counter of its own
+#pragma unroll
+        for (int e = 0; e < E; ++e) others = others || (g[e] != 0.f && (int)row[3 * e + 2] != top[tensor_of(e)]);
+        const bool any_others = __ballot(others) != 0ull;
 #pragma unroll
         for (int e = 0; e < E; ++e)
         {
-            const int t = e < 4 ? 0 : e == 4 ? 1 : e < 5 + C ? 2 : 3;
-            float m = __uint_as_float(row[3 * e]), v = __uint_as_float(row[3 * e + 1]), nw;
-            long long s = (long long)(int)row[3 * e + 2];
-            if (adam_element(p.h[t], g[e], w[e], m, v, s, nw, (uint32_t)(top[t] + 1), top_lr[t]))
+            const int t     = tensor_of(e);
+            const bool seen = g[e] != 0.f;
+            AdamRate r      = top_r[t];
+            if (any_others)  // (skipped by the whole wavefront in the usual case)
             {
-                w[e]           = nw;
-                row[3 * e]     = __float_as_uint(m);
-                row[3 * e + 1] = __float_as_uint(v);
-                row[3 * e + 2] = (uint32_t)(int)s;
+                asm volatile("");
+                const uint32_t own = row[3 * e + 2];
+                if (seen && (int)own != top[t]) r = adam_rate(p.h[t], adam_corrected_lr(p.h[t], own + 1u));
             }
+            float nw = w[e], nm = __uint_as_float(row[3 * e]), nv = __uint_as_float(row[3 * e + 1]);
+            adam_update(p.h[t], r, g[e], nw, nm, nv);
+            w[e]           = seen ? nw : w[e];
+            row[3 * e]     = seen ? __float_as_uint(nm) : row[3 * e];
+            row[3 * e + 1] = seen ? __float_as_uint(nv) : row[3 * e + 1];
+            row[3 * e + 2] += seen ? 1u : 0u;
         }
         reinterpret_cast<float4*>(p.w_pos)[point] = make_float4(w[0], w[1], w[2], w[3]);
         p.w_size[point]                          = w[4];
@@ -350,7 +435,7 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
         for (int c = 0; c < C; ++c) p.w_tex[c * p.tex_stride + point] = w[5 + c];
         p.w_conf[point] = w[5 + C];
 #pragma unroll
-        for (int j = 0; j < CHUNKS; ++j)
+        for (int j = 0; j < USED; ++j)
             s_rows[wave][lane * LS + j] = make_uint4(row[4 * j], row[4 * j + 1], row[4 * j + 2], row[4 * j + 3]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -362,7 +447,7 @@ __global__ __launch_bounds__(256) void adam_points_kernel(const AdamPointsParams
         if (my_r < RPP && r < nlive)
         {
             const int src                          = s_list[wave][r];
-            p.state[(first + src) * CHUNKS + my_c] = s_rows[wave][src * LS + my_c];
+            nt_store(s_rows[wave][src * LS + my_c], p.state + (first + src) * CHUNKS + my_c);
         }
     }
 }
@@ -383,20 +468,24 @@ hipError_t launch_adam_points(const TripsAdamTensor tensors[4], int num_points, 
     p.state      = reinterpret_cast<uint4*>(state);
     p.tex_stride = num_points;
     p.num_points = num_points;
+    p.scaled     = 0;
     for (int i = 0; i < 4; ++i)
     {
         const TripsAdamTensor& T = tensors[i];
+        if (T.loss_scale != 1.f) p.scaled = 1;
         p.h[i] = AdamScalars{T.lr, T.beta1, T.beta2, T.eps, T.relative_weight_decay, T.absolute_weight_decay,
                              T.weight_clipping_magnitude, T.lower_lr_bound, T.upper_lr_bound, T.loss_scale};
     }
-    const unsigned blocks = (unsigned)((num_points + 255) / 256);
+    // (a wavefront keeps to itself: with sixteen channels its rows take 22 KB of LDS, and workgroups of one wavefront fit
+    // seven to a CU where those of four fit one)
+    const unsigned blocks = (unsigned)((num_points + 255) / 256), blocks64 = (unsigned)((num_points + 63) / 64);
     switch (channels)
     {
-        case 3: hipLaunchKernelGGL((adam_points_kernel<3, 8>), dim3(blocks), dim3(256), 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((adam_points_kernel<4, 8>), dim3(blocks), dim3(256), 0, stream, p); break;
-        case 6: hipLaunchKernelGGL((adam_points_kernel<6, 16>), dim3(blocks), dim3(256), 0, stream, p); break;
-        case 8: hipLaunchKernelGGL((adam_points_kernel<8, 16>), dim3(blocks), dim3(256), 0, stream, p); break;
-        case 16: hipLaunchKernelGGL((adam_points_kernel<16, 24>), dim3(blocks), dim3(256), 0, stream, p); break;
+        case 3: hipLaunchKernelGGL((adam_points_kernel<3, 8, 4>), dim3(blocks), dim3(256), 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((adam_points_kernel<4, 8, 4>), dim3(blocks), dim3(256), 0, stream, p); break;
+        case 6: hipLaunchKernelGGL((adam_points_kernel<6, 16, 4>), dim3(blocks), dim3(256), 0, stream, p); break;
+        case 8: hipLaunchKernelGGL((adam_points_kernel<8, 16, 4>), dim3(blocks), dim3(256), 0, stream, p); break;
+        case 16: hipLaunchKernelGGL((adam_points_kernel<16, 24, 1>), dim3(blocks64), dim3(64), 0, stream, p); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
