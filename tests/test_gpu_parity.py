@@ -387,6 +387,31 @@ def test_tight_cluster_long_lists_and_split_tiles(oracle):
         small.ctx.check(small.workspace)
 
 
+@pytest.mark.parametrize("K", [8, 16])
+@pytest.mark.parametrize("channels", [4, 16])
+def test_lists_that_end_around_the_staged_keys(oracle, channels, K):
+    """Cells of one layer that hold 0 to 600 points, alone and beside each other: lists that end just before, at and after
+    the eight keys of a cell that the blend stages, pixels all of whose entries come from one cell, and from four."""
+    counts = [1, 7, 8, 9, 15, 16, 17, 33, 600]
+    cells = [(3 + 6 * i, 5, c) for i, c in enumerate(counts)]                                   # alone
+    cells += [(3 + 6 * i, 20, c) for i, c in enumerate(counts)] + [(4 + 6 * i, 20, d) for i, d in enumerate(counts[::-1])]
+    cells += [(3 + 6 * i + dx, 35 + dy, c) for i, c in enumerate([1, 2, 4, 8, 9, 16, 5, 3, 7]) for dx in (0, 1) for dy in (0, 1)]
+    n = sum(c for _, _, c in cells)
+    sc = scenes.tiny(n=n, w=64, h=48, f=60.0, num_layers=1, list_depth=K, seed=29, channels=channels, radius=(0.004, 0.02))
+    rng = np.random.default_rng(6)
+    at = np.concatenate([np.tile([[x, y]], (c, 1)) for x, y, c in cells]) + rng.uniform(0.05, 0.95, (n, 2))
+    z = rng.uniform(-0.2, 0.2, n)
+    order = rng.permutation(n)  # ids unrelated to the cells
+    # the camera looks along +z from z = -3; undo its projection (pixel = 60 x / depth + centre)
+    sc.position[order, 0] = ((at[:, 0] - 32.0) * (z + 3.0) / 60.0).astype(np.float32)
+    sc.position[order, 1] = ((at[:, 1] - 24.0) * (z + 3.0) / 60.0).astype(np.float32)
+    sc.position[order, 2] = z.astype(np.float32)
+    d = abi.desc_for_scene(sc)
+    _, ref, _ = _check_forward(oracle, sc, d)
+    assert {1, 7, 8, 9, 15, 16, 17, 33, 600} <= set(ref["lengths"][0].tolist())
+    _check_backward(oracle, sc, d, seed=5)
+
+
 def test_footprints_on_tile_and_image_borders_with_equal_depths(oracle):
     """A dense grid of points in a plane that faces the camera: footprints start at every pixel, also at the last
     column and row of a 32-pixel tile (their other pixels belong to the neighbouring tiles) and at the last pixels of

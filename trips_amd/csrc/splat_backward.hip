@@ -250,9 +250,6 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
 #pragma unroll
             for (int b = 0; b < BATCH; ++b)
             {
-                r0[b] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) rd[b][q] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (j0 + b < mmax && j0 + b < m)
                 {
                     const float4* rec = reinterpret_cast<const float4*>(p.rec + (size_t)(unsigned)id[j0 + b] * RF);

@@ -833,12 +833,11 @@ __global__ __launch_bounds__(THREADS) void tile_lists_kernel(const ForwardParams
 //   cell_sort_kernel   every cell's list sorted in place, ascending, and cut to its 16 smallest keys: a list of up to
 //                      8 keys by one lane (a sorting network over registers), a longer one by a 16-lane DPP row that
 //                      streams it in chunks of 16.
-//   blend_kernel       a wavefront owns an 8 x 8 block of pixels, one pixel per lane: a pixel with up to 8 entries
-//                      sorts them with a network, any other merges the (sorted, cut) lists of its four cells; then the
-//                      alpha blend front to back (RenderForward.cu:820-1048).
+//   blend_kernel       a wavefront owns an 8 x 8 block of pixels, one pixel per lane: a pixel merges the (sorted, cut) lists
+//                      of its four cells, then the alpha blend front to back (RenderForward.cu:820-1048).
 // A pixel's colour is summed in the order of a balanced binary tree over the list positions.
 constexpr int kLaneSortMax = 8;   // longest list that a lane sorts with a network
-constexpr int kStagedKeys  = 8;   // keys per cell that blend_kernel stages in LDS for the merging lanes
+constexpr int kStagedKeys  = 8;   // keys per cell that blend_kernel stages in LDS
 
 // {first key (negative: a long list, whose candidates are in `cand`), readable keys, entries} of a cell
 __device__ __forceinline__ int4 cell_info(const ForwardParams& p, int cell)
@@ -897,19 +896,6 @@ __device__ __forceinline__ void sort_pair(u64& a, u64& b)
 {
     const bool sw = b < a;
     const u64 lo = sw ? b : a, hi = sw ? a : b;
-    a = lo;
-    b = hi;
-}
-// a key with a tag that travels with it
-struct TaggedKey
-{
-    u64 key;
-    int tag;
-};
-__device__ __forceinline__ void sort_pair(TaggedKey& a, TaggedKey& b)
-{
-    const bool sw = b.key < a.key;
-    const TaggedKey lo{sw ? b.key : a.key, sw ? b.tag : a.tag}, hi{sw ? a.key : b.key, sw ? a.tag : b.tag};
     a = lo;
     b = hi;
 }
@@ -1200,6 +1186,15 @@ __global__ __launch_bounds__(256) void cell_sort_kernel(const ForwardParams p)
 }
 
 // One pixel per lane, 8 x 8 pixels per wavefront, a quarter of a tile per workgroup (the four of a tile on one XCD).
+// A wavefront stages the first kStagedKeys keys of its 9 x 9 sorted cell lists in LDS, each lane one cell's, and a pixel
+// merges its four: the smallest of the four heads is the next list position, and the list that gave it moves on. The
+// records of BATCH positions are requested as the merge finds them, then those positions are blended.
+// What bounds it: vector instructions where neighbouring lanes share the records' lines, the gathers of the records where
+// points are in no order. Every key is thus read once per wavefront instead of by up to four pixels, and no lane waits for
+// another's way of sorting (pixels of up to eight keys used to sort them with a network, the others to merge behind a staging
+// loop that waited for memory eleven times): 1920 x 1080, without / with the saved state, 6M points in Morton order 107 ->
+// 91 us, 9M 134 -> 120, 1M in a ball 99 -> 89; 6M in no order 191 -> 191. A position's saved list leaves as soon as four are
+// known: with all sixteen kept the kernel took 140 registers of a lane, and a fourth wavefront per SIMD is worth 4 %.
 template <int C, bool TRAIN>
 __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
 {
@@ -1207,8 +1202,10 @@ __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
     constexpr int RF   = 4 + CPAD;  // floats per blend record
     constexpr int NQ   = CPAD / 4;
     constexpr int BATCH = CPAD <= 8 ? 8 : 4;  // list positions whose records are requested together
-    __shared__ int4 s_cells[4][81];
-    __shared__ u64 s_keys[4][81 * kStagedKeys];
+    constexpr int CELLS = 81;
+    __shared__ int s_start[4][CELLS];               // as cell_info's
+    __shared__ unsigned s_info[4][CELLS];           // readable keys, at most kCellKeep, in bits 0..4; entries above
+    __shared__ u64 s_keys[4][kStagedKeys * CELLS];  // [key][cell], all-ones past a list's end
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NB   = p.geom.bin_off[p.num_layers];
@@ -1231,142 +1228,121 @@ __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
     // The block gathers from the 9 x 9 cells (gx0 - 1 .. gx0 + 7) x (gy0 - 1 .. gy0 + 7): one cell per lane, then
     // the 17 that are left; a pixel takes its four from LDS.
     {
-        const int i1 = lane, i2 = 64 + lane;
-        s_cells[wave][i1] = load_cell(p, tc, tc.x0 + bx - 1 + i1 % 9, tc.y0 + by - 1 + i1 / 9);
-        if (i2 < 81) s_cells[wave][i2] = load_cell(p, tc, tc.x0 + bx - 1 + i2 % 9, tc.y0 + by - 1 + i2 / 9);
+        const int i1 = lane, i2 = min(64 + lane, CELLS - 1);
+        const int4 a1 = load_cell(p, tc, tc.x0 + bx - 1 + i1 % 9, tc.y0 + by - 1 + i1 / 9);
+        const int4 a2 = load_cell(p, tc, tc.x0 + bx - 1 + i2 % 9, tc.y0 + by - 1 + i2 / 9);
+        // (the sum of a pixel's four lengths saturates at kMaxExportedLength: so may each of them)
+        s_start[wave][i1] = a1.x;
+        s_info[wave][i1]  = (unsigned)a1.y | ((unsigned)min(a1.z, kMaxExportedLength) << 5);
+        if (64 + lane < CELLS)
+        {
+            s_start[wave][i2] = a2.x;
+            s_info[wave][i2]  = (unsigned)a2.y | ((unsigned)min(a2.z, kMaxExportedLength) << 5);
+        }
+        // Keys and, in the place after the last of a shorter list, all-ones. Every key is requested before the first is
+        // stored.
+        const int r1 = min(a1.y, kStagedKeys), r2 = 64 + lane < CELLS ? min(a2.y, kStagedKeys) : 0;
+        const int qmax1 = wave_max_small<kStagedKeys>(r1), qmax2 = wave_max_small<kStagedKeys>(r2);
+        const u64* const k1 = cell_keys(p, a1.x);
+        const u64* const k2 = cell_keys(p, a2.x);
+        u64 v1[kStagedKeys], v2[kStagedKeys];
+#pragma unroll
+        for (int q = 0; q < kStagedKeys; ++q)
+        {
+            v1[q] = ~0ull;
+            if (q < qmax1 && q < r1) v1[q] = k1[q];
+        }
+#pragma unroll
+        for (int q = 0; q < kStagedKeys; ++q)
+        {
+            v2[q] = ~0ull;
+            if (q < qmax2 && q < r2) v2[q] = k2[q];
+        }
+#pragma unroll
+        for (int q = 0; q < kStagedKeys; ++q)
+            if (q <= qmax1) s_keys[wave][q * CELLS + i1] = v1[q];
+#pragma unroll
+        for (int q = 0; q < kStagedKeys; ++q)
+            if (q <= qmax2 && 64 + lane < CELLS) s_keys[wave][q * CELLS + i2] = v2[q];
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int ci0 = ly * 9 + lx;  // the pixel's cells: ci0, ci0 + 1, ci0 + 9, ci0 + 10
-    const int4 c0 = s_cells[wave][ci0], c1 = s_cells[wave][ci0 + 1], c2 = s_cells[wave][ci0 + 9], c3 = s_cells[wave][ci0 + 10];
-    const int total  = live ? c0.y + c1.y + c2.y + c3.y : 0;  // keys to choose from (each cell's cut to kCellKeep)
-    const int length = c0.z + c1.z + c2.z + c3.z;             // entries (0 for padding: its cells are empty)
-    const int n      = min(total, p.list_depth);              // list positions that hold an entry
-    const bool merges = total > kLaneSortMax;
+    int total = 0, length = 0;
+    {
+        const unsigned a = s_info[wave][ci0], b = s_info[wave][ci0 + 1], c = s_info[wave][ci0 + 9], d = s_info[wave][ci0 + 10];
+        total  = live ? (int)((a & 31u) + (b & 31u) + (c & 31u) + (d & 31u)) : 0;  // keys to choose from
+        length = (int)((a >> 5) + (b >> 5) + (c >> 5) + (d >> 5));                 // entries (0 for padding: its cells are empty)
+    }
+    const int n    = min(total, p.list_depth);  // list positions that hold an entry
+    const int nmax = wave_max_small<16>(n);     // longest list of the block
 
-    unsigned id[16];  // compact numbers of the pixel's entries, nearest first
+    unsigned id[4];  // compact numbers of four entries, nearest first (positions past n hold anything)
     // where each entry came from, for the backward: which of the pixel's four cells (bits 4..5) and its place in that
     // cell's sorted list (bits 0..3); one byte per list position, four positions per word
     unsigned tagw[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int j = 0; j < 16; ++j) id[j] = ~0u;
-
-    // ---- up to kLaneSortMax keys: load them all, sort with a network ----
-    {
-        const int mine = merges ? 0 : total;
-        const int nmax = wave_max_small<kLaneSortMax>(mine);
-        if (nmax > 0)
-        {
-            // position i of the concatenation of the four cell lists lies in cell (i >= o1) + (i >= o2) + (i >= o3)
-            // (sums of steps rather than a chain of selects: the compiler turns the chain into a table in memory);
-            // none of these cells has a long list
-            TaggedKey k[kLaneSortMax];
-            const int o1 = c0.y, o2 = o1 + c1.y, o3 = o2 + c2.y;
-            const int b0 = c0.x, b1 = c1.x - o1, b2 = c2.x - o2, b3 = c3.x - o3;
-#pragma unroll
-            for (int i = 0; i < kLaneSortMax; ++i)
-            {
-                k[i].key = ~0ull;
-                k[i].tag = 0;
-                if (i < nmax)
-                {
-                    const int base = b0 + (i >= o1 ? b1 - b0 : 0) + (i >= o2 ? b2 - b1 : 0) + (i >= o3 ? b3 - b2 : 0);
-                    if (i < mine) k[i].key = p.keys[(unsigned)(base + i)];
-                    // cell w, place i - (first position of cell w)
-                    if (TRAIN)
-                        k[i].tag = (((i >= o1) + (i >= o2) + (i >= o3)) << 4) |
-                                   (i - ((i >= o1 ? o1 : 0) + (i >= o2 ? o2 - o1 : 0) + (i >= o3 ? o3 - o2 : 0)));
-                }
-            }
-            lane_sort(k, nmax);
-#pragma unroll
-            for (int i = 0; i < kLaneSortMax; ++i)
-                if (i < mine)
-                {
-                    id[i] = (unsigned)k[i].key;
-                    tagw[i / 4] |= (unsigned)k[i].tag << (8 * (i & 3));
-                }
-        }
-    }
-    // ---- more: merge the four sorted cell lists. The first kStagedKeys keys of the block's cells wait in LDS; a
-    // lane that needs more of one cell reads them from memory. ----
-    const u64 merging = __ballot(merges);
-    if (merging)
-    {
-        // slot s = cell (s / kStagedKeys), key (s % kStagedKeys): kStagedKeys lanes read consecutive keys of a cell
-        static_assert(kStagedKeys == 8, "the slot arithmetic below");
-#pragma unroll 1
-        for (int s0 = 0; s0 < 81 * kStagedKeys; s0 += 64)
-        {
-            const int s = s0 + lane;
-            if (s < 81 * kStagedKeys)
-            {
-                const int4 c = s_cells[wave][s >> 3];
-                if ((s & 7) < c.y) s_keys[wave][s] = cell_keys(p, c.x)[s & 7];
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (merges)
-        {
-            const u64 kInf = ~0ull;
-            // key q of one of the pixel's cells (all-ones past its end)
-            auto key_of = [&](int ci, const int4& c, int q) -> u64
-            {
-                u64 v = kInf;
-                if (q < c.y) v = q < kStagedKeys ? s_keys[wave][ci * kStagedKeys + q] : cell_keys(p, c.x)[q];
-                return v;
-            };
-            u64 h0 = key_of(ci0, c0, 0), h1 = key_of(ci0 + 1, c1, 0), h2 = key_of(ci0 + 9, c2, 0), h3 = key_of(ci0 + 10, c3, 0);
-            int q0 = 0, q1 = 0, q2 = 0, q3 = 0;  // heads of the four lists
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-            {
-                if (j < n)
-                {
-                    const bool b01 = h1 < h0, b23 = h3 < h2;
-                    const u64 m01 = b01 ? h1 : h0, m23 = b23 ? h3 : h2;
-                    const bool hi = m23 < m01;
-                    id[j]         = (unsigned)(hi ? m23 : m01);
-                    const int w   = hi ? (b23 ? 3 : 2) : (b01 ? 1 : 0);  // the list that gave the key
-                    if (TRAIN) tagw[j / 4] |= (unsigned)((w << 4) | (w == 0 ? q0 : w == 1 ? q1 : w == 2 ? q2 : q3)) << (8 * (j & 3));
-                    q0 += w == 0, q1 += w == 1, q2 += w == 2, q3 += w == 3;
-                    if (j + 1 < n)
-                    {
-                        const int ci   = ci0 + (w & 1) + 9 * (w >> 1);
-                        const int4 c   = w == 0 ? c0 : w == 1 ? c1 : w == 2 ? c2 : c3;
-                        const int q    = w == 0 ? q0 : w == 1 ? q1 : w == 2 ? q2 : q3;
-                        const u64 next = key_of(ci, c, q);
-                        h0 = w == 0 ? next : h0, h1 = w == 1 ? next : h1, h2 = w == 2 ? next : h2, h3 = w == 3 ? next : h3;
-                    }
-                }
-            }
-        }
-    }
+    for (int j = 0; j < 4; ++j) id[j] = ~0u;
+    const u64* const keys = s_keys[wave] + ci0;
+    u64 h0 = keys[0], h1 = keys[1], h2 = keys[9], h3 = keys[10];
+    unsigned heads = 0x01010101u;  // a byte per list: place of the key after its head
 
     // ---- blend (RenderForward.cu:820-1048), front to back ----
-    const int nmax = wave_max_small<16>(n);  // longest list of the block
     TreeSum<C, 5> sum;  // (five levels: up to 16 positions)
     float T       = 1.f;
     float bgw     = 1.f;  // empty list -> 1
     int ret       = 0;    // length of the leading run of kept entries
     bool run_open = true;
     float4 r0[BATCH], rd[BATCH][NQ];
-    // one list position, its number a compile-time constant (the arrays indexed by it stay in registers)
+    // The next list position, its number a compile-time constant (the arrays indexed by it stay in registers): the smallest
+    // head, and the next key of the list that gave it. A lane whose list ends before walks on over what it finds.
+    auto merge = [&](auto jc)
+    {
+        constexpr int j = decltype(jc)::value;
+        const bool b01 = h1 < h0, b23 = h3 < h2;
+        const u64 m01 = b01 ? h1 : h0, m23 = b23 ? h3 : h2;
+        const bool hi = m23 < m01;
+        id[j % 4]     = (unsigned)(hi ? m23 : m01);
+        if (j < n)
+        {
+            const float4* rec = reinterpret_cast<const float4*>(p.rec + (size_t)id[j % 4] * RF);
+            r0[j % BATCH]     = rec[0];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) rd[j % BATCH][q] = rec[1 + q];
+        }
+        const unsigned shift = hi ? (b23 ? 24u : 16u) : (b01 ? 8u : 0u);  // 8 x the list that gave the key
+        const unsigned place = (heads >> shift) & 0xFFu;
+        if (TRAIN) tagw[j / 4] |= ((shift << 1) | (place - 1u)) << (8 * (j & 3));
+        heads += 1u << shift;
+        if (j == 15) return;
+        const unsigned cell = (0x0A090100u >> shift) & 0xFFu;  // of the list, from ci0
+        u64 next            = keys[__umul24(min(place, (unsigned)kStagedKeys - 1u), (unsigned)CELLS) + cell];
+        const bool further  = place >= (unsigned)kStagedKeys;
+        if (__ballot(further && j + 1 < n))  // keys that are not staged (few: of one list past its eighth)
+        {
+            if (further)
+            {
+                next           = ~0ull;
+                const int from = s_start[wave][ci0 + (int)cell];
+                if (place < (s_info[wave][ci0 + (int)cell] & 31u)) next = cell_keys(p, from)[place];
+            }
+        }
+        const bool w0 = !hi && !b01, w1 = !hi && b01, w2 = hi && !b23, w3 = hi && b23;
+        h0 = w0 ? next : h0, h1 = w1 ? next : h1, h2 = w2 ? next : h2, h3 = w3 ? next : h3;
+    };
     auto position = [&](auto jc)
     {
         constexpr int j = decltype(jc)::value;
         constexpr int b = j % BATCH;
-        const bool has  = j < n;
+        const bool has  = j < n;  // (otherwise the records of the position hold anything)
         float a         = 0.f;
         if (has) a = entry_alpha(r0[b], tc.layer, p.num_layers, gx, gy);
         const float Tc  = (T >= kAlphaDestCutoff) ? T : 0.f;
         const bool kept = has && Tc >= kAlphaDestCutoff;
         run_open        = run_open && kept;
         if (run_open) ret = j + 1;
-        const float wgt = has ? Tc * a : 0.f;
+        const float wgt = Tc * a;
         float pr[C];
 #pragma unroll
         for (int c = 0; c < C; ++c)
@@ -1380,24 +1356,25 @@ __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
         if (j == n - 1) bgw = (p.background_mode == TRIPS_BG_REFERENCE) ? Tc : T * (1.f - a);
         T = T * (1.f - a);
     };
-    // the records of BATCH positions are requested together, then the positions are walked
+    // four positions found and their records requested; the saved list holds four positions of the block's 64 pixels side by
+    // side (list_word)
+    auto merge4 = [&](auto first)
+    {
+        constexpr int j0 = decltype(first)::value;
+        if (j0 + 0 < nmax) merge(std::integral_constant<int, j0 + 0>{});
+        if (j0 + 1 < nmax) merge(std::integral_constant<int, j0 + 1>{});
+        if (j0 + 2 < nmax) merge(std::integral_constant<int, j0 + 2>{});
+        if (j0 + 3 < nmax) merge(std::integral_constant<int, j0 + 3>{});
+        if (TRAIN && j0 < nmax && j0 < n)
+            __builtin_nontemporal_store(vi4{(int)id[0], (int)id[1], (int)id[2], (int)id[3]},
+                                        reinterpret_cast<vi4*>(p.lists + list_word((unsigned)pix, j0, p.list_depth)));
+    };
+    // BATCH positions: found, their records requested, then blended
     auto batch = [&](auto first)
     {
         constexpr int j0 = decltype(first)::value;
-#pragma unroll
-        for (int b = 0; b < BATCH; ++b)
-        {
-            r0[b] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) rd[b][q] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (j0 + b < nmax && j0 + b < n)
-            {
-                const float4* rec = reinterpret_cast<const float4*>(p.rec + (size_t)id[j0 + b] * RF);
-                r0[b]             = rec[0];
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) rd[b][q] = rec[1 + q];
-            }
-        }
+        merge4(std::integral_constant<int, j0>{});
+        if constexpr (BATCH > 4) merge4(std::integral_constant<int, j0 + 4>{});
         if (j0 + 0 < nmax) position(std::integral_constant<int, j0 + 0>{});
         if (j0 + 1 < nmax) position(std::integral_constant<int, j0 + 1>{});
         if (j0 + 2 < nmax) position(std::integral_constant<int, j0 + 2>{});
@@ -1441,12 +1418,6 @@ __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
                                                  ((unsigned)min(length, kMaxExportedLength) << (2 * kRetainedBits)))
                                          : 0,
                                     p.retained + pix);
-        // four positions at a time, the block's 64 pixels side by side (list_word)
-        vi4* const mine = reinterpret_cast<vi4*>(p.lists + list_word((unsigned)pix, 0, p.list_depth));
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (4 * q < nmax && 4 * q < n)
-                __builtin_nontemporal_store(vi4{(int)id[4 * q], (int)id[4 * q + 1], (int)id[4 * q + 2], (int)id[4 * q + 3]}, mine + (q << 6));
         if (n > 0) __builtin_nontemporal_store(vu4{tagw[0], tagw[1], tagw[2], tagw[3]}, reinterpret_cast<vu4*>(p.tags) + (unsigned)pix);
         // the view's retained entries, for the backward's choice of how it keeps its pair rows: estimated from every
         // kRetainedSample-th workgroup, one atomic per wavefront (the sum of 64 values of at most 16, a ballot per bit),

@@ -65,35 +65,26 @@ __device__ __forceinline__ void log2_floor_ceil(float s, int& lo, int& hi)
 }
 
 // compute_point_size_fac (PointBlending.h:81-149) for s > 1 and more than one layer, the branch that interpolates
-// between two layers; written with selects only. (The other branch, 0.75 exp(s - 1) + 0.25 for a point that lands
-// in layer 0 only, is evaluated once per point by encode_size_field below.)
-// Between two layers the reference divides by 2^higher - 2^lower, which is 2^lower whenever the two differ (then
-// neither is clamped): multiplying by 2^-lower instead gives the same bits, the scaling being exact.
+// between two layers. (The other branch, 0.75 exp(s - 1) + 0.25 for a point that lands in layer 0 only, is evaluated once
+// per point by encode_size_field below.) `layer` must be one that the point is written to: at most ceil(log2 s).
+// With q = s / 2^layer (exact) the reference's cases are: q >= 2, a layer below both, 1; 1 <= q < 2, the lower layer,
+// 1 - (s - 2^layer) / 2^layer = 2 - q with the same rounding, or 1 if it is the last layer, where both are clamped to it;
+// 1/2 < q < 1, the higher layer, (s - 2^(layer - 1)) / 2^(layer - 1) = 2 q - 1, exact. The reference's derivative where the
+// two layers are the same is 1. (Size and layer are compared through q instead of through the bits of log2 s: 9 vector
+// instructions instead of 20, once per list entry of every pixel.)
 __device__ __forceinline__ float layer_factor_interpolated(float s, int layer, int max_layers, float* grad)
 {
-    int lo, hi;
-    log2_floor_ceil(s, lo, hi);  // lo >= 0 as s > 1
-    const int layer_lower = min(lo, max_layers - 1), layer_higher = min(hi, max_layers - 1);
-    const float l_l = __uint_as_float((uint32_t)(127 + layer_lower) << 23);  // 2^lower
-    const float inv = __uint_as_float((uint32_t)(127 - layer_lower) << 23);  // 2^-lower
-    float f         = (s - l_l) * inv;
-    float J         = inv;
-    if (layer == layer_lower)
+    const float m   = __uint_as_float((uint32_t)(127 - layer) << 23);  // 2^-layer
+    const float q   = s * m;
+    const bool last = layer == max_layers - 1;
+    float f         = (q < 2.f && !last) ? 2.f - q : 1.f;
+    f               = q < 1.f ? 2.f * q - 1.f : f;
+    if (grad)
     {
-        f = 1.f - f;
-        J = -J;
+        float J = q < 2.f ? -m : 0.f;
+        J       = (q == 1.f || last) ? 1.f : J;
+        *grad   = q < 1.f ? 2.f * m : J;
     }
-    if (layer_lower == layer_higher)
-    {
-        f = 1.f;
-        J = 1.f;
-    }
-    if (layer < layer_lower)
-    {
-        f = 1.f;
-        J = 0.f;
-    }
-    if (grad) *grad = J;
     return f;
 }
 
@@ -132,9 +123,9 @@ __device__ __forceinline__ float entry_alpha(const float4& r0, int layer, int nu
 {
     const float m  = __uint_as_float((uint32_t)(127 - layer) << 23);  // 2^-layer
     const float ux = r0.x * m, uy = r0.y * m;
-    float w        = (1.f - fabsf(ux - float(gx))) * (1.f - fabsf(uy - float(gy)));
-    if (fabsf(ux - float(gx)) > 1.f || fabsf(uy - float(gy)) > 1.f) w = 0.f;
-    float a = w * r0.w;
+    // (the reference's test for a distance above 1 never holds: the pixel is one of the four around (ux, uy))
+    const float w = (1.f - fabsf(ux - float(gx))) * (1.f - fabsf(uy - float(gy)));
+    float a       = w * r0.w;
     a *= layer_factor_encoded(r0.z, layer, num_layers);
     return a;
 }
