@@ -240,6 +240,36 @@ def test_backward_pair_row_forms_agree(oracle, scene):
             assert rel_err(got[2][k], got[1][k]) < 1e-6 and rel_err(got[0][k], got[1][k]) < 1e-6, k
 
 
+@pytest.mark.parametrize("n", [262144 + 64, 600011])
+def test_backward_points_queued_over_several_steps(oracle, n):
+    """More points than one step of the point pass takes: what a step queues and does not work off stays for the next, up
+    to the last, partly filled round. Both forms of the pair rows, overwriting (where one of them goes without the queue)
+    and adding, two views of which each culls most points: the same bits, and the oracle's."""
+    from tests.gpu_util import GpuRun, assert_grads_close
+    sc = scenes.tiny(n=n, w=120, h=90, f=300.0, num_layers=4, list_depth=16, seed=n % 97, radius=(0.002, 0.05), views=2)
+    d = abi.desc_for_scene(sc)
+    ref = oracle.forward(sc, d)
+    seen = [int(c[0]) for c in ref["counters"]]
+    assert all(100 < v < n // 2 for v in seen)
+    rng = np.random.default_rng(n)
+    grads = [rng.normal(0, 1, (2, d.num_channels, h, w)).astype(np.float32) for (w, h) in ref["sizes"]]
+    g_ref = oracle.backward(sc, d, ref, grads)
+    run = GpuRun(sc, d)
+    run.forward()
+    got = {}
+    try:
+        for mode in (1, 2):
+            run.ctx.pair_rows_mode(mode)
+            for overwrite in (False, True):
+                got[mode, overwrite] = {k: np.array(v, copy=True) for k, v in run.backward(grads, overwrite=overwrite).items()}
+    finally:
+        run.ctx.pair_rows_mode(0)
+    assert_grads_close(got[1, False], g_ref)
+    for k in ("d_texture", "d_confidence", "d_position", "d_point_size"):
+        for other in got.values():
+            np.testing.assert_array_equal(other[k], got[1, False][k], err_msg=k)
+
+
 @pytest.mark.parametrize("channels", [4, 16])
 def test_backward_points_written_to_many_layers(oracle, channels):
     """Every point is large enough for four to eight layers: a wavefront of the point pass then has several hundred

@@ -18,7 +18,7 @@
 //      the lanes, a lane collects the four corner pixels' entries and writes ONE row per pair: sum over the corners of
 //      T alpha dL/dimage and the four dL/dalpha. The rows of a point's first two layers sit at its compact number,
 //      further layers in an overflow table.
-//   2. points: the (point, layer) pairs of 64 consecutive points are dealt out to the lanes; a lane reads its pair's
+//   2. points: the (point, layer) pairs of 64 points are dealt out to the lanes; a lane reads its pair's
 //      row, evaluates the bilinear weights' Jacobian and the layer factor per corner (PointBlending.h:216-264,
 //      RenderBackward.cu:366-438); the point's own lane sums the image-space gradient of all its entries and runs the
 //      projection chain ONCE (the chain is linear in the image-space gradient, RenderBackward.cu:385-417), then stores
@@ -453,12 +453,20 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Pass 2: per point. A wavefront takes 64 consecutive points. The work of a point is one item per layer it was written
-// to; points differ in the layers they reach, so the items of the 64 points are dealt out to the lanes through LDS,
-// one item per lane and round (usually one or two rounds): the items of a round are consecutive (point, layer) pairs,
-// whose rows are consecutive in memory, and every lane works instead of all lanes walking the layers of the deepest
-// point. An item's sums return through LDS and each point adds its items up in layer order. What does not change from
-// point to point (camera, rotation matrix) waits in LDS rather than in registers.
+// Pass 2: per point. A wavefront walks 64 consecutive points at a time. Where only some of them have work (the flagged ones of
+// a view with few retained pairs, or the valid ones where gradients are added to what earlier views left) they are
+// queued, and worked off 64 together: all lanes work however many points a view culls or hides. What the others get in
+// overwrite mode is zero, stored at once. With rows for all pairs and overwriting, the 64 points of a step are worked off
+// as they are: through the queue their outputs would leave in parts of lines (6M points: 238 us instead of 175).
+// The work of a point is one item per layer it was written to; points differ in the layers they reach, so the items of the
+// 64 points are dealt out to the lanes through LDS, one item per lane and round: the items of a round are consecutive
+// (point, layer) pairs, whose rows are consecutive in memory. An item's sums return through LDS and each point adds its
+// items up in layer order. The camera's rotation is the same for all points and sits in scalar registers.
+// What bounds it: vector instructions and memory together. 6M points in no order (0.85 GB) 202 -> 175 us, 9M in Morton order
+// 200 -> 184, four crops of 2M 211 -> 157, four views of 4M clustered points, of which a view retains one in five, 602 ->
+// 299, against a step per 64 points whatever they hold, with the camera in LDS and the weights, their derivatives and the
+// layer factor worked out corner by corner. (Products and sums stay uncontracted and in this order: gradients of points that
+// many pixels pull apart are small differences of large terms.)
 constexpr int kItemFloats(int cpad) { return 4 + cpad; }  // {confidence, ip.x, ip.y, size} sums, then the descriptor's
 
 struct PointPassCamera
@@ -466,6 +474,20 @@ struct PointPassCamera
     Camera cam;
     float R[9];
 };
+
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
+// the camera of a view and its rotation matrix, in scalar registers
+__device__ __forceinline__ PointPassCamera load_uniform_camera(const BackwardParams& p)
+{
+    PointPassCamera u;
+    const Camera c = load_camera_bw(p.pose, p.intrinsics, p.view, p.dist_cutoff);
+    rotation_matrix(c.V, u.R);
+    for (int i = 0; i < 9; ++i) u.R[i] = uniform(u.R[i]);
+    u.cam   = c;
+    u.cam.V = Pose{uniform(c.V.qx), uniform(c.V.qy), uniform(c.V.qz), uniform(c.V.qw), uniform(c.V.tx), uniform(c.V.ty), uniform(c.V.tz)};
+    return u;
+}
 
 template <int C>
 __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardParams p)
@@ -477,267 +499,55 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
     constexpr int NACC = 6 + 5 + 8;  // pose, K, distortion
     constexpr int NIT  = kItemFloats(CPAD);
     const int lane     = threadIdx.x & 63;
-    const int wave     = threadIdx.x >> 6;
+    const int wave     = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool want_pose = p.d_pose != nullptr;
     const bool want_intr = p.d_intrinsics != nullptr;
     const bool want_size = p.d_point_size != nullptr;
     const bool identity  = p.header->not_identity == 0;  // index[pid] == pid for every point
     const bool overwrite = p.overwrite != 0;             // outputs are written, not added to
     const bool sparse    = *p.mode != 0;  // only the flagged rows exist
-    // In that mode every point stores all its outputs (zeros where it has no gradient), all lanes at one place, so that
-    // whole lines are written. (Descriptor columns other than the points' own, and all of them when the index is not
-    // the identity, were cleared by the prologue kernel.)
+    const bool direct    = overwrite && !sparse;  // every point's outputs are stored: as whole lines, without the queue
+    // In overwrite mode every point stores all its outputs, zeros where it has no gradient. (Descriptor columns other than
+    // the points' own, and all of them when the index is not the identity, were cleared by the prologue kernel.)
 
-    __shared__ PointPassCamera s_cam;
+    constexpr int kQueue = 128;  // fewer than 64 that wait and up to 64 more
+    __shared__ int s_pid[4][kQueue], s_cid[4][kQueue];
+    __shared__ unsigned char s_mask[4][kQueue];  // the layers whose rows the point's items read
     // what an item needs of its point {ip.x, ip.y, size field, confidence, size_px, softplus' * d size_px / d size,
-    // number of its first overflow row, compact number}, then the point in view space, kept here for the point's own lane
-    __shared__ float s_point[4][64][11];
+    // number of its first overflow row, compact number}
+    __shared__ float s_point[4][64][9];
     __shared__ unsigned short s_item[4][64 * TRIPS_MAX_LAYERS];  // lane of the point | layer << 8
     __shared__ __align__(16) float s_sums[4][64][NIT];           // sums of the items of one round
-    if (threadIdx.x == 0)
+    const PointPassCamera u = load_uniform_camera(p);
+    auto wave_fence         = []()
     {
-        s_cam.cam = load_camera_bw(p.pose, p.intrinsics, p.view, p.dist_cutoff);
-        rotation_matrix(s_cam.cam.V, s_cam.R);
-    }
-    __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
 
     // a thread sees a handful of points: its own sums stay in single precision, everything across threads is double
     float acc[NACC];
 #pragma unroll
     for (int i = 0; i < NACC; ++i) acc[i] = 0.f;
 
-    const int stride = (int)gridDim.x * 256;
-    // The compact number of a point is requested two steps ahead and its point record one step ahead, so that a step
-    // starts with both in hand (a step otherwise begins with two dependent round trips to memory).
-    const float4 kNoRecord = make_float4(0.f, -1.f, 0.f, 0.f);
-    int cid_cur = -1, cid_next = -1;
-    float4 tail_cur = kNoRecord;
+    auto store_gradients = [&](int pid, bool any, float conf_grad, float size_grad, const float (&tex_grad)[C], const float (&g_point)[3])
     {
-        const long long pid0 = (long long)blockIdx.x * 256 + (int)threadIdx.x;
-        if (pid0 < p.num_points) cid_cur = p.cid_of[pid0];
-        if (pid0 + stride < p.num_points) cid_next = p.cid_of[pid0 + stride];
-        if (cid_cur >= 0) tail_cur = reinterpret_cast<const float4*>(p.prec)[cid_cur];
-    }
-    for (int base = blockIdx.x * 256; base < p.num_points; base += stride)
-    {
-        asm volatile("" ::: "memory");  // what waits in LDS is read where it is used, in every step
-        const int pid = base + (int)threadIdx.x;
-        // the records of a valid point sit at its compact number (valid points numbered in point order: lanes that are
-        // neighbours here are neighbours there)
-        const int cid   = cid_cur;
-        const bool live = cid >= 0;
-        // {softplus'(raw size), depth, layers written, size_px}
-        const float4 tail = tail_cur;
-        {
-            // in flight during this step: the next step's point record, the compact number of the step after it
-            cid_cur              = cid_next;
-            tail_cur             = cid_cur >= 0 ? reinterpret_cast<const float4*>(p.prec)[cid_cur] : kNoRecord;
-            const long long pid3 = (long long)pid + 2ll * stride;
-            cid_next             = pid3 < p.num_points ? p.cid_of[pid3] : -1;
-        }
-        // {ip.x, ip.y, size field, confidence} of the blend record and the position: requested here, beside the point
-        // record, unless the flags decide first whether the point has any row at all
-        float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), pos = make_float4(0.f, 0.f, 0.f, 0.f);
-        auto load_point_inputs = [&]()
-        {
-            r0  = *reinterpret_cast<const float4*>(p.rec + (size_t)(unsigned)cid * RF);
-            pos = p.position[pid];
-            if (p.displacement)
-            {
-                const float* dsp = p.displacement + (size_t)pid * 3;
-                pos.x += dsp[0];
-                pos.y += dsp[1];
-                pos.z += dsp[2];
-            }
-        };
-        if (live && !sparse) load_point_inputs();
-        int max_layer = live ? __float_as_int(tail.z) : 0;
-        // (a point of one or two layers has no overflow rows, and its number there is not looked at)
-        const int first = max_layer > kInlineLayers ? p.over_first[cid] : 0;
-        // (rows past the capacity of the overflow table do not exist: the forward reported the overflow)
-        if (max_layer > kInlineLayers && (long long)first + (max_layer - kInlineLayers) > p.over_capacity)
-            max_layer = kInlineLayers + (int)max(0ll, p.over_capacity - first);
-        // the layers whose rows the point's items read: all it was written to, or those whose flag the tile pass set
-        unsigned layer_mask = (1u << max_layer) - 1u;
-        if (sparse && live)
-        {
-            // (one byte per layer at the point's compact number)
-            const unsigned long long eight = *reinterpret_cast<const unsigned long long*>(p.flags + (size_t)(unsigned)cid * TRIPS_MAX_LAYERS);
-            unsigned flagged = 0;
-#pragma unroll
-            for (int l = 0; l < TRIPS_MAX_LAYERS; ++l)
-                if ((eight >> (8 * l)) & 0xFFull) flagged |= 1u << l;
-            layer_mask &= flagged;
-            if (layer_mask) load_point_inputs();
-        }
-        if (live && layer_mask)
-        {
-            // the point in view space, exactly as the projection kernel computed it
-            float view[3];
-            transform_point(s_cam.cam.V, pos.x, pos.y, pos.z, view);
-            const float J_softmax_proj = s_cam.cam.fx * s_cam.cam.cfx / fmaxf(view[2], 0.f);
-            float* sp = s_point[wave][lane];
-            sp[0] = r0.x, sp[1] = r0.y, sp[2] = r0.z, sp[3] = r0.w, sp[4] = tail.w, sp[5] = tail.x * J_softmax_proj;
-            sp[6] = __int_as_float(first);
-            sp[7] = view[0], sp[8] = view[1], sp[9] = view[2];
-            sp[10] = __int_as_float(cid);
-        }
-
-        // ---- the point's items: the layers it was written to ----
-        const int my_items = (int)__popc(layer_mask);
-        int first_item     = my_items;  // inclusive prefix over the wavefront, then made exclusive
-        for (int o = 1; o < 64; o <<= 1)
-        {
-            const int t = __shfl_up(first_item, o);
-            if (lane >= o) first_item += t;
-        }
-        const int num_items = __builtin_amdgcn_readlane(first_item, 63);  // <= 64 * 8
-        first_item -= my_items;
-        {
-            int at = first_item;
-            for (int l = 0; l < max_layer; ++l)
-                if ((layer_mask >> l) & 1u) s_item[wave][at++] = (unsigned short)(lane | (l << 8));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        float conf_grad = 0.f, size_grad = 0.f, d0 = 0.f, d1 = 0.f;
-        float tex_grad[C];
-#pragma unroll
-        for (int c = 0; c < C; ++c) tex_grad[c] = 0.f;
-        bool any = false;  // some pixel retained the point
-
-        for (int round = 0; round < num_items; round += 64)
-        {
-            float i_conf = 0.f, i_d0 = 0.f, i_d1 = 0.f, i_size = 0.f;
-            float i_tex[CPAD];
-#pragma unroll
-            for (int c = 0; c < CPAD; ++c) i_tex[c] = 0.f;
-            if (round + lane < num_items)
-            {
-                // one layer of one point: its row holds the descriptor sums, then dL/dalpha of the four corners (zeros
-                // where no pixel retained the point)
-                const unsigned item = s_item[wave][round + lane];
-                const int layer     = (int)(item >> 8);
-                const float* sp     = s_point[wave][item & 63u];
-                const float ipx = sp[0], ipy = sp[1], size_field = sp[2], conf = sp[3], size_px = sp[4], size_chain = sp[5];
-                const vf4* row = reinterpret_cast<const vf4*>(
-                    layer < kInlineLayers ? p.rows_inline + ((size_t)(unsigned)__float_as_int(sp[10]) * kInlineLayers + layer) * PRF
-                                          : p.rows_over + ((size_t)__float_as_int(sp[6]) + (layer - kInlineLayers)) * PRF);
-                vf4 tq[NQ];
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) tq[q] = __builtin_nontemporal_load(row + q);
-                const vf4 gav     = __builtin_nontemporal_load(row + NQ);
-                const float ga[4] = {gav.x, gav.y, gav.z, gav.w};
-                const float mfac = 1.f / float(1 << layer);
-                const float ux = ipx * mfac, uy = ipy * mfac;
-                const float fx = floorf(ux), fy = floorf(uy);
-                const int px = (int)fx, py = (int)fy;
-                const float sx = ux - fx, sy = uy - fy;
-                float lfac = 1.f, J_lf = 0.f;
-                if (want_size) lfac = layer_factor_encoded_grad(size_field, size_px, layer, p.num_layers, &J_lf);
-#pragma unroll
-                for (int corner = 0; corner < 4; ++corner)
-                {
-                    const int gx = px + (corner & 1), gy = py + (corner >> 1);
-                    const float grad_alpha = ga[corner];
-                    // blend_fac_index / compute_blending_fac (PointBlending.h:216-264)
-                    // the four cases of the reference's switch on y_i + x_i as selects (same products, exact negations)
-                    const bool x_hi = !(float(gx) < ux), y_hi = !(float(gy) < uy);
-                    const float wx = x_hi ? sx : 1.f - sx, wy = y_hi ? sy : 1.f - sy;
-                    float blend    = wx * wy;
-                    const float J0 = x_hi ? wy : -wy;
-                    const float J1 = y_hi ? wx : -wx;
-                    if (fabsf(ux - float(gx)) > 1.f || fabsf(uy - float(gy)) > 1.f) blend *= 0.f;
-                    i_conf += blend * lfac * grad_alpha;
-                    const float gbs = conf * lfac * grad_alpha;
-                    i_d0 += J0 * gbs;
-                    i_d1 += J1 * gbs;
-                    if (want_size)
-                    {
-                        const float grad_layer_ps = size_chain * J_lf * grad_alpha;
-                        i_size += blend * conf * grad_layer_ps;
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < CPAD; ++c)
-                {
-                    const vf4 t4 = tq[c / 4];
-                    i_tex[c]     = (c & 3) == 0 ? t4.x : (c & 3) == 1 ? t4.y : (c & 3) == 2 ? t4.z : t4.w;
-                }
-                float4* out = reinterpret_cast<float4*>(s_sums[wave][lane]);
-                out[0]      = make_float4(i_conf, i_d0, i_d1, i_size);
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) out[1 + q] = make_float4(i_tex[4 * q], i_tex[4 * q + 1], i_tex[4 * q + 2], i_tex[4 * q + 3]);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // the point's items of this round, in layer order
-            const int j_end = min(first_item + my_items, round + 64);
-            for (int j = max(first_item, round); j < j_end; ++j)
-            {
-                const float4* in = reinterpret_cast<const float4*>(s_sums[wave][j - round]);
-                const float4 a   = in[0];
-                bool nz          = a.x != 0.f || a.y != 0.f || a.z != 0.f || a.w != 0.f;
-                conf_grad += a.x;
-                d0 += a.y;
-                d1 += a.z;
-                size_grad += a.w;
-#pragma unroll
-                for (int q = 0; q < NQ; ++q)
-                {
-                    const float4 t = in[1 + q];
-                    nz             = nz || t.x != 0.f || t.y != 0.f || t.z != 0.f || t.w != 0.f;
-                    if (4 * q < C) tex_grad[4 * q] += t.x;
-                    if (4 * q + 1 < C) tex_grad[4 * q + 1] += t.y;
-                    if (4 * q + 2 < C) tex_grad[4 * q + 2] += t.z;
-                    if (4 * q + 3 < C) tex_grad[4 * q + 3] += t.w;
-                }
-                any = any || nz;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        if (pid >= p.num_points || (!live && !overwrite)) continue;
-        const int tex = identity ? pid : p.index[pid];  // (a column outside the table: the point was culled)
-        if (!any && !overwrite) continue;
-
-        float g_point[3] = {0.f, 0.f, 0.f}, g_pose[6], g_k[5], g_dis[8];
-        if (any)
-        {
-            const float* sp = s_point[wave][lane];
-            project_backward(s_cam.cam, s_cam.R, sp[7], sp[8], sp[9], d0, d1, g_point, g_pose, g_k, g_dis, want_intr);
-            if (want_pose)
-            {
-#pragma unroll
-                for (int k = 0; k < 6; ++k) acc[k] += g_pose[k];
-            }
-            if (want_intr)
-            {
-#pragma unroll
-                for (int k = 0; k < 5; ++k) acc[6 + k] += g_k[k];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc[11 + k] += g_dis[k];
-            }
-        }
-
         if (identity && overwrite)
         {
 #pragma unroll
-            for (int c = 0; c < C; ++c) p.d_texture[(size_t)c * p.num_texels + tex] = tex_grad[c];
-            p.d_confidence[tex] = conf_grad;
+            for (int c = 0; c < C; ++c) p.d_texture[(size_t)c * p.num_texels + pid] = tex_grad[c];
+            p.d_confidence[pid] = conf_grad;
         }
         else if (identity)
         {
 #pragma unroll
-            for (int c = 0; c < C; ++c) p.d_texture[(size_t)c * p.num_texels + tex] += tex_grad[c];
-            p.d_confidence[tex] += conf_grad;
+            for (int c = 0; c < C; ++c) p.d_texture[(size_t)c * p.num_texels + pid] += tex_grad[c];
+            p.d_confidence[pid] += conf_grad;
         }
         else if (any)
         {
+            const int tex = p.index[pid];  // (a column outside the table: the point was culled)
 #pragma unroll
             for (int c = 0; c < C; ++c) unsafeAtomicAdd(p.d_texture + (size_t)c * p.num_texels + tex, tex_grad[c]);
             unsafeAtomicAdd(p.d_confidence + tex, conf_grad);
@@ -758,6 +568,221 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
             v.z += g_point[2];
             *dp = v;
         }
+    };
+
+    // one point per lane: number, compact number, the layers whose rows its items read (none: the point gets zeros)
+    auto work_off = [&](int pid, int cid, unsigned mask)
+    {
+        const bool has = mask != 0u;
+        int first      = 0;
+        // {softplus'(raw size), depth, layers written, size_px}; {ip.x, ip.y, size field, confidence} of the blend record
+        float4 tail = make_float4(0.f, 0.f, 0.f, 0.f), r0 = tail, pos = tail;
+        if (has)
+        {
+            // (a point of one or two layers has no overflow rows, and its number there is not looked at)
+            if (mask >> kInlineLayers) first = p.over_first[cid];
+            tail = reinterpret_cast<const float4*>(p.prec)[cid];
+            r0   = *reinterpret_cast<const float4*>(p.rec + (size_t)(unsigned)cid * RF);
+            pos  = p.position[pid];
+            if (p.displacement)
+            {
+                const float* dsp = p.displacement + (size_t)pid * 3;
+                pos.x += dsp[0];
+                pos.y += dsp[1];
+                pos.z += dsp[2];
+            }
+        }
+        // (rows past the capacity of the overflow table do not exist: the forward reported the overflow)
+        if (mask >> kInlineLayers)
+        {
+            const long long fit = p.over_capacity - first;
+            if (fit < TRIPS_MAX_LAYERS - kInlineLayers) mask &= (1u << (kInlineLayers + (int)max(0ll, fit))) - 1u;
+        }
+        // ---- the point's items: the layers it was written to ----
+        const int my_items = (int)__popc(mask);
+        int first_item     = my_items;  // inclusive prefix over the wavefront, then made exclusive
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const int t = __shfl_up(first_item, o);
+            if (lane >= o) first_item += t;
+        }
+        const int num_items = __builtin_amdgcn_readlane(first_item, 63);  // <= 64 * 8
+        first_item -= my_items;
+        {
+            int at = first_item;
+            for (unsigned m = mask; m; m &= m - 1u) s_item[wave][at++] = (unsigned short)(lane | ((__ffs((int)m) - 1) << 8));
+        }
+        // the point in view space, exactly as the projection kernel computed it
+        float view[3];
+        transform_point(u.cam.V, pos.x, pos.y, pos.z, view);
+        {
+            const float J_softmax_proj = u.cam.fx * u.cam.cfx / fmaxf(view[2], 0.f);
+            float* sp = s_point[wave][lane];
+            sp[0] = r0.x, sp[1] = r0.y, sp[2] = r0.z, sp[3] = r0.w, sp[4] = tail.w, sp[5] = tail.x * J_softmax_proj;
+            sp[6] = __int_as_float(first);
+            sp[7] = __int_as_float(cid);
+        }
+        wave_fence();
+
+        float conf_grad = 0.f, size_grad = 0.f, d0 = 0.f, d1 = 0.f;
+        float tex_grad[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) tex_grad[c] = 0.f;
+        for (int round = 0; round < num_items; round += 64)
+        {
+            if (round + lane < num_items)
+            {
+                // one layer of one point: its row holds the descriptor sums, then dL/dalpha of the four corners (zeros
+                // where no pixel retained the point)
+                const unsigned item = s_item[wave][round + lane];
+                const int layer     = (int)(item >> 8);
+                const float* sp     = s_point[wave][item & 63u];
+                const float ipx = sp[0], ipy = sp[1], size_field = sp[2], conf = sp[3], size_px = sp[4], size_chain = sp[5];
+                const vf4* row = reinterpret_cast<const vf4*>(
+                    layer < kInlineLayers ? p.rows_inline + ((size_t)(unsigned)__float_as_int(sp[7]) * kInlineLayers + layer) * PRF
+                                          : p.rows_over + ((size_t)__float_as_int(sp[6]) + (layer - kInlineLayers)) * PRF);
+                vf4 tq[NQ];
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) tq[q] = __builtin_nontemporal_load(row + q);
+                const vf4 ga = __builtin_nontemporal_load(row + NQ);
+                const float mfac = __uint_as_float((uint32_t)(127 - layer) << 23);
+                const float ux = ipx * mfac, uy = ipy * mfac;
+                const float sx = ux - floorf(ux), sy = uy - floorf(uy);
+                float lfac = 1.f, J_lf = 0.f;
+                if (want_size) lfac = layer_factor_encoded_grad(size_field, size_px, layer, p.num_layers, &J_lf);
+                // blend_fac_index / compute_blending_fac (PointBlending.h:216-264) at the corners x = floor(ux) + 0, 1: weight 1 -
+                // s and s, derivative -1 and 1; of a coordinate that is a whole number the reference takes s and 1 for both
+                const bool ex = sx == 0.f, ey = sy == 0.f;
+                const float wx0 = ex ? 0.f : 1.f - sx, wy0 = ey ? 0.f : 1.f - sy;
+                const float gl = conf * lfac, gs = size_chain * J_lf;
+                float i_conf = 0.f, i_d0 = 0.f, i_d1 = 0.f, i_size = 0.f;
+#pragma unroll
+                for (int corner = 0; corner < 4; ++corner)
+                {
+                    const bool x1 = (corner & 1) != 0, y1 = corner >= 2;
+                    const float wx = x1 ? sx : wx0, wy = y1 ? sy : wy0, blend = wx * wy;
+                    i_conf += blend * lfac * ga[corner];
+                    const float gbs = gl * ga[corner];
+                    i_d0 += (x1 ? wy : ex ? wy : -wy) * gbs;
+                    i_d1 += (y1 ? wx : ey ? wx : -wx) * gbs;
+                    if (want_size) i_size += blend * conf * (gs * ga[corner]);
+                }
+                float4* out = reinterpret_cast<float4*>(s_sums[wave][lane]);
+                out[0]      = make_float4(i_conf, i_d0, i_d1, i_size);
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) out[1 + q] = make_float4(tq[q].x, tq[q].y, tq[q].z, tq[q].w);
+            }
+            wave_fence();
+            // the point's items of this round, in layer order
+            const int j_end = min(first_item + my_items, round + 64);
+            for (int j = max(first_item, round); j < j_end; ++j)
+            {
+                const float4* in = reinterpret_cast<const float4*>(s_sums[wave][j - round]);
+                const float4 a   = in[0];
+                conf_grad += a.x;
+                d0 += a.y;
+                d1 += a.z;
+                size_grad += a.w;
+#pragma unroll
+                for (int q = 0; q < NQ; ++q)
+                {
+                    const float4 t = in[1 + q];
+                    if (4 * q < C) tex_grad[4 * q] += t.x;
+                    if (4 * q + 1 < C) tex_grad[4 * q + 1] += t.y;
+                    if (4 * q + 2 < C) tex_grad[4 * q + 2] += t.z;
+                    if (4 * q + 3 < C) tex_grad[4 * q + 3] += t.w;
+                }
+            }
+            wave_fence();
+        }
+        // some gradient reached the point
+        bool any = conf_grad != 0.f || d0 != 0.f || d1 != 0.f || size_grad != 0.f;
+#pragma unroll
+        for (int c = 0; c < C; ++c) any = any || tex_grad[c] != 0.f;
+        if (pid < 0 || (!any && !overwrite)) return;
+
+        float g_point[3] = {0.f, 0.f, 0.f}, g_pose[6], g_k[5], g_dis[8];
+        if (any)
+        {
+            project_backward(u.cam, u.R, view[0], view[1], view[2], d0, d1, g_point, g_pose, g_k, g_dis, want_intr);
+            if (want_pose)
+            {
+#pragma unroll
+                for (int k = 0; k < 6; ++k) acc[k] += g_pose[k];
+            }
+            if (want_intr)
+            {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) acc[6 + k] += g_k[k];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[11 + k] += g_dis[k];
+            }
+        }
+        store_gradients(pid, any, conf_grad, size_grad, tex_grad, g_point);
+    };
+
+    const int stride = (int)gridDim.x * 256;
+    // The compact number of a point is requested two steps ahead, and the layers it was written to (or the flags of its rows)
+    // one step ahead, so that a step starts with both in hand.
+    auto cid_at   = [&](long long pid) { return pid < p.num_points ? p.cid_of[pid] : -1; };
+    auto layers_of = [&](int cid) -> unsigned
+    {
+        if (cid < 0) return 0u;
+        if (!sparse) return (1u << __float_as_int(p.prec[(size_t)(unsigned)cid * kPointRecordFloats + 2])) - 1u;
+        const uint2 eight = *reinterpret_cast<const uint2*>(p.flags + (size_t)(unsigned)cid * TRIPS_MAX_LAYERS);
+        unsigned flagged  = 0;  // (a byte of 0 or 1 per layer)
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+        {
+            flagged |= ((eight.x >> (8 * l)) & 1u) << l;
+            flagged |= ((eight.y >> (8 * l)) & 1u) << (4 + l);
+        }
+        return flagged;
+    };
+    const long long pid0 = (long long)blockIdx.x * 256 + (int)threadIdx.x;
+    int cid_cur = cid_at(pid0), cid_next = cid_at(pid0 + stride);
+    unsigned mask_cur = layers_of(cid_cur);
+    int waiting = 0;  // queued points (the same in every lane)
+    // (the last steps, past the end, empty the queue)
+    for (int base = blockIdx.x * 256; base < p.num_points || waiting > 0; base = min(base, p.num_points) + stride)
+    {
+        int pid       = base + (int)threadIdx.x;
+        int cid       = cid_cur;
+        unsigned mask = mask_cur;
+        cid_cur       = cid_next;
+        mask_cur      = layers_of(cid_cur);
+        cid_next      = cid_at((long long)pid + 2ll * stride);
+        if (!direct)
+        {
+            const bool queued = mask != 0u;
+            const unsigned long long qm = __ballot(queued);
+            if (queued)
+            {
+                const int at     = waiting + (int)__popcll(qm & ((1ull << lane) - 1ull));
+                s_pid[wave][at]  = pid;
+                s_cid[wave][at]  = cid;
+                s_mask[wave][at] = (unsigned char)mask;
+            }
+            waiting += (int)__popcll(qm);
+            if (overwrite && !queued && pid < p.num_points)
+            {
+                const float none[C] = {}, nowhere[3] = {0.f, 0.f, 0.f};
+                store_gradients(pid, false, 0.f, 0.f, none, nowhere);
+            }
+            if (waiting < 64 && base < p.num_points) continue;
+            wave_fence();
+            // 64 leave the queue, the others move up
+            const int next  = 64 + lane;
+            const bool here = lane < waiting, moves = next < waiting;
+            pid = here ? s_pid[wave][lane] : p.num_points, cid = s_cid[wave][lane], mask = here ? s_mask[wave][lane] : 0u;
+            int mpid = 0, mcid = 0;
+            unsigned char mmask = 0;
+            if (moves) mpid = s_pid[wave][next], mcid = s_cid[wave][next], mmask = s_mask[wave][next];
+            wave_fence();
+            if (moves) s_pid[wave][lane] = mpid, s_cid[wave][lane] = mcid, s_mask[wave][lane] = mmask;
+            waiting = max(waiting - 64, 0);
+        }
+        work_off(pid < p.num_points ? pid : -1, cid, mask);
     }
 
     if (!want_pose && !want_intr) return;

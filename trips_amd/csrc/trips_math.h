@@ -305,17 +305,45 @@ __device__ __forceinline__ void project_backward(const Camera& cam, const float 
 {
     float iz = 1.f / vz, iz2 = 1.f / (vz * vz);
     float nx = vx * iz, ny = vy * iz;
-    float Jp[4], Jd[16];
-    float dx, dy;
-    distort(nx, ny, cam.dist, cam.dist_cutoff, dx, dy, Jp, Jd);  // a pointer chosen at run time would put the arrays in scratch memory
     float gr0 = cam.r00 * g0 + cam.r10 * g1;
     float gr1 = cam.r01 * g0 + cam.r11 * g1;
     float a   = cam.cfx * gr0;
     float b   = cam.cs * gr0 + cam.cfy * gr1;
     float k0  = cam.fx * a;
     float k1  = cam.s * a + cam.fy * b;
-    float d0  = Jp[0] * k0 + Jp[2] * k1;
-    float d1  = Jp[1] * k0 + Jp[3] * k1;
+    float dx, dy, d0, d1;
+    if (cam.no_distortion)
+    {
+        // all eight coefficients are zero: the distortion is the identity, and of the Jacobian of its coefficients only the
+        // powers of the radius are left (the same bits as through distort() and its matrices)
+        const float x2 = nx * nx, y2 = ny * ny, r2 = x2 + y2, r4 = r2 * r2, r6 = r4 * r2;
+        const bool cut = r2 > cam.dist_cutoff * cam.dist_cutoff;  // (never of a point that the projection kept)
+        dx = cut ? 100000.f : nx;
+        dy = cut ? 100000.f : ny;
+        d0 = cut ? 0.f : k0;
+        d1 = cut ? 0.f : k1;
+        if (want_intrinsics)
+        {
+            const float xy2 = 2.f * nx * ny;
+            g_dis[0] = nx * r2 * d0 + ny * r2 * d1;
+            g_dis[1] = nx * r4 * d0 + ny * r4 * d1;
+            g_dis[2] = nx * r6 * d0 + ny * r6 * d1;
+            g_dis[3] = -g_dis[0];
+            g_dis[4] = -g_dis[1];
+            g_dis[5] = -g_dis[2];
+            g_dis[6] = xy2 * d0 + (r2 + 2.f * y2) * d1;
+            g_dis[7] = (r2 + 2.f * x2) * d0 + xy2 * d1;
+        }
+    }
+    else
+    {
+        float Jp[4], Jd[16];
+        distort(nx, ny, cam.dist, cam.dist_cutoff, dx, dy, Jp, Jd);  // a pointer chosen at run time would put the arrays in scratch memory
+        d0 = Jp[0] * k0 + Jp[2] * k1;
+        d1 = Jp[1] * k0 + Jp[3] * k1;
+        if (want_intrinsics)
+            for (int i = 0; i < 8; ++i) g_dis[i] = Jd[i] * k0 + Jd[8 + i] * k1;
+    }
     float v0  = iz * d0;
     float v1  = iz * d1;
     float v2  = (-vx * iz2) * d0 + (-vy * iz2) * d1;
@@ -335,7 +363,6 @@ __device__ __forceinline__ void project_backward(const Camera& cam, const float 
         g_k[2] = a;
         g_k[3] = b;
         g_k[4] = dy * a;
-        for (int i = 0; i < 8; ++i) g_dis[i] = Jd[i] * k0 + Jd[8 + i] * k1;
     }
 }
 
