@@ -95,16 +95,17 @@ __device__ __forceinline__ int wave_max_small(int v)
 constexpr int kBlockSide   = 16;                       // pixels per side of a workgroup's block: one pixel per lane
 constexpr int kBlockCells  = kBlockSide - 1;           // cells per side whose footprints lie inside those pixels
 constexpr int kBlockPixels = kBlockSide * kBlockSide;  // 256
-constexpr int kListMax     = 16;                       // entries of a pixel's list (the larger list depth)
 
-// LDS of a block: {dL/dalpha, T alpha} per (list position, pixel); dL/dimage per (channel, pixel); per (place in the
-// cell's sorted list, cell) the list positions of that point's entry in its four corner pixels (0xFF: none). The pixel or the cell is the fastest index everywhere: neighbouring lanes, neighbouring banks.
-__host__ __device__ constexpr size_t tiles_lds_bytes(int cpad)
+// LDS of a block for lists of up to K entries: {dL/dalpha, T alpha} per (list position, pixel); dL/dimage per pixel, four
+// channels at a time; per (place in the cell's sorted list, cell) the list positions of that point's entry in its four
+// corner pixels (0xFF: none; an entry at list position j has a place of at most j). The pixel or the cell is the fastest
+// index everywhere: neighbouring lanes, neighbouring banks.
+__host__ __device__ constexpr size_t tiles_lds_bytes(int cpad, int K)
 {
-    return (size_t)kBlockPixels * kListMax * 8 + (size_t)kBlockPixels * cpad * 4 + (size_t)kBlockCells * kBlockCells * kCellKeep * 4;
+    return (size_t)kBlockPixels * K * 8 + (size_t)kBlockPixels * cpad * 4 + (size_t)kBlockCells * kBlockCells * K * 4;
 }
 
-template <int C>
+template <int C, int kListMax>
 __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParams p)
 {
     constexpr int CPAD  = (C + 3) & ~3;
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
     constexpr int BATCH = CPAD <= 4 ? 8 : 4;
     extern __shared__ __align__(16) unsigned char s_mem[];
     float2* const s_ex     = reinterpret_cast<float2*>(s_mem);
-    float* const s_g       = reinterpret_cast<float*>(s_mem + (size_t)kBlockPixels * kListMax * 8);
+    vf4* const s_g         = reinterpret_cast<vf4*>(s_mem + (size_t)kBlockPixels * kListMax * 8);
     unsigned* const s_rank = reinterpret_cast<unsigned*>(s_mem + (size_t)kBlockPixels * kListMax * 8 + (size_t)kBlockPixels * CPAD * 4);
     __shared__ double s_acc[4][C];
     // (point, layer) pairs that wait for a lane of their wavefront: slot = place * 225 + cell, and the point's compact
@@ -197,14 +198,14 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
             }
         }
         // no entry yet under any (cell, place): cleared while the loads above travel
-        for (int i = threadIdx.x; i < kBlockCells * kBlockCells * kCellKeep / 4; i += 256)
+        for (int i = threadIdx.x; i < kBlockCells * kBlockCells * kListMax / 4; i += 256)
             reinterpret_cast<uint4*>(s_rank)[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
         __syncthreads();
         const int m    = word & kRetainedMask;
         const int mmax = wave_max_small<kListMax>(m);
         // (two thirds of the pixels of a typical view retain at most four entries: the rest of a list only where needed)
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
+        for (int q = 1; q < kListMax / 4; ++q)
         {
             if (4 * q < mmax && 4 * q < m)
             {
@@ -213,7 +214,14 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
             }
         }
 #pragma unroll
-        for (int c = 0; c < CPAD; ++c) s_g[c * kBlockPixels + t] = c < C ? g[c] : 0.f;
+        for (int q = 0; q < NQ; ++q)
+        {
+            vf4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (4 * q + i < C) v[i] = g[4 * q + i];
+            s_g[q * kBlockPixels + t] = v;
+        }
         float sbg = 0.f;
 #pragma unroll
         for (int c = 0; c < C; ++c) sbg += p.background[c] * g[c];
@@ -274,11 +282,16 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
         if constexpr (BATCH == 4)
         {
             if (mmax > 4) batch(std::integral_constant<int, 4>{});
-            if (mmax > 8) batch(std::integral_constant<int, 8>{});
-            if (mmax > 12) batch(std::integral_constant<int, 12>{});
+            if constexpr (kListMax > 8)
+            {
+                if (mmax > 8) batch(std::integral_constant<int, 8>{});
+                if (mmax > 12) batch(std::integral_constant<int, 12>{});
+            }
         }
-        else if (mmax > 8)
-            batch(std::integral_constant<int, 8>{});
+        else if constexpr (kListMax > 8)
+        {
+            if (mmax > 8) batch(std::integral_constant<int, 8>{});
+        }
 
         // transmittance after the m retained entries decides whether the background is reached
         // (RenderBackward.cu:205-210,302-308); T is that product (1 for an empty list)
@@ -345,20 +358,32 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
                 const unsigned w4 = s_rank[slot];
                 // past the second layer: the number of the point's first row in the overflow table
                 if (!inline_row) row_of = p.over_first[row_of];
+                // the four corners' entries, all requested before the first is looked at (of a corner that did not retain the
+                // point, an entry of its list that is not used)
+                float2 e[4];
+                vf4 g4[4][NQ];
+#pragma unroll
+                for (int corner = 0; corner < 4; ++corner)
+                {
+                    const int tp = (cyl + (corner >> 1)) * kBlockSide + cxl + (corner & 1);
+                    e[corner]    = s_ex[(int)((w4 >> (8 * corner)) & (unsigned)(kListMax - 1)) * kBlockPixels + tp];
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) g4[corner][q] = s_g[q * kBlockPixels + tp];
+                }
                 float tex[CPAD], ga[4];
 #pragma unroll
                 for (int c = 0; c < CPAD; ++c) tex[c] = 0.f;
 #pragma unroll
                 for (int corner = 0; corner < 4; ++corner)
                 {
-                    const unsigned r = (w4 >> (8 * corner)) & 0xFFu;
-                    ga[corner]       = 0.f;
-                    if (r == 0xFFu) continue;
-                    const int tp   = (cyl + (corner >> 1)) * kBlockSide + cxl + (corner & 1);
-                    const float2 e = s_ex[(int)r * kBlockPixels + tp];
-                    ga[corner]     = e.x;
+                    const bool is = ((w4 >> (8 * corner)) & 0xFFu) != 0xFFu;
+                    ga[corner]    = is ? e[corner].x : 0.f;
 #pragma unroll
-                    for (int c = 0; c < C; ++c) tex[c] += e.y * s_g[c * kBlockPixels + tp];
+                    for (int c = 0; c < C; ++c)
+                    {
+                        const float more = tex[c] + e[corner].y * g4[corner][c / 4][c & 3];
+                        tex[c]           = is ? more : tex[c];
+                    }
                 }
                 const long long over = (long long)row_of + (layer - kInlineLayers);
                 if (inline_row || over < p.over_capacity)
@@ -394,10 +419,17 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
         for (int q4 = 0; q4 < kListMax / 4; ++q4)
         {
             if (4 * q4 >= mmax) break;
-            const unsigned tw = q4 == 0 ? tagw[0] : q4 == 1 ? tagw[1] : q4 == 2 ? tagw[2] : tagw[3];
+            unsigned tw = tagw[0];
             int idq[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) idq[i] = q4 == 0 ? id[i] : q4 == 1 ? id[4 + i] : q4 == 2 ? id[8 + i] : id[12 + i];
+            for (int i = 0; i < 4; ++i) idq[i] = id[i];
+#pragma unroll
+            for (int k = 1; k < kListMax / 4; ++k)
+            {
+                tw = q4 == k ? tagw[k] : tw;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) idq[i] = q4 == k ? id[4 * k + i] : idq[i];
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
             {
@@ -891,14 +923,20 @@ __global__ __launch_bounds__(256) void backward_prologue_kernel(const ViewHeader
     }
 }
 
+template <int C, int K>
+hipError_t launch_tiles(const BackwardParams& p, int blocks, hipStream_t stream)
+{
+    const size_t lds = tiles_lds_bytes((C + 3) & ~3, K);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&backward_tiles_kernel<C, K>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((backward_tiles_kernel<C, K>), dim3(blocks), dim3(256), lds, stream, p);
+    return hipSuccess;
+}
+// (a list of eight takes half of the LDS and a fourth of a lane's registers less: four workgroups per CU instead of two or three)
 template <int C>
 hipError_t launch_tiles(const BackwardParams& p, int blocks, hipStream_t stream)
 {
-    const size_t lds = tiles_lds_bytes((C + 3) & ~3);
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&backward_tiles_kernel<C>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((backward_tiles_kernel<C>), dim3(blocks), dim3(256), lds, stream, p);
-    return hipSuccess;
+    return p.list_depth <= 8 ? launch_tiles<C, 8>(p, blocks, stream) : launch_tiles<C, 16>(p, blocks, stream);
 }
 
 #define TRIPS_BW_DISPATCH(KERNEL, BLOCKS)                                                                      \
