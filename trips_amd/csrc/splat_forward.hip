@@ -629,15 +629,17 @@ __device__ __forceinline__ void for_entries(const T* __restrict__ entries, int n
 // The keys of a tile are filed by cell: the cell (px, py) holds the points whose 2 x 2 footprint starts at that pixel,
 // so that a (point, layer) pair is written once and the four pixels it covers gather it from the cell. There is one key
 // per bin entry: the keys of a tile start where its bin entries do.
-// One workgroup per tile (blocks [0, NB)) plus one per slice of a split tile (blocks from NB on; those past the
+// One workgroup per tile (blocks [0, NB)) plus one per slice of a split tile (blocks from there on; those past the
 // number of slices the plan found return at once). Pass `SCATTER == false`: count the entries of the tile's 1024
 // cells in LDS and write the counts (split tiles only). Pass `SCATTER == true`: the counts of a tile that is not
 // split, then the exclusive scan of the 1024 counts, per-cell list starts, and the 64-bit keys (depth bits << 32 | compact point number) into their lists. A slice adds its counts to the
 // tile's with atomics; when it places its keys it first counts its own entries per cell again and claims that many
 // slots of each cell's list with one atomic.
-// (THREADS: 256 for the counting pass, whose idle workgroups for unused slices are cheaper that way; 1024 for the
-// placement pass, where two workgroups per CU with their 64 KB of LDS then make 32 wavefronts instead of 8)
-constexpr int kScatterThreads = 1024;
+// (THREADS: 256 for the counting pass, whose idle workgroups for unused slices are cheaper that way. The placement pass is a
+// chain of round trips and barriers per tile, so as many tiles as possible should be under way on a CU: four workgroups of
+// 512 with 39 KB of LDS each. Two of 1024 with 64 KB, and these: 6M points
+// in no order 57 -> 50 us, in Morton order without the saved state 36 -> 26, 1M in a ball 37 -> 30.)
+constexpr int kScatterThreads = 512;
 template <bool SCATTER, int THREADS, bool PACKED>
 __global__ __launch_bounds__(THREADS) void tile_lists_kernel(const ForwardParams p)
 {
@@ -653,7 +655,12 @@ __global__ __launch_bounds__(THREADS) void tile_lists_kernel(const ForwardParams
     int slice    = -1;  // -1: the tile's own workgroup
     if (bin >= NB)
     {
-        const int e = bin - NB;
+        // Runs of eight consecutive slices share an XCD (workgroups are dealt to the eight of them in turn): the slices of a
+        // tile store their keys side by side all over the tile's lists, and an L2 that sees them all writes whole lines (a
+        // render of 3.3M points at 1112 x 583: 64 -> 56 us).
+        const int tiles8 = (NB + kNumXcd - 1) / kNumXcd * kNumXcd;
+        if (bin < tiles8) return;
+        const int e = (int)xcd_tile_block(bin - tiles8, 8);
         if (e >= p.slice_start[NB]) return;
         // the tile with slice_start[t] <= e < slice_start[t + 1]: a split one, tiles without slices have empty ranges
         int lo = 0, hi = NB;
@@ -798,29 +805,26 @@ __global__ __launch_bounds__(THREADS) void tile_lists_kernel(const ForwardParams
         if (dropped) atomicAdd(&p.status->overflow, (u64)dropped);
         return;
     }
-    // Keys of a tile whose lists fit into LDS are staged there and copied out with full-line stores; the keys of
-    // bigger tiles go to their lists directly (8-byte stores scattered over the tile's region).
+    // The tile's first kStageKeys keys are staged in LDS and copied out with full-line stores; the others of a bigger tile
+    // go to their lists directly (8-byte stores scattered over the tile's region).
     extern __shared__ u64 s_keys[];
     const int tile_total = p.bin_start[bin + 1] - key_start;
-    const bool staged    = tile_total <= kStageKeys && (long long)key_start + tile_total <= p.capacity;
+    const int staged     = (int)max(0ll, min((long long)min(tile_total, kStageKeys), p.capacity - key_start));
     for_mine(
                 [&](const ET& e)
                 {
                     const u64 key  = E::key(e);
                     const int slot = atomicAdd(&s_cnt[E::cell(e)], 1);
-                    if (staged)
+                    if (slot - key_start < staged)
                         s_keys[slot - key_start] = key;
                     else if ((unsigned long long)(unsigned)slot < (unsigned long long)p.capacity)
                         p.keys[slot] = key;
                     else
                         dropped += 1;
                 });
-    if (staged)
-    {
-        __syncthreads();
-        u64* dst = p.keys + key_start;
-        for (int i = threadIdx.x; i < tile_total; i += THREADS) __builtin_nontemporal_store(s_keys[i], dst + i);
-    }
+    __syncthreads();
+    u64* dst = p.keys + key_start;
+    for (int i = threadIdx.x; i < staged; i += THREADS) __builtin_nontemporal_store(s_keys[i], dst + i);
     if (dropped) atomicAdd(&p.status->overflow, (u64)dropped);
 }
 
@@ -1483,26 +1487,21 @@ hipError_t launch_forward_view(const ForwardParams& p, int channels, bool train,
     // workgroups for the slices of split tiles: at most capacity / kSliceEntries full slices plus one partial slice
     // per split tile
     const int max_slices = (int)std::min<long long>(2 * (p.capacity / kSliceEntries) + 1, 1 << 20);
+    const int list_blocks = (NB + kNumXcd - 1) / kNumXcd * kNumXcd + (max_slices + 63) / 64 * 64;  // (whole runs of eight on eight XCDs)
     {
         ProfScope ps(prof, "tile_count", stream);
         if (packed)
-            hipLaunchKernelGGL((tile_lists_kernel<false, 256, true>), dim3(NB + max_slices), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((tile_lists_kernel<false, 256, true>), dim3(list_blocks), dim3(256), 0, stream, p);
         else
-            hipLaunchKernelGGL((tile_lists_kernel<false, 256, false>), dim3(NB + max_slices), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((tile_lists_kernel<false, 256, false>), dim3(list_blocks), dim3(256), 0, stream, p);
     }
     {
         ProfScope ps(prof, "tile_scatter", stream);
-        // (64 KB of LDS with the static tables: above the default limit of a launch)
-        const void* fn = packed ? reinterpret_cast<const void*>(&tile_lists_kernel<true, kScatterThreads, true>)
-                                : reinterpret_cast<const void*>(&tile_lists_kernel<true, kScatterThreads, false>);
-        const hipError_t lds = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kStageKeys * sizeof(u64)));
-        if (lds != hipSuccess) return lds;
+        constexpr size_t lds = kStageKeys * sizeof(u64);
         if (packed)
-            hipLaunchKernelGGL((tile_lists_kernel<true, kScatterThreads, true>), dim3(NB + max_slices), dim3(kScatterThreads),
-                               kStageKeys * sizeof(u64), stream, p);
+            hipLaunchKernelGGL((tile_lists_kernel<true, kScatterThreads, true>), dim3(list_blocks), dim3(kScatterThreads), lds, stream, p);
         else
-            hipLaunchKernelGGL((tile_lists_kernel<true, kScatterThreads, false>), dim3(NB + max_slices), dim3(kScatterThreads),
-                               kStageKeys * sizeof(u64), stream, p);
+            hipLaunchKernelGGL((tile_lists_kernel<true, kScatterThreads, false>), dim3(list_blocks), dim3(kScatterThreads), lds, stream, p);
     }
     {
         ProfScope ps(prof, "long_lists", stream);

@@ -127,7 +127,7 @@ constexpr int kSliceEntries = 8192;
 // smallest keys of every segment (a 16-lane row each), and the blend kernel then sorts those instead of the list.
 constexpr int kLongList    = 512;
 constexpr int kLongSegment = 256;
-constexpr int kStageKeys  = 7168;   // keys of one tile staged in LDS before they are written (56 KB)
+constexpr int kStageKeys  = 3968;   // keys of one tile staged in LDS before they are written (31 KB)
 // keys of a cell that can reach a pixel's list (the larger list depth): the forward sorts every cell's list and keeps
 // this many
 constexpr int kCellKeep = 16;
