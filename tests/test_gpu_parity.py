@@ -442,6 +442,25 @@ def test_lists_that_end_around_the_staged_keys(oracle, channels, K):
     _check_backward(oracle, sc, d, seed=5)
 
 
+@pytest.mark.parametrize("n", [3967, 3968, 3969, 8191, 8192, 8193, 70000])
+def test_keys_of_a_tile_around_the_staged_ones(oracle, n):
+    """A single tile that holds exactly n points (one layer, footprints inside 32 x 32 pixels): as many keys as are staged,
+    one more, the last tile that is not split, the first that is, and one in nine slices."""
+    sc = scenes.tiny(n=n, w=33, h=33, f=30.0, num_layers=1, list_depth=16, seed=n % 89, radius=(0.004, 0.02))
+    rng = np.random.default_rng(n)
+    z = rng.uniform(-0.5, 0.5, n)
+    at = rng.uniform(0.1, 31.9, (n, 2))
+    sc.position[:, 0] = ((at[:, 0] - 16.0) * (z + 3.0) / 30.0).astype(np.float32)
+    sc.position[:, 1] = ((at[:, 1] - 16.0) * (z + 3.0) / 30.0).astype(np.float32)
+    sc.position[:, 2] = z.astype(np.float32)
+    sc.intrinsics[0, 2:4] = 16.0
+    d = abi.desc_for_scene(sc)
+    run, ref, _ = _check_forward(oracle, sc, d)
+    assert run.ctx.counters(d, run.saved, 0)["valid"] == n
+    ip = ref["ip"][0]
+    assert ip.min() >= 0 and ip.max() < 32
+
+
 def test_footprints_on_tile_and_image_borders_with_equal_depths(oracle):
     """A dense grid of points in a plane that faces the camera: footprints start at every pixel, also at the last
     column and row of a 32-pixel tile (their other pixels belong to the neighbouring tiles) and at the last pixels of
