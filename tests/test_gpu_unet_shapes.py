@@ -123,3 +123,56 @@ def test_upsampling_of_neighbours_far_apart():
     g = torch.Generator().manual_seed(81)
     inputs = [torch.sign(torch.rand(t.shape, generator=g) - 0.5) * (4e4 + 2e4 * t) for t in _pyramid(45, 37, 2, 4, batch=1, seed=82)]
     _compare(net, inputs)
+
+
+@pytest.mark.parametrize("filters,w,h,batch", [
+    ([32, 32, 32, 32, 32], 160, 120, 1),  # one instance for all levels, a workgroup per tile
+    ([32, 32, 32, 32], 545, 273, 2),      # ... more tiles than workgroups
+    ([16, 32, 48, 64], 300, 200, 2),      # levels of several instances, two of which share one, a level of two shares
+])
+def test_weight_gradients_of_some_levels(filters, w, h, batch):
+    """Levels whose weight gradients are the same instance of the kernel run in one launch: without the gradients of some
+    levels (weights, biases or both), the others are the same bits as with all of them."""
+    import ctypes as C
+
+    from trips_amd import _lib, abi
+    from trips_amd.renderer import get_context
+    from trips_amd.unet import _buffer_sizes, _ptr, _stream_ptr
+    L = len(filters)
+    net = _net(filters, L, seed=5).cuda()
+    ins = [t.cuda() for t in _pyramid(w, h, L, 4, batch=batch, seed=6)]
+    ctx, dev, d, params = get_context(0), ins[0].device, net.desc(ins), net.ordered_parameters()
+    sizes = _buffer_sizes(bytes(d))
+    saved, ws = ctx.alloc_bytes(sizes[1]), ctx.alloc_bytes(sizes[2])
+    with torch.no_grad():
+        net._run_forward(d, ins, params, saved)
+    d_out = torch.randn((batch, 3, h, w), generator=torch.Generator().manual_seed(7)).cuda() * 1e-3
+    wts, _ = net._weights_struct(params)
+
+    def backward(wanted):
+        """wanted: (weights, biases) per level"""
+        outs = [torch.full_like(p, float("nan")) for p in params]
+        g, d_ins = abi.TripsUnetGrads(), [torch.empty_like(t) for t in ins]
+        for i, (weights, biases) in enumerate(wanted):
+            f, fb, m, mb = (t.data_ptr() for t in outs[4 * i:4 * i + 4])
+            g.feature_weight[i], g.mask_weight[i] = (f, m) if weights else (None, None)
+            g.feature_bias[i], g.mask_bias[i] = (fb, mb) if biases else (None, None)
+        g.inputs[:L] = [t.data_ptr() for t in d_ins]
+        _lib.check(ctx.lib.trips_unet_backward(ctx.ctx, C.byref(d), C.byref(wts), net._input_ptrs(ins), _ptr(saved), _ptr(d_out),
+                                               C.c_float(net.grad_scale), C.byref(g), _ptr(ws), sizes[2], _stream_ptr(dev)))
+        return outs, d_ins
+    full, full_ins = backward([(True, True)] * L)
+    assert all(bool(torch.isfinite(t).all()) for t in full[:4 * L])
+    for wanted in ([(i != 1, True) for i in range(L)], [(True, i != 0) for i in range(L)], [(i % 2 == 0, i < 2) for i in range(L)],
+                   [(i == L - 1, False) for i in range(L)]):
+        part, part_ins = backward(wanted)
+        assert all(torch.equal(a, b) for a, b in zip(part_ins, full_ins))
+        for i, (weights, biases) in enumerate(wanted):
+            for k in range(4):
+                a, b = part[4 * i + k], full[4 * i + k]
+                if not (weights if k % 2 == 0 else biases):
+                    assert bool(torch.isnan(a).all())
+                elif k % 2 == 1 and not weights:  # summed by a kernel of its own: single precision, another order
+                    assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max()) + 1e-12
+                else:
+                    assert torch.equal(a, b), (wanted, i, k)

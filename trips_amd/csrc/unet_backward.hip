@@ -1088,11 +1088,19 @@ struct BwdWeightParams
     int batch;           // images, one after the other in every array
     const float* feat;
     const _Float16* below;  // rows of the level below, [Hb][Wb][below_stride]
-    int npad;               // pre-activations of a pixel, of which a workgroup takes NPAD (the grid's y dimension the others)
+    int npad;               // pre-activations of a pixel, of which a workgroup takes NPAD
     const _Float16* dpre;   // [H][W][npad]
-    float* part;           // [gridDim.x][9][npad][CIN]
+    int groups;            // workgroups of each share of NPAD pre-activations
+    float* part;           // [groups][9][npad][CIN]
     // bias gradients = sums of dpre over the pixels, taken from the transposed tile while it is in LDS
-    float* bias_part;      // [gridDim.x][npad] or nullptr
+    float* bias_part;      // [groups][npad] or nullptr
+};
+// The levels of a launch, one after the other in its workgroups: level, share, group.
+struct BwdWeightTable
+{
+    BwdWeightParams lv[TRIPS_UNET_MAX_LEVELS];
+    int first[TRIPS_UNET_MAX_LEVELS];  // first workgroup of every level
+    int n;
 };
 
 // Pixel-major tiles and the transposing LDS read. Both operands of the weight-gradient GEMM are needed with eight
@@ -1183,8 +1191,12 @@ __device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8
 
 // CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
-__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightParams p)
+__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightTable tab)
 {
+    int level = 0;
+    while (level + 1 < tab.n && (int)blockIdx.x >= tab.first[level + 1]) ++level;
+    const BwdWeightParams p = tab.lv[level];
+    const int in_level = (int)blockIdx.x - tab.first[level];
     constexpr int ROW    = CIN + kLdsChanPad;   // halves per pixel of the input patch
     constexpr int DS     = NPAD + kLdsChanPad;  // halves per pixel of the gradient tile
     constexpr int GROUPS = CIN / 8;
@@ -1217,7 +1229,7 @@ __global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(C
     const int cb0 = (wave % CBW) * MYCB, nb0 = (RW == 1 ? wave / CBW : (wave / CBW) % NBW) * MYNB;
     const int share = RW == 1 ? 0 : wave / (CBW * NBW);
     const int row0  = share * MYROWS;           // this wavefront's rows of a tile
-    const int set   = blockIdx.x;               // the workgroup's set of partial sums
+    const int set   = in_level % p.groups;      // the workgroup's set of partial sums
     floatx4 acc[9][MYNB][MYCB];
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -1251,7 +1263,7 @@ __global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(C
     const int below_groups = p.below_stride / 8;  // groups of eight that a row of the level below has
     // the images of the batch are walked as one run of tiles: a workgroup keeps its sums from one image to the next
     // (image after image, every image paid for a set of partial sums of its own and for a last round of its own)
-    const int n0      = (int)blockIdx.y * NPAD;  // this workgroup's first pre-activation
+    const int n0      = in_level / p.groups * NPAD;  // this workgroup's first pre-activation
     const float* feat = p.feat;
     const _Float16 *below = p.below, *dpre = p.dpre + n0;
     auto of_image = [&](int& tile)
@@ -1381,9 +1393,9 @@ __global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(C
         }
 
     TileLoads cur;
-    const int tiles = p.tiles * p.batch;
-    if ((int)blockIdx.x < tiles) issue_loads(blockIdx.x, cur);
-    for (int tile0 = blockIdx.x; tile0 < tiles; tile0 += gridDim.x)
+    const int tiles = p.tiles * p.batch, groups = p.groups;
+    if (set < tiles) issue_loads(set, cur);
+    for (int tile0 = set; tile0 < tiles; tile0 += groups)
     {
         int tile = tile0;
         of_image(tile);
@@ -1391,7 +1403,7 @@ __global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(C
         const int x0 = tx * kConvTileW, y0 = ty * kConvTileH;
         __syncthreads();  // the previous tile's operands have been consumed (and the zero fill is done)
         commit_loads(cur);
-        if (tile0 + (int)gridDim.x < tiles) issue_loads(tile0 + gridDim.x, cur);  // travels during stage 2 and the taps
+        if (tile0 + groups < tiles) issue_loads(tile0 + groups, cur);  // travels during stage 2 and the taps
         if (has_below)
         {
             __syncthreads();
@@ -1660,7 +1672,7 @@ hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, i
 }
 
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
-hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, hipStream_t stream)
+hipError_t launch_bwd_weight(const BwdWeightTable& t, int blocks, hipStream_t stream)
 {
     const size_t lds = ((size_t)(kConvPatchH * kConvPatchW + kBelowH * kBelowW) * (CIN + kLdsChanPad) +
                         (size_t)kConvTileH * kConvTileW * (NPAD + kLdsChanPad)) *
@@ -1668,28 +1680,30 @@ hipError_t launch_bwd_weight(const BwdWeightParams& p, int groups, int splits, h
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>), dim3(groups, splits), dim3(kWgradThreads), lds, stream, p);
+    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>), dim3(blocks), dim3(kWgradThreads), lds, stream, t);
     return hipGetLastError();
 }
 
 template <int CI, bool FOUR>
-hipError_t dispatch_bwd_weight_ci(const BwdWeightParams& p, const LevelPlan& lv, hipStream_t stream)
+hipError_t dispatch_bwd_weight_ci(const BwdWeightTable& t, int blocks, int cin_pad, int tile, hipStream_t stream)
 {
 #define TRIPS_BW(CIN_, NT_)                                                                    \
-    if (lv.cin_pad == CIN_ && lv.wgrad_tile == NT_)                                            \
-        return p.bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(p, lv.groups, lv.npad / NT_, stream) \
-                           : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(p, lv.groups, lv.npad / NT_, stream);
+    if (cin_pad == CIN_ && tile == NT_)                                                        \
+        return t.lv[0].bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(t, blocks, stream) \
+                                 : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(t, blocks, stream);
     TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 128) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
 #undef TRIPS_BW
     return hipErrorInvalidValue;
 }
 
-hipError_t dispatch_bwd_weight(const BwdWeightParams& p, const LevelPlan& lv, hipStream_t stream)
+// the levels of a launch are the same instance of the kernel, all with bias gradients or all without
+hipError_t dispatch_bwd_weight(const BwdWeightTable& t, int blocks, const LevelPlan& lv, hipStream_t stream)
 {
-    if (p.c_feat == 4) return dispatch_bwd_weight_ci<4, true>(p, lv, stream);
-    if (p.c_feat < 4) return dispatch_bwd_weight_ci<4, false>(p, lv, stream);
-    if (p.c_feat <= 8) return dispatch_bwd_weight_ci<8, false>(p, lv, stream);
-    return dispatch_bwd_weight_ci<16, false>(p, lv, stream);
+    const int C = t.lv[0].c_feat;
+    if (C == 4) return dispatch_bwd_weight_ci<4, true>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
+    if (C < 4) return dispatch_bwd_weight_ci<4, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
+    if (C <= 8) return dispatch_bwd_weight_ci<8, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
+    return dispatch_bwd_weight_ci<16, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -1845,45 +1859,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     for (int i = 0; i < L; ++i)
     {
         const LevelPlan& lv = np.lv[i];
-        const size_t plane  = (size_t)lv.H * lv.W;
         const bool below    = i < L - 1;
-        {
-            ProfScope ps(prof, kWeightNames[i], stream);
-            BiasGradParams bp;
-            bp.pixels    = plane * d.batch;
-            bp.npad      = lv.npad;
-            bp.cout      = lv.cout;
-            bp.scale_inv = scale_inv;
-            bp.dpre      = dpre_ptr(i);
-            bp.d_bias_f  = grads->feature_bias[i];
-            bp.d_bias_m  = grads->mask_bias[i];
-            const bool want_w = grads->feature_weight[i] || grads->mask_weight[i];
-            if ((bp.d_bias_f || bp.d_bias_m) && !want_w)  // otherwise the weight-gradient kernel sums them on its way
-                hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((bp.pixels + kBiasChunk - 1) / kBiasChunk)), dim3(256), 0, stream, bp);
-
-            BwdWeightParams wp;
-            std::memset(&wp, 0, sizeof(wp));
-            wp.H = lv.H, wp.W = lv.W, wp.c_feat = C;
-            wp.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
-            wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
-            wp.batch   = d.batch;
-            wp.feat    = inputs[i];
-            wp.npad    = lv.npad;
-            wp.dpre    = dpre_ptr(i);
-            wp.part    = reinterpret_cast<float*>(ws + lv.part_off);
-            if (bp.d_bias_f || bp.d_bias_m) wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off);
-            if (below)
-            {
-                const LevelPlan& lb = np.lv[i + 1];
-                wp.Hb = lb.H, wp.Wb = lb.W, wp.below_stride = lb.row_stride;
-                wp.below = rows_ptr(i + 1);
-            }
-            if (want_w)
-            {
-                hipError_t e = dispatch_bwd_weight(wp, lv, stream);
-                if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
-            }
-        }
         {
             ProfScope ps(prof, kDataNames[i], stream);
             BwdDataParams dp;
@@ -1940,6 +1916,63 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "backward launch (level %d): %s", i, hipGetErrorString(e));
+    }
+    // The weight gradients need the pre-activation gradients alone: all behind the data gradients, levels that are the same
+    // instance of the kernel in one launch.
+    bool launched[TRIPS_UNET_MAX_LEVELS] = {};
+    for (int i = 0; i < L; ++i)
+    {
+        if (launched[i]) continue;
+        ProfScope ps(prof, kWeightNames[i], stream);
+        const bool bias = grads->feature_bias[i] || grads->mask_bias[i];
+        if (!grads->feature_weight[i] && !grads->mask_weight[i])
+        {
+            if (!bias) continue;
+            // (otherwise the weight-gradient kernel sums them on its way)
+            const LevelPlan& lv = np.lv[i];
+            BiasGradParams bp;
+            bp.pixels    = (size_t)lv.H * lv.W * d.batch;
+            bp.npad      = lv.npad;
+            bp.cout      = lv.cout;
+            bp.scale_inv = scale_inv;
+            bp.dpre      = dpre_ptr(i);
+            bp.d_bias_f  = grads->feature_bias[i];
+            bp.d_bias_m  = grads->mask_bias[i];
+            hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((bp.pixels + kBiasChunk - 1) / kBiasChunk)), dim3(256), 0, stream, bp);
+            continue;
+        }
+        BwdWeightTable t;
+        std::memset(&t, 0, sizeof(t));
+        int blocks = 0;
+        for (int k = i; k < L; ++k)
+        {
+            const LevelPlan& lv = np.lv[k];
+            if (launched[k] || !same_wgrad_kernel(lv, np.lv[i]) || !(grads->feature_weight[k] || grads->mask_weight[k]) ||
+                (grads->feature_bias[k] || grads->mask_bias[k]) != bias)
+                continue;
+            launched[k]         = true;
+            t.first[t.n]        = blocks;
+            BwdWeightParams& wp = t.lv[t.n++];
+            wp.H = lv.H, wp.W = lv.W, wp.c_feat = C;
+            wp.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
+            wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
+            wp.batch   = d.batch;
+            wp.feat    = inputs[k];
+            wp.npad    = lv.npad;
+            wp.groups  = lv.groups;
+            wp.dpre    = dpre_ptr(k);
+            wp.part    = reinterpret_cast<float*>(ws + lv.part_off);
+            if (bias) wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off);
+            if (k < L - 1)
+            {
+                const LevelPlan& lb = np.lv[k + 1];
+                wp.Hb = lb.H, wp.Wb = lb.W, wp.below_stride = lb.row_stride;
+                wp.below = rows_ptr(k + 1);
+            }
+            blocks += lv.groups * (lv.npad / lv.wgrad_tile);
+        }
+        hipError_t e = dispatch_bwd_weight(t, blocks, np.lv[i], stream);
+        if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
     }
     // the partial weight and bias gradients of all levels are summed at the end, one launch per step of the sum
     {

@@ -110,7 +110,8 @@ struct LevelPlan
     size_t sliced_off;  // partial sums of the partials [16][9][npad][cin_pad] fp32
     size_t bias_part_off;  // per-workgroup sums of the pre-activation gradients [groups][npad] fp32
     int wgrad_tile;     // pre-activations of a workgroup of the weight-gradient kernel
-    int groups;         // persistent workgroups of the weight-gradient kernel, for all images of the batch
+    long long tiles;    // 8 x 32 tiles of all images of the batch
+    int groups;         // persistent workgroups of the weight-gradient kernel for each of its npad / wgrad_tile shares
 };
 
 // Whether the data gradient of a block and the adjoint of the upsampling below it run as one kernel
@@ -166,6 +167,33 @@ inline int check_unet_desc(const TripsUnetDesc* d)
     return TRIPS_OK;
 }
 
+// Levels whose weight gradients are the same instance of the kernel run in one launch, whose workgroups are as many as are
+// resident at once (two per CU for the smallest shape, else one; every further one would only add a set of partial sums to
+// write and reduce) and are dealt to the levels by their tiles. With a launch per level the coarser ones were a handful of
+// tiles each, begun and ended 256 workgroups at a time: all weight gradients and the sums of their partials, default net
+// of five levels at 1245 x 825 155 -> 110 us, at 105 x 74 (32/64/64/64/64) 85 -> 46, 16/32/64/64 at 1920 x 1080 217 -> 205.
+inline bool same_wgrad_kernel(const LevelPlan& a, const LevelPlan& b) { return a.cin_pad == b.cin_pad && a.wgrad_tile == b.wgrad_tile; }
+inline void plan_wgrad_groups(NetPlan& np, int levels)
+{
+    for (int i = 0; i < levels; ++i)
+    {
+        LevelPlan& lv      = np.lv[i];
+        const int resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1);
+        // one workgroup for every share of every level, the others by the tiles (rounded down: one that has to wait for
+        // another to end would take as long again)
+        long long work = 0, shares = 0;
+        for (int k = 0; k < levels; ++k)
+            if (same_wgrad_kernel(np.lv[k], lv))
+            {
+                const int s = np.lv[k].npad / np.lv[k].wgrad_tile;
+                work += np.lv[k].tiles * s;
+                shares += s;
+            }
+        const long long g = 1 + (resident - shares) * lv.tiles / work;
+        lv.groups         = (int)(g < lv.tiles ? g : lv.tiles);
+    }
+}
+
 // Block i convolves cat(in[i], up2(x_{i+1})) (F[i+1] channels; C for the start block) to F[i] - 2C outputs
 // (F[0] - C for the last block when it is not also the start block), Networks.h:1034-1037,1104-1118.
 inline NetPlan make_plan(const TripsUnetDesc& d)
@@ -213,13 +241,13 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         lv.din_off = bw;
         if (i < L - 1 && !bwd_data_up_fits(lv.npad, lv.cin_pad, true)) bw += align256(pixels * lv.cin_pad * sizeof(_Float16));
         const long long tiles = (long long)d.batch * ((lv.W + kConvTileW - 1) / kConvTileW) * ((lv.H + kConvTileH - 1) / kConvTileH);
-        // persistent workgroups of the weight-gradient kernel: as many as are resident at once (two per CU for the
-        // smallest shape, else one; those that share the pre-activations of a tile between them count together); every
-        // further one would only add a set of partial sums to write and reduce (32 x 64 with two per CU: 64 instead of
-        // 70 us at 1245 x 825, and 7 us more for the sums)
-        lv.wgrad_tile      = wgrad_tile(lv.cin_pad, lv.npad, tiles);
-        const int resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1) / (lv.npad / lv.wgrad_tile);
-        lv.groups          = tiles < resident ? (int)tiles : resident;
+        lv.wgrad_tile = wgrad_tile(lv.cin_pad, lv.npad, tiles);
+        lv.tiles      = tiles;
+    }
+    plan_wgrad_groups(np, L);
+    for (int i = 0; i < L; ++i)
+    {
+        LevelPlan& lv = np.lv[i];
         lv.part_off     = bw;
         bw += align256((size_t)lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
         lv.sliced_off = bw;
