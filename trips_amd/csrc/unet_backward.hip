@@ -101,8 +101,13 @@ struct FinalBwdParams
 // WGRAD, the weight and bias gradients of the 1x1 convolution. Every thread keeps the cout x cin products of its
 // pixels in registers, a workgroup folds them through LDS and writes its sums once (final_reduce_kernel adds the
 // workgroups up: atomics of a thousand workgroups on these few addresses would serialise in one L2 channel).
-// (The library is compiled without contraction of products and sums; this kernel is bound by its arithmetic
-// instructions, and its sums are written as fused multiply-adds.)
+// (The library is compiled without contraction of products and sums; here the sums are written as fused multiply-adds.)
+// Bound by the memory: about 300 bytes a pixel at 64 gates, most of them the rows that it reads and the rows that it
+// writes. The rows it reads are read for the last time, whole lines of them by a wavefront, and are loaded past the caches:
+// loaded as usual they push out the rows that are written, which the data gradient reads next. 1245 x 825 pixels: 96 us, 71
+// with the loads past the caches (and the data gradient of the level 113, now 106), 4.3 TB/s; four crops of 512^2: 83, now
+// 64; 1717 x 783 at 32 gates: 71, now 57. Two or four pixels of a lane requested together gave nothing (86 and 93 us where
+// one gave 84): the registers cost as many wavefronts as they add loads.
 // CI = image channels the kernel has room for (4, 8 or 16).
 template <int NPAD, bool WGRAD, int CI>
 __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParams p)
@@ -128,7 +133,9 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
     const size_t plane = (size_t)p.H * p.W;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane % LPP, sub = lane / LPP;
-    const bool in_row = g < NPAD / 8;  // lanes past the row idle (rows of 96 halves on 16 lanes)
+    // lanes past the row (rows of 96 halves on 16 lanes) work on its first word again and store nothing
+    const bool in_row = NPAD / 8 == LPP || g < NPAD / 8;
+    const int row_word = in_row ? 8 * g : 0;
     const int c0      = 4 * g;         // first of this lane's four channels
     // ... and the image channels g, g + LPP, ... (one each for up to LPP image channels)
     constexpr int NI = (CI + LPP - 1) / LPP;
@@ -155,46 +162,56 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[k][i] = 0.f;
 
-    // the arrays of the image at hand
-    const float *d_out = p.d_out, *feat = p.feat;
-    const _Float16* pre = p.pre;
-    float* d_feat       = p.d_feat;
-    _Float16* dpre      = p.dpre;
     struct Loaded
     {
         float g[4], x[NI];
         half8 mine;
     };
-    auto load = [&](size_t pix, bool valid)
-    {
-        Loaded l;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) l.g[k] = (valid && k < p.cout) ? d_out[k * plane + pix] : 0.f;
-#pragma unroll
-        for (int j = 0; j < NI; ++j) l.x[j] = (WGRAD && valid && has_img[j]) ? feat[(size_t)(g + LPP * j) * plane + pix] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) l.mine[i] = _Float16(0.f);
-        if (valid && in_row) l.mine = *reinterpret_cast<const half8*>(pre + pix * NPAD + 8 * g);
-        return l;
-    };
     constexpr int STEP = 4 * PPW;  // pixels per iteration of the workgroup
     for (int item = blockIdx.x; item < p.chunks * p.batch; item += gridDim.x)
     {
         const int image = item / p.chunks, chunk = item - image * p.chunks;
-        d_out  = p.d_out + (size_t)image * p.cout * plane;
-        feat   = p.feat + (size_t)image * p.c_feat * plane;
-        d_feat = p.d_feat + (size_t)image * p.c_feat * plane;
-        pre    = p.pre + (size_t)image * plane * p.npad;
-        dpre   = p.dpre + (size_t)image * plane * p.npad;
-        const size_t p1 = std::min(plane, (size_t)(chunk + 1) * kFinalPixelsPerBlock);
-        size_t base     = (size_t)chunk * kFinalPixelsPerBlock + wave * PPW;
-        Loaded next     = load(base + sub, base + sub < p1);
-        for (; base < p1; base += STEP)
+        const size_t first = (size_t)chunk * kFinalPixelsPerBlock;
+        const int n        = (int)std::min(plane - first, (size_t)kFinalPixelsPerBlock);
+        // the arrays from the chunk's first pixel on: what a lane adds to them fits in 32 bits
+        const float* d_out  = p.d_out + (size_t)image * p.cout * plane + first;
+        const float* feat   = p.feat + (size_t)image * p.c_feat * plane + first;
+        float* d_feat       = p.d_feat + (size_t)image * p.c_feat * plane + first;
+        const _Float16* pre = p.pre + ((size_t)image * plane + first) * NPAD;
+        _Float16* dpre      = p.dpre + ((size_t)image * plane + first) * NPAD;
+        const float* x_of[NI];
+        float* dx_of[NI];
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
         {
-            const size_t pix = base + sub;
-            const bool valid = pix < p1;
+            const size_t at = has_img[j] ? (size_t)(g + LPP * j) * plane : 0;
+            x_of[j]  = feat + at;
+            dx_of[j] = d_feat + at;
+        }
+        // (pixels past the end: the last one's values, which are not used; a load behind a condition of the lane costs more
+        // than the load)
+        auto load = [&](unsigned pix)
+        {
+            Loaded l;
+            const unsigned at = min(pix, (unsigned)n - 1u);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                l.g[k] = 0.f;
+                if (k < p.cout) l.g[k] = (d_out + k * plane)[at];
+            }
+#pragma unroll
+            for (int j = 0; j < NI; ++j) l.x[j] = WGRAD ? x_of[j][at] : 0.f;
+            l.mine = __builtin_nontemporal_load(reinterpret_cast<const half8*>(pre + (at * NPAD + row_word)));
+            return l;
+        };
+        unsigned pix = wave * PPW + sub;
+        Loaded next  = load(pix);
+        for (int base = 0; base < n; base += STEP, pix += STEP)
+        {
             const Loaded cur = next;
-            if (base + STEP < p1) next = load(pix + STEP, pix + STEP < p1);  // in flight while this pixel is worked on
+            if (base + STEP < n) next = load(pix + STEP);  // in flight while this pixel is worked on
+            if (pix >= (unsigned)n) continue;
             half8 out;   // gradients of the four features, then of the four masks
             float v[4];  // the block's output as the forward's 1x1 convolution read it (fp16)
 #pragma unroll
@@ -207,19 +224,16 @@ __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParam
                 gate_backward(da * p.scale, float(cur.mine[i]), float(cur.mine[4 + i]), df, dm, a);
                 out[i]     = _Float16(df);
                 out[4 + i] = _Float16(dm);
-                v[i]       = (valid && c0 + i < p.cact) ? float(_Float16(a)) : 0.f;
+                v[i]       = float(_Float16(a));  // (sums of padding channels are not read)
             }
-            if (valid && in_row) *reinterpret_cast<half8*>(dpre + pix * NPAD + 8 * g) = out;
+            if (in_row) *reinterpret_cast<half8*>(dpre + (pix * NPAD + row_word)) = out;
 #pragma unroll
             for (int j = 0; j < NI; ++j)
             {
-                if (valid && has_img[j])
-                {
-                    float d = 0.f;
+                float d = 0.f;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) d = __builtin_fmaf(wimg[k][j], cur.g[k], d);
-                    d_feat[(size_t)(g + LPP * j) * plane + pix] = d;
-                }
+                for (int k = 0; k < 4; ++k) d = __builtin_fmaf(wimg[k][j], cur.g[k], d);
+                if (has_img[j]) dx_of[j][pix] = d;
             }
             if (WGRAD)
             {

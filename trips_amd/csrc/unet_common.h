@@ -18,7 +18,7 @@ constexpr int kConvPatchH  = kConvTileH + 2;
 constexpr int kConvPatchW  = kConvTileW + 2;
 constexpr int kBelowH      = kConvTileH / 2 + 2;  // rows / columns of the level below that an upsampled patch touches
 constexpr int kBelowW      = kConvTileW / 2 + 2;
-constexpr int kFinalPixelsPerBlock = 512;   // pixels a workgroup of the 1x1 convolution's backward takes at a time
+constexpr int kFinalPixelsPerBlock = 256;   // pixels a workgroup of the 1x1 convolution's backward takes at a time
 constexpr int kUnetMaxImageChannels = 16;  // channels of the splat images (the descriptor widths of the splat: 3, 4, 6, 8, 16)
 constexpr int kFinalPartFloats     = 4 * (kUnetMaxImageChannels + 64) + 4;  // its partial sums: [4 outputs][<= 16 image + <= 64 block channels], 4 biases
 constexpr int kMaxGridImages = 32768;  // images of a batch that one launch takes (the y and z dimensions of a grid end at 65535)
@@ -257,10 +257,11 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
     }
     {
         const size_t chunks = d.batch * (((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
-        // as many workgroups as are resident at once walk the chunks (three per CU at the 162 registers of the instance for
-        // 16 image channels; the others, at 109 to 125, would leave room for a fourth): a second, partly filled round of
-        // one-chunk workgroups cost a third of the kernel's time
-        np.final_groups     = chunks < 768 ? (int)chunks : 768;
+        // as many workgroups as are resident at once walk the chunks (four per CU at the 100 to 118 registers of most
+        // instances): a second, partly filled round of one-chunk workgroups cost a third of the kernel's time. Three per CU
+        // with chunks of 512 pixels 95 us at 1245 x 825, four 90, four with chunks of 256 (less difference between the
+        // workgroup with the most and the one with the fewest) 84; five, at 96 registers, no faster.
+        np.final_groups     = chunks < 1024 ? (int)chunks : 1024;
         np.final_part_off   = bw;
         bw += align256((size_t)np.final_groups * kFinalPartFloats * sizeof(float));
     }
