@@ -341,158 +341,105 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Everything between the projection and the scatter that ONE workgroup can do, in one launch:
-//   * the view's counters, written (not added to, so that nothing has to clear them first): valid points and flags
-//     summed over the chunks of the projection, entries from the scan; on the first view of a call the status block
-//     of the whole call as well;
-//   * exclusive scan of the tile totals: bin_start[i] = sum_{k<i} bin_count[k], bin_start[NB] = total;
-//   * slices of split tiles: a tile with more than kSliceEntries bin entries (hundreds of points per pixel, e.g.
-//     tight clusters) would keep a single workgroup busy for milliseconds; it is cut into slices of kSliceEntries
-//     entries, each a workgroup of its own. slice_start[t] = number of slices of split tiles before tile t.
-// Its time is a chain of barriers and round trips, so every thread takes its share of the tiles at once (all loads in
-// flight together) and the scans over chunks and tiles share their barriers.
-// The workgroups after the first clear the per-cell counters `counts` and `run` of the tiles that may be split: the
-// slices add to them. Those of any other tile are written, not added to, where its keys are placed (clearing all of
-// them was 22 MB at 1920 x 1080 and eight layers: with that and a scan of 1024 tiles at a time, 13.8 us there; now 6).
-constexpr int kPlanPer = (kMaxBins + 1023) / 1024;  // tiles of a thread
-__global__ __launch_bounds__(1024) void scan_plan_kernel(const int32_t* __restrict__ bin_count, int32_t* __restrict__ bin_start,
-                                                         int32_t* __restrict__ slice_start, int NB, long long capacity,
-                                                         int32_t* __restrict__ chunk_valid, int G, ViewHeader* header,
-                                                         ViewHeader* status, int first_view, int32_t* __restrict__ long_count,
-                                                         int32_t* __restrict__ counts, int32_t* __restrict__ run,
-                                                         int32_t* __restrict__ saved_chunk_valid)
-{
-    if (blockIdx.x > 0)
-    {
-        // (a superset of the tiles that are split: entries past the capacity may leave a tile whole)
-        static_assert(kTilePixels == 1024, "a thread per cell");
-        for (int t = blockIdx.x - 1; t < NB; t += gridDim.x - 1)
-            if (bin_count[t] > kSliceEntries)
-            {
-                counts[(size_t)t * kTilePixels + threadIdx.x] = 0;
-                run[(size_t)t * kTilePixels + threadIdx.x]    = 0;
-            }
-        return;
-    }
-    __shared__ int s_over[16], s_tiles[16], s_slices[16], s_valid[16], s_flag[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int per  = (NB + 1023) / 1024;
-    const int t0   = (int)threadIdx.x * per;
-    int v[kPlanPer];
-#pragma unroll
-    for (int j = 0; j < kPlanPer; ++j) v[j] = j < per && t0 + j < NB ? bin_count[t0 + j] : 0;
-    const bool chunk = (int)threadIdx.x < G;  // (G <= 1024)
-    const int valid = chunk ? chunk_valid[threadIdx.x] : 0;
-    const int flags = chunk ? chunk_valid[G + threadIdx.x] : 0;
-    const int over  = chunk ? chunk_valid[2 * G + threadIdx.x] : 0;
-
-    auto wave_scan = [&](int x)
-    {
-        for (int o = 1; o < 64; o <<= 1)
-        {
-            const int t = __shfl_up(x, o);
-            if (lane >= o) x += t;
-        }
-        return x;
-    };
-    // sum over the wavefronts before this one, and over all of them
-    auto wave_prefix = [&](const int* waves, int& all)
-    {
-        int before = 0;
-        all        = 0;
-#pragma unroll
-        for (int w = 0; w < 16; ++w)
-        {
-            const int x = waves[w];
-            before += w < wave ? x : 0;
-            all += x;
-        }
-        return before;
-    };
-    int sum = 0;
-#pragma unroll
-    for (int j = 0; j < kPlanPer; ++j) sum += v[j];
-    const int inc_tiles = wave_scan(sum), inc_over = wave_scan(over), inc_valid = wave_scan(valid);
-    const int wave_flags = (__ballot(flags & 1) ? 1 : 0) | (__ballot(flags & 2) ? 2 : 0);
-    if (lane == 63) s_tiles[wave] = inc_tiles, s_over[wave] = inc_over, s_valid[wave] = inc_valid, s_flag[wave] = wave_flags;
-    __syncthreads();
-    int total, total_over, total_valid, total_slices;
-    int first = wave_prefix(s_tiles, total) + inc_tiles - sum;  // first slot of the thread's first tile
-    // number of every chunk's first overflow row
-    const int first_over = wave_prefix(s_over, total_over) + inc_over - over;
-    if (chunk) chunk_valid[3 * G + threadIdx.x] = first_over;
-    if (saved_chunk_valid && chunk) saved_chunk_valid[threadIdx.x] = valid;
-    if (saved_chunk_valid && (int)threadIdx.x < kRetainedParts) saved_chunk_valid[G + threadIdx.x] = 0;  // (the blend adds)
-    // slices of the tiles' entries that fit the capacity
-    int sl[kPlanPer], slices = 0;
-#pragma unroll
-    for (int j = 0; j < kPlanPer; ++j)
-    {
-        sl[j] = 0;
-        if (j < per && t0 + j < NB)
-        {
-            bin_start[t0 + j]    = first;
-            const long long last = min((long long)first + v[j], capacity);
-            const long long n    = max(last - (long long)first, 0ll);
-            sl[j]                = n > kSliceEntries ? (int)((n + kSliceEntries - 1) / kSliceEntries) : 0;
-        }
-        first += v[j];
-        slices += sl[j];
-    }
-    const int inc_slices = wave_scan(slices);
-    if (lane == 63) s_slices[wave] = inc_slices;
-    __syncthreads();
-    int first_slice = wave_prefix(s_slices, total_slices) + inc_slices - slices;
-#pragma unroll
-    for (int j = 0; j < kPlanPer; ++j)
-    {
-        if (j < per && t0 + j < NB) slice_start[t0 + j] = first_slice;
-        first_slice += sl[j];
-    }
-    if (threadIdx.x == 0)
-    {
-        wave_prefix(s_valid, total_valid);
-        int any_flags = 0;
-        for (int w = 0; w < 16; ++w) any_flags |= s_flag[w];
-        *long_count     = 0;
-        bin_start[NB]   = total;
-        slice_start[NB] = total_slices;
-        const unsigned long long bad = (unsigned long long)((any_flags >> 1) & 1);
-        header->n_valid       = (unsigned long long)(unsigned)total_valid;
-        header->n_entries     = (unsigned long long)(unsigned)total;
-        header->overflow      = 0;
-        header->retained      = 0;
-        header->not_identity  = (unsigned long long)(any_flags & 1);
-        header->bad_index     = 0;
-        header->overflow_rows = (unsigned long long)(unsigned)total_over;
-        if (first_view)
-        {
-            status->n_valid = status->n_entries = status->overflow = status->retained = status->not_identity = 0;
-            status->bad_index                                                       = bad;
-            status->overflow_rows                                                   = 0;
-        }
-        else if (bad)
-            status->bad_index = 1;  // (the views of a call run one after the other on the stream)
-    }
-}
-
-// ---------------------------------------------------------------------------------------------------------
 // Column-wise exclusive prefix of the histogram matrix [workgroup][bin]: afterwards hist[g][bin] = entries of
 // `bin` that come from workgroups before g, and bin_count[bin] = the column total. No atomics anywhere in the
 // binning, since atomics on a few thousand hot counters serialise. A workgroup owns 16 columns; its 16 row
 // segments are summed side by side, prefixed through LDS, then each segment writes its rows' prefixes (one thread
 // walking a whole column is a chain of G dependent-latency steps).
+// A workgroup also clears the per-cell counters `counts` and `run` of those of its tiles that may be split: their slices add
+// to them. Those of any other tile are written, not added to, where its keys are placed (clearing all of them is 22 MB at
+// 1920 x 1080 and eight layers).
+//
+// The last workgroup adds up the chunks of the projection: the number of every chunk's first overflow row, and the view's
+// counters, written (not added to, so that nothing has to clear them first); on the first view of a call the status block of
+// the whole call as well. The scan over the tiles' totals is the scatter pass's (BinPlan).
 constexpr int kScanCols = 16, kScanSegs = 16;
-__global__ __launch_bounds__(256) void bin_column_scan_kernel(int32_t* __restrict__ hist, int32_t* __restrict__ bin_count,
-                                                              int NB, int G)
+__device__ __forceinline__ int wave_inclusive_scan(int x)
 {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+    {
+        const int t = __shfl_up(x, o);
+        if (lane >= o) x += t;
+    }
+    return x;
+}
+// sum over the wavefronts before this one, and over all of them
+template <int WAVES>
+__device__ __forceinline__ int waves_before(const int* waves, int& all)
+{
+    const int wave = threadIdx.x >> 6;
+    int before     = 0;
+    all            = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+    {
+        const int x = waves[w];
+        before += w < wave ? x : 0;
+        all += x;
+    }
+    return before;
+}
+
+__device__ __forceinline__ void sum_chunks(const ForwardParams& p, bool first_view)
+{
+    static_assert(kBinGroups == 256 && kRetainedParts == 256, "a thread per chunk, and per part");
+    constexpr int G = kBinGroups;
+    __shared__ int s_over[4], s_valid[4], s_flag[4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int valid = p.chunk_valid[t], flags = p.chunk_valid[G + t], over = p.chunk_valid[2 * G + t];
+    const int inc_over = wave_inclusive_scan(over), inc_valid = wave_inclusive_scan(valid);
+    const int wave_flags = (__ballot(flags & 1) ? 1 : 0) | (__ballot(flags & 2) ? 2 : 0);
+    if (lane == 63) s_over[wave] = inc_over, s_valid[wave] = inc_valid, s_flag[wave] = wave_flags;
+    __syncthreads();
+    int total_over, total_valid;
+    p.chunk_valid[3 * G + t] = waves_before<4>(s_over, total_over) + inc_over - over;
+    waves_before<4>(s_valid, total_valid);
+    if (p.saved_chunk_valid)
+    {
+        p.saved_chunk_valid[t]     = valid;
+        p.saved_chunk_valid[G + t] = 0;  // (the blend adds)
+    }
+    if (t == 0)
+    {
+        const int any_flags = s_flag[0] | s_flag[1] | s_flag[2] | s_flag[3];
+        *p.long_count       = 0;
+        const unsigned long long bad = (unsigned long long)((any_flags >> 1) & 1);
+        p.header->n_valid       = (unsigned long long)(unsigned)total_valid;
+        p.header->overflow      = 0;
+        p.header->retained      = 0;
+        p.header->not_identity  = (unsigned long long)(any_flags & 1);
+        p.header->bad_index     = 0;
+        p.header->overflow_rows = (unsigned long long)(unsigned)total_over;
+        if (first_view)
+        {
+            ViewHeader* status = p.status;
+            status->n_valid = status->n_entries = status->overflow = status->retained = status->not_identity = 0;
+            status->bad_index                                                       = bad;
+            status->overflow_rows                                                   = 0;
+        }
+        else if (bad)
+            p.status->bad_index = 1;  // (the views of a call run one after the other on the stream)
+    }
+}
+
+__global__ __launch_bounds__(256) void bin_column_scan_kernel(const ForwardParams p, int first_view)
+{
+    if (blockIdx.x == gridDim.x - 1)
+    {
+        sum_chunks(p, first_view != 0);
+        return;
+    }
     __shared__ int s_seg[kScanSegs][kScanCols];
+    __shared__ int s_total[kScanCols];
+    const int NB = p.geom.bin_off[p.num_layers], G = p.bin_groups;
     const int c = threadIdx.x % kScanCols, seg = threadIdx.x / kScanCols;
-    const int bin = blockIdx.x * kScanCols + c;
+    const int bin0 = blockIdx.x * kScanCols, bin = bin0 + c;
     const int rows = (G + kScanSegs - 1) / kScanSegs;
     const int g0 = seg * rows, g1 = min(G, g0 + rows);
     const bool live = bin < NB;
-    int32_t* col    = hist + bin;
+    int32_t* col    = p.bin_hist + bin;
     int sum         = 0;
     if (live)
         for (int g = g0; g < g1; g += 8)
@@ -507,20 +454,34 @@ __global__ __launch_bounds__(256) void bin_column_scan_kernel(int32_t* __restric
     __syncthreads();
     int run = 0;
     for (int k = 0; k < seg; ++k) run += s_seg[k][c];
-    if (!live) return;
-    for (int g = g0; g < g1; g += 8)
-    {
-        int v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = (g + k < g1) ? col[(size_t)(g + k) * NB] : 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
+    if (live)
+        for (int g = g0; g < g1; g += 8)
         {
-            if (g + k < g1) col[(size_t)(g + k) * NB] = run;
-            run += v[k];
+            int v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = (g + k < g1) ? col[(size_t)(g + k) * NB] : 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                if (g + k < g1) col[(size_t)(g + k) * NB] = run;
+                run += v[k];
+            }
         }
+    if (seg == kScanSegs - 1)
+    {
+        s_total[c] = run;  // (of columns past the last: 0)
+        if (live) p.bin_count[bin] = run;
     }
-    if (seg == kScanSegs - 1) bin_count[bin] = run;
+    __syncthreads();
+    // (a superset of the tiles that are split: entries past the capacity may leave a tile whole)
+    static_assert(kTilePixels == 4 * 256, "four cells of a thread");
+    for (int k = 0; k < kScanCols; ++k)
+        if (s_total[k] > kSliceEntries)
+        {
+            const size_t at = (size_t)(bin0 + k) * (kTilePixels / 4) + threadIdx.x;
+            reinterpret_cast<int4*>(p.counts)[at] = make_int4(0, 0, 0, 0);
+            reinterpret_cast<int4*>(p.run)[at]    = make_int4(0, 0, 0, 0);
+        }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -558,6 +519,86 @@ struct BinEntry<false>
 };
 static_assert(kTilePixels == 1 << (2 * kTileShift), "a cell number takes 2 kTileShift bits");
 
+// The plan of the view's tiles, from their totals:
+//   * exclusive scan: bin_start[i] = sum_{k<i} bin_count[k], bin_start[NB] = total;
+//   * slices of split tiles: a tile with more than kSliceEntries bin entries (hundreds of points per pixel, e.g.
+//     tight clusters) would keep a single workgroup busy for milliseconds; it is cut into slices of kSliceEntries
+//     entries, each a workgroup of its own. slice_start[t] = number of slices of split tiles before tile t.
+// Every workgroup of the scatter pass makes the scan for itself (a few values of a thread, two barriers) and keeps its
+// cursors in `s_cur`; the first one writes scan and slices for the kernels behind. Bound by its round trips: 1.7 us longer the
+// scatter (2.6 at 2700 tiles) and a launch between column scan and scatter less, whose single workgroup took 4.5: 100k
+// points at 512^2 53.9 -> 52.1 us for the whole render, 20k at 160 x 120 with the network 98.7 -> 94.7, 1M at 1920 x 1080
+// 237.5 -> 234.4.
+constexpr int kPlanPer = (kMaxBins + kBinThreads - 1) / kBinThreads;  // tiles of a thread
+__device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t* __restrict__ row, int NB, int* __restrict__ s_cur)
+{
+    constexpr int WAVES = kBinThreads / 64;
+    __shared__ int s_tiles[WAVES], s_slices[WAVES];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per  = (NB + kBinThreads - 1) / kBinThreads;
+    const int t0   = (int)threadIdx.x * per;
+    int v[kPlanPer], before[kPlanPer], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j)
+    {
+        const bool live = j < per && t0 + j < NB;
+        v[j]      = live ? p.bin_count[t0 + j] : 0;
+        before[j] = live ? row[t0 + j] : 0;  // entries of the chunks before this one
+    }
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j) sum += v[j];
+    const int inc_tiles = wave_inclusive_scan(sum);
+    if (lane == 63) s_tiles[wave] = inc_tiles;
+    __syncthreads();
+    int total;
+    const int first0 = waves_before<WAVES>(s_tiles, total) + inc_tiles - sum;  // first slot of the thread's first tile
+    int first = first0;
+#pragma unroll
+    for (int j = 0; j < kPlanPer; ++j)
+    {
+        if (j < per && t0 + j < NB) s_cur[t0 + j] = first + before[j];
+        first += v[j];
+    }
+    if (blockIdx.x == 0)
+    {
+        // slices of the tiles' entries that fit the capacity
+        int sl[kPlanPer], slices = 0;
+        first = first0;
+#pragma unroll
+        for (int j = 0; j < kPlanPer; ++j)
+        {
+            sl[j] = 0;
+            if (j < per && t0 + j < NB)
+            {
+                p.bin_start[t0 + j]  = first;
+                const long long last = min((long long)first + v[j], p.capacity);
+                const long long n    = max(last - (long long)first, 0ll);
+                sl[j]                = n > kSliceEntries ? (int)((n + kSliceEntries - 1) / kSliceEntries) : 0;
+            }
+            first += v[j];
+            slices += sl[j];
+        }
+        const int inc_slices = wave_inclusive_scan(slices);
+        if (lane == 63) s_slices[wave] = inc_slices;
+        __syncthreads();
+        int total_slices;
+        int first_slice = waves_before<WAVES>(s_slices, total_slices) + inc_slices - slices;
+#pragma unroll
+        for (int j = 0; j < kPlanPer; ++j)
+        {
+            if (j < per && t0 + j < NB) p.slice_start[t0 + j] = first_slice;
+            first_slice += sl[j];
+        }
+        if (threadIdx.x == 0)
+        {
+            p.bin_start[NB]     = total;
+            p.slice_start[NB]   = total_slices;
+            p.header->n_entries = (unsigned long long)(unsigned)total;
+        }
+    }
+    __syncthreads();
+}
+
 // One bin entry per (point, layer), in the tile of the footprint's first pixel. A workgroup walks
 // the records that its chunk of the points left at the compact numbers; its slots inside every bin are contiguous
 // and start at bin_start[bin] + hist[workgroup][bin].
@@ -567,11 +608,9 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     using E = BinEntry<PACKED>;
     typename E::T* __restrict__ entries = reinterpret_cast<typename E::T*>(p.bin_entries);
     extern __shared__ int s_cur[];
-    const int NB       = p.geom.bin_off[p.num_layers];
-    const int chunk    = chunk_of_workgroup();
-    const int32_t* row = p.bin_hist + (size_t)chunk * NB;
-    for (int i = threadIdx.x; i < NB; i += kBinThreads) s_cur[i] = p.bin_start[i] + row[i];
-    __syncthreads();
+    const int NB    = p.geom.bin_off[p.num_layers];
+    const int chunk = chunk_of_workgroup();
+    plan_tiles(p, p.bin_hist + (size_t)chunk * NB, NB, s_cur);
     int begin, end;
     chunk_point_range(p, chunk, begin, end);
     const int n      = p.chunk_valid[chunk];
@@ -1487,10 +1526,7 @@ hipError_t launch_forward_view(const ForwardParams& p, int channels, bool train,
     }
     {
         ProfScope ps(prof, "bin_scan", stream);
-        hipLaunchKernelGGL(bin_column_scan_kernel, dim3((NB + kScanCols - 1) / kScanCols), dim3(256), 0, stream, p.bin_hist, p.bin_count, NB, G);
-        hipLaunchKernelGGL(scan_plan_kernel, dim3(1 + std::min(NB, 255)), dim3(1024), 0, stream, p.bin_count, p.bin_start,
-                           p.slice_start, NB, p.capacity, p.chunk_valid, G, p.header, p.status, first_view ? 1 : 0, p.long_count,
-                           p.counts, p.run, p.saved_chunk_valid);
+        hipLaunchKernelGGL(bin_column_scan_kernel, dim3((NB + kScanCols - 1) / kScanCols + 1), dim3(256), 0, stream, p, first_view ? 1 : 0);
     }
     {
         ProfScope ps(prof, "bin_scatter", stream);
