@@ -31,18 +31,18 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "14f2165ef7675dbf5de03cbc4b7e7224bee2e22f3e62b9af4fbd4273fb754787"
+PMC_SOURCES_SHA256 = "3ad2b3d3ad5acae111af3338bcda4037c306940632267f7d429e6518841c30b8"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129116, 237345),
-    "bin_scatter": (95985, 166944),
-    "tile_count": (13148, 2296),
-    "tile_scatter": (26677, 105766),
-    "cell_sort": (35344, 42151),
-    "blend": (319572, 195403),
-    "backward_prologue": (55, 265130),
-    "backward_tiles": (425689, 121568),
-    "backward_points": (297354, 234503),
-    "adam_fused": (383788, 498420),
+    "project_bin": (129103, 236068),
+    "bin_scatter": (94971, 191274),
+    "tile_count": (13115, 2295),
+    "tile_scatter": (26033, 89345),
+    "cell_sort": (35349, 42136),
+    "blend": (367709, 196692),
+    "backward_prologue": (54, 265165),
+    "backward_tiles": (427122, 121568),
+    "backward_points": (309723, 234503),
+    "adam_fused": (383764, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
                         "splat_internal.h", "trips_math.h", "row16.h")

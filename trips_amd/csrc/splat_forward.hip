@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     // The loads of the next step's points, their descriptors and dropout flags among them (whether a point is visible or
     // not), are in flight while this step's are projected. (With the dropout flag and the descriptor requested in the
     // step itself, its waits were a part of every step: 9M points with dropout 225 us, now 197; 6M without 152, now 150,
-    // which its vector instructions, 100 us, and the 520 MB that it moves, 105 us at a copy's rate, bound together.)
+    // which its vector instructions, 100 us, and the 520 MB that it moves, 84 us at a copy's rate, bound together.)
     PointInputs<CPAD> nxt;
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)

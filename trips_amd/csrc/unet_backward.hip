@@ -728,7 +728,7 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
 // A wavefront owns 4 x 16 pixels and half of the outputs and keeps the weights of those in registers for the whole strip:
 // an operand read from the patch then serves up to three taps, and the sums run in the order of conv_taps_mfma.
 //
-// Bound at the finest level of a large image by memory (1920 x 1080: 484 MB in 124 us, 81 % of a copy's rate, halos that
+// Bound at the finest level of a large image by memory (1920 x 1080: 484 MB in 124 us, 63 % of a copy's rate, halos that
 // neighbouring strips read as well among them), elsewhere by the steps' latencies (two barriers each) at one or two
 // workgroups per CU. As two kernels and as one: 1920 x 1080, 32 pre-activations x 32 inputs: 90 + 68 and 125 us;
 // 960 x 540, 64 x 64: 54 + 36 and 83 us; 1245 x 825 and the levels below it, 64 x 32: 119 + 60 and 164 us. The gather as
