@@ -106,8 +106,10 @@ struct FinalBwdParams
 // writes. The rows it reads are read for the last time, whole lines of them by a wavefront, and are loaded past the caches:
 // loaded as usual they push out the rows that are written, which the data gradient reads next. 1245 x 825 pixels: 96 us, 71
 // with the loads past the caches (and the data gradient of the level 113, now 106), 4.3 TB/s; four crops of 512^2: 83, now
-// 64; 1717 x 783 at 32 gates: 71, now 57. Two or four pixels of a lane requested together gave nothing (86 and 93 us where
-// one gave 84): the registers cost as many wavefronts as they add loads.
+// 64; 1717 x 783 at 32 gates: 71, now 57, all with caches that other data has been through; in a loop over the same buffers
+// the loads past the caches change nothing and the workgroups and chunks (unet_common.h) save 1 % of a training step on the crops. Two or four pixels
+// of a lane requested together gave nothing (86 and 93 us where one gave 84): the registers cost as many wavefronts as they
+// add loads.
 // CI = image channels the kernel has room for (4, 8 or 16).
 template <int NPAD, bool WGRAD, int CI>
 __global__ __launch_bounds__(256) void final_backward_kernel(const FinalBwdParams p)
