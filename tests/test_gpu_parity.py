@@ -303,6 +303,43 @@ def test_backward_views_crop_distortion_optional_outputs(oracle):
     _check_backward(oracle, sc, d, want_position=False, want_pose=False, want_intrinsics=False)
 
 
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_gradients_out_of_range_reach_both_axes(oracle, axis, mode):
+    """The image gradient changes its sign from pixel to pixel along one axis and is so large that the gradient of a point on
+    the image plane overflows along it and not along the other (nothing before it does). The Jacobian of the distortion, the
+    identity here, multiplies what is not finite by zero: the point's gradient is NaN in all components, as the oracle's, and
+    so is the pose's; the other points' gradients are the oracle's."""
+    from tests.gpu_util import GRAD_FLOOR, GRAD_RTOL, GpuRun
+    sc = scenes.tiny(n=200, w=96, h=64, f=8000.0, num_layers=1, list_depth=8, seed=12, radius=(0.00002, 0.00012))
+    sc.position[:, :3] *= 0.01
+    sc.confidence[:] = np.exp(np.random.default_rng(0).uniform(np.log(1e-4), np.log(0.9), 200))
+    sc.poses_se3[0] = scenes.look_at_pose((0.9, 0.4, -3.0), (0.0, 0.0, 0.0))  # (no zeros in the rotation)
+    d = abi.desc_for_scene(sc)
+    assert not sc.intrinsics[0, 5:].any()
+    sign = np.where((np.arange(96)[None, :] if axis == 0 else np.arange(64)[:, None]) % 2, 1.0, -1.0)
+    grads = [np.broadcast_to(1e36 * sign, (1, 4, 64, 96)).astype(np.float32)]
+    ref = oracle.forward(sc, d)
+    want = oracle.backward(sc, d, ref, grads)
+    run = GpuRun(sc, d)
+    run.forward()
+    try:
+        run.ctx.pair_rows_mode(mode)
+        got = run.backward(grads)
+    finally:
+        run.ctx.pair_rows_mode(0)
+    # (the oracle runs the chain per pixel, the kernels once per point on the sum over its pixels: a point whose single
+    # gradients stay in range may leave it in their sum)
+    w, g = want["d_position"][:, :3], got["d_position"][:, :3]
+    out, clear = np.isnan(w).all(axis=1), np.abs(np.nan_to_num(w, nan=np.inf)).max(axis=1) < 3e38 / 64
+    assert out.sum() > 40 and (clear & (w != 0).any(axis=1)).sum() > 40
+    assert np.isnan(g[out]).all()
+    assert (np.isnan(g).all(axis=1) | np.isfinite(g).all(axis=1))[out | clear].all()
+    w, g = w[clear].astype(np.float64), g[clear].astype(np.float64)
+    assert (np.abs(g - w) <= GRAD_RTOL * np.abs(w) + GRAD_FLOOR * np.abs(w).max()).all()
+    assert np.isnan(want["d_pose"]).all() and np.isnan(got["d_pose"]).all()
+
+
 @pytest.mark.parametrize("case", ["two_views", "shared_columns", "spare_columns", "bad_index", "no_size_no_position"])
 def test_backward_overwrite_mode_equals_adding_into_zeros(case):
     """overwrite_point_grads: the per-point outputs start as NaN and must come out bit-equal to what adding into

@@ -315,24 +315,26 @@ __device__ __forceinline__ void project_backward(const Camera& cam, const float 
     if (cam.no_distortion)
     {
         // all eight coefficients are zero: the distortion is the identity, and of the Jacobian of its coefficients only the
-        // powers of the radius are left (the same bits as through distort() and its matrices)
-        const float x2 = nx * nx, y2 = ny * ny, r2 = x2 + y2, r4 = r2 * r2, r6 = r4 * r2;
-        const bool cut = r2 > cam.dist_cutoff * cam.dist_cutoff;  // (never of a point that the projection kept)
+        // powers of the radius are left (the same bits as through distort() and its matrices, whose zeros stay in the
+        // sums: they carry a gradient of one axis that is not finite to the other)
+        const bool cut = nx * nx + ny * ny > cam.dist_cutoff * cam.dist_cutoff;  // (never of a point that the projection kept)
         dx = cut ? 100000.f : nx;
         dy = cut ? 100000.f : ny;
-        d0 = cut ? 0.f : k0;
-        d1 = cut ? 0.f : k1;
+        const float j = cut ? 0.f : 1.f;
+        d0 = j * k0 + 0.f * k1;
+        d1 = 0.f * k0 + j * k1;
         if (want_intrinsics)
         {
-            const float xy2 = 2.f * nx * ny;
-            g_dis[0] = nx * r2 * d0 + ny * r2 * d1;
-            g_dis[1] = nx * r4 * d0 + ny * r4 * d1;
-            g_dis[2] = nx * r6 * d0 + ny * r6 * d1;
+            const float x = cut ? 0.f : nx, y = cut ? 0.f : ny;
+            const float x2 = x * x, y2 = y * y, r2 = x2 + y2, r4 = r2 * r2, r6 = r4 * r2, xy2 = 2.f * x * y;
+            g_dis[0] = x * r2 * k0 + y * r2 * k1;
+            g_dis[1] = x * r4 * k0 + y * r4 * k1;
+            g_dis[2] = x * r6 * k0 + y * r6 * k1;
             g_dis[3] = -g_dis[0];
             g_dis[4] = -g_dis[1];
             g_dis[5] = -g_dis[2];
-            g_dis[6] = xy2 * d0 + (r2 + 2.f * y2) * d1;
-            g_dis[7] = (r2 + 2.f * x2) * d0 + xy2 * d1;
+            g_dis[6] = xy2 * k0 + (r2 + 2.f * y2) * k1;
+            g_dis[7] = (r2 + 2.f * x2) * k0 + xy2 * k1;
         }
     }
     else
