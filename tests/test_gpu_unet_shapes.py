@@ -131,8 +131,9 @@ def test_upsampling_of_neighbours_far_apart():
     ([16, 32, 48, 64], 300, 200, 2),      # levels of several instances, two of which share one, a level of two shares
 ])
 def test_weight_gradients_of_some_levels(filters, w, h, batch):
-    """Levels whose weight gradients are the same instance of the kernel run in one launch: without the gradients of some
-    levels (weights, biases or both), the others are the same bits as with all of them."""
+    """Levels whose weight gradients are the same instance of the kernel run in one launch, whose workgroups are dealt to the
+    levels that are asked for: without the gradients of some levels (weights, biases or both), the others are those that all
+    of them together give, the same bits where the tiles are dealt alike."""
     import ctypes as C
 
     from trips_amd import _lib, abi
@@ -163,10 +164,13 @@ def test_weight_gradients_of_some_levels(filters, w, h, batch):
         return outs, d_ins
     full, full_ins = backward([(True, True)] * L)
     assert all(bool(torch.isfinite(t).all()) for t in full[:4 * L])
+    # 8 x 32 tiles, at most two shares of each: up to 240 of them find a workgroup of their own whatever is asked for
+    few = 2 * batch * sum(-(-t.shape[2] // 8) * -(-t.shape[3] // 32) for t in ins) <= 240
     for wanted in ([(i != 1, True) for i in range(L)], [(True, i != 0) for i in range(L)], [(i % 2 == 0, i < 2) for i in range(L)],
                    [(i == L - 1, False) for i in range(L)]):
         part, part_ins = backward(wanted)
         assert all(torch.equal(a, b) for a, b in zip(part_ins, full_ins))
+        dealt_alike = few or all(weights for weights, _ in wanted)
         for i, (weights, biases) in enumerate(wanted):
             for k in range(4):
                 a, b = part[4 * i + k], full[4 * i + k]
@@ -174,5 +178,10 @@ def test_weight_gradients_of_some_levels(filters, w, h, batch):
                     assert bool(torch.isnan(a).all())
                 elif k % 2 == 1 and not weights:  # summed by a kernel of its own: single precision, another order
                     assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max()) + 1e-12
-                else:
+                elif dealt_alike:
                     assert torch.equal(a, b), (wanted, i, k)
+                else:
+                    # The same products (exact in fp32) summed in another order. A sum is a chain of about 100 additions (a
+                    # workgroup's tiles, then the workgroups): rounding errors of sqrt(100) 2^-24 = 6e-7 of partial sums that
+                    # are no larger than the largest result (terms of either sign); 16 times that.
+                    assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()), (wanted, i, k)

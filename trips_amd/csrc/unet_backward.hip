@@ -1109,7 +1109,7 @@ struct BwdWeightParams
     int groups;            // workgroups of each share of NPAD pre-activations
     float* part;           // [groups][9][npad][CIN]
     // bias gradients = sums of dpre over the pixels, taken from the transposed tile while it is in LDS
-    float* bias_part;      // [groups][npad] or nullptr
+    float* bias_part;      // [groups][npad]
 };
 // The levels of a launch, one after the other in its workgroups: level, share, group.
 struct BwdWeightTable
@@ -1701,25 +1701,25 @@ hipError_t launch_bwd_weight(const BwdWeightTable& t, int blocks, hipStream_t st
 }
 
 template <int CI, bool FOUR>
-hipError_t dispatch_bwd_weight_ci(const BwdWeightTable& t, int blocks, int cin_pad, int tile, hipStream_t stream)
+hipError_t dispatch_bwd_weight_ci(const BwdWeightTable& t, int blocks, const LevelPlan& lv, bool bias, hipStream_t stream)
 {
-#define TRIPS_BW(CIN_, NT_)                                                                    \
-    if (cin_pad == CIN_ && tile == NT_)                                                        \
-        return t.lv[0].bias_part ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(t, blocks, stream) \
-                                 : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(t, blocks, stream);
+#define TRIPS_BW(CIN_, NT_)                                                                 \
+    if (lv.cin_pad == CIN_ && lv.wgrad_tile == NT_)                                         \
+        return bias ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(t, blocks, stream)       \
+                    : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(t, blocks, stream);
     TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 128) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
 #undef TRIPS_BW
     return hipErrorInvalidValue;
 }
 
-// the levels of a launch are the same instance of the kernel, all with bias gradients or all without
-hipError_t dispatch_bwd_weight(const BwdWeightTable& t, int blocks, const LevelPlan& lv, hipStream_t stream)
+// `lv`: any level of the launch (all are the same instance of the kernel)
+hipError_t dispatch_bwd_weight(const BwdWeightTable& t, int blocks, const LevelPlan& lv, bool bias, hipStream_t stream)
 {
     const int C = t.lv[0].c_feat;
-    if (C == 4) return dispatch_bwd_weight_ci<4, true>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
-    if (C < 4) return dispatch_bwd_weight_ci<4, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
-    if (C <= 8) return dispatch_bwd_weight_ci<8, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
-    return dispatch_bwd_weight_ci<16, false>(t, blocks, lv.cin_pad, lv.wgrad_tile, stream);
+    if (C == 4) return dispatch_bwd_weight_ci<4, true>(t, blocks, lv, bias, stream);
+    if (C < 4) return dispatch_bwd_weight_ci<4, false>(t, blocks, lv, bias, stream);
+    if (C <= 8) return dispatch_bwd_weight_ci<8, false>(t, blocks, lv, bias, stream);
+    return dispatch_bwd_weight_ci<16, false>(t, blocks, lv, bias, stream);
 }
 }  // namespace
 }  // namespace trips
@@ -1757,9 +1757,13 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     if (!weights->final_weight) return set_error(TRIPS_ERR_INVALID_ARG, "final weights are NULL");
     if ((reinterpret_cast<uintptr_t>(workspace) & 255) || (reinterpret_cast<uintptr_t>(saved) & 255))
         return set_error(TRIPS_ERR_INVALID_ARG, "workspace / saved must be 256-byte aligned");
-    const NetPlan np = make_plan(d);
+    NetPlan np = make_plan(d);
     if (workspace_bytes < np.backward_bytes)
         return set_error(TRIPS_ERR_WORKSPACE_SMALL, "workspace has %zu bytes, %zu needed", workspace_bytes, np.backward_bytes);
+    unsigned wanted = 0;  // levels whose weight gradients are asked for
+    for (int i = 0; i < L; ++i)
+        if (grads->feature_weight[i] || grads->mask_weight[i]) wanted |= 1u << i;
+    plan_wgrad(np, L, wanted, np.wgrad_off);
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     char* ws           = reinterpret_cast<char*>(workspace);
     const char* sv     = reinterpret_cast<const char*>(saved);
@@ -1808,7 +1812,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         for (int i = 0; i < L; ++i)
         {
             const LevelPlan& lv = np.lv[i];
-            if (!grads->feature_weight[i] && !grads->mask_weight[i])  // bias_grad_kernel accumulates; otherwise they are written
+            if (!((wanted >> i) & 1u))  // bias_grad_kernel accumulates; otherwise they are written
             {
                 fill(grads->feature_bias[i], lv.cout);
                 fill(grads->mask_bias[i], lv.cout);
@@ -1934,18 +1938,16 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "backward launch (level %d): %s", i, hipGetErrorString(e));
     }
     // The weight gradients need the pre-activation gradients alone: all behind the data gradients, levels that are the same
-    // instance of the kernel in one launch.
-    bool launched[TRIPS_UNET_MAX_LEVELS] = {};
+    // instance of the kernel in one launch, which the profiler names after the finest of them. It sums the pre-activation
+    // gradients as well if a bias gradient of any of its levels is asked for.
+    unsigned launched = 0;
     for (int i = 0; i < L; ++i)
     {
-        if (launched[i]) continue;
-        ProfScope ps(prof, kWeightNames[i], stream);
-        const bool bias = grads->feature_bias[i] || grads->mask_bias[i];
-        if (!grads->feature_weight[i] && !grads->mask_weight[i])
+        const LevelPlan& lv = np.lv[i];
+        if (!((wanted >> i) & 1u))
         {
-            if (!bias) continue;
-            // (otherwise the weight-gradient kernel sums them on its way)
-            const LevelPlan& lv = np.lv[i];
+            if (!grads->feature_bias[i] && !grads->mask_bias[i]) continue;
+            ProfScope ps(prof, kWeightNames[i], stream);
             BiasGradParams bp;
             bp.pixels    = (size_t)lv.H * lv.W * d.batch;
             bp.npad      = lv.npad;
@@ -1957,37 +1959,39 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
             hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((bp.pixels + kBiasChunk - 1) / kBiasChunk)), dim3(256), 0, stream, bp);
             continue;
         }
+        if ((launched >> i) & 1u) continue;
+        ProfScope ps(prof, kWeightNames[i], stream);
         BwdWeightTable t;
         std::memset(&t, 0, sizeof(t));
         int blocks = 0;
+        bool bias  = false;
         for (int k = i; k < L; ++k)
         {
-            const LevelPlan& lv = np.lv[k];
-            if (launched[k] || !same_wgrad_kernel(lv, np.lv[i]) || !(grads->feature_weight[k] || grads->mask_weight[k]) ||
-                (grads->feature_bias[k] || grads->mask_bias[k]) != bias)
-                continue;
-            launched[k]         = true;
+            const LevelPlan& lk = np.lv[k];
+            if (!((wanted >> k) & 1u) || !same_wgrad_kernel(lk, lv)) continue;
+            launched |= 1u << k;
+            bias                = bias || grads->feature_bias[k] || grads->mask_bias[k];
             t.first[t.n]        = blocks;
             BwdWeightParams& wp = t.lv[t.n++];
-            wp.H = lv.H, wp.W = lv.W, wp.c_feat = C;
-            wp.tiles_x = (lv.W + kConvTileW - 1) / kConvTileW;
-            wp.tiles   = wp.tiles_x * ((lv.H + kConvTileH - 1) / kConvTileH);
-            wp.batch   = d.batch;
-            wp.feat    = inputs[k];
-            wp.npad    = lv.npad;
-            wp.groups  = lv.groups;
-            wp.dpre    = dpre_ptr(k);
-            wp.part    = reinterpret_cast<float*>(ws + lv.part_off);
-            if (bias) wp.bias_part = reinterpret_cast<float*>(ws + lv.bias_part_off);
+            wp.H = lk.H, wp.W = lk.W, wp.c_feat = C;
+            wp.tiles_x   = (lk.W + kConvTileW - 1) / kConvTileW;
+            wp.tiles     = wp.tiles_x * ((lk.H + kConvTileH - 1) / kConvTileH);
+            wp.batch     = d.batch;
+            wp.feat      = inputs[k];
+            wp.npad      = lk.npad;
+            wp.groups    = lk.groups;
+            wp.dpre      = dpre_ptr(k);
+            wp.part      = reinterpret_cast<float*>(ws + lk.part_off);
+            wp.bias_part = reinterpret_cast<float*>(ws + lk.bias_part_off);
             if (k < L - 1)
             {
                 const LevelPlan& lb = np.lv[k + 1];
                 wp.Hb = lb.H, wp.Wb = lb.W, wp.below_stride = lb.row_stride;
                 wp.below = rows_ptr(k + 1);
             }
-            blocks += lv.groups * (lv.npad / lv.wgrad_tile);
+            blocks += lk.groups * (lk.npad / lk.wgrad_tile);
         }
-        hipError_t e = dispatch_bwd_weight(t, blocks, np.lv[i], stream);
+        hipError_t e = dispatch_bwd_weight(t, blocks, lv, bias, stream);
         if (e != hipSuccess) return set_error(TRIPS_ERR_HIP, "weight gradient launch (level %d): %s", i, hipGetErrorString(e));
     }
     // the partial weight and bias gradients of all levels are summed at the end, one launch per step of the sum
@@ -1999,7 +2003,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         for (int i = 0; i < L; ++i)
         {
             const LevelPlan& lv = np.lv[i];
-            if (!grads->feature_weight[i] && !grads->mask_weight[i]) continue;
+            if (!((wanted >> i) & 1u)) continue;
             ReduceLevel& r = rt.lv[n++];
             r.part      = reinterpret_cast<const float*>(ws + lv.part_off);
             r.sliced    = reinterpret_cast<float*>(ws + lv.sliced_off);

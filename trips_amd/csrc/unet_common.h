@@ -3,6 +3,8 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/trips_unet.h"
 #include "splat_internal.h"
 
@@ -126,6 +128,7 @@ struct NetPlan
     size_t fin_off;         // forward workspace: packed weights of the 1x1 output convolution
     size_t saved_bytes;     // saved state
     size_t backward_bytes;  // backward workspace
+    size_t wgrad_off;       // backward workspace: the levels' partial weight and bias gradients (plan_wgrad)
     size_t final_part_off;  // backward workspace: per-workgroup sums of the 1x1 convolution's weight and bias gradients
     int final_groups;       // persistent workgroups of the finest level's first backward kernel, for all images of the batch
 };
@@ -172,26 +175,48 @@ inline int check_unet_desc(const TripsUnetDesc* d)
 // write and reduce) and are dealt to the levels by their tiles. With a launch per level the coarser ones were a handful of
 // tiles each, begun and ended 256 workgroups at a time: all weight gradients and the sums of their partials, default net
 // of five levels at 1245 x 825 155 -> 110 us, at 105 x 74 (32/64/64/64/64) 85 -> 46, 16/32/64/64 at 1920 x 1080 217 -> 205.
+// `wanted` holds a bit per level whose weight gradients are asked for: the workgroups are dealt to those alone. (Dealt as if
+// all were asked for, a level on its own got a fifth of the GPU. Whole backward of the default net at 1245 x 825 with the weight
+// gradients of all levels but the finest 307 -> 256 us, of the second level alone 303 -> 250, of the finest alone 310 -> 291;
+// the finest without its bias gradients, then a launch of its own, 387 -> 316.)
+// The partial sums lie from `at` on; returns where they end, which does not depend on `wanted`: an instance has at most
+// `resident` workgroups, and at most one for each tile and share of its levels, and a workgroup writes one set of sums.
 inline bool same_wgrad_kernel(const LevelPlan& a, const LevelPlan& b) { return a.cin_pad == b.cin_pad && a.wgrad_tile == b.wgrad_tile; }
-inline void plan_wgrad_groups(NetPlan& np, int levels)
+inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
 {
     for (int i = 0; i < levels; ++i)
     {
-        LevelPlan& lv      = np.lv[i];
-        const int resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1);
-        // one workgroup for every share of every level, the others by the tiles (rounded down: one that has to wait for
-        // another to end would take as long again)
-        long long work = 0, shares = 0;
-        for (int k = 0; k < levels; ++k)
+        const LevelPlan& lv = np.lv[i];
+        bool first          = true;  // of its instance
+        for (int k = 0; k < i; ++k) first = first && !same_wgrad_kernel(np.lv[k], lv);
+        if (!first) continue;
+        const long long resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1);
+        long long all = 0, work = 0, shares = 0;
+        for (int k = i; k < levels; ++k)
             if (same_wgrad_kernel(np.lv[k], lv))
             {
-                const int s = np.lv[k].npad / np.lv[k].wgrad_tile;
+                const int s = np.lv[k].npad / lv.wgrad_tile;
+                all += np.lv[k].tiles * s;
+                if (!((wanted >> k) & 1u)) continue;
                 work += np.lv[k].tiles * s;
                 shares += s;
             }
-        const long long g = 1 + (resident - shares) * lv.tiles / work;
-        lv.groups         = (int)(g < lv.tiles ? g : lv.tiles);
+        size_t o = at;
+        for (int k = i; k < levels; ++k)
+        {
+            LevelPlan& l = np.lv[k];
+            if (!same_wgrad_kernel(l, lv) || !((wanted >> k) & 1u)) continue;
+            // one workgroup for every share, the others by the tiles (rounded down: one that has to wait for another to end
+            // would take as long again)
+            l.groups   = (int)std::min(1 + (resident - shares) * l.tiles / work, l.tiles);
+            l.part_off = o;
+            o += (size_t)l.groups * 9 * l.npad * l.cin_pad * sizeof(float);
+            l.bias_part_off = o;
+            o += (size_t)l.groups * l.npad * sizeof(float);
+        }
+        at += align256((size_t)std::min(resident, all) * lv.wgrad_tile * (9 * lv.cin_pad + 1) * sizeof(float));
     }
+    return at;
 }
 
 // Block i convolves cat(in[i], up2(x_{i+1})) (F[i+1] channels; C for the start block) to F[i] - 2C outputs
@@ -244,17 +269,13 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         lv.wgrad_tile = wgrad_tile(lv.cin_pad, lv.npad, tiles);
         lv.tiles      = tiles;
     }
-    plan_wgrad_groups(np, L);
     for (int i = 0; i < L; ++i)
     {
-        LevelPlan& lv = np.lv[i];
-        lv.part_off     = bw;
-        bw += align256((size_t)lv.groups * 9 * lv.npad * lv.cin_pad * sizeof(float));
-        lv.sliced_off = bw;
-        bw += align256((size_t)16 * 9 * lv.npad * lv.cin_pad * sizeof(float));
-        lv.bias_part_off = bw;
-        bw += align256((size_t)lv.groups * lv.npad * sizeof(float));
+        np.lv[i].sliced_off = bw;
+        bw += align256((size_t)16 * 9 * np.lv[i].npad * np.lv[i].cin_pad * sizeof(float));
     }
+    np.wgrad_off = bw;
+    bw           = plan_wgrad(np, L, ~0u, bw);
     {
         const size_t chunks = d.batch * (((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
         // as many workgroups as are resident at once walk the chunks (four per CU at the 100 to 118 registers of most
