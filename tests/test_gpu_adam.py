@@ -59,7 +59,7 @@ def test_fused_adam_matches_oracle(oracle):
 @pytest.mark.parametrize("steps_dtype", [np.int64, np.int32])
 @pytest.mark.parametrize("n", [1, 3, 31, 32, 33, 255, 1024, 4099])
 def test_fused_adam_runs_of_unseen_elements(oracle, n, steps_dtype):
-    """Eight lanes (32 elements) skip or write a line together: elements without gradient keep their bits wherever the runs
+    """Four lanes (16 elements) skip or write a piece of 64 bytes together: elements without gradient keep their bits wherever the runs
     begin and end, whatever they hold, also under a loss scale that is divided out; the others follow the oracle (tolerances
     as above)."""
     from tests.oracle_lib import fill_adam_tensor

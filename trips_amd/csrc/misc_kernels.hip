@@ -143,14 +143,19 @@ __device__ __forceinline__ void adam_block(const AdamTable& tab, int ti)
         const float4 g4 = nt_load(reinterpret_cast<const float4*>(g + i0));
         float ge[4]     = {g4.x, g4.y, g4.z, g4.w};
         adam_unscale(h.loss_scale, ge);
-        // (A parameter not seen in this step stays as it is, MyAdam.cu:57-61.) Eight lanes share the 128-byte lines of every
-        // float array: they skip a line together or write all of it, unseen elements as they were read. (Lane by lane, the
-        // lines of a cloud with culled points leave in pieces, and non-temporal accesses then cost time instead of saving it:
-        // 10M elements with 64-bit counters, 39 % of them without a gradient, 98 us with ordinary accesses, 111 with
-        // non-temporal ones, 80 = 5.5 TB/s with whole lines.)
+        // (A parameter not seen in this step stays as it is, MyAdam.cu:57-61.) Four lanes share a piece of 64 bytes, the unit
+        // that memory transfers, of every float array: they skip it together or write all of it, unseen elements as they were
+        // read, so that nothing smaller leaves. 10M elements with 64-bit counters (1M points), us:
+        //                                       other buffers between two steps      a loop over the same 240 MB
+        //   share of points with a gradient         5 %   61 %    all                 5 %   61 %    all
+        //   lane by lane, ordinary accesses          57    101     89                  39     75     76
+        //   lines of 128 bytes, non-temporal         53     80     80                  54     81     81
+        //   pieces of 64 bytes, non-temporal         46     79     80                  46     80     81
+        // In a step with anything else in it the state is not in the caches when its turn comes; what fits the last-level
+        // cache and is stepped over and over is better off with ordinary accesses.
         const bool some             = !(ge[0] == 0.f && ge[1] == 0.f && ge[2] == 0.f && ge[3] == 0.f);
         const unsigned long long by = __ballot(some);
-        if (((by >> (threadIdx.x & 56u)) & 0xFFull) == 0) return;
+        if (((by >> (threadIdx.x & 60u)) & 0xFull) == 0) return;
         const float4 w4 = nt_load(reinterpret_cast<const float4*>(w + i0));
         const float4 m4 = nt_load(reinterpret_cast<const float4*>(mo + i0));
         const float4 v4 = nt_load(reinterpret_cast<const float4*>(vo + i0));
