@@ -501,18 +501,29 @@ def test_keys_of_a_tile_around_the_staged_ones(oracle, n):
 @pytest.mark.parametrize("tx, ty, n", [(1, 1, 700), (33, 31, 3000), (32, 32, 3000), (41, 25, 3000), (64, 32, 12000), (41, 50, 12000)])
 def test_plan_of_as_many_tiles_as_threads(oracle, tx, ty, n):
     """One tile, 1023, 1024 and 1025 (a tile for every thread of the plan, and two for some), 2048 and 2050 with a split tile
-    behind the first thousand: three views, whose counters and slices must not mix."""
+    behind the first thousand: three views, whose counters and slices must not mix. The first two views split the same tile,
+    the third another one, and finds the tile that was split before with no more than its share of the other points."""
     w, h = 32 * tx - 5, 32 * ty - 3
     sc = scenes.tiny(n=n, w=w, h=h, f=0.5 * w, num_layers=1, list_depth=8, views=3, seed=tx + ty, radius=(0.004, 0.02))
-    if n > 8192:  # more than 8192 of the points inside 12 x 12 pixels in the lower right
+    split = n > 8192
+    if split:  # more than 8192 of the points inside 12 x 12 pixels of a tile in the lower right
         rng = np.random.default_rng(tx)
         z = rng.uniform(-0.2, 0.2, 9000)
         at = np.array([w - 20.0, h - 20.0]) + rng.uniform(0.1, 11.9, (9000, 2))
         sc.position[:9000, 0] = ((at[:, 0] - w / 2) * (z + 3.0) / (0.5 * w)).astype(np.float32)
         sc.position[:9000, 1] = ((at[:, 1] - h / 2) * (z + 3.0) / (0.5 * w)).astype(np.float32)
         sc.position[:9000, 2] = z.astype(np.float32)
+        for view in sc.views:
+            view["image_index"] = 0
+        sc.views[2]["crop_transform"] = (1.0, 1.0, -96.0, -64.0, 0.0)  # three tiles to the left, two up
     d = abi.desc_for_scene(sc)
-    _check_forward(oracle, sc, d)
+    _, ref, _ = _check_forward(oracle, sc, d)
+    if not split:
+        return
+    for b, (x, y) in enumerate([(tx - 1, ty - 1), (tx - 1, ty - 1), (tx - 4, ty - 3)]):
+        tile = np.floor(ref["ip"][b][ref["depth"][b] > 0] / 32).astype(int)
+        entries = np.bincount(tile[:, 1] * tx + tile[:, 0], minlength=tx * ty)
+        assert entries[y * tx + x] >= 9000 and np.sort(entries)[-2] < 100
 
 
 def test_footprints_on_tile_and_image_borders_with_equal_depths(oracle):
