@@ -222,6 +222,51 @@ def test_packed_point_adam_equals_per_tensor_adam(oracle, n, c):
     assert packed.packed_state.shape[0] == m + 5 and int(packed.packed_state[m:].abs().sum()) == 0
 
 
+@pytest.mark.parametrize("c", [4, 8, 16])
+@pytest.mark.parametrize("scales", [(1.0, 1.0, 128.0, 1.0), (2.0, 128.0, 1024.0, 3.0), (1.0, 1e30, 1.0, 1e30)])
+def test_packed_point_adam_loss_scales(c, scales):
+    """Loss scales of the packed step, one tensor's among three of 1, all four different, and one so large that its tensors'
+    gradients are zero after the division: weights, moments and counters bit for bit those of the per-tensor step on the same
+    descriptors."""
+    from tests.oracle_lib import fill_adam_tensor
+    from trips_amd.renderer import get_context
+    ctx = get_context(0)
+    n = 1003
+    rng = np.random.default_rng(c)
+    w0 = _point_params(n, c, rng)
+    fused, packed = [], []
+    for i, (x, scale) in enumerate(zip(w0, scales)):
+        for out in (fused, packed):
+            out.append(dict(w=torch.as_tensor(x.reshape(-1)).cuda(), g=torch.zeros(x.size, device="cuda"), n=x.size, lr=1e-3 * (i + 1),
+                            loss_scale=scale, m=torch.zeros(x.size, device="cuda"), v=torch.zeros(x.size, device="cuda"),
+                            steps=torch.zeros(x.size, dtype=torch.int32, device="cuda"), steps_dtype=abi.TRIPS_STEPS_I32))
+    nbytes, row = ctx.adam_points_state_size(n, c)
+    state = torch.zeros((n, row // 4), dtype=torch.int32, device="cuda")
+
+    def descs(tensors):
+        out = [abi.TripsAdamTensor() for _ in tensors]
+        for d, t in zip(out, tensors):
+            fill_adam_tensor(d, t, lambda a: a.data_ptr())
+        return out
+    for _ in range(3):
+        # (after 1e30 the gradients are below half of the smallest number above zero: zero, whether or not subnormals are kept)
+        for i, gi in enumerate(_point_grads(n, c, rng, 0.4)):
+            g = torch.as_tensor(gi.reshape(-1) * (1e-17 if scales[i] == 1e30 else scales[i])).cuda()
+            fused[i]["g"], packed[i]["g"] = g, g.clone()
+        ctx.adam_step(descs(fused))
+        ctx.adam_step_points(descs(packed), n, c, state)
+    torch.cuda.synchronize()
+    # a row: {first moment, second moment, counter} of the four position elements, the size, the descriptor, the confidence
+    rows = state.cpu().numpy()[:, :3 * (6 + c)].reshape(n, 6 + c, 3)
+    for i, (a, b, part) in enumerate(zip(fused, packed, (rows[:, :4], rows[:, 4:5], rows[:, 5:5 + c], rows[:, 5 + c:]))):
+        part = np.ascontiguousarray(part.transpose(1, 0, 2) if i >= 2 else part).reshape(-1, 3)
+        assert torch.equal(a["w"], b["w"]), i
+        for k, name in enumerate(("m", "v", "steps")):
+            assert a[name].cpu().numpy().view(np.int32).tobytes() == np.ascontiguousarray(part[:, k]).tobytes(), (i, name)
+        moved = not np.array_equal(a["w"].cpu().numpy(), w0[i].reshape(-1))
+        assert moved == (scales[i] != 1e30), i
+
+
 def test_packed_point_adam_state_dict_round_trip():
     """A checkpoint of MyAdamPoints carries the rows of the four point parameters: an optimiser restored from
     state_dict() continues bit for bit like the one that never stopped."""
