@@ -957,15 +957,13 @@ __device__ __forceinline__ void sort_pair(u64& a, u64& b)
     a = lo;
     b = hi;
 }
-template <typename T>
-__device__ __forceinline__ void lane_sort4(T (&k)[kLaneSortMax])
+__device__ __forceinline__ void lane_sort4(u64 (&k)[kLaneSortMax])
 {
     sort_pair(k[0], k[1]), sort_pair(k[2], k[3]);
     sort_pair(k[0], k[2]), sort_pair(k[1], k[3]);
     sort_pair(k[1], k[2]);
 }
-template <typename T>
-__device__ __forceinline__ void lane_sort8(T (&k)[kLaneSortMax])
+__device__ __forceinline__ void lane_sort8(u64 (&k)[kLaneSortMax])
 {
     sort_pair(k[0], k[1]), sort_pair(k[2], k[3]), sort_pair(k[4], k[5]), sort_pair(k[6], k[7]);
     sort_pair(k[0], k[2]), sort_pair(k[1], k[3]), sort_pair(k[4], k[6]), sort_pair(k[5], k[7]);
@@ -975,8 +973,7 @@ __device__ __forceinline__ void lane_sort8(T (&k)[kLaneSortMax])
     sort_pair(k[1], k[2]), sort_pair(k[3], k[4]), sort_pair(k[5], k[6]);
 }
 // ascending sort of the first nmax (wave-uniform) of the lane's keys
-template <typename T>
-__device__ __forceinline__ void lane_sort(T (&k)[kLaneSortMax], int nmax)
+__device__ __forceinline__ void lane_sort(u64 (&k)[kLaneSortMax], int nmax)
 {
     if (nmax > 4)
         lane_sort8(k);

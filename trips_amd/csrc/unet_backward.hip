@@ -84,14 +84,14 @@ __global__ __launch_bounds__(256) void fill_f32_kernel(float* __restrict__ p, fl
 
 struct FinalBwdParams
 {
-    int H, W, c_feat, cact, cout, npad;
+    int H, W, c_feat, cact, cout;
     float scale;
     const float* feat;        // [C][H][W]
-    const _Float16* pre;      // [H][W][npad]
+    const _Float16* pre;      // [H][W][NPAD]
     const float* weight;      // [cout][c_feat + cact]
     const float* d_out;       // [cout][H][W]
     float* d_feat;            // [C][H][W], written
-    _Float16* dpre;           // [H][W][npad], written
+    _Float16* dpre;           // [H][W][NPAD], written
     float* part;              // [gridDim.x][4 * (4 + CS) + 4] sums of this launch's workgroups (WGRAD)
     int chunks;               // of one image: ceil(pixels / kFinalPixelsPerBlock)
     int batch;                // images, one after the other in every array
@@ -1825,7 +1825,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
         const size_t plane  = (size_t)lv.H * lv.W;
         FinalBwdParams p;
         std::memset(&p, 0, sizeof(p));
-        p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cout = K, p.npad = lv.npad;
+        p.H = lv.H, p.W = lv.W, p.c_feat = C, p.cact = lv.cout, p.cout = K;
         p.scale    = grad_scale;
         p.feat     = inputs[0];
         p.pre      = pre_ptr(0);
