@@ -207,9 +207,12 @@ __device__ __forceinline__ void chunk_point_range(const ForwardParams& p, int ch
     begin = min(p.num_points, chunk * p.points_per_block);
     end   = min(p.num_points, begin + p.points_per_block);
 }
-// The chunk of a workgroup: consecutive chunks share an XCD (workgroups are dealt to the eight of them in turn). Their
-// records follow each other, and what they file under a tile lies in the order of the chunks, a few entries each, so that
-// most lines hold entries of two or three of them. (Projection and scatter of 5.8M points together 286 -> 280 us.)
+// The chunk of a workgroup: consecutive chunks share an XCD (workgroups are dealt to the eight of them in turn). Worth about 1 %
+// of the projection where it saves a training step's records: 6M points in no order 139.0 -> 137.7 us, 3M in a ball 83.1 ->
+// 81.8, 4M clustered 112.8 -> 111.6; without the saved state, and at 9M in Morton order, nothing (128.7 and 129.0, 189.3 and 190.4).
+// The scatter's time does not change (a few entries of a chunk under every tile: 108.6 and 109.4 us at 6M in no order, others
+// alike), but its lines leave in more parts: 198 MB written instead of 169 there (without the saved state 184 instead of 151), as
+// much as before in Morton order and of clusters.
 __device__ __forceinline__ int chunk_of_workgroup()
 {
     static_assert(kBinGroups % kNumXcd == 0, "equal shares");
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 //
 // The last workgroup adds up the chunks of the projection: the number of every chunk's first overflow row, and the view's
 // counters, written (not added to, so that nothing has to clear them first); on the first view of a call the status block of
-// the whole call as well. The scan over the tiles' totals is the scatter pass's (BinPlan).
+// the whole call as well. The scan over the tiles' totals is the scatter pass's (plan_tiles).
 constexpr int kScanCols = 16, kScanSegs = 16;
 __device__ __forceinline__ int wave_inclusive_scan(int x)
 {
@@ -617,9 +620,10 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     const int pair_base = p.chunk_valid[3 * p.bin_groups + chunk];
     unsigned dropped = 0;
     // Records of a thread that are requested together. Loads and stores of a wavefront return in the order of their issue: a
-    // load that follows scattered stores waits for them, so there are as few such turns as registers allow (one for clouds
-    // of up to 4M valid points). Two at a time / 8 / 16: 6M points in no order 106 / 104 / 93 us, four views of 4M clustered
-    // points 396 / 373 / 342.
+    // load that follows scattered stores waits for them, so there are as few such turns as registers allow: one where no chunk
+    // has more than U * kBinThreads = 16384 valid points, which clouds of up to 4.19M points never do. Two at a time / 8 / 16,
+    // us: 6M points in no order 103 / 89 / 81 and with the saved state 109 / 113 / 109, 4M clustered 91 / 84 / 79, 3M in a ball
+    // 61 / 58 / 55, 1M 22 / 21 / 21; 9M in Morton order 40 / 35 / 39.
     constexpr int U = 16;
     for (int cid0 = begin + (int)threadIdx.x; cid0 < begin + n; cid0 += U * kBinThreads)
     {
@@ -1250,6 +1254,11 @@ __global__ __launch_bounds__(256) void cell_sort_kernel(const ForwardParams p)
 // loop that waited for memory eleven times): 1920 x 1080, without / with the saved state, 6M points in Morton order 107 ->
 // 91 us, 9M 134 -> 120, 1M in a ball 99 -> 89; 6M in no order 191 -> 191. A position's saved list leaves as soon as four are
 // known: with all sixteen kept the kernel took 140 registers of a lane, and a fourth wavefront per SIMD is worth 4 %.
+// What it costs: the requests lie a merge step apart, and a fourth wavefront shares the L1, so neighbouring pixels' requests of
+// a line meet there less often than when eight positions were requested in a row: at 6M points in no order 10.1 M reads of the
+// L2 instead of 7.7 M and 769 MB of memory instead of 663. All four of a group requested behind their merge: 8.6 M, 743 MB
+// and 182 us; three wavefronts: 9.5 M, 733 MB, 197 us; both: 8.3 M, 717 MB, 193 us. (The former takes registers that cost the
+// instances for 3 and 6 channels without the saved state and for 8 with it a wavefront, 1 to 3 % of a whole pass.)
 template <int C, bool TRAIN>
 __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
 {
