@@ -152,7 +152,9 @@ __device__ __forceinline__ void adam_block(const AdamTable& tab, int ti)
         //   lines of 128 bytes, non-temporal         53     80     80                  54     81     81
         //   pieces of 64 bytes, non-temporal         46     79     80                  46     80     81
         // In a step with anything else in it the state is not in the caches when its turn comes; what fits the last-level
-        // cache and is stepped over and over is better off with ordinary accesses.
+        // cache and is stepped over and over is better off with ordinary accesses (64-bit counters, 61 %, pieces either way:
+        // 300k points 22 and 24 us, with other buffers in between 35 and 29). Whole splat steps of 20k to 300k points take the
+        // same time with both, of 1M 484 us instead of 501.
         const bool some             = !(ge[0] == 0.f && ge[1] == 0.f && ge[2] == 0.f && ge[3] == 0.f);
         const unsigned long long by = __ballot(some);
         if (((by >> (threadIdx.x & 60u)) & 0xFull) == 0) return;

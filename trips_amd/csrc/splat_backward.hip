@@ -755,7 +755,8 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
 
     const int stride = (int)gridDim.x * 256;
     // The compact number of a point is requested two steps ahead, and the layers it was written to (or the flags of its rows)
-    // one step ahead, so that a step starts with both in hand.
+    // one step ahead, so that a step starts with both in hand. (The rest of the point's record follows in work_off, in a request
+    // of its own: where every point is worked off as it comes, 634 MB read instead of 609 at 6M points in no order.)
     auto cid_at   = [&](long long pid) { return pid < p.num_points ? p.cid_of[pid] : -1; };
     auto layers_of = [&](int cid) -> unsigned
     {
