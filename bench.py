@@ -31,17 +31,17 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "3ad2b3d3ad5acae111af3338bcda4037c306940632267f7d429e6518841c30b8"
+PMC_SOURCES_SHA256 = "7e8a90c362fb9d6ae3fe9dae55a751015a4baacf058b9abd0ff78ed0260f5dcd"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129103, 236068),
-    "bin_scatter": (94971, 191274),
-    "tile_count": (13115, 2295),
-    "tile_scatter": (26033, 89345),
-    "cell_sort": (35349, 42136),
-    "blend": (367709, 196692),
-    "backward_prologue": (54, 265165),
-    "backward_tiles": (427122, 121568),
-    "backward_points": (309723, 234503),
+    "project_bin": (129103, 235458),
+    "bin_scatter": (94882, 191464),
+    "tile_count": (13116, 2296),
+    "tile_scatter": (26022, 89639),
+    "cell_sort": (35349, 42140),
+    "blend": (372892, 196630),
+    "backward_prologue": (54, 265150),
+    "backward_tiles": (426498, 121594),
+    "backward_points": (309661, 234503),
     "adam_fused": (383764, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
