@@ -71,6 +71,32 @@ def test_forward_radius_dropout_and_floor_layers(oracle):
     assert 0 < ref["counters"][0, 0] < 3000
 
 
+def test_sizes_and_depths_over_the_range_of_floats(oracle):
+    """Softplus, the quotients by the depth and the size field to the last bit: raw sizes of all magnitudes and signs, next to
+    the limits of the branches (20, -200, steps of the logarithm's table), and depths whose reciprocal is not normal. (Sizes in
+    pixels stay above the denormals.)"""
+    n = 6000
+    sc = scenes.tiny(n=n, w=70, h=50, f=60.0, num_layers=8, list_depth=16, seed=31)
+    rng = np.random.default_rng(31)
+    sc.poses_se3[:] = [0, 0, 0, 1, 0, 0, 0, 0]
+    z = 10.0 ** rng.uniform(-12, 12, n)
+    z[:2000] = rng.uniform(0.5, 20.0, 2000)
+    z[2000:2012] = [2e-20, 3e-25, 7e-39, 1e-38, 2.0 ** -60, 2.0 ** 60, 3e18, 3e19, 1e20, 1.0, 1.5, 3.0]
+    z[2012:2040] = -z[2012:2040]
+    x, y = rng.uniform(-0.55, 0.55, n), rng.uniform(-0.4, 0.4, n)
+    sc.position[:] = np.stack([x * z, y * z, z, 0.01 * np.abs(z)], axis=1).astype(np.float32)
+    raw = rng.uniform(-50.0, 25.0, n)
+    raw[::3] = rng.choice((-1.0, 1.0), raw[::3].shape) * 10.0 ** rng.uniform(-9, 1.3, raw[::3].shape)
+    raw[1::9] = np.log(np.expm1(np.clip(np.abs(z[1::9]) * 10.0 ** rng.uniform(-3, 0.5, z[1::9].shape), 1e-20, 15.0)))  # a few pixels
+    edge = np.float32([20.0, -200.0, 0.0, np.log(1.0 / 128), np.log(127.0 / 128), np.log(1.0), np.log(255.0 / 256)])
+    edges = np.concatenate([edge, np.nextafter(edge, np.float32(np.inf)), np.nextafter(edge, np.float32(-np.inf)),
+                            np.float32([-1e30, -np.inf, -0.0, 1e-40, 30.0, 1e6])])
+    raw[:edges.size] = edges
+    sc.point_size[:] = raw.astype(np.float32).reshape(sc.point_size.shape)
+    run, ref, _ = _check_forward(oracle, sc, abi.desc_for_scene(sc))
+    assert (ref["depth"][0] > 0).sum() > 0.9 * n and ref["max_layer"][0].max() >= 4
+
+
 def test_forward_distortion(oracle):
     # non-zero distortion: parity with Saiga's model is unpinned; this checks HIP == oracle for the restated model
     sc = scenes.tiny(n=3000, w=64, h=48, f=60.0, num_layers=3, list_depth=16, seed=10)

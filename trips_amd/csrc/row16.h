@@ -37,6 +37,16 @@ __device__ __forceinline__ u64 dpp_u64(u64 v)
     return ((u64)hi << 32) | lo;
 }
 
+// sum over the lanes of the row up to this one
+__device__ __forceinline__ int row_inclusive_scan(int v)
+{
+    v += dpp_i<kDppShr1>(v);  // lanes without a source read 0
+    v += dpp_i<kDppShr1 + 1>(v);
+    v += dpp_i<kDppShr1 + 3>(v);
+    v += dpp_i<kDppShr1 + 7>(v);
+    return v;
+}
+
 // value of lane (i ^ M) of the same row, M in {1, 2, 4, 8, 15}
 template <int M>
 __device__ __forceinline__ u64 row_xor_u64(u64 v)

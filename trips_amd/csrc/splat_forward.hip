@@ -105,11 +105,30 @@ __device__ __forceinline__ void load_point(const ForwardParams& p, int pid, int 
     }
 }
 
+// The last pixels, first tile and tile columns of all layers, layer l's in lane l of four registers (the whole wavefront makes
+// them, outside of any branch): a loop over the layers gets them with v_readlane, where loads of kernel arguments are four
+// round trips of the scalar cache per layer, one behind the other, which wait for the wavefront's LDS atomics as well.
+struct LayerTable
+{
+    int last_x, last_y, bin_off, tiles_x;
+};
+__device__ __forceinline__ LayerTable layer_table(const PyramidGeom& g)
+{
+    const int l = min((int)(threadIdx.x & 63), TRIPS_MAX_LAYERS - 1);
+    LayerTable t;
+    t.last_x  = g.w[l] - 1;
+    t.last_y  = g.h[l] - 1;
+    t.bin_off = g.bin_off[l];
+    t.tiles_x = g.tiles_x[l];
+    return t;
+}
+
 // `s_hist`: LDS counters, one per tile; every layer the point is written to adds one to the tile of the footprint's
 // first pixel (px, py). (The footprint (px..px+1, py..py+1) lies inside the image because px < w-1 and py < h-1.)
 template <bool TRAIN, int CPAD>
 __device__ __forceinline__ PointProjection project_point(const ForwardParams& p, const Camera& cam, int pid, const PointInputs<CPAD>& in,
-                                                         int* s_hist, bool& not_identity, bool& bad_index)
+                                                         int* s_hist, const double2* log_table, const LayerTable& layers,
+                                                         bool& not_identity, bool& bad_index)
 {
     PointProjection o;
     o.valid  = false;
@@ -130,12 +149,8 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
         not_identity = true;  // the backward then never uses the point's own number as a column
         skip         = true;
     }
-    if (p.viewer_only && !skip)
-    {
-        if (in.conf < p.stability_cutoff_value) skip = true;
-    }
+    if (p.viewer_only && in.conf < p.stability_cutoff_value) skip = true;
     if (TRAIN && in.dropout == 1.f) skip = true;
-    if (skip) return o;
     float4 pos = in.pos;
     if (p.displacement)
     {
@@ -144,43 +159,39 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
         pos.y += dsp[1];
         pos.z += dsp[2];
     }
-    float d_softplus    = 0.f;
-    const float size    = TRAIN ? softplus_and_derivative(in.raw_size, &d_softplus) : softplus(in.raw_size);
-    const Projected pr  = project(cam, pos.x, pos.y, pos.z);
-    const float z       = pr.z;
-    float radius_px     = pr.scale * pos.w / z;
-    const float size_px = pr.scale * size / z;
-
-    auto valid = [&](float x, float y, int layer, float radius) -> bool
-    {
-        if (z <= 0.f) return false;
-        if (!(x >= 0.f) || x >= float(p.geom.w[layer] - 1) || !(y >= 0.f) || y >= float(p.geom.h[layer] - 1)) return false;
-        if (p.drop_out_points_by_radius && float(trunc_sat(radius)) < p.drop_out_radius_threshold) return false;
-        return true;
-    };
-    if (!valid(pr.ipx, pr.ipy, 0, radius_px)) return o;
+    const Projected pr = project(cam, pos.x, pos.y, pos.z);
+    float radius_px    = quotient(pr.scale * pos.w, pr.iz);
+    auto small = [&](float radius) { return p.drop_out_points_by_radius && float(trunc_sat(radius)) < p.drop_out_radius_threshold; };
+    o.valid = !skip && pr.z > 0.f && pr.ipx >= 0.f && pr.ipx < float(p.geom.w[0] - 1) && pr.ipy >= 0.f &&
+              pr.ipy < float(p.geom.h[0] - 1) && !small(radius_px);
+    if (!o.valid) return o;
+    o.ipx = pr.ipx;
+    o.ipy = pr.ipy;
+    o.z   = pr.z;
+    const float size = softplus(in.raw_size, log_table, TRAIN ? &o.d_softplus : nullptr);
+    o.size_px        = quotient(pr.scale * size, pr.iz);
     int layer_higher = 0;
-    if (size_px > 1.f)
+    if (o.size_px > 1.f)
     {
         int lo, hi;
-        log2_floor_ceil(size_px, lo, hi);
+        log2_floor_ceil(o.size_px, lo, hi);
         layer_higher = min(hi, L - 1);
     }
-    int layer = 0;
-    float lx = pr.ipx, ly = pr.ipy;
-    for (; layer < layer_higher + 1; ++layer, lx *= 0.5f, ly *= 0.5f, radius_px *= 0.5f)
+    float lx = o.ipx, ly = o.ipy;
+    bool more = true;
+    for (int layer = 0; layer < L; ++layer, lx *= 0.5f, ly *= 0.5f, radius_px *= 0.5f)
     {
-        const int px = (int)floorf(lx), py = (int)floorf(ly);
-        if (!valid(float(px), float(py), layer, radius_px)) break;
-        atomicAdd(s_hist + p.geom.bin_off[layer] + (py >> kTileShift) * p.geom.tiles_x[layer] + (px >> kTileShift), 1);
+        const int px = (int)lx, py = (int)ly;
+        more = more && layer <= layer_higher && px < __builtin_amdgcn_readlane(layers.last_x, layer) &&
+               py < __builtin_amdgcn_readlane(layers.last_y, layer) && !small(radius_px);
+        if (__ballot(more) == 0) break;
+        if (more)
+        {
+            const int row = (int)__umul24((unsigned)(py >> kTileShift), (unsigned)__builtin_amdgcn_readlane(layers.tiles_x, layer));
+            atomicAdd(s_hist + __builtin_amdgcn_readlane(layers.bin_off, layer) + row + (px >> kTileShift), 1);
+            o.layers = layer + 1;
+        }
     }
-    o.valid   = true;
-    o.layers  = layer;
-    o.ipx     = pr.ipx;
-    o.ipy     = pr.ipy;
-    o.z       = z;
-    o.size_px = size_px;
-    o.d_softplus = d_softplus;
     return o;
 }
 
@@ -229,6 +240,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     constexpr int WAVES = kBinThreads / 64;
     extern __shared__ int s_hist[];  // bin entries of this workgroup's points, one counter per tile
     __shared__ int s_valid[2][WAVES];  // valid points of every wavefront in this step (two steps in flight)
+    __shared__ double2 s_log[kLogTable];
     __shared__ int s_flags;            // bit 0: not_identity, bit 1: bad_index, of any point of the chunk
     const Camera cam  = load_camera(p.pose, p.intrinsics, p.view, p.dist_cutoff);
     const int L       = p.num_layers;
@@ -236,6 +248,8 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     bool not_identity = false;  // some point's descriptor column differs from its own index
     bool bad_index    = false;
     for (int i = threadIdx.x; i < NB; i += kBinThreads) s_hist[i] = 0;
+    const LayerTable layers = layer_table(p.geom);
+    if (threadIdx.x < kLogTable) s_log[threadIdx.x] = log_table_entry(threadIdx.x);
     if (threadIdx.x == 0) s_flags = 0;
     __syncthreads();
 
@@ -248,8 +262,11 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     int step       = 0;
     // The loads of the next step's points, their descriptors and dropout flags among them (whether a point is visible or
     // not), are in flight while this step's are projected. (With the dropout flag and the descriptor requested in the
-    // step itself, its waits were a part of every step: 9M points with dropout 225 us, now 197; 6M without 152, now 150,
-    // which its vector instructions, 100 us, and the 520 MB that it moves, 84 us at a copy's rate, bound together.)
+    // step itself, its waits were a part of every step: 9M points with dropout 225 -> 197 us.) What bounds it: without the saved
+    // state the 447 MB that it moves at 6M points, 4.5 TB/s; with it the stores, 507 MB at 3.9 TB/s (that the next step waits for
+    // them is not it: without branches around loads and stores, so that nothing waits for a store, it takes 137 us instead of
+    // 131). Before the short exp and log and the layers' table it was its vector instructions, 91 us of them: eval 6M in Morton
+    // order 126 -> 99 us, train 6M 138 -> 131, 9M 191 -> 173, 4M clustered 111 -> 105 a view.
     PointInputs<CPAD> nxt;
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)
@@ -267,7 +284,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
         PointProjection o;
         o.valid  = false;
         o.layers = 0;
-        if (pid < end) o = project_point<TRAIN>(p, cam, pid, in, s_hist, not_identity, bad_index);
+        if (pid < end) o = project_point<TRAIN>(p, cam, pid, in, s_hist, s_log, layers, not_identity, bad_index);
         const unsigned long long vm = __ballot(o.valid);
         const unsigned long long below = (1ull << lane) - 1ull;
         // rows of the backward's overflow table (one per layer past the second) of the wavefront's points before this
@@ -285,20 +302,14 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
             }
         }
         // both counts of a wavefront in one word (at most 64 valid points and 384 rows per wavefront, 1024 and 6144 per
-        // step: 16 bits each); every wavefront then takes the prefix over the 16 words in its first 16 lanes
+        // step: 16 bits each); every wavefront then takes the prefix over the 16 words in its 16-lane rows
         if (lane == 0) s_valid[step][wave] = (int)__popcll(vm) | (pairs_wave << 16);
         __syncthreads();
         static_assert(WAVES == 16, "the prefix below runs over one 16-lane row");
-        const int word = lane < WAVES ? s_valid[step][lane] : 0;  // the counts of wavefront w in lane w
-        int inc        = word;
-#pragma unroll
-        for (int o = 1; o < WAVES; o <<= 1)
-        {
-            const int t = __shfl_up(inc, o);
-            if (lane >= o) inc += t;
-        }
-        const int upto = __shfl(inc, WAVES - 1);     // the step's totals
-        const int excl = __shfl(inc - word, wave);   // the wavefronts before this one
+        const int word = s_valid[step][lane & (WAVES - 1)];  // the counts of wavefront w in lane w of every row
+        const int inc  = row_inclusive_scan(word);
+        const int upto = __builtin_amdgcn_readlane(inc, WAVES - 1);                                    // the step's totals
+        const int excl = __builtin_amdgcn_readlane(inc - word, __builtin_amdgcn_readfirstlane(wave));  // the wavefronts before this one
         const int before = excl & 0xFFFF, pbefore = excl >> 16, total = upto & 0xFFFF, ptotal = upto >> 16;
         const int cid        = next + before + (int)__popcll(vm & below);
         const int first_pair = next_pair + pbefore + pairs_before;  // within the chunk; the scatter pass adds the chunk's first

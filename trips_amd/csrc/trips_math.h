@@ -18,34 +18,88 @@ namespace trips
 {
 constexpr float kAlphaDestCutoff = 0.001f;  // ALPHA_DEST_CUTOFF, RenderForward.cu:907
 
-// exp / log evaluated in double and rounded once, so that results do not depend on a libm's float path
-__device__ __forceinline__ float exp_rn(float x) { return (float)exp((double)x); }
-__device__ __forceinline__ float log_rn(float x) { return (float)log((double)x); }
+// exp / log evaluated in double and rounded once, so that results do not depend on a libm's float path. The projection is bound by
+// its vector instructions, and the two functions for any double were a third of them: a float's exponential and the logarithm
+// of 1 + exp(x) need no second word of the argument, no range tests and, with a table of reciprocals, no division. Their errors
+// stay below 2^-51 of the value, and over all floats the rounded results are those of exp() and log() in double.
 
-__device__ __forceinline__ float softplus(float x)
+// A constant kept in scalar registers: as an operand of a multiply-add it then costs nothing, where the compiler would copy
+// it into two vector registers first.
+__device__ __forceinline__ double scalar_const(double c)
 {
-    if (x > 20.f) return x;
-    return log_rn(1.f + exp_rn(x));
+    asm("" : "+s"(c));
+    return c;
 }
 
-__device__ __forceinline__ float softplus_backward(float y)
+// exp(x) for -200 <= x <= 200 (or NaN): 2^n 2^f with n = rint(x log2 e), |f| <= 1/2, and for 2^f a polynomial that interpolates
+// it in the Chebyshev nodes (relative error 2^-55).
+__device__ __forceinline__ float exp_rn(float x)
 {
-    if (y > 20.f) return 1.f;
-    float z = exp_rn(y);
-    return z / (z + 1.f);
+    const double xd = (double)x, log2e = scalar_const(0x1.71547652b82fep+0);
+    const double n = rint(xd * log2e);
+    const double f = fma(xd, scalar_const(0x1.777d0ffda0d24p-56), fma(xd, log2e, -n));
+    double q       = scalar_const(0x1.e9d3fe3952179p-32);
+    q              = fma(q, f, scalar_const(0x1.e6063f7217bc6p-28));
+    q              = fma(q, f, scalar_const(0x1.b524fae627834p-24));
+    q              = fma(q, f, scalar_const(0x1.62bfd47773353p-20));
+    q              = fma(q, f, scalar_const(0x1.ffcbfc670dcd4p-17));
+    q              = fma(q, f, scalar_const(0x1.430913096fd9fp-13));
+    q              = fma(q, f, scalar_const(0x1.5d87fe78a5276p-10));
+    q              = fma(q, f, scalar_const(0x1.3b2ab6fba1ddap-7));
+    q              = fma(q, f, scalar_const(0x1.c6b08d704a0c2p-5));
+    q              = fma(q, f, scalar_const(0x1.ebfbdff82c598p-3));
+    q              = fma(q, f, scalar_const(0x1.62e42fefa39efp-1));
+    return (float)__builtin_amdgcn_ldexp(fma(q, f, 1.0), (int)n);
 }
 
-// both at once, with the one exponential that they share (same bits as the two functions above)
-__device__ __forceinline__ float softplus_and_derivative(float x, float* derivative)
+// {c, -log c} for c = 1 / (1 + i / 128) rounded to float, which makes the product with another float exact in double
+constexpr int kLogTable = 128;
+__device__ __forceinline__ double2 log_table_entry(int i)
 {
-    if (x > 20.f)
-    {
-        *derivative = 1.f;
-        return x;
-    }
-    const float z = exp_rn(x);
-    *derivative   = z / (z + 1.f);
-    return log_rn(1.f + z);
+    const double c = (double)(float)(1.0 / (1.0 + (double)i / kLogTable));
+    return make_double2(c, -log(c));
+}
+
+// log(z) for finite z >= 1 (or NaN): with z = 2^k m, m in [1 - 2^-8, 2 - 2^-8), and the table's c next to 1 / m,
+// k log 2 - log c + log(1 + r), r = m c - 1 (exact), |r| <= 2^-7, and the series of log(1 + r) to the eighth power
+__device__ __forceinline__ float log_rn(float z, const double2* table)
+{
+    const uint32_t u = __float_as_uint(z) + 0x8000u;
+    const int minus_k = 127 - (int)(u >> 23);
+    const double2 t   = table[(u >> 16) & (kLogTable - 1)];
+    const double r    = fma(__builtin_amdgcn_ldexp((double)z, minus_k), t.x, -1.0);
+    double q          = scalar_const(-1.0 / 8);
+    q                 = fma(q, r, scalar_const(1.0 / 7));
+    q                 = fma(q, r, scalar_const(-1.0 / 6));
+    q                 = fma(q, r, scalar_const(1.0 / 5));
+    q                 = fma(q, r, scalar_const(-1.0 / 4));
+    q                 = fma(q, r, scalar_const(1.0 / 3));
+    q                 = fma(q, r, -0.5);
+    return (float)(fma((double)minus_k, scalar_const(-0x1.62e42fefa39efp-1), t.y) + fma(r * r, q, r));
+}
+
+// 1 / b in double for a float b > 0, within two units of the last place: the hardware's reciprocal (an error e of 2^-23) times
+// 1 + e + e^2. A float times it is within 2^-51 of the quotient, which is never that close to the middle between two
+// floats (25-bit numbers; quotients of floats keep 2^-49 of themselves away from these): rounded to float it is the IEEE quotient.
+// Quotients by the same number share it: three operations each instead of eleven.
+__device__ __forceinline__ double reciprocal_of(float b)
+{
+    const double bd = (double)b;
+    if (!(b > 0x1p-60f && b < 0x1p60f)) return 1.0 / bd;  // where the hardware's has no more to give (infinity among them)
+    const double r = (double)__builtin_amdgcn_rcpf(b);
+    const double e = fma(-bd, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+__device__ __forceinline__ float quotient(float a, double reciprocal) { return (float)((double)a * reciprocal); }
+
+// softplus and its derivative, with the one exponential that they share (derivative may be nullptr)
+__device__ __forceinline__ float softplus(float x, const double2* table, float* derivative)
+{
+    const float z   = exp_rn(x < -200.f ? -200.f : x > 20.f ? 20.f : x);
+    const float sum = 1.f + z;
+    if (derivative) *derivative = x > 20.f ? 1.f : z / sum;
+    const float y = log_rn(sum, table);
+    return x > 20.f ? x : y;
 }
 
 // floor(log2 s), ceil(log2 s) for finite s > 0 from the bit pattern (exact; the reference rounds log2f first)
@@ -95,7 +149,8 @@ __device__ __forceinline__ float layer_factor_interpolated(float s, int layer, i
 __device__ __forceinline__ float encode_size_field(float size_px, int max_layers)
 {
     const bool small_branch = !(size_px > 1.f) || max_layers == 1;
-    return small_branch ? -(0.75f * exp_rn(size_px - 1.f) + 0.25f) : size_px;
+    const float x = size_px - 1.f;
+    return small_branch ? -(0.75f * exp_rn(x < -200.f ? -200.f : x > 200.f ? 200.f : x) + 0.25f) : size_px;
 }
 
 // layer factor from the encoded size field
@@ -257,7 +312,7 @@ struct Camera
 struct Projected
 {
     float ipx, ipy, z, scale;  // scale = K.fx * crop.fx (divide by z after multiplying with a radius)
-    float vx, vy, vz;          // view-space point
+    double iz;                 // 1 / z where z > 0
 };
 
 __device__ __forceinline__ Projected project(const Camera& cam, float px, float py, float pz)
@@ -265,7 +320,8 @@ __device__ __forceinline__ Projected project(const Camera& cam, float px, float 
     float view[3];
     transform_point(cam.V, px, py, pz, view);
     float z  = fmaxf(view[2], 0.f);
-    float iz = 1.f / view[2];
+    const double izd = reciprocal_of(view[2]);  // (a point that is not in front of the camera is culled, wherever it falls)
+    const float iz   = (float)izd;
     float nx = view[0] * iz, ny = view[1] * iz;
     float dx, dy;
     if (cam.no_distortion)
@@ -292,9 +348,7 @@ __device__ __forceinline__ Projected project(const Camera& cam, float px, float 
     P.ipy   = ry + cam.centre_y;
     P.z     = z;
     P.scale = cam.fx * cam.cfx;
-    P.vx    = view[0];
-    P.vy    = view[1];
-    P.vz    = view[2];
+    P.iz    = izd;
     return P;
 }
 
