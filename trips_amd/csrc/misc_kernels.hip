@@ -581,16 +581,16 @@ __global__ __launch_bounds__(256) void export_points_kernel(const float* __restr
     const int cid   = cid_of[pid];
     const bool ok   = cid >= 0;
     const float* r  = rec + (size_t)(ok ? cid : 0) * rec_floats;
-    // {softplus'(raw size), depth, max_layer, size_px}
-    const float4 tl = ok ? reinterpret_cast<const float4*>(prec)[cid] : make_float4(0.f, -1.f, 0.f, 0.f);
+    // {depth, layers written | .. << 4, softplus'(raw size), size_px}
+    const float4 tl = ok ? reinterpret_cast<const float4*>(prec)[cid] : make_float4(-1.f, 0.f, 0.f, 0.f);
     if (ip)
     {
         ip[2 * (size_t)pid]     = ok ? r[0] : 0.f;
         ip[2 * (size_t)pid + 1] = ok ? r[1] : 0.f;
     }
-    if (depth) depth[pid] = tl.y;
+    if (depth) depth[pid] = tl.x;
     if (size_px) size_px[pid] = ok ? tl.w : 0.f;
-    if (max_layer) max_layer[pid] = ok ? __float_as_int(tl.z) : 0;
+    if (max_layer) max_layer[pid] = ok ? (int)(__float_as_uint(tl.y) & kLayersMask) : 0;
 }
 
 hipError_t launch_export_points(const float* rec, int rec_floats, const float* prec, const int32_t* cid_of, int n, float* ip,
@@ -605,9 +605,26 @@ hipError_t launch_export_points(const float* rec, int rec_floats, const float* p
 // saved tables are tile-major (padded); the exports are row-major, layer by layer
 __global__ __launch_bounds__(256) void export_lists_kernel(const PyramidGeom g, int K, const int32_t* __restrict__ lists,
                                                            const int32_t* __restrict__ retained,
-                                                           const int32_t* __restrict__ pid_of, int32_t* out_lists,
-                                                           int32_t* out_retained, int32_t* out_lengths)
+                                                           const int32_t* __restrict__ cid_of, int num_points,
+                                                           int points_per_block, int32_t* out_lists, int32_t* out_retained,
+                                                           int32_t* out_lengths)
 {
+    // the point of a compact number: cid_of, which counts on over culled points (~number of the next valid one), is searched
+    // within the number's chunk for the last point that does not exceed it from below
+    auto point_of = [&](int cid)
+    {
+        int lo = cid / points_per_block * points_per_block, hi = min(num_points, lo + points_per_block);  // the point is in [lo, hi)
+        while (lo < hi)
+        {
+            const int mid = lo + (hi - lo) / 2, c = cid_of[mid];
+            if (c == cid) return mid;
+            if ((c < 0 ? ~c : c + 1) <= cid)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return -1;
+    };
     const int P = g.off[g.num_layers];
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r >= P) return;
@@ -624,18 +641,18 @@ __global__ __launch_bounds__(256) void export_lists_kernel(const PyramidGeom g, 
         for (int k = 0; k < K; ++k)
         {
             const int cid                = k < filled ? lists[list_word((unsigned)ip, k, K)] : -1;  // compact number of the point
-            out_lists[(size_t)r * K + k] = cid >= 0 ? pid_of[cid] : -1;
+            out_lists[(size_t)r * K + k] = cid >= 0 ? point_of(cid) : -1;
         }
 }
 
 hipError_t launch_export_lists(const PyramidGeom& g, int K, const int32_t* lists, const int32_t* retained,
-                               const int32_t* pid_of, int32_t* out_lists, int32_t* out_retained,
-                               int32_t* out_lengths, hipStream_t stream)
+                               const int32_t* cid_of, int num_points, int points_per_block, int32_t* out_lists,
+                               int32_t* out_retained, int32_t* out_lengths, hipStream_t stream)
 {
     const int P = g.off[g.num_layers];
     if (P <= 0) return hipSuccess;
-    hipLaunchKernelGGL(export_lists_kernel, dim3((P + 255) / 256), dim3(256), 0, stream, g, K, lists, retained, pid_of,
-                       out_lists, out_retained, out_lengths);
+    hipLaunchKernelGGL(export_lists_kernel, dim3((P + 255) / 256), dim3(256), 0, stream, g, K, lists, retained, cid_of,
+                       num_points, points_per_block, out_lists, out_retained, out_lengths);
     return hipGetLastError();
 }
 

@@ -105,6 +105,15 @@ __host__ __device__ constexpr size_t tiles_lds_bytes(int cpad, int K)
     return (size_t)kBlockPixels * K * 8 + (size_t)kBlockPixels * cpad * 4 + (size_t)kBlockCells * kBlockCells * K * 4;
 }
 
+// The chunk of the binning kernels that a compact number (below 256 chunks) belongs to: the factor exceeds the quotient's by less
+// than 2^-49 of it, the product by less than 2^-40, and no quotient is closer than 2^-23 below a whole number.
+__device__ __forceinline__ int chunk_of_point(const BackwardParams& p, int cid) { return (int)((double)cid * p.chunk_per_point); }
+// The point's first row in the overflow table, `word` being the second of its point record.
+__device__ __forceinline__ int first_overflow_row(const BackwardParams& p, int cid, unsigned word)
+{
+    return (int)(word >> kLayersBits) + p.chunk_valid[kBinGroups + kRetainedParts + chunk_of_point(p, cid)];
+}
+
 template <int C, int kListMax>
 __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParams p)
 {
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
                 const int cyl = c2 / kBlockCells, cxl = c2 - cyl * kBlockCells;
                 const unsigned w4 = s_rank[slot];
                 // past the second layer: the number of the point's first row in the overflow table
-                if (!inline_row) row_of = p.over_first[row_of];
+                if (!inline_row) row_of = first_overflow_row(p, cid, __float_as_uint(p.prec[(size_t)(unsigned)cid * kPointRecordFloats + 1]));
                 // the four corners' entries, all requested before the first is looked at (of a corner that did not retain the
                 // point, an entry of its list that is not used)
                 float2 e[4];
@@ -607,12 +616,11 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
     {
         const bool has = mask != 0u;
         int first      = 0;
-        // {softplus'(raw size), depth, layers written, size_px}; {ip.x, ip.y, size field, confidence} of the blend record
+        // {depth, layers written and first overflow row, softplus'(raw size), size_px}; {ip.x, ip.y, size field, confidence}
+        // of the blend record
         float4 tail = make_float4(0.f, 0.f, 0.f, 0.f), r0 = tail, pos = tail;
         if (has)
         {
-            // (a point of one or two layers has no overflow rows, and its number there is not looked at)
-            if (mask >> kInlineLayers) first = p.over_first[cid];
             tail = reinterpret_cast<const float4*>(p.prec)[cid];
             r0   = *reinterpret_cast<const float4*>(p.rec + (size_t)(unsigned)cid * RF);
             pos  = p.position[pid];
@@ -624,9 +632,11 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
                 pos.z += dsp[2];
             }
         }
-        // (rows past the capacity of the overflow table do not exist: the forward reported the overflow)
+        // (rows past the capacity of the overflow table do not exist: the forward reported the overflow; a point of one or two
+        // layers has none, and its number there is not looked at)
         if (mask >> kInlineLayers)
         {
+            first               = first_overflow_row(p, cid, __float_as_uint(tail.y));
             const long long fit = p.over_capacity - first;
             if (fit < TRIPS_MAX_LAYERS - kInlineLayers) mask &= (1u << (kInlineLayers + (int)max(0ll, fit))) - 1u;
         }
@@ -650,7 +660,7 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
         {
             const float J_softmax_proj = u.cam.fx * u.cam.cfx / fmaxf(view[2], 0.f);
             float* sp = s_point[wave][lane];
-            sp[0] = r0.x, sp[1] = r0.y, sp[2] = r0.z, sp[3] = r0.w, sp[4] = tail.w, sp[5] = tail.x * J_softmax_proj;
+            sp[0] = r0.x, sp[1] = r0.y, sp[2] = r0.z, sp[3] = r0.w, sp[4] = tail.w, sp[5] = tail.z * J_softmax_proj;
             sp[6] = __int_as_float(first);
             sp[7] = __int_as_float(cid);
         }
@@ -761,7 +771,7 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
     auto layers_of = [&](int cid) -> unsigned
     {
         if (cid < 0) return 0u;
-        if (!sparse) return (1u << __float_as_int(p.prec[(size_t)(unsigned)cid * kPointRecordFloats + 2])) - 1u;
+        if (!sparse) return (1u << (__float_as_uint(p.prec[(size_t)(unsigned)cid * kPointRecordFloats + 1]) & kLayersMask)) - 1u;
         const uint2 eight = *reinterpret_cast<const uint2*>(p.flags + (size_t)(unsigned)cid * TRIPS_MAX_LAYERS);
         unsigned flagged  = 0;  // (a byte of 0 or 1 per layer)
 #pragma unroll

@@ -31,6 +31,7 @@ namespace trips
 {
 typedef unsigned vu4 __attribute__((ext_vector_type(4)));
 typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef float vf2 __attribute__((ext_vector_type(2)));
 typedef int vi4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ Camera load_camera(const double* pose, const float* intr, const TripsView& v,
@@ -263,10 +264,10 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     // The loads of the next step's points, their descriptors and dropout flags among them (whether a point is visible or
     // not), are in flight while this step's are projected. (With the dropout flag and the descriptor requested in the
     // step itself, its waits were a part of every step: 9M points with dropout 225 -> 197 us.) What bounds it: without the saved
-    // state the 447 MB that it moves at 6M points, 4.5 TB/s; with it the stores, 507 MB at 3.9 TB/s (that the next step waits for
-    // them is not it: without branches around loads and stores, so that nothing waits for a store, it takes 137 us instead of
+    // state the 447 MB that it moves at 6M points, 4.5 TB/s; with it the stores, 477 MB at 3.9 TB/s (that the next step waits for
+    // them is not it: without branches around loads and stores, so that nothing waits for a store, it took 137 us instead of
     // 131). Before the short exp and log and the layers' table it was its vector instructions, 91 us of them: eval 6M in Morton
-    // order 126 -> 99 us, train 6M 138 -> 131, 9M 191 -> 173, 4M clustered 111 -> 105 a view.
+    // order 126 -> 99 us, train 6M 138 -> 131, 9M 191 -> 173, 4M clustered 111 -> 105 a view (then two stores less: see prec).
     PointInputs<CPAD> nxt;
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)
@@ -312,11 +313,11 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
         const int excl = __builtin_amdgcn_readlane(inc - word, __builtin_amdgcn_readfirstlane(wave));  // the wavefronts before this one
         const int before = excl & 0xFFFF, pbefore = excl >> 16, total = upto & 0xFFFF, ptotal = upto >> 16;
         const int cid        = next + before + (int)__popcll(vm & below);
-        const int first_pair = next_pair + pbefore + pairs_before;  // within the chunk; the scatter pass adds the chunk's first
+        const int first_pair = next_pair + pbefore + pairs_before;  // within the chunk
         next += total;
         next_pair += ptotal;
         if (pid >= end) continue;
-        if (TRAIN) p.cid_of[pid] = o.valid ? cid : -1;
+        if (TRAIN) p.cid_of[pid] = o.valid ? cid : ~cid;
         if (!o.valid) continue;
 
         // record for the blend (and the pixel pass of the backward)
@@ -327,14 +328,9 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
         float4* rec = reinterpret_cast<float4*>(p.rec + (size_t)cid * p.rec_floats);
 #pragma unroll
         for (int q = 0; q < NREC; ++q) __builtin_nontemporal_store(vf4{recv[q].x, recv[q].y, recv[q].z, recv[q].w}, reinterpret_cast<vf4*>(rec) + q);
-        // point record: depth and layers for the scatter pass; softplus' and the size for the backward
-        __builtin_nontemporal_store(vf4{TRAIN ? o.d_softplus : 0.f, o.z, __int_as_float(o.layers), o.size_px},
+        // point record: depth and layers for the scatter pass; first overflow row, softplus' and the size for the backward
+        __builtin_nontemporal_store(vf4{o.z, __uint_as_float((unsigned)o.layers | (unsigned)first_pair << kLayersBits), TRAIN ? o.d_softplus : 0.f, o.size_px},
                                     reinterpret_cast<vf4*>(p.prec) + cid);
-        if (TRAIN)
-        {
-            __builtin_nontemporal_store(pid, p.pid_of + cid);
-            __builtin_nontemporal_store(first_pair, p.over_first + cid);
-        }
     }
     {
         const int flags = (__ballot(not_identity) != 0 ? 1 : 0) | (__ballot(bad_index) != 0 ? 2 : 0);
@@ -408,10 +404,11 @@ __device__ __forceinline__ void sum_chunks(const ForwardParams& p, bool first_vi
     if (lane == 63) s_over[wave] = inc_over, s_valid[wave] = inc_valid, s_flag[wave] = wave_flags;
     __syncthreads();
     int total_over, total_valid;
-    p.chunk_valid[3 * G + t] = waves_before<4>(s_over, total_over) + inc_over - over;
+    const int first_over = waves_before<4>(s_over, total_over) + inc_over - over;
     waves_before<4>(s_valid, total_valid);
     if (p.saved_chunk_valid)
     {
+        p.saved_chunk_valid[G + kRetainedParts + t] = first_over;
         p.saved_chunk_valid[t]     = valid;
         p.saved_chunk_valid[G + t] = 0;  // (the blend adds)
     }
@@ -628,7 +625,6 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     int begin, end;
     chunk_point_range(p, chunk, begin, end);
     const int n      = p.chunk_valid[chunk];
-    const int pair_base = p.chunk_valid[3 * p.bin_groups + chunk];
     unsigned dropped = 0;
     // Records of a thread that are requested together. Loads and stores of a wavefront return in the order of their issue: a
     // load that follows scattered stores waits for them, so there are as few such turns as registers allow: one where no chunk
@@ -638,18 +634,16 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     constexpr int U = 16;
     for (int cid0 = begin + (int)threadIdx.x; cid0 < begin + n; cid0 += U * kBinThreads)
     {
-        float2 tail[U], ip[U];  // {depth, layers}
-        int over[U];
+        vf2 tail[U];  // {depth, layers}
+        float2 ip[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
             const int cid = cid0 + u * kBinThreads;
             if (cid < begin + n)
             {
-                tail[u] = make_float2(__builtin_nontemporal_load(p.prec + (size_t)cid * kPointRecordFloats + 1),
-                                      __builtin_nontemporal_load(p.prec + (size_t)cid * kPointRecordFloats + 2));
+                tail[u] = __builtin_nontemporal_load(reinterpret_cast<const vf2*>(p.prec + (size_t)cid * kPointRecordFloats));
                 ip[u]   = *reinterpret_cast<const float2*>(p.rec + (size_t)cid * p.rec_floats);
-                if (p.over_first) over[u] = p.over_first[cid];
             }
         }
 #pragma unroll
@@ -657,12 +651,10 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
         {
             const int cid = cid0 + u * kBinThreads;
             if (cid >= begin + n) break;
-            // the point's first overflow row: the projection numbered it within the chunk, the scan found the chunk's first
-            if (p.over_first) p.over_first[cid] = over[u] + pair_base;
             PointProjection o;
             o.ipx    = ip[u].x;
             o.ipy    = ip[u].y;
-            o.layers = __float_as_int(tail[u].y);
+            o.layers = (int)(__float_as_uint(tail[u].y) & kLayersMask);
             const unsigned zbits = __float_as_uint(tail[u].x);
             for_point_tiles(p.geom, o, s_cur,
                             [&](int px, int py, int* bc)

@@ -91,7 +91,7 @@ struct TripsCtx
 namespace trips
 {
 // Per-point records written by the projection kernel, for the VALID points of a view only, at the point's compact
-// number cid (see chunk_point_range: dense runs in point order; cid_of / pid_of translate). The 64-bit sort key of a
+// number cid (see chunk_point_range: dense runs in point order; cid_of translates). The 64-bit sort key of a
 // list entry is depth bits << 32 | cid: cid grows with the point id, so the order is that of depth bits << 32 |
 // point id.
 //   rec[cid]   4 + Cpad floats {ip.x, ip.y, size field (see encode_size_field), confidence, descriptor[0..C)}:
@@ -99,11 +99,21 @@ namespace trips
 //              C = 4 (the reference reads a 5-float record, the confidence and C descriptor planes,
 //              src/lib/rendering/RenderForward.cu:875-899,952). Kept apart from the rest because a scattered gather
 //              costs the bytes of the whole aligned block it touches.
-//   prec[cid]  4 floats {softplus'(raw size), depth, layers written, size_px}: read by the kernel that makes the bin
-//              entries and, in point order, by the point pass of the backward, which transforms the point into view
-//              space again rather than have the projection kernel write those 12 bytes per point as well.
+//   prec[cid]  4 words {depth, layers written | first overflow row << 4, softplus'(raw size), size_px}: the first two are
+//              read by the kernel that makes the bin entries, all in point order by the point pass of the backward, which
+//              transforms the point into view space again rather than have the projection kernel write those 12 bytes
+//              per point as well. The first overflow row (of the backward's table, for a point written to more than two
+//              layers) is counted from its chunk's, which the saved state holds (a chunk has at most 2^23 points of 6
+//              such rows: 26 bits). In an array of their own, to which the entries' kernel added the chunk's, the numbers
+//              cost that kernel a load and a store per point, and the projection, which is bound by its stores in a
+//              training step, one more (as did an array with the point of every compact number, which only the exports
+//              need: they search cid_of instead). us a view: projection 131 -> 123 and entries 109 -> 102 at 6M points in no
+//              order, 105 -> 98 and 79 -> 74 at 4M clustered, 173 -> 169 and 39 -> 37 at 9M in Morton order. The tile pass,
+//              whose rows past the second layer look the number up, gathers it from a larger array: 6M 330 -> 339; the others
+//              as before.
 __host__ __device__ inline int record_floats(int channels) { return 4 + ((channels + 3) & ~3); }
 constexpr int kPointRecordFloats = 4;
+constexpr unsigned kLayersBits = 4, kLayersMask = (1u << kLayersBits) - 1u;
 
 // Pixels are binned into 32 x 32 tiles per layer. Internally a pixel is numbered tile-major:
 // (bin << 10) | (y & 31) << 5 | (x & 31), bin = bin_off[layer] + tile_y * tiles_x[layer] + tile_x, so that a
@@ -259,13 +269,12 @@ struct SavedLayout
     size_t retained;  // int32 [Pi]: retained entries in bits 0..4, list positions that hold an id (min(length, K)) in bits 5..9, list length from bit 10
     size_t tags;      // uint8 [Pi, 16]  where a list position came from: which of the pixel's four cells (bits 4..5) and its
                       // place in that cell's sorted list (bits 0..3); a row's positions past its ids are undefined
-    size_t cid_of;    // int32 [N] compact number of every point (-1 = culled)
-    size_t pid_of;    // int32 [N] point of every compact number (the first n_valid are defined)
-    size_t over_first;  // int32 [N] by compact number: for a point written to more than two layers, the number of its
-                        // first row in the backward's overflow table (rows numbered densely in point order)
+    size_t cid_of;    // int32 [N] compact number of every point (culled: ~number of the chunk's next valid point, so that the point
+                      // of a compact number can be searched for)
     size_t chunk_valid;  // int32 [kBinGroups] valid points of every chunk of the binning kernels (their compact numbers
                          // start at the chunk's first point number), then [kRetainedParts] partial sums of the view's
-                         // retained entries
+                         // retained entries, then [kBinGroups] the first overflow row of every chunk (rows are numbered
+                         // densely in point order)
     size_t bytes_per_view;
 };
 
@@ -289,8 +298,7 @@ struct BackwardWorkspaceLayout
 
 struct WorkspaceLayout
 {
-    size_t chunk_valid;   // int32 [4 G]  per chunk of the binning kernels: valid points, flags, overflow rows of the
-                          //              backward, and (from the scan) the number of the chunk's first overflow row
+    size_t chunk_valid;   // int32 [3 G]  per chunk of the binning kernels: valid points, flags, overflow rows of the backward
     size_t prec;         // float4 [N]         point records, when there is no saved state to hold them
     size_t counts;       // int32 [Pi]   list length per cell (the points whose 2 x 2 footprint starts at that pixel): added up
                          //              by the slices of tiles with more than kSliceEntries bin entries, whose counters are
@@ -337,8 +345,7 @@ struct ForwardParams
     float drop_out_radius_threshold, dist_cutoff, stability_cutoff_value;
     // buffers
     int32_t* chunk_valid;
-    int32_t* cid_of;  // training only: compact number of every point, -1 = culled
-    int32_t* pid_of;  // training only: point of every compact number
+    int32_t* cid_of;  // training only: compact number of every point, negative = culled
     int32_t* counts;
     int32_t* cursor;
     int32_t* bin_count;
@@ -360,8 +367,7 @@ struct ForwardParams
     int32_t* lists;
     int32_t* retained;
     unsigned char* tags;  // training only
-    int32_t* over_first;  // training only
-    int32_t* saved_chunk_valid;  // training only: [kBinGroups + kRetainedParts]
+    int32_t* saved_chunk_valid;  // training only: [2 kBinGroups + kRetainedParts]
     ViewHeader* header;  // counters of this view
     ViewHeader* status;  // overflow flag of the whole forward call (start of the workspace)
     float* image[TRIPS_MAX_LAYERS];
@@ -390,8 +396,8 @@ struct BackwardParams
     const ViewHeader* header;
     const float* grad_image[TRIPS_MAX_LAYERS];
     const unsigned char* tags;  // [Pi, 16] (saved state) cell and place in the cell's list of every list position
-    const int32_t* over_first;   // [N] (saved state) by compact number
-    const int32_t* chunk_valid;  // [kBinGroups + kRetainedParts] (saved state)
+    const int32_t* chunk_valid;  // [2 kBinGroups + kRetainedParts] (saved state)
+    double chunk_per_point;      // 1 / points_per_block, rounded up (see chunk_of_point)
     int32_t* mode;               // (workspace) 1 = only flagged rows exist
     int32_t force_mode;          // 0 = chosen per view from the retained entries, 1 = rows of all pairs, 2 = flagged rows
     int32_t bin_groups, points_per_block;

@@ -24,7 +24,7 @@ hipError_t launch_export_points(const float* rec, int rec_floats, const float* p
                                 float* depth, float* size_px, int32_t* max_layer, hipStream_t stream);
 hipError_t launch_sum_i32(const int32_t* v, long long n, unsigned mask, unsigned long long* out, hipStream_t stream);
 hipError_t launch_export_lists(const PyramidGeom& g, int K, const int32_t* lists, const int32_t* retained,
-                               const int32_t* pid_of, int32_t* out_lists, int32_t* out_retained,
+                               const int32_t* cid_of, int num_points, int points_per_block, int32_t* out_lists, int32_t* out_retained,
                                int32_t* out_lengths, hipStream_t stream);
 }  // namespace trips
 
@@ -196,6 +196,8 @@ long long pyramid_pixels_checked(const TripsSplatDesc& d)
     return P;
 }
 
+int points_per_chunk(const TripsSplatDesc& d) { return (d.num_points + kBinGroups - 1) / kBinGroups; }
+
 SavedLayout saved_layout(const TripsSplatDesc& d, const PyramidGeom& g)
 {
     SavedLayout s;
@@ -216,12 +218,8 @@ SavedLayout saved_layout(const TripsSplatDesc& d, const PyramidGeom& g)
     o += align256(P * 16);
     s.cid_of = o;
     o += align256(N * sizeof(int32_t));
-    s.pid_of = o;
-    o += align256(N * sizeof(int32_t));
-    s.over_first = o;
-    o += align256(N * sizeof(int32_t));
     s.chunk_valid = o;
-    o += align256((size_t)(kBinGroups + kRetainedParts) * sizeof(int32_t));
+    o += align256((size_t)(2 * kBinGroups + kRetainedParts) * sizeof(int32_t));
     s.bytes_per_view = o;
     return s;
 }
@@ -239,7 +237,7 @@ WorkspaceLayout workspace_layout(const TripsSplatDesc& d, const PyramidGeom& g)
     o += align256(sizeof(ViewHeader));
     o += align256(N * (size_t)record_floats(d.num_channels) * sizeof(float));
     w.chunk_valid = o;
-    o += align256((size_t)kBinGroups * 4 * sizeof(int32_t));
+    o += align256((size_t)kBinGroups * 3 * sizeof(int32_t));
     w.prec = o;
     o += align256(N * kPointRecordFloats * sizeof(float));
     w.counts = o;
@@ -440,7 +438,7 @@ int forward_impl(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsSplatIn* 
         p.bin_start  = reinterpret_cast<int32_t*>(ws + wl.bin_start);
         p.bin_hist   = reinterpret_cast<int32_t*>(ws + wl.bin_hist);
         p.bin_groups = kBinGroups;
-        p.points_per_block = (d.num_points + kBinGroups - 1) / kBinGroups;
+        p.points_per_block = points_per_chunk(d);
         p.run         = reinterpret_cast<int32_t*>(ws + wl.run);
         p.slice_start = reinterpret_cast<int32_t*>(ws + wl.slice_start);
         p.long_count  = reinterpret_cast<int32_t*>(ws + wl.long_count);
@@ -460,10 +458,8 @@ int forward_impl(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsSplatIn* 
             p.lists      = reinterpret_cast<int32_t*>(sv + sl.lists);
             p.retained   = reinterpret_cast<int32_t*>(sv + sl.retained);
             p.tags       = reinterpret_cast<unsigned char*>(sv + sl.tags);
-            p.over_first = reinterpret_cast<int32_t*>(sv + sl.over_first);
             p.saved_chunk_valid = reinterpret_cast<int32_t*>(sv + sl.chunk_valid);
             p.cid_of     = reinterpret_cast<int32_t*>(sv + sl.cid_of);
-            p.pid_of     = reinterpret_cast<int32_t*>(sv + sl.pid_of);
         }
         else
         {
@@ -569,10 +565,10 @@ int trips_splat_backward(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsS
         p.cid_of       = reinterpret_cast<const int32_t*>(sv + sl.cid_of);
         p.header       = reinterpret_cast<const ViewHeader*>(sv + sl.header);
         p.tags         = reinterpret_cast<const unsigned char*>(sv + sl.tags);
-        p.over_first   = reinterpret_cast<const int32_t*>(sv + sl.over_first);
         p.chunk_valid  = reinterpret_cast<const int32_t*>(sv + sl.chunk_valid);
         p.bin_groups   = kBinGroups;
-        p.points_per_block = (d.num_points + kBinGroups - 1) / kBinGroups;
+        p.points_per_block = points_per_chunk(d);
+        p.chunk_per_point  = (1.0 + 0x1p-50) / std::max(p.points_per_block, 1);
         p.rows_inline  = reinterpret_cast<float*>(ws + bl.rows_inline);
         p.rows_over    = reinterpret_cast<float*>(ws + bl.rows_over);
         p.flags        = reinterpret_cast<unsigned char*>(ws + bl.flags);
@@ -685,8 +681,8 @@ int trips_splat_export_lists(TripsCtx* ctx, const TripsSplatDesc* desc, const vo
     const char* sv       = reinterpret_cast<const char*>(saved) + sl.bytes_per_view * (size_t)view;
     hipError_t e = launch_export_lists(g, desc->list_depth, reinterpret_cast<const int32_t*>(sv + sl.lists),
                                        reinterpret_cast<const int32_t*>(sv + sl.retained),
-                                       reinterpret_cast<const int32_t*>(sv + sl.pid_of), device_lists, device_retained,
-                                       device_lengths, stream);
+                                       reinterpret_cast<const int32_t*>(sv + sl.cid_of), desc->num_points,
+                                       points_per_chunk(*desc), device_lists, device_retained, device_lengths, stream);
     if (e != hipSuccess) return hip_fail(e, "export copy");
     return TRIPS_OK;
 }
