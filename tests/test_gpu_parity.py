@@ -430,6 +430,31 @@ def test_backward_clearing_the_block_sums_equals_adding_into_zeros(views, overwr
     assert not cleared["d_pose"][-1].any() and not cleared["d_intrinsics"][-1].any()
 
 
+@pytest.mark.parametrize("w,h,n,channels,views", [(960, 960, 255, 4, 1), (975, 960, 257, 16, 1), (975, 960, 1, 6, 1),
+                                                  (31, 17, 262144 + 300, 4, 3), (15, 15, 1, 3, 16)])
+def test_block_sums_around_the_rows_of_a_workgroup(oracle, w, h, n, channels, views):
+    """64 x 64 blocks of the tile pass and one column of them more, 256 points and one more, more points than the point pass's
+    1024 workgroups take at once; several views that share a camera. The sums add to what the outputs hold, and repeat to the last
+    bit where one workgroup adds them up (double sums of floats: 1e-6 is a few units in the last place of the float output)."""
+    from tests.gpu_util import GpuRun, assert_grads_close, rel_err
+    sc = scenes.tiny(n=n, w=w, h=h, f=0.9 * w, num_layers=1, list_depth=8, seed=w + n, views=views, channels=channels,
+                     radius=(0.27 / w, 2.0 / w))
+    desc = abi.desc_for_scene(sc)
+    run = GpuRun(sc, desc)
+    run.forward()
+    rng = np.random.default_rng(w)
+    grads = [rng.normal(0.3, 1, (views, channels, h, w)).astype(np.float32)]
+    got, again = run.backward(grads), run.backward(grads, clear=True)
+    ref = oracle.forward(sc, desc)
+    want = oracle.backward(sc, desc, ref, grads)
+    assert_grads_close(got, want)
+    for k in ("d_pose", "d_intrinsics", "d_background"):
+        if views == 1 and w * h <= 960 * 960:
+            assert np.array_equal(got[k], again[k]), k
+        else:
+            assert rel_err(again[k], got[k]) < 1e-6, k
+
+
 def test_displacement_forward_backward(oracle):
     """Per-view displacements of the point positions (dynamic_refinement_t, PointRenderer.cu:703-713)."""
     sc = scenes.tiny(n=4000, w=70, h=50, f=60.0, num_layers=4, list_depth=16, seed=77, views=3, radius=(0.004, 0.4))

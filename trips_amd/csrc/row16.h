@@ -47,6 +47,39 @@ __device__ __forceinline__ int row_inclusive_scan(int v)
     return v;
 }
 
+// The lanes 32..63 of a change places with the lanes 0..31 of b (32), or the odd rows of a with the even rows of b (16).
+template <int LANES>
+__device__ __forceinline__ void swap_lanes(double& a, double& b)
+{
+    static_assert(LANES == 16 || LANES == 32, "a row or two");
+    const u64 x = (u64)__double_as_longlong(a), y = (u64)__double_as_longlong(b);
+    auto swapped = [](unsigned u, unsigned v)
+    {
+        if constexpr (LANES == 32) return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+        if constexpr (LANES == 16) return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+    };
+    const auto lo = swapped((unsigned)x, (unsigned)y), hi = swapped((unsigned)(x >> 32), (unsigned)(y >> 32));
+    a = __longlong_as_double((long long)(((u64)hi[0] << 32) | lo[0]));
+    b = __longlong_as_double((long long)(((u64)hi[1] << 32) | lo[1]));
+}
+
+// Sums of four values over the wavefront: every lane of row r holds that of v_r. Three steps of one value each less than a
+// butterfly of the four, and no lane crosses through LDS.
+__device__ __forceinline__ double wave_sum4(double v0, double v1, double v2, double v3)
+{
+    swap_lanes<32>(v0, v2);
+    swap_lanes<32>(v1, v3);
+    double a = v0 + v2, b = v1 + v3;  // lower half: v0 and v1, upper half: v2 and v3
+    swap_lanes<16>(a, b);
+    double v = a + b;
+    auto add = [&](u64 other) { v += __longlong_as_double((long long)other); };
+    add(dpp_u64<kDppXor1>((u64)__double_as_longlong(v)));
+    add(dpp_u64<kDppXor2>((u64)__double_as_longlong(v)));
+    add(dpp_u64<kDppHalfMirror>((u64)__double_as_longlong(v)));
+    add(dpp_u64<kDppMirror>((u64)__double_as_longlong(v)));
+    return v;
+}
+
 // value of lane (i ^ M) of the same row, M in {1, 2, 4, 8, 15}
 template <int M>
 __device__ __forceinline__ u64 row_xor_u64(u64 v)

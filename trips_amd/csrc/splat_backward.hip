@@ -23,15 +23,17 @@
 //      RenderBackward.cu:366-438); the point's own lane sums the image-space gradient of all its entries and runs the
 //      projection chain ONCE (the chain is linear in the image-space gradient, RenderBackward.cu:385-417), then stores
 //      or adds its gradients. Pose / intrinsics partials stay in registers over a grid-stride loop before one
-//      block-level reduction and one atomic per value and block (the reference keeps them in shared double arrays,
+//      block-level reduction; a workgroup leaves a row of sums (the reference keeps them in shared double arrays,
 //      :160-187,546-617).
+//   3. sums: adds up those rows, and the ones that the first pass's workgroups leave for the background.
 // A prologue kernel clears the rows (or, for a view in which few pairs are retained, one flag byte per row) beforehand.
-// The per-point gradients are summed in a fixed order and are bit-reproducible from run to run; the few block sums
-// (background, pose, intrinsics) are added with one atomic per workgroup, in an order that varies.
+// The per-point gradients are summed in a fixed order and are bit-reproducible from run to run; so are the block sums
+// (background, pose, intrinsics) but for the order in which several views, or images of more than kSumRows blocks, add to one.
 #include "row16.h"
 #include "splat_internal.h"
 #include "trips_math.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -72,12 +74,6 @@ __device__ __forceinline__ Camera load_camera_bw(const double* pose, const float
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef int vi4 __attribute__((ext_vector_type(4)));
 typedef unsigned vu4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
 
 // largest value of v (0 .. LIMIT) over the wavefront's lanes, as a scalar
 template <int LIMIT>
@@ -128,7 +124,7 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
     float2* const s_ex     = reinterpret_cast<float2*>(s_mem);
     vf4* const s_g         = reinterpret_cast<vf4*>(s_mem + (size_t)kBlockPixels * kListMax * 8);
     unsigned* const s_rank = reinterpret_cast<unsigned*>(s_mem + (size_t)kBlockPixels * kListMax * 8 + (size_t)kBlockPixels * CPAD * 4);
-    __shared__ double s_acc[4][C];
+    __shared__ double s_acc[4][CPAD];
     // (point, layer) pairs that wait for a lane of their wavefront: slot = place * 225 + cell, and the point's compact
     // number. The queue is emptied down to fewer than kQueueSlack pairs before a list position adds up to 64.
     constexpr int kQueueSlack = 32, kQueue = kQueueSlack + 64;
@@ -478,18 +474,19 @@ __global__ __launch_bounds__(256) void backward_tiles_kernel(const BackwardParam
         while (waiting > 0) pop64();
     }
 
+    // the block's row of the background's sums (backward_sums_kernel adds them up)
 #pragma unroll
-    for (int i = 0; i < C; ++i)
+    for (int q = 0; q < NQ; ++q)
     {
-        double v = wave_sum((double)acc_bg[i]);
-        if (lane == 0) s_acc[threadIdx.x >> 6][i] = v;
+        auto of = [&](int i) { return 4 * q + i < C ? (double)acc_bg[min(4 * q + i, C - 1)] : 0.0; };
+        const double v = wave_sum4(of(0), of(1), of(2), of(3));
+        if ((lane & 15) == 0) s_acc[wave][4 * q + (lane >> 4)] = v;
     }
     __syncthreads();
-    if (threadIdx.x < C)
+    if (threadIdx.x < CPAD)
     {
         const int i = threadIdx.x;
-        double v    = s_acc[0][i] + s_acc[1][i] + s_acc[2][i] + s_acc[3][i];
-        if (v != 0.0) unsafeAtomicAdd(p.d_background + i, (float)v);
+        p.background_sums[(size_t)lblock * CPAD + i] = (float)(s_acc[0][i] + s_acc[1][i] + s_acc[2][i] + s_acc[3][i]);
     }
 }
 
@@ -828,32 +825,86 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
         work_off(pid < p.num_points ? pid : -1, cid, mask);
     }
 
+    // the workgroup's row of the pose's and the intrinsics' sums (backward_sums_kernel adds them up)
     if (!want_pose && !want_intr) return;
-    __shared__ double s_acc[4][NACC];
+    __shared__ double s_acc[4][kCameraSums];
 #pragma unroll
-    for (int i = 0; i < NACC; ++i)
+    for (int q = 0; q < kCameraSums / 4; ++q)
     {
-        const bool used = (i < 6) ? want_pose : want_intr;
-        if (!used) continue;
-        double v = wave_sum((double)acc[i]);
-        if (lane == 0) s_acc[threadIdx.x >> 6][i] = v;
+        auto of = [&](int i) { return 4 * q + i < NACC ? (double)acc[min(4 * q + i, NACC - 1)] : 0.0; };
+        const double v = wave_sum4(of(0), of(1), of(2), of(3));
+        if ((lane & 15) == 0) s_acc[wave][4 * q + (lane >> 4)] = v;
     }
     __syncthreads();
-    if (threadIdx.x < NACC)
+    if (threadIdx.x < kCameraSums)
     {
-        const int i     = threadIdx.x;
-        const bool used = (i < 6) ? want_pose : want_intr;
-        if (used)
+        const int i = threadIdx.x;
+        p.camera_sums[(size_t)blockIdx.x * kCameraSums + i] = s_acc[0][i] + s_acc[1][i] + s_acc[2][i] + s_acc[3][i];
+    }
+}
+
+// After the passes of all views of a call: the rows that the workgroups of the two passes left for the background, the poses and
+// the intrinsics are added up, up to kSumRows rows to a workgroup (x: a share of the background's rows, the one after the last
+// share the camera's rows; y: the view), and added to the outputs with one atomic per value. (The passes used to end on these atomics
+// themselves: 12 thousand workgroups of a full-HD view add to one line of memory, which serves some 10^8 of them a second. Tile pass 6M points
+// 339 -> 324 us, four crops of 512 x 512 150 -> 114, four views of clusters 444 -> 330; point pass 300k points 32.6 -> 27, crops
+// 153 -> 134.) Rows that lie in a fixed order are summed in it, so a view of up to kSumRows blocks has the same sums in every run.
+constexpr int kSumThreads = 1024;  // (a chain of round trips: the more rows requested together the shorter)
+__global__ __launch_bounds__(kSumThreads) void backward_sums_kernel(const SumsParams p)
+{
+    const int view = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ double s_acc[kSumThreads];
+    if ((int)blockIdx.x < p.background_shares)
+    {
+        const int quads     = p.cpad / 4;  // 1, 2 or 4: a thread stays with one quad of channels
+        const long long end = min((long long)p.background_rows, ((long long)blockIdx.x + 1) * kSumRows) * quads;
+        const vf4* rows     = reinterpret_cast<const vf4*>(p.background_sums + (size_t)view * p.background_stride);
+        double sum[4]       = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (long long i = (long long)blockIdx.x * kSumRows * quads + threadIdx.x; i < end; i += kSumThreads)
         {
-            double v = s_acc[0][i] + s_acc[1][i] + s_acc[2][i] + s_acc[3][i];
-            if (v != 0.0)
-            {
-                if (i < 6)
-                    unsafeAtomicAdd(p.d_pose + i, v);
-                else
-                    unsafeAtomicAdd(p.d_intrinsics + (i - 6), (float)v);
-            }
+            const vf4 v = rows[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sum[k] += (double)v[k];
         }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            for (int o = 32; o >= quads; o >>= 1) sum[k] += __shfl_xor(sum[k], o);
+            if (lane < quads) s_acc[wave * 16 + 4 * lane + k] = sum[k];
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < p.channels)
+        {
+            const int i = threadIdx.x;
+            double v = 0.0;
+            for (int w = 0; w < kSumThreads / 64; ++w) v += s_acc[16 * w + i];
+            if (v != 0.0) unsafeAtomicAdd(p.d_background + i, (float)v);
+        }
+        return;
+    }
+    // a value per lane, the rows dealt to the groups of kCameraSums threads
+    constexpr int kGroups = kSumThreads / kCameraSums;
+    const int group = (int)threadIdx.x / kCameraSums, i = (int)threadIdx.x - group * kCameraSums;
+    const double* rows = p.camera_sums + (size_t)view * kCameraRows * kCameraSums;
+    double v           = 0.0;
+    if (group < kGroups)
+    {
+#pragma unroll 8
+        for (int r = group; r < p.camera_rows; r += kGroups) v += rows[(size_t)r * kCameraSums + i];
+    }
+    s_acc[threadIdx.x] = v;
+    __syncthreads();
+    if ((int)threadIdx.x >= kCameraSums) return;
+    for (int g = 1; g < kGroups; ++g) v += s_acc[g * kCameraSums + i];
+    if (v == 0.0) return;
+    if (i < 6)
+    {
+        if (p.d_pose) unsafeAtomicAdd(p.d_pose + 6 * (size_t)p.image_index[view] + i, v);
+    }
+    else if (i < 6 + 13)
+    {
+        if (p.d_intrinsics) unsafeAtomicAdd(p.d_intrinsics + 13 * (size_t)p.camera_index[view] + (i - 6), (float)v);
     }
 }
 
@@ -961,6 +1012,9 @@ hipError_t launch_tiles(const BackwardParams& p, int blocks, hipStream_t stream)
         default: return hipErrorInvalidValue;                                                                  \
     }
 
+// (four workgroups per CU, each walking its share of the points: every further one leaves another row of sums)
+int point_pass_blocks(int num_points) { return std::min((num_points + 255) / 256, kCameraRows); }
+
 hipError_t launch_backward_view(const BackwardParams& p, int channels, hipStream_t stream, Profiler* prof)
 {
     const int N = p.num_points;
@@ -992,11 +1046,19 @@ hipError_t launch_backward_view(const BackwardParams& p, int channels, hipStream
     if (N > 0)
     {
         ProfScope ps(prof, "backward_points", stream);
-        // (four workgroups per CU, each walking its share of the points: every further workgroup adds its atomics on the
-        // pose and intrinsics sums)
-        const int blocks = min((N + 255) / 256, 1024);
+        const int blocks = point_pass_blocks(N);
         TRIPS_BW_DISPATCH(backward_points_kernel, blocks);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_backward_sums(SumsParams& p, int num_points, hipStream_t stream, Profiler* prof)
+{
+    ProfScope ps(prof, "backward_sums", stream);
+    const bool camera   = num_points > 0 && (p.d_pose || p.d_intrinsics);
+    p.background_shares = (p.background_rows + kSumRows - 1) / kSumRows;
+    p.camera_rows       = point_pass_blocks(num_points);
+    hipLaunchKernelGGL(backward_sums_kernel, dim3(p.background_shares + (camera ? 1 : 0), p.num_views), dim3(kSumThreads), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -285,6 +285,12 @@ struct SavedLayout
 __host__ __device__ constexpr int pair_row_floats(int cpad) { return cpad + 4; }
 constexpr int kInlineLayers = 2;
 
+// The tile pass's workgroups leave their sums for the background, the point pass's (at most kCameraRows) theirs for pose (6),
+// intrinsics (5) and distortion (8), in whole quads; backward_sums_kernel adds them up, kSumRows rows to a workgroup.
+constexpr int kCameraRows = 1024;
+constexpr int kCameraSums = 20;
+constexpr int kSumRows    = 4096;
+
 struct BackwardWorkspaceLayout
 {
     size_t rows_inline;  // float [N, kInlineLayers, pair_row_floats] by compact number
@@ -292,6 +298,8 @@ struct BackwardWorkspaceLayout
     size_t flags;         // uint8 [N, TRIPS_MAX_LAYERS] by compact number: 1 where the tile pass wrote the pair's row
                           // (only for views in which few pairs are retained)
     size_t mode;          // int32: 1 = only flagged rows exist (written by the prologue kernel)
+    size_t background_sums;  // float [views][blocks of the tile pass][channels in whole quads]: a workgroup's sums
+    size_t camera_sums;      // double [views][kCameraRows][kCameraSums]: a workgroup's sums in the point pass
     size_t over_capacity;
     size_t bytes;
 };
@@ -408,6 +416,8 @@ struct BackwardParams
     int32_t blocks_off[TRIPS_MAX_LAYERS + 1];
     int32_t blocks_x[TRIPS_MAX_LAYERS];
     long long over_capacity;
+    float* background_sums;  // [blocks][channels in whole quads] (workspace, this view's)
+    double* camera_sums;     // [kCameraRows][kCameraSums] (workspace, this view's)
     float* d_texture;
     float* d_confidence;
     float* d_background;
@@ -421,6 +431,20 @@ struct BackwardParams
     double* d_pose_all;       // [num_images][6] or nullptr
     float* d_intrinsics_all;  // [num_cameras][13] or nullptr
     int32_t num_images, num_cameras;
+};
+
+// what backward_sums_kernel adds up, for all views of a call
+struct SumsParams
+{
+    const float* background_sums;
+    const double* camera_sums;
+    long long background_stride;  // floats from a view's rows to the next one's
+    int32_t background_rows, background_shares, camera_rows;
+    int32_t channels, cpad, num_views;
+    float* d_background;
+    double* d_pose;       // [num_images][6] or nullptr
+    float* d_intrinsics;  // [num_cameras][13] or nullptr
+    int32_t image_index[TRIPS_MAX_VIEWS], camera_index[TRIPS_MAX_VIEWS];
 };
 
 }  // namespace trips

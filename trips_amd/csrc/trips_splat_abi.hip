@@ -15,6 +15,7 @@ namespace trips
 hipError_t launch_forward_view(const ForwardParams& p, int channels, bool train, bool first_view, hipStream_t stream,
                                Profiler* prof);
 hipError_t launch_backward_view(const BackwardParams& p, int channels, hipStream_t stream, Profiler* prof);
+hipError_t launch_backward_sums(SumsParams& p, int num_points, hipStream_t stream, Profiler* prof);
 hipError_t launch_adam(const TripsAdamTensor* tensors, int n_tensors, hipStream_t stream, Profiler* prof);
 int adam_points_row_chunks(int channels);
 hipError_t launch_adam_points(const TripsAdamTensor tensors[4], int num_points, int channels, void* state, hipStream_t stream,
@@ -273,6 +274,19 @@ WorkspaceLayout workspace_layout(const TripsSplatDesc& d, const PyramidGeom& g)
 
 namespace
 {
+// Blocks of the tile pass, 16 x 16 pixels, 15 apart, so that every pixel is the first-15 part of exactly one: first block of each
+// layer, blocks per block row of each layer.
+void tile_pass_blocks(const PyramidGeom& g, int num_layers, int32_t (&off)[TRIPS_MAX_LAYERS + 1], int32_t (&per_row)[TRIPS_MAX_LAYERS])
+{
+    off[0] = 0;
+    for (int l = 0; l < TRIPS_MAX_LAYERS; ++l)
+    {
+        const int nx = l < num_layers ? (g.w[l] + 14) / 15 : 0, ny = l < num_layers ? (g.h[l] + 14) / 15 : 0;
+        per_row[l] = nx;
+        off[l + 1] = off[l] + nx * ny;
+    }
+}
+
 BackwardWorkspaceLayout backward_workspace_layout(const TripsSplatDesc& d, const PyramidGeom& g)
 {
     BackwardWorkspaceLayout w;
@@ -290,6 +304,12 @@ BackwardWorkspaceLayout backward_workspace_layout(const TripsSplatDesc& d, const
     o += align256((size_t)d.num_points * TRIPS_MAX_LAYERS);
     w.mode = o;
     o += 256;
+    int32_t blocks_off[TRIPS_MAX_LAYERS + 1], blocks_x[TRIPS_MAX_LAYERS];
+    tile_pass_blocks(g, d.num_layers, blocks_off, blocks_x);
+    w.background_sums = o;
+    o += align256((size_t)d.num_views * blocks_off[d.num_layers] * (size_t)((d.num_channels + 3) & ~3) * sizeof(float));
+    w.camera_sums = o;
+    o += align256((size_t)d.num_views * kCameraRows * kCameraSums * sizeof(double));
     w.bytes = o;
     return w;
 }
@@ -535,6 +555,16 @@ int trips_splat_backward(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsS
         return fail(TRIPS_ERR_WORKSPACE_SMALL, "workspace has %zu bytes, %zu needed", workspace_bytes, bl.bytes);
     char* ws             = reinterpret_cast<char*>(workspace);
     hipStream_t stream   = reinterpret_cast<hipStream_t>(stream_);
+    SumsParams sums;
+    std::memset(&sums, 0, sizeof(sums));
+    sums.background_sums = reinterpret_cast<const float*>(ws + bl.background_sums);
+    sums.camera_sums     = reinterpret_cast<const double*>(ws + bl.camera_sums);
+    sums.channels        = d.num_channels;
+    sums.cpad            = (d.num_channels + 3) & ~3;
+    sums.num_views       = d.num_views;
+    sums.d_background    = grads->d_background;
+    sums.d_pose          = grads->d_pose;
+    sums.d_intrinsics    = grads->d_intrinsics;
     for (int b = 0; b < d.num_views; ++b)
     {
         BackwardParams p;
@@ -575,14 +605,14 @@ int trips_splat_backward(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsS
         p.mode         = reinterpret_cast<int32_t*>(ws + bl.mode);
         p.force_mode   = ctx->pair_rows_mode;
         p.over_capacity = (long long)bl.over_capacity;
-        p.blocks_off[0] = 0;
-        for (int l = 0; l < TRIPS_MAX_LAYERS; ++l)
-        {
-            // blocks of 16 x 16 pixels, 15 apart, so that every pixel is the first-15 part of exactly one block
-            const int nx = l < d.num_layers ? (g.w[l] + 14) / 15 : 0, ny = l < d.num_layers ? (g.h[l] + 14) / 15 : 0;
-            p.blocks_x[l]       = nx;
-            p.blocks_off[l + 1] = p.blocks_off[l] + nx * ny;
-        }
+        tile_pass_blocks(g, d.num_layers, p.blocks_off, p.blocks_x);
+        const size_t background_floats = (size_t)p.blocks_off[d.num_layers] * (size_t)((d.num_channels + 3) & ~3);
+        p.background_sums = reinterpret_cast<float*>(ws + bl.background_sums) + background_floats * (size_t)b;
+        p.camera_sums     = reinterpret_cast<double*>(ws + bl.camera_sums) + (size_t)kCameraRows * kCameraSums * (size_t)b;
+        sums.background_stride = (long long)background_floats;
+        sums.background_rows   = p.blocks_off[d.num_layers];
+        sums.image_index[b]    = d.views[b].image_index;
+        sums.camera_index[b]   = d.views[b].camera_index;
         for (int l = 0; l < d.num_layers; ++l) p.grad_image[l] = grad_image[l];
         p.d_texture    = grads->d_texture;
         p.d_confidence = grads->d_confidence;
@@ -600,6 +630,8 @@ int trips_splat_backward(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsS
         hipError_t e   = launch_backward_view(p, d.num_channels, stream, ctx->prof.enabled ? &ctx->prof : nullptr);
         if (e != hipSuccess) return hip_fail(e, "backward launch");
     }
+    if (hipError_t e = launch_backward_sums(sums, d.num_points, stream, ctx->prof.enabled ? &ctx->prof : nullptr); e != hipSuccess)
+        return hip_fail(e, "backward launch");
     return TRIPS_OK;
 }
 
