@@ -846,9 +846,10 @@ __global__ __launch_bounds__(256) void backward_points_kernel(const BackwardPara
 // After the passes of all views of a call: the rows that the workgroups of the two passes left for the background, the poses and
 // the intrinsics are added up, up to kSumRows rows to a workgroup (x: a share of the background's rows, the one after the last
 // share the camera's rows; y: the view), and added to the outputs with one atomic per value. (The passes used to end on these atomics
-// themselves: 12 thousand workgroups of a full-HD view add to one line of memory, which serves some 10^8 of them a second. Tile pass 6M points
-// 339 -> 324 us, four crops of 512 x 512 150 -> 114, four views of clusters 444 -> 330; point pass 300k points 32.6 -> 27, crops
-// 153 -> 134.) Rows that lie in a fixed order are summed in it, so a view of up to kSumRows blocks has the same sums in every run.
+// themselves: 12 thousand workgroups of a full-HD view add to one line of memory, which serves some 10^8 of them a second. us,
+// tile pass: 6M points 331 -> 318, 9M 252 -> 210, four crops of 512 x 512 151 -> 103, four views of clusters 443 -> 308; point
+// pass: 300k points 33 -> 22, crops 149 -> 111, clusters 289 -> 269; this kernel: 4 to 8 a call.) The rows are summed in a fixed
+// order, so a view of up to kSumRows blocks has the same sums in every run.
 constexpr int kSumThreads = 1024;  // (a chain of round trips: the more rows requested together the shorter)
 __global__ __launch_bounds__(kSumThreads) void backward_sums_kernel(const SumsParams p)
 {
