@@ -726,14 +726,16 @@ __global__ __launch_bounds__(256) void up2_adjoint_gate_kernel(UpAdjointParams p
 // data gradient of 8 x 32 pixels (30 columns of its own and one at each side, which the neighbour works out too) goes
 // into a ring of ten rows in LDS, rounded to fp16 as it was in memory; four rows of the coarser level then gather their
 // 4 x 4 finer pixels from it, in the order of up2_adjoint_gate_kernel, and leave gated. The patch of pre-activation
-// gradients is a ring of ten rows too, and the eight rows of the next step travel in registers during the products.
+// gradients is a ring of ten rows too. The eight rows of the next step travel in registers during the products where a CU
+// holds one workgroup; where it holds two they go straight to LDS during the gather, which leaves the registers for the
+// second workgroup: its products then run beside the first one's gather.
 // A wavefront owns 4 x 16 pixels and half of the outputs and keeps the weights of those in registers for the whole strip:
 // an operand read from the patch then serves up to three taps, and the sums run in the order of conv_taps_mfma.
 //
-// Bound at the finest level of a large image by memory (1920 x 1080: 484 MB in 124 us, 63 % of a copy's rate, halos that
-// neighbouring strips read as well among them), elsewhere by the steps' latencies (two barriers each) at one or two
-// workgroups per CU. As two kernels and as one: 1920 x 1080, 32 pre-activations x 32 inputs: 90 + 68 and 125 us;
-// 960 x 540, 64 x 64: 54 + 36 and 83 us; 1245 x 825 and the levels below it, 64 x 32: 119 + 60 and 164 us. The gather as
+// Bound at the finest level of a large image by memory, elsewhere by the steps' latencies (two barriers each). As two kernels and as
+// one: 1920 x 1080, 32 pre-activations x 32 inputs: 90 + 68 and 125 us; 960 x 540, 64 x 64: 54 + 36 and 82 us; 1245 x 825 and
+// the levels below it, 64 x 32: 119 + 60 and 142 us. Of these two workgroups on a CU at 64 x 32, 168 -> 145 (four crops of 512 x 512
+// 189 -> 152); neighbouring strips on one XCD, whose L2 then holds the halos that they share, 145 -> 142 and 127 -> 125. The gather as
 // matrix products from a ring with the pixels innermost took 358 us where this takes 164.
 struct BwdDataUpParams
 {
@@ -758,10 +760,20 @@ constexpr int strip_lds_bytes(int kc, int nn, int ci)
     return kConvPatchH * kConvPatchW * (kc + kLdsChanPad) * 2 + kRingRows * kConvTileW * (nn + kLdsChanPad) * 2 + kConvTileH * kConvTileW * ci * 4;
 }
 // Workgroups of a CU: two where LDS and registers (the weights take 36 (kc / 32) (nn / 32) of a lane) hold them.
-constexpr int strip_resident(int kc, int nn, int ci) { return 2 * strip_lds_bytes(kc, nn, ci) <= 160 * 1024 && kc * nn <= 32 * 32 ? 2 : 1; }
+// (LDS is given out in 128 pieces of 1280 bytes.)
+constexpr int strip_resident(int kc, int nn, int ci) { return strip_lds_bytes(kc, nn, ci) <= 64 * 1280 && nn == 32 ? 2 : 1; }
 
-// ALIGNED: 2 C is a multiple of 8, so that a group of eight block outputs is one aligned read (both forms in one kernel
-// took 40 registers more).
+__device__ const _Float16 k_zeros[8] = {};  // what lies outside the image
+
+// 16 bytes of each active lane, from its address to LDS: at `to` (the same for all lanes), in the order of the lanes, the places of
+// inactive ones left as they are. In flight until wait_for_loads.
+__device__ __forceinline__ void load_to_lds16(const void* from, void* to)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// ALIGNED: 2 C is a multiple of 4, so that a group of four block outputs is one aligned read.
 template <int KC, int NN, int CI, bool ALIGNED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_resident(KC, NN, CI)))) void conv_bwd_data_up_kernel(BwdDataUpParams q)
 {
@@ -770,7 +782,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
     constexpr int GROUPS = KC / 8, KB = KC / 32, NBW = NN / 32;
     constexpr int kPixels = kConvTileH * kConvTileW;
     const int H = q.fine.H, W = q.fine.W, C = q.fine.c_feat, Hb = q.up.Hb, Wb = q.up.Wb, npad_b = q.up.npad;
-    const size_t image  = (size_t)q.fine.first_image + blockIdx.z;
+    // Neighbouring strips share halos: they go to one XCD (workgroups are dealt to the eight of them in turn).
+    const int all = gridDim.x * gridDim.y * gridDim.z, dealt = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int at_block = (dealt & 7) * (all >> 3) + min(dealt & 7, all & 7) + (dealt >> 3);
+    const int strip_x = at_block % gridDim.x, strip_yz = at_block / gridDim.x, strip_y = strip_yz % gridDim.y;
+    const size_t image  = (size_t)q.fine.first_image + strip_yz / gridDim.y;
     const size_t plane  = (size_t)H * W, plane_b = (size_t)Hb * Wb;
     const _Float16* dpre  = q.fine.dpre + image * plane * KC;
     float* d_feat         = q.fine.d_feat + image * plane * C;
@@ -779,17 +795,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
     float* d_feat_b       = q.up.d_feat + image * plane_b * C;
     const float scale_inv = q.fine.scale_inv;
 
-    extern __shared__ _Float16 smem[];
-    _Float16* s_patch = smem;                                       // [10 rows][34][ROW]
-    _Float16* s_ring  = s_patch + kConvPatchH * kConvPatchW * ROW;  // [10 rows][32][OS]
-    float* s_img      = reinterpret_cast<float*>(s_ring + kRingRows * kConvTileW * OS);  // [CI][8 x 32]
+    // (arrays of their own: the loads into the patch are then known to leave what is read from the ring alone)
+    __shared__ __align__(16) _Float16 s_patch[kConvPatchH * kConvPatchW * ROW];  // [10 rows][34][ROW]
+    __shared__ __align__(16) _Float16 s_ring[kRingRows * kConvTileW * OS];       // [10 rows][32][OS]
+    __shared__ float s_img[CI * kPixels];                                        // [CI][8 x 32]
+    constexpr bool kAlone = strip_resident(KC, NN, CI) == 1;  // one workgroup on a CU
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lrow = lane & 15, lk = (lane >> 4) * 8;
     const int wr = (wave & 1) * 4, wc = ((wave >> 1) & 1) * 16, wn = (wave >> 2) * NBW;  // this wavefront's rows, columns, output blocks
     const int rows_own = 4 * q.steps - 1;                      // rows of the coarser level
-    const int Y0 = blockIdx.y * rows_own, Y1 = min(Y0 + rows_own, Hb);
-    const int yf = 2 * Y0 - 1, xf = blockIdx.x * kStripFine - 1;  // the strip's first computed pixel
+    const int Y0 = strip_y * rows_own, Y1 = min(Y0 + rows_own, Hb);
+    const int yf = 2 * Y0 - 1, xf = strip_x * kStripFine - 1;  // the strip's first computed pixel
     const int steps = (2 * (Y1 - Y0) + 2 + kConvTileH - 1) / kConvTileH;
 
     half8 b[9][KB][NBW];
@@ -840,33 +857,55 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
             if (kRowItems % 64 == 0 || px < kConvPatchW) *reinterpret_cast<uint4*>(dst + j * (64 / GROUPS) * ROW) = v;
         }
     };
-    if (wave < 2)
+    // The same without registers on the way: a wavefront's loads write LDS in the order of its lanes, so the lanes are dealt to
+    // whole rows of the patch, and those of the padding sit out.
+    auto load_row = [&](int row, int slot)
     {
-        fetch_row(wave);
-        put_row(wave, wave);
-    }
-    fetch_row(wave + 2);
-    put_row(wave + 2, wave + 2);
+        constexpr int kWords = GROUPS + kLdsChanPad / 8;  // of 16 bytes, of a pixel
+        const int tl = thread() & 63;
+        const int y  = yf - 1 + row;
+#pragma unroll
+        for (int j = 0; j < (kConvPatchW * kWords + 63) / 64; ++j)
+        {
+            const int i = tl + 64 * j, px = i / kWords, g = i - px * kWords, x = xf - 1 + px;
+            const _Float16* src = y >= 0 && y < H && x >= 0 && x < W ? dpre + ((size_t)y * W + x) * KC + 8 * g : k_zeros;
+            if (px < kConvPatchW && g < GROUPS) load_to_lds16(src, s_patch + slot * kConvPatchW * ROW + 64 * 8 * j);
+        }
+    };
+    auto first_row = [&](int row)
+    {
+        if (kAlone)
+        {
+            fetch_row(row);
+            put_row(row, row);
+        }
+        else
+            load_row(row, row);
+    };
+    if (wave < 2) first_row(wave);
+    first_row(wave + 2);
 
-    // the items of the adjoint: a pixel of the coarser level and eight positions (see up2_adjoint_gate_kernel)
-    const int g0 = C / 8, ig = (2 * C - 1) / 8 - g0 + 1;
-    const int groups = ig + npad_b / 16;
-    const int items  = 4 * kStripCoarse * groups;
+    // the items of the adjoint: a pixel of the coarser level and four positions (see up2_adjoint_gate_kernel), the gated
+    // ones before those of the image. (Eight positions to an item are 300 items of a step at 64 pre-activations: five of the eight
+    // wavefronts work, and one SIMD does the work of two: 960 x 540, 64 x 64, 88 -> 82 us, 1920 x 1080, 32 x 32, 132 -> 127.)
+    const int gates = npad_b / 8;
+    const int g0 = C / 4, ig = (2 * C - 1) / 4 - g0 + 1;
+    const int gate_items = 4 * kStripCoarse * gates;
+    const int items      = gate_items + 4 * kStripCoarse * ig;
     struct Item
     {
         int q, c, cx;
     };
     auto item_of = [&](int item)
     {
-        const int bp = item / groups;
-        return Item{item - bp * groups, bp / kStripCoarse, bp % kStripCoarse};
+        const int past = item - gate_items, per = past < 0 ? gates : ig, i = past < 0 ? item : past;
+        const int bp   = i / per;
+        return Item{i - bp * per + (past < 0 ? 0 : gates), bp / kStripCoarse, bp % kStripCoarse};
     };
-    auto load_pre = [&](const Item& it, int Yk, half8& lo, half8& hi)
+    auto load_pre = [&](const Item& it, int Yk)
     {
-        const int Y = min(max(Yk + it.c, 0), Hb - 1), X = min((int)blockIdx.x * kStripCoarse + it.cx, Wb - 1);
-        const _Float16* src = pre_b + ((size_t)Y * Wb + X) * npad_b + 16 * max(it.q - ig, 0);
-        lo = *reinterpret_cast<const half8*>(src);
-        hi = *reinterpret_cast<const half8*>(src + 8);
+        const int Y = min(max(Yk + it.c, 0), Hb - 1), X = min(strip_x * kStripCoarse + it.cx, Wb - 1);
+        return *reinterpret_cast<const half8*>(pre_b + ((size_t)Y * Wb + X) * npad_b + 8 * min(it.q, gates - 1));
     };
     const Item first_item = item_of(threadIdx.x);
     const int packed      = first_item.q | first_item.c << 8 | first_item.cx << 16;
@@ -876,6 +915,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
         asm volatile("" : "+v"(t));
         return Item{t & 255, t >> 8 & 255, t >> 16};
     };
+    if (!kAlone) wait_for_loads();
     __syncthreads();
 
     int slot = 0;  // of the step's first row, in both rings
@@ -884,13 +924,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
         const int yk = yf + kConvTileH * k;  // the step's first row of the finer level
         const int Yk = Y0 - 1 + 4 * k;       // ... and of the coarser one (k = 0: the strip above owns that row)
         const bool more = k + 1 < steps;
-        // in flight during the products: the next step's rows
-        if (more) fetch_row(kConvTileH * (k + 1) + 2 + wave);
-        half8 lo, hi;
+        // rows 2 .. 9 of the next step, a row per wavefront, into the slots of rows 0 .. 7 of this one: in flight during the
+        // products, where no other workgroup hides the latency, else during the adjoint
+        const int next_row = kConvTileH * (k + 1) + 2 + wave, next_slot = slot + wave < kConvPatchH ? slot + wave : slot + wave - kConvPatchH;
+        if (kAlone && more) fetch_row(next_row);
+        half8 pre;  // four features, four masks
         float old[kPixels * CI / THREADS];
         auto load_rest = [&]()
         {
-            load_pre(mine(), Yk, lo, hi);
+            pre = load_pre(mine(), Yk);
             const int tid_load = thread();
 #pragma unroll
             for (int j = 0; j < kPixels * CI / THREADS; ++j)
@@ -900,8 +942,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
                 old[j] = d_feat[min(v / kPixels, C - 1) * plane + (size_t)y * W + x];
             }
         };
-        // (before the products where there are registers for it: nothing else hides this latency with one workgroup per CU)
-        constexpr bool kEarly = strip_resident(KC, NN, CI) == 1 && KC * NN <= 64 * 32;
+        // (before the products where there are registers for it)
+        constexpr bool kEarly = kAlone && KC * NN <= 64 * 32;
         if (kEarly) load_rest();
         floatx4 acc[4][NBW];
 #pragma unroll
@@ -910,22 +952,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
             for (int n = 0; n < NBW; ++n) acc[r][n] = floatx4{0.f, 0.f, 0.f, 0.f};
         // step t: column dx = t % 3 of patch row pr = t / 3; its operands are requested two steps ahead (and no further:
         // the registers would not do)
-        half8 a3[3][KB];
+        constexpr int kAhead = kAlone || KC * NN <= 32 * 32 ? 2 : 1;
+        half8 a3[kAhead + 1][KB];
         auto operands = [&](int t)
         {
             const int pr  = t / 3, dx = t - 3 * pr;
             const int at  = slot + wr + pr < kConvPatchH ? slot + wr + pr : slot + wr + pr - kConvPatchH;
             const _Float16* src = s_patch + (at * kConvPatchW + wc + lrow + dx) * ROW + lk;
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb) a3[t % 3][kb] = *reinterpret_cast<const half8*>(src + kb * 32);
+            for (int kb = 0; kb < KB; ++kb) a3[t % (kAhead + 1)][kb] = *reinterpret_cast<const half8*>(src + kb * 32);
         };
-        operands(0);
-        operands(1);
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t) operands(t);
 #pragma unroll
         for (int t = 0; t < 18; ++t)
         {
             const int pr = t / 3, dx = t - 3 * pr;
-            if (t + 2 < 18) operands(t + 2);
+            if (t + kAhead < 18) operands(t + kAhead);
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -933,7 +976,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
                     if (pr - dy >= 0 && pr - dy < 4)
 #pragma unroll
                         for (int n = 0; n < NBW; ++n)
-                            acc[pr - dy][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy * 3 + dx][kb][n], a3[t % 3][kb], acc[pr - dy][n], 0, 0, 0);
+                            acc[pr - dy][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[dy * 3 + dx][kb][n], a3[t % (kAhead + 1)][kb], acc[pr - dy][n], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (!kEarly)
@@ -963,7 +1006,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
             }
         }
         __syncthreads();  // the step's rows are in the ring; nobody reads the patch any more
-        if (more) put_row(kConvTileH * (k + 1) + 2 + wave, slot + wave < kConvPatchH ? slot + wave : slot + wave - kConvPatchH);  // (rows 2 .. 9 of the next step: the slots of rows 0 .. 7 of this one)
+        if (more)
+        {
+            if (kAlone)
+                put_row(next_row, next_slot);
+            else
+                load_row(next_row, next_slot);
+        }
 
         // the finer level's own image
         const int tid_store = thread();
@@ -979,16 +1028,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
         for (int item = threadIdx.x; item < items; item += THREADS)
         {
             const Item it = item < THREADS ? mine() : item_of(item);
-            const int Y = Yk + it.c, X = (int)blockIdx.x * kStripCoarse + it.cx;
+            const int Y = Yk + it.c, X = strip_x * kStripCoarse + it.cx;
             if (Y < Y0 || Y >= Y1 || X >= Wb) continue;
-            if (item >= THREADS) load_pre(it, Yk, lo, hi);
-            const int ch0 = 8 * (it.q - ig);
-            const int pos = it.q < ig ? 8 * (g0 + it.q) : 2 * C + ch0;  // first of the eight positions
-            float wy[4], wx[4], a[8];
+            if (item >= THREADS && it.q < gates) pre = load_pre(it, Yk);
+            const int pos = it.q < gates ? 2 * C + 4 * it.q : 4 * (g0 + it.q - gates);  // first of the four positions
+            float wy[4], wx[4], a[4];
             up2_adjoint_weights(Y, H, Hb, wy);
             up2_adjoint_weights(X, W, Wb, wx);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a[i] = 0.f;
+            for (int i = 0; i < 4; ++i) a[i] = 0.f;
             if (pos < NN)  // (a row ends with eight unused halves: the last group may reach into them, past the block's outputs)
             {
 #pragma unroll
@@ -998,30 +1046,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
                     int at = slot + 8 + 2 * it.c + ky;
                     at -= at >= 2 * kRingRows ? 2 * kRingRows : at >= kRingRows ? kRingRows : 0;
                     const _Float16* src = s_ring + (at * kConvTileW + 2 * it.cx) * OS + pos;
-                    __builtin_amdgcn_sched_barrier(0);  // one row's reads at a time: sixteen in flight cost 64 registers
+                    if (!kAlone) __builtin_amdgcn_sched_barrier(0);  // one row's reads at a time: more would take the weights' registers
 #pragma unroll
                     for (int kx = 0; kx < 4; ++kx)
                     {
-                        half8 v;
+                        half4 v;
                         if (ALIGNED)
-                            v = *reinterpret_cast<const half8*>(src + kx * OS);
+                            v = *reinterpret_cast<const half4*>(src + kx * OS);
                         else
                         {
                             // (2 C is even: words of four bytes)
-                            const unsigned* w4 = reinterpret_cast<const unsigned*>(src + kx * OS);
-                            v = __builtin_bit_cast(half8, make_uint4(w4[0], w4[1], w4[2], w4[3]));
+                            const unsigned* w2 = reinterpret_cast<const unsigned*>(src + kx * OS);
+                            v = __builtin_bit_cast(half4, make_uint2(w2[0], w2[1]));
                         }
                         const float w = wy[ky] * wx[kx];  // (0 for pixels outside the image only: the ring holds zeros there)
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) a[i] = __builtin_fmaf(w, float(v[i]), a[i]);
+                        for (int i = 0; i < 4; ++i) a[i] = __builtin_fmaf(w, float(v[i]), a[i]);
                     }
                 }
             }
             const size_t bp = (size_t)Y * Wb + X;
-            if (it.q < ig)
+            if (it.q >= gates)
             {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < 4; ++i)
                 {
                     const int c = pos + i - C;
                     if (c >= 0 && c < C) d_feat_b[(size_t)c * plane_b + bp] = a[i] * scale_inv;
@@ -1029,20 +1077,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2 * strip_r
             }
             else
             {
-                half8 of, om;
+                half8 out;
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < 4; ++i)
                 {
                     float df, dm;
-                    gate_backward(ch0 + i < q.up.cout ? a[i] : 0.f, float(i < 4 ? lo[i & 3] : hi[i & 3]), float(i < 4 ? lo[4 + (i & 3)] : hi[4 + (i & 3)]), df, dm);
-                    of[i] = _Float16(df);
-                    om[i] = _Float16(dm);
+                    gate_backward(4 * it.q + i < q.up.cout ? a[i] : 0.f, float(pre[i]), float(pre[4 + i]), df, dm);
+                    out[i]     = _Float16(df);
+                    out[4 + i] = _Float16(dm);
                 }
-                _Float16* dp = dpre_b + bp * npad_b + 2 * ch0;
-                *reinterpret_cast<half8*>(dp)     = half8{of[0], of[1], of[2], of[3], om[0], om[1], om[2], om[3]};
-                *reinterpret_cast<half8*>(dp + 8) = half8{of[4], of[5], of[6], of[7], om[4], om[5], om[6], om[7]};
+                *reinterpret_cast<half8*>(dpre_b + bp * npad_b + 8 * it.q) = out;
             }
         }
+        if (!kAlone) wait_for_loads();
         slot = slot + kConvTileH < kRingRows ? slot + kConvTileH : slot + kConvTileH - kRingRows;
         __syncthreads();  // the next step's patch is in place; nobody reads the ring any more
     }
@@ -1646,11 +1693,7 @@ hipError_t dispatch_bwd_data(const BwdDataParams& p, int batch, int npad, int ci
 template <int KC, int NN, int CI, bool ALIGNED>
 hipError_t launch_bwd_data_up(const BwdDataUpParams& p, int batch, hipStream_t stream)
 {
-    constexpr int lds = strip_lds_bytes(KC, NN, CI);
-    static_assert(lds <= 160 * 1024, "the rings do not fit");
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_data_up_kernel<KC, NN, CI, ALIGNED>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return e;
+    static_assert(strip_lds_bytes(KC, NN, CI) <= 160 * 1024, "the rings do not fit");
     const int strips = (p.up.Wb + kStripCoarse - 1) / kStripCoarse;
     for (int b = 0; b < batch; b += kMaxGridImages)
     {
@@ -1664,14 +1707,14 @@ hipError_t launch_bwd_data_up(const BwdDataUpParams& p, int batch, hipStream_t s
         auto segments            = [&](int steps) { return (p.up.Hb + 4 * steps - 2) / (4 * steps - 1); };
         q.steps                  = 1;
         while (q.steps < most && (long long)strips * images * segments(q.steps) > resident) ++q.steps;
-        hipLaunchKernelGGL((conv_bwd_data_up_kernel<KC, NN, CI, ALIGNED>), dim3(strips, segments(q.steps), images), dim3(512), lds, stream, q);
+        hipLaunchKernelGGL((conv_bwd_data_up_kernel<KC, NN, CI, ALIGNED>), dim3(strips, segments(q.steps), images), dim3(512), 0, stream, q);
     }
     return hipGetLastError();
 }
 
 hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, int cin_pad, hipStream_t stream)
 {
-    const bool aligned = p.fine.c_feat % 4 == 0;
+    const bool aligned = p.fine.c_feat % 2 == 0;
 #define TRIPS_BDU_CI(KC_, NN_, CI_) \
     return aligned ? launch_bwd_data_up<KC_, NN_, CI_, true>(p, batch, stream) : launch_bwd_data_up<KC_, NN_, CI_, false>(p, batch, stream)
 #define TRIPS_BDU(KC_, NN_)                                     \
