@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8
 
 // CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
 template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
-__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(CIN == 32 && NPAD == 32 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightTable tab)
+__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(2 * wgrad_resident(CIN, NPAD)))) void conv_bwd_weight_kernel(const BwdWeightTable tab)
 {
     int level = 0;
     while (level + 1 < tab.n && (int)blockIdx.x >= tab.first[level + 1]) ++level;

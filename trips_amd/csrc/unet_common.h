@@ -170,9 +170,13 @@ inline int check_unet_desc(const TripsUnetDesc* d)
     return TRIPS_OK;
 }
 
+// Workgroups of the weight gradient on a CU: two where LDS (75 KB at 32 x 64) and registers (128 of a lane) allow it; one waits for
+// its loads and barriers while the other multiplies. 32 inputs x 64 pre-activations, levels of 1245 x 825 and of four 512 x 512 crops
+// 98 -> 86 us and 99 -> 87, the sums of twice the partials 10 -> 12.
+constexpr int wgrad_resident(int cin_pad, int npad) { return cin_pad == 32 && npad <= 64 ? 2 : 1; }
+
 // Levels whose weight gradients are the same instance of the kernel run in one launch, whose workgroups are as many as are
-// resident at once (two per CU for the smallest shape, else one; every further one would only add a set of partial sums to
-// write and reduce) and are dealt to the levels by their tiles. With a launch per level the coarser ones were a handful of
+// resident at once (every further one would only add a set of partial sums to write and reduce) and are dealt to the levels by their tiles. With a launch per level the coarser ones were a handful of
 // tiles each, begun and ended 256 workgroups at a time: all weight gradients and the sums of their partials, default net
 // of five levels at 1245 x 825 155 -> 110 us, at 105 x 74 (32/64/64/64/64) 85 -> 46, 16/32/64/64 at 1920 x 1080 217 -> 205.
 // `wanted` holds a bit per level whose weight gradients are asked for: the workgroups are dealt to those alone. (Dealt as if
@@ -190,7 +194,7 @@ inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
         bool first          = true;  // of its instance
         for (int k = 0; k < i; ++k) first = first && !same_wgrad_kernel(np.lv[k], lv);
         if (!first) continue;
-        const long long resident = 256 * (lv.cin_pad == 32 && lv.wgrad_tile == 32 ? 2 : 1);
+        const long long resident = 256 * wgrad_resident(lv.cin_pad, lv.wgrad_tile);
         long long all = 0, work = 0, shares = 0;
         for (int k = i; k < levels; ++k)
             if (same_wgrad_kernel(np.lv[k], lv))
