@@ -191,6 +191,13 @@ def test_extreme_image_shapes(oracle, w, h, L, n):
     _check_backward(oracle, sc, d, seed=1)
 
 
+@pytest.mark.parametrize("channels,train", [(16, True), (4, False)])
+def test_as_many_tiles_as_there_may_be(oracle, channels, train):
+    """15265 of at most 15360 tiles: the counters and the records of a workgroup of the projection take the most LDS there is."""
+    sc = scenes.tiny(n=3000, w=4096, h=2848, f=3000.0, num_layers=8, list_depth=8, seed=41, channels=channels, radius=(1e-4, 0.3))
+    _check_forward(oracle, sc, abi.desc_for_scene(sc, train=train))
+
+
 def test_transmittance_cutoff_matches(oracle):
     n = 12
     sc = scenes.tiny(n=n, w=16, h=16, f=30.0, num_layers=1, list_depth=16, seed=3, background=0.5)

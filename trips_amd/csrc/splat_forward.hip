@@ -198,13 +198,17 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
 
 // Calls f(px, py, counter of the tile of (px, py)) for the layers a point is written to.
 template <typename F>
-__device__ __forceinline__ void for_point_tiles(const PyramidGeom& g, const PointProjection& o, int* tile_table, F&& f)
+__device__ __forceinline__ void for_point_tiles(const LayerTable& t, float lx, float ly, int layers, int* tile_table, F&& f)
 {
-    float lx = o.ipx, ly = o.ipy;
-    for (int layer = 0; layer < o.layers; ++layer, lx *= 0.5f, ly *= 0.5f)
+    for (int layer = 0; layer < TRIPS_MAX_LAYERS; ++layer, lx *= 0.5f, ly *= 0.5f)
     {
-        const int px = (int)floorf(lx), py = (int)floorf(ly);
-        f(px, py, tile_table + g.bin_off[layer] + (py >> kTileShift) * g.tiles_x[layer] + (px >> kTileShift));
+        if (__ballot(layer < layers) == 0) break;
+        const int bin_off = __builtin_amdgcn_readlane(t.bin_off, layer), tiles_x = __builtin_amdgcn_readlane(t.tiles_x, layer);
+        if (layer < layers)
+        {
+            const int px = (int)lx, py = (int)ly;  // (not negative)
+            f(px, py, tile_table + bin_off + (int)__umul24((unsigned)(py >> kTileShift), (unsigned)tiles_x) + (px >> kTileShift));
+        }
     }
 }
 
@@ -242,6 +246,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     extern __shared__ int s_hist[];  // bin entries of this workgroup's points, one counter per tile
     __shared__ int s_valid[2][WAVES];  // valid points of every wavefront in this step (two steps in flight)
     __shared__ double2 s_log[kLogTable];
+    __shared__ vf4 s_rec[WAVES][64 * NREC];  // a wavefront's records of a step
     __shared__ int s_flags;            // bit 0: not_identity, bit 1: bad_index, of any point of the chunk
     const Camera cam  = load_camera(p.pose, p.intrinsics, p.view, p.dist_cutoff);
     const int L       = p.num_layers;
@@ -264,10 +269,13 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     // The loads of the next step's points, their descriptors and dropout flags among them (whether a point is visible or
     // not), are in flight while this step's are projected. (With the dropout flag and the descriptor requested in the
     // step itself, its waits were a part of every step: 9M points with dropout 225 -> 197 us.) What bounds it: without the saved
-    // state the 447 MB that it moves at 6M points, 4.5 TB/s; with it the stores, 477 MB at 3.9 TB/s (that the next step waits for
+    // state the 430 MB that it moves at 6M points, 4.5 TB/s; with it the stores, 477 MB at 3.8 TB/s (that the next step waits for
     // them is not it: without branches around loads and stores, so that nothing waits for a store, it took 137 us instead of
     // 131). Before the short exp and log and the layers' table it was its vector instructions, 91 us of them: eval 6M in Morton
     // order 126 -> 99 us, train 6M 138 -> 131, 9M 191 -> 173, 4M clustered 111 -> 105 a view (then two stores less: see prec).
+    // With a point's record stored by its own lane, 16 bytes of 32 (80 at 16 channels) at a time, a store touched twice (five
+    // times) the lines that it filled: as runs of the wavefront 4M clustered 100 -> 91 us a view, 9M 170 -> 163, 1M without the saved
+    // state 27.6 -> 26, 500k of sixteen channels 51 -> 22; 6M in no order, of which a view culls two in five, 125 both ways.
     PointInputs<CPAD> nxt;
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)
@@ -316,21 +324,32 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
         const int first_pair = next_pair + pbefore + pairs_before;  // within the chunk
         next += total;
         next_pair += ptotal;
-        if (pid >= end) continue;
-        if (TRAIN) p.cid_of[pid] = o.valid ? cid : ~cid;
-        if (!o.valid) continue;
-
-        // record for the blend (and the pixel pass of the backward)
-        float4 recv[NREC];
-        recv[0] = make_float4(o.ipx, o.ipy, encode_size_field(o.size_px, L), in.conf);
+        if (TRAIN && pid < end) p.cid_of[pid] = o.valid ? cid : ~cid;
+        // records for the blend (and the pixel pass of the backward): those of the wavefront's valid points follow each other, and
+        // leave through LDS as one run of 16 bytes a lane
+        vf4* const mine = s_rec[wave];
+        const int rank  = (int)__popcll(vm & below), words = (int)__popcll(vm) * NREC;
+        if (o.valid)
+        {
+            vf4* const to = mine + rank * NREC;
+            to[0]         = vf4{o.ipx, o.ipy, encode_size_field(o.size_px, L), in.conf};
 #pragma unroll
-        for (int q = 0; q < CPAD / 4; ++q) recv[1 + q] = make_float4(in.d[4 * q], in.d[4 * q + 1], in.d[4 * q + 2], in.d[4 * q + 3]);
-        float4* rec = reinterpret_cast<float4*>(p.rec + (size_t)cid * p.rec_floats);
+            for (int q = 0; q < CPAD / 4; ++q) to[1 + q] = vf4{in.d[4 * q], in.d[4 * q + 1], in.d[4 * q + 2], in.d[4 * q + 3]};
+            // point record: depth and layers for the scatter pass; first overflow row, softplus' and the size for the backward (without
+            // it 8 bytes: a frame of 6M points 1.5 us less here and in the scatter)
+            if constexpr (TRAIN)
+                __builtin_nontemporal_store(vf4{o.z, __uint_as_float((unsigned)o.layers | (unsigned)first_pair << kLayersBits), o.d_softplus, o.size_px},
+                                            reinterpret_cast<vf4*>(p.prec) + cid);
+            else
+                __builtin_nontemporal_store(vf2{o.z, __uint_as_float((unsigned)o.layers)}, reinterpret_cast<vf2*>(p.prec) + cid);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        vf4* const rec = reinterpret_cast<vf4*>(p.rec + (size_t)(cid - rank) * p.rec_floats);
 #pragma unroll
-        for (int q = 0; q < NREC; ++q) __builtin_nontemporal_store(vf4{recv[q].x, recv[q].y, recv[q].z, recv[q].w}, reinterpret_cast<vf4*>(rec) + q);
-        // point record: depth and layers for the scatter pass; first overflow row, softplus' and the size for the backward
-        __builtin_nontemporal_store(vf4{o.z, __uint_as_float((unsigned)o.layers | (unsigned)first_pair << kLayersBits), TRAIN ? o.d_softplus : 0.f, o.size_px},
-                                    reinterpret_cast<vf4*>(p.prec) + cid);
+        for (int q = 0; q < NREC; ++q)
+            if (64 * q + lane < words) __builtin_nontemporal_store(mine[64 * q + lane], rec + 64 * q + lane);
     }
     {
         const int flags = (__ballot(not_identity) != 0 ? 1 : 0) | (__ballot(bad_index) != 0 ? 2 : 0);
@@ -355,7 +374,8 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 // `bin` that come from workgroups before g, and bin_count[bin] = the column total. No atomics anywhere in the
 // binning, since atomics on a few thousand hot counters serialise. A workgroup owns 16 columns; its 16 row
 // segments are summed side by side, prefixed through LDS, then each segment writes its rows' prefixes (one thread
-// walking a whole column is a chain of G dependent-latency steps).
+// walking a whole column is a chain of G dependent-latency steps). A thread requests its 16 rows together and keeps them for the
+// prefix: read twice, eight at a time, 5.5 us instead of 4.3 at 512 x 512, 9.7 instead of 8.7 at 1920 x 1080.
 // A workgroup also clears the per-cell counters `counts` and `run` of those of its tiles that may be split: their slices add
 // to them. Those of any other tile are written, not added to, where its keys are placed (clearing all of them is 22 MB at
 // 1920 x 1080 and eight layers).
@@ -364,6 +384,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
 // counters, written (not added to, so that nothing has to clear them first); on the first view of a call the status block of
 // the whole call as well. The scan over the tiles' totals is the scatter pass's (plan_tiles).
 constexpr int kScanCols = 16, kScanSegs = 16;
+static_assert(kBinGroups % kScanSegs == 0, "equal segments");
 __device__ __forceinline__ int wave_inclusive_scan(int x)
 {
     const int lane = threadIdx.x & 63;
@@ -444,40 +465,28 @@ __global__ __launch_bounds__(256) void bin_column_scan_kernel(const ForwardParam
     }
     __shared__ int s_seg[kScanSegs][kScanCols];
     __shared__ int s_total[kScanCols];
-    const int NB = p.geom.bin_off[p.num_layers], G = p.bin_groups;
+    const int NB = p.geom.bin_off[p.num_layers];
     const int c = threadIdx.x % kScanCols, seg = threadIdx.x / kScanCols;
     const int bin0 = blockIdx.x * kScanCols, bin = bin0 + c;
-    const int rows = (G + kScanSegs - 1) / kScanSegs;
-    const int g0 = seg * rows, g1 = min(G, g0 + rows);
+    constexpr int kRows = kBinGroups / kScanSegs;
     const bool live = bin < NB;
-    int32_t* col    = p.bin_hist + bin;
-    int sum         = 0;
-    if (live)
-        for (int g = g0; g < g1; g += 8)
-        {
-            int v[8];
+    int32_t* col    = p.bin_hist + (size_t)(seg * kRows) * NB + bin;
+    int v[kRows], sum = 0;  // (all requested together, and kept for the prefix)
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = (g + k < g1) ? col[(size_t)(g + k) * NB] : 0;
+    for (int k = 0; k < kRows; ++k) v[k] = live ? col[(size_t)k * NB] : 0;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) sum += v[k];
-        }
+    for (int k = 0; k < kRows; ++k) sum += v[k];
     s_seg[seg][c] = sum;
     __syncthreads();
     int run = 0;
-    for (int k = 0; k < seg; ++k) run += s_seg[k][c];
-    if (live)
-        for (int g = g0; g < g1; g += 8)
-        {
-            int v[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = (g + k < g1) ? col[(size_t)(g + k) * NB] : 0;
+    for (int k = 0; k < kScanSegs; ++k) run += k < seg ? s_seg[k][c] : 0;
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-            {
-                if (g + k < g1) col[(size_t)(g + k) * NB] = run;
-                run += v[k];
-            }
-        }
+    for (int k = 0; k < kRows; ++k)
+    {
+        if (live) col[(size_t)k * NB] = run;
+        run += v[k];
+    }
     if (seg == kScanSegs - 1)
     {
         s_total[c] = run;  // (of columns past the last: 0)
@@ -612,7 +621,8 @@ __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t
 
 // One bin entry per (point, layer), in the tile of the footprint's first pixel. A workgroup walks
 // the records that its chunk of the points left at the compact numbers; its slots inside every bin are contiguous
-// and start at bin_start[bin] + hist[workgroup][bin].
+// and start at bin_start[bin] + hist[workgroup][bin]. (The layers' tiles come from registers, see LayerTable: 4M clustered 77 ->
+// 73 us a view.)
 template <bool PACKED>
 __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardParams p)
 {
@@ -621,6 +631,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     extern __shared__ int s_cur[];
     const int NB    = p.geom.bin_off[p.num_layers];
     const int chunk = chunk_of_workgroup();
+    const LayerTable layers = layer_table(p.geom);
     plan_tiles(p, p.bin_hist + (size_t)chunk * NB, NB, s_cur);
     int begin, end;
     chunk_point_range(p, chunk, begin, end);
@@ -642,7 +653,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
             const int cid = cid0 + u * kBinThreads;
             if (cid < begin + n)
             {
-                tail[u] = __builtin_nontemporal_load(reinterpret_cast<const vf2*>(p.prec + (size_t)cid * kPointRecordFloats));
+                tail[u] = __builtin_nontemporal_load(reinterpret_cast<const vf2*>(p.prec + (size_t)cid * p.prec_floats));
                 ip[u]   = *reinterpret_cast<const float2*>(p.rec + (size_t)cid * p.rec_floats);
             }
         }
@@ -651,12 +662,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
         {
             const int cid = cid0 + u * kBinThreads;
             if (cid >= begin + n) break;
-            PointProjection o;
-            o.ipx    = ip[u].x;
-            o.ipy    = ip[u].y;
-            o.layers = (int)(__float_as_uint(tail[u].y) & kLayersMask);
             const unsigned zbits = __float_as_uint(tail[u].x);
-            for_point_tiles(p.geom, o, s_cur,
+            for_point_tiles(layers, ip[u].x, ip[u].y, (int)(__float_as_uint(tail[u].y) & kLayersMask), s_cur,
                             [&](int px, int py, int* bc)
                             {
                                 const int slot = atomicAdd(bc, 1);

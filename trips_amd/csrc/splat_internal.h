@@ -113,6 +113,7 @@ namespace trips
 //              as before.
 __host__ __device__ inline int record_floats(int channels) { return 4 + ((channels + 3) & ~3); }
 constexpr int kPointRecordFloats = 4;
+constexpr int kDepthRecordFloats = 2;  // without the saved state: the first two words alone
 constexpr unsigned kLayersBits = 4, kLayersMask = (1u << kLayersBits) - 1u;
 
 // Pixels are binned into 32 x 32 tiles per layer. Internally a pixel is numbered tile-major:
@@ -307,7 +308,7 @@ struct BackwardWorkspaceLayout
 struct WorkspaceLayout
 {
     size_t chunk_valid;   // int32 [3 G]  per chunk of the binning kernels: valid points, flags, overflow rows of the backward
-    size_t prec;         // float4 [N]         point records, when there is no saved state to hold them
+    size_t prec;         // float [N * kPointRecordFloats] point records, when there is no saved state to hold them: kDepthRecordFloats of a point
     size_t counts;       // int32 [Pi]   list length per cell (the points whose 2 x 2 footprint starts at that pixel): added up
                          //              by the slices of tiles with more than kSliceEntries bin entries, whose counters are
                          //              cleared per view, and written by one workgroup for every other tile
@@ -372,6 +373,7 @@ struct ForwardParams
     float* rec;
     float* prec;
     int32_t rec_floats;
+    int32_t prec_floats;  // kPointRecordFloats with the saved state, else kDepthRecordFloats
     int32_t* lists;
     int32_t* retained;
     unsigned char* tags;  // training only

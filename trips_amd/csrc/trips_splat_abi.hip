@@ -475,6 +475,7 @@ int forward_impl(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsSplatIn* 
             p.rec        = reinterpret_cast<float*>(sv + sl.rec);
             p.prec       = reinterpret_cast<float*>(sv + sl.prec);
             p.rec_floats = record_floats(d.num_channels);
+            p.prec_floats = kPointRecordFloats;
             p.lists      = reinterpret_cast<int32_t*>(sv + sl.lists);
             p.retained   = reinterpret_cast<int32_t*>(sv + sl.retained);
             p.tags       = reinterpret_cast<unsigned char*>(sv + sl.tags);
@@ -487,6 +488,7 @@ int forward_impl(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsSplatIn* 
             p.rec        = reinterpret_cast<float*>(ws + 2 * align256(sizeof(ViewHeader)));
             p.prec       = reinterpret_cast<float*>(ws + wl.prec);
             p.rec_floats = record_floats(d.num_channels);
+            p.prec_floats = kDepthRecordFloats;
         }
         p.status = reinterpret_cast<ViewHeader*>(ws);
         for (int l = 0; l < d.num_layers; ++l) p.image[l] = out->image[l];
