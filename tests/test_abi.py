@@ -40,6 +40,36 @@ def test_library_exports_every_unet_symbol():
         assert hasattr(lib, n), f"{n} declared in trips_unet.h but not exported"
 
 
+def test_parameters_of_the_net_are_those_of_the_module():
+    """The net's own walk over its parameters against the module's: added modules, one of them twice, a shared parameter and an
+    empty one among them; the convolutions in the order of the C structs, a parametrised weight computed."""
+    import torch
+    from torch.nn.utils import parametrize
+    from trips_amd.unet import MultiScaleUnet2dDecOnlySmallFixed, MultiScaleUnet2dParams
+    net = MultiScaleUnet2dDecOnlySmallFixed(MultiScaleUnet2dParams(num_input_layers=4, num_layers=3, filters_network=[16, 32, 32]))
+    plain = net.ordered_parameters()
+    assert [id(p) for p in sorted(plain, key=id)] == [id(p) for p in sorted(net.parameters(), key=id)]
+    extra = torch.nn.Linear(2, 2, bias=False)
+    net.extra, net.again, net.scale = extra, torch.nn.ModuleList([extra, torch.nn.Identity()]), extra.weight
+    net.register_module("nothing", None)
+    for recurse in (True, False):
+        want = list(torch.nn.Module.parameters(net, recurse))
+        assert [id(p) for p in net.parameters(recurse)] == [id(p) for p in want]
+    for p in net.parameters():
+        p.grad = torch.zeros_like(p)
+    net.zero_grad(set_to_none=True)
+    assert all(p.grad is None for p in torch.nn.Module.parameters(net))
+
+    class Twice(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+    conv = net.final_conv
+    before = conv.weight.detach().clone()
+    parametrize.register_parametrization(conv, "weight", Twice())
+    got = net.ordered_parameters()
+    assert torch.equal(got[-2], 2 * before) and got[-1] is conv.bias and all(a is b for a, b in zip(got[:-2], plain))
+
+
 def test_unet_ctypes_mirrors_and_host_checks(tmp_path):
     prog = tmp_path / "sizes.c"
     prog.write_text('#include <stdio.h>\n#include "trips_unet.h"\nint main(){printf("%zu %zu %zu %zu\\n",'

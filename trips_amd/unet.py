@@ -147,17 +147,37 @@ class MultiScaleUnet2dDecOnlySmallFixed(torch.nn.Module):
         """Parameters in the order of the C structs: per level feature weight, bias, mask weight, bias; then final."""
         # (through the modules' own tables: an attribute of a module is looked up in three of them, and a small frame
         # spent a quarter of its time on that)
+        def tensors_of(conv):
+            own = conv._parameters
+            w, b = own.get("weight"), own.get("bias")
+            return (conv.weight if w is None else w), (conv.bias if b is None else b)  # (a parametrised one is computed)
+
         mods, L, out = self._modules, self.params.num_layers, []
         for i in range(L):
             blk = mods["start"]._modules["conv"] if i == L - 1 else mods[f"up{i + 1}"]._modules["convolution"]
             for branch in ("feature_transform", "mask_transform"):
-                conv = blk._modules[branch]._modules["0"]
-                out.append(conv.weight)
-                out.append(conv.bias)
-        conv = mods["final"]._modules["0"]
-        out.append(conv.weight)
-        out.append(conv.bias)
+                out.extend(tensors_of(blk._modules[branch]._modules["0"]))
+        out.extend(tensors_of(mods["final"]._modules["0"]))
         return out
+
+    def parameters(self, recurse=True):
+        """As torch.nn.Module gives them, in its order, each once. (Its own walk goes through five generators a parameter: a
+        training step of the net alone, which clears its gradients and reads them, spent a fifth of its host time there.)"""
+        if not recurse:
+            return super().parameters(recurse)
+        found, seen = {}, set()
+
+        def walk(module):
+            seen.add(module)
+            for p in module._parameters.values():
+                if p is not None:
+                    found[id(p)] = p
+            for child in module._modules.values():
+                if child is not None and child not in seen:
+                    walk(child)
+
+        walk(self)
+        return iter(found.values())
 
     def he_normal_(self, generator=None):
         """He-normal weights, zero biases (the initialisation the benchmark configuration names)."""
