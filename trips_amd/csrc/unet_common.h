@@ -172,8 +172,15 @@ inline int check_unet_desc(const TripsUnetDesc* d)
 
 // Workgroups of the weight gradient on a CU: two where LDS (75 KB at 32 x 64) and registers (128 of a lane) allow it; one waits for
 // its loads and barriers while the other multiplies. 32 inputs x 64 pre-activations, levels of 1245 x 825 and of four 512 x 512 crops
-// 98 -> 86 us and 99 -> 87, the sums of twice the partials 10 -> 12.
+// 98 -> 86 us and 99 -> 87, the sums of twice the partials 10 -> 12. With fewer than three tiles for each of two, one: the second
+// one's partials cost more than it gives (504 tiles 21 us either way, the sums 20 -> 23; 1972 tiles of two levels 43 and 40, 12.5
+// and 15.5).
 constexpr int wgrad_resident(int cin_pad, int npad) { return cin_pad == 32 && npad <= 64 ? 2 : 1; }
+inline long long wgrad_workgroups(int cin_pad, int npad, long long tiles)
+{
+    const long long most = 256 * wgrad_resident(cin_pad, npad);
+    return npad == 64 && tiles < 3 * most ? 256 : most;
+}
 
 // Levels whose weight gradients are the same instance of the kernel run in one launch, whose workgroups are as many as are
 // resident at once (every further one would only add a set of partial sums to write and reduce) and are dealt to the levels by their tiles. With a launch per level the coarser ones were a handful of
@@ -194,7 +201,6 @@ inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
         bool first          = true;  // of its instance
         for (int k = 0; k < i; ++k) first = first && !same_wgrad_kernel(np.lv[k], lv);
         if (!first) continue;
-        const long long resident = 256 * wgrad_resident(lv.cin_pad, lv.wgrad_tile);
         long long all = 0, work = 0, shares = 0;
         for (int k = i; k < levels; ++k)
             if (same_wgrad_kernel(np.lv[k], lv))
@@ -205,6 +211,7 @@ inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
                 work += np.lv[k].tiles * s;
                 shares += s;
             }
+        const long long resident = wgrad_workgroups(lv.cin_pad, lv.wgrad_tile, all);
         size_t o = at;
         for (int k = i; k < levels; ++k)
         {
