@@ -543,7 +543,13 @@ static_assert(kTilePixels == 1 << (2 * kTileShift), "a cell number takes 2 kTile
 //   * exclusive scan: bin_start[i] = sum_{k<i} bin_count[k], bin_start[NB] = total;
 //   * slices of split tiles: a tile with more than kSliceEntries bin entries (hundreds of points per pixel, e.g.
 //     tight clusters) would keep a single workgroup busy for milliseconds; it is cut into slices of kSliceEntries
-//     entries, each a workgroup of its own. slice_start[t] = number of slices of split tiles before tile t.
+//     entries, each a workgroup of its own. slice_start[t] = number of slices of split tiles before tile t;
+//   * coarse_first: whether cell sort and blend begin with the coarsest layer, whose lists are the longest, so that no few
+//     workgroups are left over at the end. Not where fewer than a third of the tiles hold anything: what they hold is long in
+//     every layer, and side by side on a CU the heaviest slow each other down. us, cell sort and blend, finest layer first and
+//     coarsest: 1M in a ball 48 + 89 and 35 + 79, 6M in no order 57 + 190 and 51 + 176, 9M in Morton order 37 + 119 and 35 + 105,
+//     500k at 700 x 500 15 + 48 and 12 + 39, four views of 64 tight clusters 197 + 208 and 208 + 219. (Both spread evenly among each
+//     other: between the two.)
 // Every workgroup of the scatter pass makes the scan for itself (a few values of a thread, two barriers) and keeps its
 // cursors in `s_cur`; the first one writes scan and slices for the kernels behind. Bound by its round trips: 1.7 us longer the
 // scatter (2.6 at 2700 tiles) and a launch between column scan and scatter less, whose single workgroup took 4.5: 100k
@@ -553,7 +559,7 @@ constexpr int kPlanPer = (kMaxBins + kBinThreads - 1) / kBinThreads;  // tiles o
 __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t* __restrict__ row, int NB, int* __restrict__ s_cur)
 {
     constexpr int WAVES = kBinThreads / 64;
-    __shared__ int s_tiles[WAVES], s_slices[WAVES];
+    __shared__ int s_tiles[WAVES], s_slices[WAVES], s_filled[WAVES];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int per  = (NB + kBinThreads - 1) / kBinThreads;
     const int t0   = (int)threadIdx.x * per;
@@ -581,8 +587,8 @@ __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t
     }
     if (blockIdx.x == 0)
     {
-        // slices of the tiles' entries that fit the capacity
-        int sl[kPlanPer], slices = 0;
+        // slices of the tiles' entries that fit the capacity; tiles with any
+        int sl[kPlanPer], slices = 0, filled = 0;
         first = first0;
 #pragma unroll
         for (int j = 0; j < kPlanPer; ++j)
@@ -597,7 +603,9 @@ __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t
             }
             first += v[j];
             slices += sl[j];
+            filled += (int)__popcll(__ballot(v[j] > 0));
         }
+        if (lane == 0) s_filled[wave] = filled;
         const int inc_slices = wave_inclusive_scan(slices);
         if (lane == 63) s_slices[wave] = inc_slices;
         __syncthreads();
@@ -614,6 +622,9 @@ __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t
             p.bin_start[NB]     = total;
             p.slice_start[NB]   = total_slices;
             p.header->n_entries = (unsigned long long)(unsigned)total;
+            int all_filled;
+            waves_before<WAVES>(s_filled, all_filled);
+            *p.coarse_first = 3 * all_filled >= NB ? 1 : 0;
         }
     }
     __syncthreads();
@@ -1170,8 +1181,10 @@ __global__ __launch_bounds__(256) void cell_sort_kernel(const ForwardParams p)
     __shared__ int s_num_long, s_next;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NB   = p.geom.bin_off[p.num_layers];
-    const long long lblock = xcd_tile_block(blockIdx.x, 16);
+    const bool coarse_first = *p.coarse_first != 0;
+    long long lblock        = xcd_tile_block(blockIdx.x, 16);
     if (lblock >= (long long)NB * 16) return;
+    if (coarse_first) lblock = (long long)NB * 16 - 1 - lblock;
     int4 info = make_int4(0, 0, 0, 0);
     if (wave == 0)
     {
@@ -1283,8 +1296,10 @@ __global__ __launch_bounds__(256) void blend_kernel(const ForwardParams p)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NB   = p.geom.bin_off[p.num_layers];
-    const long long lblock = xcd_tile_block(blockIdx.x, 4);
+    const bool coarse_first = *p.coarse_first != 0;
+    long long lblock        = xcd_tile_block(blockIdx.x, 4);
     if (lblock >= (long long)NB * 4) return;
+    if (coarse_first) lblock = (long long)NB * 4 - 1 - lblock;
     const int bin = (int)(lblock >> 2), quarter = (int)(lblock & 3);
     const TileCtx tc = tile_ctx(p.geom, bin);
     const int bx = ((quarter & 1) << 4) + ((wave & 1) << 3), by = ((quarter >> 1) << 4) + ((wave >> 1) << 3);

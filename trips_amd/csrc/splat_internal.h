@@ -316,7 +316,7 @@ struct WorkspaceLayout
     size_t run;          // int32 [Pi]   keys of a cell already claimed by slices of a split tile (cleared per view for tiles with
                          //              more than kSliceEntries bin entries; undefined for every other tile)
     size_t slice_start;  // int32 [NB+1] exclusive scan of the slices of split tiles (0 for a tile that is not split)
-    size_t long_count;   // int32 [1]    segments of long lists handed out so far
+    size_t long_count;   // int32 [2]    segments of long lists handed out so far; 1 = the coarsest layer's tiles first (see coarse_first)
     size_t long_items;   // int2  [max_long_items] {first key, number of keys} of each segment of a long list
     size_t cand;         // uint64 [max_long_items * 16] the 16 smallest keys of each segment
     size_t max_long_items;
@@ -364,6 +364,7 @@ struct ForwardParams
     int32_t* run;
     int32_t* slice_start;
     int32_t* long_count;
+    int32_t* coarse_first;  // 1: cell sort and blend take the tiles from the last one on
     int2* long_items;
     unsigned long long* cand;
     int32_t max_long_items;

@@ -462,6 +462,7 @@ int forward_impl(TripsCtx* ctx, const TripsSplatDesc* desc, const TripsSplatIn* 
         p.run         = reinterpret_cast<int32_t*>(ws + wl.run);
         p.slice_start = reinterpret_cast<int32_t*>(ws + wl.slice_start);
         p.long_count  = reinterpret_cast<int32_t*>(ws + wl.long_count);
+        p.coarse_first = p.long_count + 1;
         p.long_items  = reinterpret_cast<int2*>(ws + wl.long_items);
         p.cand        = reinterpret_cast<unsigned long long*>(ws + wl.cand);
         p.max_long_items = (int32_t)wl.max_long_items;
