@@ -763,7 +763,7 @@ constexpr int strip_lds_bytes(int kc, int nn, int ci)
 // (LDS is given out in 128 pieces of 1280 bytes.)
 constexpr int strip_resident(int kc, int nn, int ci) { return strip_lds_bytes(kc, nn, ci) <= 64 * 1280 && nn == 32 ? 2 : 1; }
 
-__device__ const _Float16 k_zeros[8] = {};  // what lies outside the image
+alignas(16) __device__ const _Float16 k_zeros[8] = {};  // what lies outside the image
 
 // 16 bytes of each active lane, from its address to LDS: at `to` (the same for all lanes), in the order of the lanes, the places of
 // inactive ones left as they are. In flight until wait_for_loads.
