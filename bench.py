@@ -31,18 +31,18 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "7e8a90c362fb9d6ae3fe9dae55a751015a4baacf058b9abd0ff78ed0260f5dcd"
+PMC_SOURCES_SHA256 = "a41803904653c40c2ff50a1afadee7cebb393eaf67b3030e5e2c5c3f3c686c25"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129103, 235458),
-    "bin_scatter": (94882, 191464),
-    "tile_count": (13116, 2296),
-    "tile_scatter": (26022, 89639),
-    "cell_sort": (35349, 42140),
-    "blend": (372892, 196630),
-    "backward_prologue": (54, 265150),
-    "backward_tiles": (426498, 121594),
-    "backward_points": (309661, 234503),
-    "adam_fused": (383764, 498420),
+    "project_bin": (129103, 205081),
+    "bin_scatter": (87647, 177753),
+    "tile_count": (13109, 2296),
+    "tile_scatter": (26080, 88451),
+    "cell_sort": (35350, 42079),
+    "blend": (358872, 194218),
+    "backward_prologue": (50, 265142),
+    "backward_tiles": (434079, 121514),
+    "backward_points": (316658, 234535),
+    "adam_fused": (383767, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
                         "splat_internal.h", "trips_math.h", "row16.h")
