@@ -97,6 +97,14 @@ def test_gradients_through_strips_of_many_steps(filters, preact, inputs, w, h, c
     _held_to_restatement(filters, w, h, cin, batch)
 
 
+@pytest.mark.parametrize("batch", [10, 11, 24])
+def test_gradients_with_two_workgroups_on_a_cu(batch):
+    """32 inputs and 64 pre-activations, two levels of 100 and 50 tiles an image: 1500 and 1650 tiles, of which 512 workgroups of the
+    weight gradient get three each from 1536 on; 24 images leave the 512 strips of the data gradient six steps, after which their
+    rings are back at row 0."""
+    _held_to_restatement([32, 32], 30, 800, 4, batch)
+
+
 @pytest.mark.parametrize("filters,w,h,cin,batch", [
     ([16, 32], 37, 29, 4, 2), ([24, 32], 40, 24, 3, 1), ([32, 48], 33, 17, 8, 1), ([48, 64], 32, 8, 16, 1), ([16, 32], 1, 1, 4, 1),
 ])
