@@ -106,9 +106,10 @@ __device__ __forceinline__ void load_point(const ForwardParams& p, int pid, int 
     }
 }
 
-// The last pixels, first tile and tile columns of all layers, layer l's in lane l of four registers (the whole wavefront makes
-// them, outside of any branch): a loop over the layers gets them with v_readlane, where loads of kernel arguments are four
-// round trips of the scalar cache per layer, one behind the other, which wait for the wavefront's LDS atomics as well.
+// The last pixels, first tile and tile columns of all layers, layer l's in lane l of four registers: a loop over the layers gets
+// them with v_readlane, where loads of kernel arguments are four round trips of the scalar cache per layer, one behind the
+// other, which wait for the wavefront's LDS atomics as well. The whole wavefront makes them, and the whole wavefront runs the
+// loops that read them: a copy or a spill of such a register where only some lanes run would leave the other layers behind.
 struct LayerTable
 {
     int last_x, last_y, bin_off, tiles_x;
@@ -126,8 +127,9 @@ __device__ __forceinline__ LayerTable layer_table(const PyramidGeom& g)
 
 // `s_hist`: LDS counters, one per tile; every layer the point is written to adds one to the tile of the footprint's
 // first pixel (px, py). (The footprint (px..px+1, py..py+1) lies inside the image because px < w-1 and py < h-1.)
+// Called by the whole wavefront (see LayerTable); lanes with `live` unset have no point.
 template <bool TRAIN, int CPAD>
-__device__ __forceinline__ PointProjection project_point(const ForwardParams& p, const Camera& cam, int pid, const PointInputs<CPAD>& in,
+__device__ __forceinline__ PointProjection project_point(const ForwardParams& p, const Camera& cam, int pid, bool live, const PointInputs<CPAD>& in,
                                                          int* s_hist, const double2* log_table, const LayerTable& layers,
                                                          bool& not_identity, bool& bad_index)
 {
@@ -139,10 +141,10 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
     o.size_px = 0.f;
     o.d_softplus = 0.f;
     const int L = p.num_layers;
-    bool skip   = false;
+    bool skip   = !live;
     o.tex       = in.tex;
-    not_identity |= (o.tex != pid);
-    if ((unsigned)o.tex >= (unsigned)p.num_texels)
+    not_identity |= live && o.tex != pid;
+    if (live && (unsigned)o.tex >= (unsigned)p.num_texels)
     {
         // a column outside the descriptor table: leave the point out (reported by the status query) rather
         // than read past the tables
@@ -153,7 +155,7 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
     if (p.viewer_only && in.conf < p.stability_cutoff_value) skip = true;
     if (TRAIN && in.dropout == 1.f) skip = true;
     float4 pos = in.pos;
-    if (p.displacement)
+    if (p.displacement && live)
     {
         const float* dsp = p.displacement + (size_t)pid * 3;
         pos.x += dsp[0];
@@ -165,38 +167,38 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
     auto small = [&](float radius) { return p.drop_out_points_by_radius && float(trunc_sat(radius)) < p.drop_out_radius_threshold; };
     o.valid = !skip && pr.z > 0.f && pr.ipx >= 0.f && pr.ipx < float(p.geom.w[0] - 1) && pr.ipy >= 0.f &&
               pr.ipy < float(p.geom.h[0] - 1) && !small(radius_px);
-    if (!o.valid) return o;
-    o.ipx = pr.ipx;
-    o.ipy = pr.ipy;
-    o.z   = pr.z;
-    const float size = softplus(in.raw_size, log_table, TRAIN ? &o.d_softplus : nullptr);
-    o.size_px        = quotient(pr.scale * size, pr.iz);
     int layer_higher = 0;
-    if (o.size_px > 1.f)
+    if (o.valid)
     {
-        int lo, hi;
-        log2_floor_ceil(o.size_px, lo, hi);
-        layer_higher = min(hi, L - 1);
+        o.ipx = pr.ipx;
+        o.ipy = pr.ipy;
+        o.z   = pr.z;
+        const float size = softplus(in.raw_size, log_table, TRAIN ? &o.d_softplus : nullptr);
+        o.size_px        = quotient(pr.scale * size, pr.iz);
+        if (o.size_px > 1.f)
+        {
+            int lo, hi;
+            log2_floor_ceil(o.size_px, lo, hi);
+            layer_higher = min(hi, L - 1);
+        }
     }
     float lx = o.ipx, ly = o.ipy;
-    bool more = true;
+    bool more = o.valid;
     for (int layer = 0; layer < L; ++layer, lx *= 0.5f, ly *= 0.5f, radius_px *= 0.5f)
     {
+        const int last_x = __builtin_amdgcn_readlane(layers.last_x, layer), last_y = __builtin_amdgcn_readlane(layers.last_y, layer);
+        const int bin_off = __builtin_amdgcn_readlane(layers.bin_off, layer), tiles_x = __builtin_amdgcn_readlane(layers.tiles_x, layer);
         const int px = (int)lx, py = (int)ly;
-        more = more && layer <= layer_higher && px < __builtin_amdgcn_readlane(layers.last_x, layer) &&
-               py < __builtin_amdgcn_readlane(layers.last_y, layer) && !small(radius_px);
+        more = more && layer <= layer_higher && px < last_x && py < last_y && !small(radius_px);
         if (__ballot(more) == 0) break;
-        if (more)
-        {
-            const int row = (int)__umul24((unsigned)(py >> kTileShift), (unsigned)__builtin_amdgcn_readlane(layers.tiles_x, layer));
-            atomicAdd(s_hist + __builtin_amdgcn_readlane(layers.bin_off, layer) + row + (px >> kTileShift), 1);
-            o.layers = layer + 1;
-        }
+        o.layers += more ? 1 : 0;  // (not layer + 1: the compiler then keeps the loop's own number per lane)
+        if (more) atomicAdd(s_hist + bin_off + (int)__umul24((unsigned)(py >> kTileShift), (unsigned)tiles_x) + (px >> kTileShift), 1);
     }
     return o;
 }
 
-// Calls f(px, py, counter of the tile of (px, py)) for the layers a point is written to.
+// Calls f(px, py, counter of the tile of (px, py)) for the layers a point is written to. Called by the whole wavefront (see
+// LayerTable); lanes without a point have 0 layers.
 template <typename F>
 __device__ __forceinline__ void for_point_tiles(const LayerTable& t, float lx, float ly, int layers, int* tile_table, F&& f)
 {
@@ -276,7 +278,9 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     // With a point's record stored by its own lane, 16 bytes of 32 (80 at 16 channels) at a time, a store touched twice (five
     // times) the lines that it filled: as runs of the wavefront 4M clustered 100 -> 91 us a view, 9M 170 -> 163, 1M without the saved
     // state 27.6 -> 26, 500k of sixteen channels 51 -> 22; 6M in no order, of which a view culls two in five, 125 both ways.
-    PointInputs<CPAD> nxt;
+    // With culled points kept in the loop over the layers instead of leaving before it: 6M in no order 125 -> 116, 4M clustered 91 -> 85
+    // a view, 9M 168 -> 160, 1M without the saved state 25.3 -> 24.0 (477 MB at 4.1 TB/s, without the saved state 430 MB at 4.4).
+    PointInputs<CPAD> nxt{};
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)
     {
@@ -290,10 +294,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
         const PointInputs<CPAD> in = nxt;
         if (pid + kBinThreads < end) load_point<C, TRAIN>(p, pid + kBinThreads, next_tex, nxt);
         if (pid + 2 * kBinThreads < end) next_tex = p.index[pid + 2 * kBinThreads];
-        PointProjection o;
-        o.valid  = false;
-        o.layers = 0;
-        if (pid < end) o = project_point<TRAIN>(p, cam, pid, in, s_hist, s_log, layers, not_identity, bad_index);
+        const PointProjection o = project_point<TRAIN>(p, cam, pid, pid < end, in, s_hist, s_log, layers, not_identity, bad_index);
         const unsigned long long vm = __ballot(o.valid);
         const unsigned long long below = (1ull << lane) - 1ull;
         // rows of the backward's overflow table (one per layer past the second) of the wavefront's points before this
@@ -633,7 +634,7 @@ __device__ __forceinline__ void plan_tiles(const ForwardParams& p, const int32_t
 // One bin entry per (point, layer), in the tile of the footprint's first pixel. A workgroup walks
 // the records that its chunk of the points left at the compact numbers; its slots inside every bin are contiguous
 // and start at bin_start[bin] + hist[workgroup][bin]. (The layers' tiles come from registers, see LayerTable: 4M clustered 77 ->
-// 73 us a view.)
+// 73 us a view; walked by whole wavefronts, 9M points with entries of 16 bytes 101 -> 104, the others as before.)
 template <bool PACKED>
 __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardParams p)
 {
@@ -654,8 +655,9 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
     // us: 6M points in no order 103 / 89 / 81 and with the saved state 109 / 113 / 109, 4M clustered 91 / 84 / 79, 3M in a ball
     // 61 / 58 / 55, 1M 22 / 21 / 21; 9M in Morton order 40 / 35 / 39.
     constexpr int U = 16;
-    for (int cid0 = begin + (int)threadIdx.x; cid0 < begin + n; cid0 += U * kBinThreads)
+    for (int first = begin; first < begin + n; first += U * kBinThreads)
     {
+        const int cid0 = first + (int)threadIdx.x;
         vf2 tail[U];  // {depth, layers}
         float2 ip[U];
 #pragma unroll
@@ -671,10 +673,11 @@ __global__ __launch_bounds__(kBinThreads) void bin_scatter_kernel(const ForwardP
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
-            const int cid = cid0 + u * kBinThreads;
-            if (cid >= begin + n) break;
+            const int cid   = cid0 + u * kBinThreads;
+            const bool live = cid < begin + n;
+            if (__ballot(live) == 0) break;
             const unsigned zbits = __float_as_uint(tail[u].x);
-            for_point_tiles(layers, ip[u].x, ip[u].y, (int)(__float_as_uint(tail[u].y) & kLayersMask), s_cur,
+            for_point_tiles(layers, ip[u].x, ip[u].y, live ? (int)(__float_as_uint(tail[u].y) & kLayersMask) : 0, s_cur,
                             [&](int px, int py, int* bc)
                             {
                                 const int slot = atomicAdd(bc, 1);
