@@ -105,6 +105,14 @@ def test_gradients_with_two_workgroups_on_a_cu(batch):
     _held_to_restatement([32, 32], 30, 800, 4, batch)
 
 
+@pytest.mark.parametrize("cin,batch", [(3, 10), (3, 11), (6, 10), (6, 11), (8, 15), (8, 16), (10, 15), (10, 16), (16, 31)])
+def test_weight_gradients_of_one_and_of_two_workgroups_on_a_cu(cin, batch):
+    """32 inputs and 64 pre-activations for each kind of image: two workgroups on a CU from 1536 tiles on and up to eight channels.
+    An image has 100 tiles and, up to six channels, 50 of the second level in the same launch; sixteen channels leave 32 inputs to
+    the second level only."""
+    _held_to_restatement([48, 64] if cin == 16 else [32, 32], 30, 800, cin, batch)
+
+
 @pytest.mark.parametrize("filters,w,h,cin,batch", [
     ([16, 32], 37, 29, 4, 2), ([24, 32], 40, 24, 3, 1), ([32, 48], 33, 17, 8, 1), ([48, 64], 32, 8, 16, 1), ([16, 32], 1, 1, 4, 1),
 ])

@@ -1252,9 +1252,9 @@ __device__ __forceinline__ void put_upsampled(_Float16* row, int g, int C, half8
     }
 }
 
-// CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4
-template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
-__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(2 * wgrad_resident(CIN, NPAD)))) void conv_bwd_weight_kernel(const BwdWeightTable tab)
+// CI: image channels the kernel has room for (4, 8 or 16; C <= CI); FOUR: C is exactly 4; RESIDENT: workgroups on a CU (wgrad_resident)
+template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR, int RESIDENT>
+__global__ __launch_bounds__(kWgradThreads) __attribute__((amdgpu_waves_per_eu(RESIDENT == 2 ? 4 : 1))) void conv_bwd_weight_kernel(const BwdWeightTable tab)
 {
     int level = 0;
     while (level + 1 < tab.n && (int)blockIdx.x >= tab.first[level + 1]) ++level;
@@ -1730,27 +1730,28 @@ hipError_t dispatch_bwd_data_up(const BwdDataUpParams& p, int batch, int npad, i
     return hipErrorInvalidValue;
 }
 
-template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR>
+template <int CIN, int NPAD, bool BIAS, int CI, bool FOUR, int RESIDENT>
 hipError_t launch_bwd_weight(const BwdWeightTable& t, int blocks, hipStream_t stream)
 {
     const size_t lds = ((size_t)(kConvPatchH * kConvPatchW + kBelowH * kBelowW) * (CIN + kLdsChanPad) +
                         (size_t)kConvTileH * kConvTileW * (NPAD + kLdsChanPad)) *
                        sizeof(_Float16);  // up to 101 KB
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR, RESIDENT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR>), dim3(blocks), dim3(kWgradThreads), lds, stream, t);
+    hipLaunchKernelGGL((conv_bwd_weight_kernel<CIN, NPAD, BIAS, CI, FOUR, RESIDENT>), dim3(blocks), dim3(kWgradThreads), lds, stream, t);
     return hipGetLastError();
 }
 
 template <int CI, bool FOUR>
 hipError_t dispatch_bwd_weight_ci(const BwdWeightTable& t, int blocks, const LevelPlan& lv, bool bias, hipStream_t stream)
 {
-#define TRIPS_BW(CIN_, NT_)                                                                 \
-    if (lv.cin_pad == CIN_ && lv.wgrad_tile == NT_)                                         \
-        return bias ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR>(t, blocks, stream)       \
-                    : launch_bwd_weight<CIN_, NT_, false, CI, FOUR>(t, blocks, stream);
-    TRIPS_BW(32, 32) TRIPS_BW(32, 64) TRIPS_BW(32, 128) TRIPS_BW(64, 32) TRIPS_BW(64, 64)
+#define TRIPS_BW(CIN_, NT_, RES_)                                                           \
+    if (lv.cin_pad == CIN_ && lv.wgrad_tile == NT_ && lv.wgrad_resident == RES_)            \
+        return bias ? launch_bwd_weight<CIN_, NT_, true, CI, FOUR, RES_>(t, blocks, stream) \
+                    : launch_bwd_weight<CIN_, NT_, false, CI, FOUR, RES_>(t, blocks, stream);
+    TRIPS_BW(32, 32, 2) TRIPS_BW(32, 64, 1) TRIPS_BW(32, 128, 1) TRIPS_BW(64, 32, 1) TRIPS_BW(64, 64, 1)
+    if constexpr (CI <= 8) TRIPS_BW(32, 64, 2)
 #undef TRIPS_BW
     return hipErrorInvalidValue;
 }
@@ -1806,7 +1807,7 @@ int trips_unet_backward(TripsCtx* ctx, const TripsUnetDesc* desc, const TripsUne
     unsigned wanted = 0;  // levels whose weight gradients are asked for
     for (int i = 0; i < L; ++i)
         if (grads->feature_weight[i] || grads->mask_weight[i]) wanted |= 1u << i;
-    plan_wgrad(np, L, wanted, np.wgrad_off);
+    plan_wgrad(np, L, C, wanted, np.wgrad_off);
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     char* ws           = reinterpret_cast<char*>(workspace);
     const char* sv     = reinterpret_cast<const char*>(saved);

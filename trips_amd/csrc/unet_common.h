@@ -114,6 +114,7 @@ struct LevelPlan
     int wgrad_tile;     // pre-activations of a workgroup of the weight-gradient kernel
     long long tiles;    // 8 x 32 tiles of all images of the batch
     int groups;         // persistent workgroups of the weight-gradient kernel for each of its npad / wgrad_tile shares
+    int wgrad_resident; // ... and how many of them share a CU
 };
 
 // Whether the data gradient of a block and the adjoint of the upsampling below it run as one kernel
@@ -170,16 +171,19 @@ inline int check_unet_desc(const TripsUnetDesc* d)
     return TRIPS_OK;
 }
 
-// Workgroups of the weight gradient on a CU: two where LDS (75 KB at 32 x 64) and registers (128 of a lane) allow it; one waits for
-// its loads and barriers while the other multiplies. 32 inputs x 64 pre-activations, levels of 1245 x 825 and of four 512 x 512 crops
-// 98 -> 86 us and 99 -> 87, the sums of twice the partials 10 -> 12. With fewer than three tiles for each of two, one: the second
-// one's partials cost more than it gives (504 tiles 21 us either way, the sums 20 -> 23; 1972 tiles of two levels 43 and 40, 12.5
-// and 15.5).
-constexpr int wgrad_resident(int cin_pad, int npad) { return cin_pad == 32 && npad <= 64 ? 2 : 1; }
-inline long long wgrad_workgroups(int cin_pad, int npad, long long tiles)
+// Workgroups of the weight gradient on a CU (`tiles`: of all its levels; `channels`: of the image). Two for 32 inputs x 32
+// pre-activations. Two for 32 x 64 too (LDS 75 KB, 128 registers of a lane, for which the kernel spills 3 to 7 of the 134 to 139 that
+// it takes with the bias gradients, 16 to 22 without) where one's loads and barriers then pass while the other multiplies: up to
+// eight channels, from three tiles for each of the 512 on. us, one of its own registers and two, kernel + sums of the partials:
+// levels of 1245 x 825, three channels 99.9 + 6.2 and 86.5 + 8.4, four 97 + 6.4 and 85 + 8.5, six 93 + 4.9 and 88 + 8.0, eight 75 + 8.8 and
+// 71 + 11; four crops of 512 x 512 94 + 6.3 and 83 + 8.5. The sixteen channels of a pixel's image leave the registers less room (17
+// to 38 spilled): ten channels 84 + 8.7 and 100 + 10.7, at 960 x 560 52 + 7.2 and 62 + 9.6. Around three tiles: four channels, 1500
+// tiles, 32.2 + 5.2 and 30.0 + 7.6, 1800 38.2 + 5.0 and 31.6 + 7.5; eight, 1200 tiles, 31.2 + 6.6 and 31.7 + 8.5, 1610 38.4 + 7.3 and 36.1 + 9.4.
+// (One on a CU, but held to 128 registers all the same: 1500 tiles of four channels 32.2 -> 33.6, 1200 of eight 31.2 -> 34.0, 650 of ten
+// 22.9 -> 29.5.)
+inline int wgrad_resident(int cin_pad, int npad, int channels, long long tiles)
 {
-    const long long most = 256 * wgrad_resident(cin_pad, npad);
-    return npad == 64 && tiles < 3 * most ? 256 : most;
+    return cin_pad == 32 && (npad == 32 || (npad == 64 && channels <= 8 && tiles >= 3 * 512)) ? 2 : 1;
 }
 
 // Levels whose weight gradients are the same instance of the kernel run in one launch, whose workgroups are as many as are
@@ -193,7 +197,7 @@ inline long long wgrad_workgroups(int cin_pad, int npad, long long tiles)
 // The partial sums lie from `at` on; returns where they end, which does not depend on `wanted`: an instance has at most
 // `resident` workgroups, and at most one for each tile and share of its levels, and a workgroup writes one set of sums.
 inline bool same_wgrad_kernel(const LevelPlan& a, const LevelPlan& b) { return a.cin_pad == b.cin_pad && a.wgrad_tile == b.wgrad_tile; }
-inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
+inline size_t plan_wgrad(NetPlan& np, int levels, int channels, unsigned wanted, size_t at)
 {
     for (int i = 0; i < levels; ++i)
     {
@@ -211,12 +215,14 @@ inline size_t plan_wgrad(NetPlan& np, int levels, unsigned wanted, size_t at)
                 work += np.lv[k].tiles * s;
                 shares += s;
             }
-        const long long resident = wgrad_workgroups(lv.cin_pad, lv.wgrad_tile, all);
+        const int on_a_cu        = wgrad_resident(lv.cin_pad, lv.wgrad_tile, channels, all);
+        const long long resident = 256 * on_a_cu;
         size_t o = at;
         for (int k = i; k < levels; ++k)
         {
             LevelPlan& l = np.lv[k];
             if (!same_wgrad_kernel(l, lv) || !((wanted >> k) & 1u)) continue;
+            l.wgrad_resident = on_a_cu;
             // one workgroup for every share, the others by the tiles (rounded down: one that has to wait for another to end
             // would take as long again)
             l.groups   = (int)std::min(1 + (resident - shares) * l.tiles / work, l.tiles);
@@ -286,7 +292,7 @@ inline NetPlan make_plan(const TripsUnetDesc& d)
         bw += align256((size_t)16 * 9 * np.lv[i].npad * np.lv[i].cin_pad * sizeof(float));
     }
     np.wgrad_off = bw;
-    bw           = plan_wgrad(np, L, ~0u, bw);
+    bw           = plan_wgrad(np, L, C, ~0u, bw);
     {
         const size_t chunks = d.batch * (((size_t)np.lv[0].H * np.lv[0].W + kFinalPixelsPerBlock - 1) / kFinalPixelsPerBlock);
         // as many workgroups as are resident at once walk the chunks (four per CU at the 100 to 118 registers of most
