@@ -70,6 +70,32 @@ def test_parameters_of_the_net_are_those_of_the_module():
     assert torch.equal(got[-2], 2 * before) and got[-1] is conv.bias and all(a is b for a, b in zip(got[:-2], plain))
 
 
+def test_parameters_of_the_net_follow_overridden_walks():
+    """What a subclass, the object or a child module makes of the walk over the parameters holds for parameters(), as it does for any
+    module: a subclass that leaves one out, a method set on the object, a child that hides a module."""
+    import torch
+    from trips_amd.unet import MultiScaleUnet2dDecOnlySmallFixed, MultiScaleUnet2dParams
+    params = MultiScaleUnet2dParams(num_input_layers=4, num_layers=3, filters_network=[16, 32, 32])
+
+    class NoBias(MultiScaleUnet2dDecOnlySmallFixed):
+        def named_parameters(self, *args, **kwargs):
+            return ((n, p) for n, p in super().named_parameters(*args, **kwargs) if not n.endswith("bias"))
+
+    class Hidden(torch.nn.ModuleList):
+        def named_modules(self, memo=None, prefix="", remove_duplicate=True):
+            yield prefix, self
+
+    a, b, c = NoBias(params), MultiScaleUnet2dDecOnlySmallFixed(params), MultiScaleUnet2dDecOnlySmallFixed(params)
+    own = b.named_parameters
+    b.named_parameters = lambda *args, **kwargs: list(own(*args, **kwargs))[:2]
+    c.hidden = Hidden([torch.nn.Linear(2, 2)])
+    for net, count in ((a, len(list(own())) // 2), (b, 2), (c, len(list(own())))):
+        want = [p for _, p in net.named_parameters()]
+        assert [id(p) for p in net.parameters()] == [id(p) for p in want] and len(want) == count
+    a.requires_grad_(False)
+    assert all(p.requires_grad == n.endswith("bias") for n, p in torch.nn.Module.named_parameters(a))
+
+
 def test_unet_ctypes_mirrors_and_host_checks(tmp_path):
     prog = tmp_path / "sizes.c"
     prog.write_text('#include <stdio.h>\n#include "trips_unet.h"\nint main(){printf("%zu %zu %zu %zu\\n",'
