@@ -97,6 +97,34 @@ def test_sizes_and_depths_over_the_range_of_floats(oracle):
     assert (ref["depth"][0] > 0).sum() > 0.9 * n and ref["max_layer"][0].max() >= 4
 
 
+def test_sizes_that_are_the_middle_between_two_denormals(oracle):
+    """A size in pixels below the normal floats can lie in the middle between two of them, where a product with the rounded reciprocal
+    of the depth goes to the wrong one now and then: softplus(raw) 64 / z = an odd number of half units, z = b 2^k."""
+    f32 = np.float32
+    raw = np.random.default_rng(0).uniform(-16, -8, 60000).astype(f32)
+    size = np.log((f32(1) + np.exp(raw.astype(np.float64)).astype(f32)).astype(np.float64)).astype(f32) * f32(64)
+    mantissa, exponent = np.frexp(size.astype(np.float64))
+    odd, exponent = (mantissa * 2.0 ** 24).astype(np.int64), exponent - 24
+    while (odd % 2 == 0).any():
+        exponent, odd = np.where(odd % 2 == 0, exponent + 1, exponent), np.where(odd % 2 == 0, odd // 2, odd)
+    raws, sizes, depths = [], [], []
+    for b in (49, 63, 75, 77, 21, 11, 3):
+        at = np.flatnonzero((odd % b == 0) & (odd > b) & (np.log2(b) + exponent + 150 < 125))
+        raws.append(raw[at])
+        sizes.append(size[at])
+        depths.append(b * 2.0 ** (exponent[at] + 150))
+    raw, size, z = np.concatenate(raws)[:4000], np.concatenate(sizes)[:4000], np.concatenate(depths)[:4000].astype(f32)
+    assert ((size * (1.0 / z.astype(np.float64))).astype(f32) != size / z).sum() > 20
+    n = raw.size
+    sc = scenes.tiny(n=n, w=70, h=50, f=64.0, num_layers=4, list_depth=16, seed=33)
+    rng = np.random.default_rng(33)
+    sc.poses_se3[:] = [0, 0, 0, 1, 0, 0, 0, 0]
+    sc.position[:] = np.stack([rng.uniform(-0.5, 0.5, n) * z, rng.uniform(-0.35, 0.35, n) * z, z, 0.01 * z], axis=1).astype(f32)
+    sc.point_size[:] = raw.reshape(sc.point_size.shape)
+    _, ref, _ = _check_forward(oracle, sc, abi.desc_for_scene(sc))
+    assert (ref["depth"][0] > 0).all() and np.array_equal(ref["size_px"][0], size / z) and (size / z < 2.0 ** -126).all()
+
+
 def test_forward_distortion(oracle):
     # non-zero distortion: parity with Saiga's model is unpinned; this checks HIP == oracle for the restated model
     sc = scenes.tiny(n=3000, w=64, h=48, f=60.0, num_layers=3, list_depth=16, seed=10)

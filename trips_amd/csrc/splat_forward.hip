@@ -163,7 +163,7 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
         pos.z += dsp[2];
     }
     const Projected pr = project(cam, pos.x, pos.y, pos.z);
-    float radius_px    = quotient(pr.scale * pos.w, pr.iz);
+    float radius_px    = quotient(pr.scale * pos.w, pr.iz);  // (only its whole pixels count)
     auto small = [&](float radius) { return p.drop_out_points_by_radius && float(trunc_sat(radius)) < p.drop_out_radius_threshold; };
     o.valid = !skip && pr.z > 0.f && pr.ipx >= 0.f && pr.ipx < float(p.geom.w[0] - 1) && pr.ipy >= 0.f &&
               pr.ipy < float(p.geom.h[0] - 1) && !small(radius_px);
@@ -174,7 +174,7 @@ __device__ __forceinline__ PointProjection project_point(const ForwardParams& p,
         o.ipy = pr.ipy;
         o.z   = pr.z;
         const float size = softplus(in.raw_size, log_table, TRAIN ? &o.d_softplus : nullptr);
-        o.size_px        = quotient(pr.scale * size, pr.iz);
+        o.size_px        = quotient_of_any_size(pr.scale * size, pr.z, pr.iz);
         if (o.size_px > 1.f)
         {
             int lo, hi;

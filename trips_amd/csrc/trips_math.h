@@ -21,7 +21,9 @@ constexpr float kAlphaDestCutoff = 0.001f;  // ALPHA_DEST_CUTOFF, RenderForward.
 // exp / log evaluated in double and rounded once, so that results do not depend on a libm's float path. The projection is bound by
 // its vector instructions, and the two functions for any double were a third of them: a float's exponential and the logarithm
 // of 1 + exp(x) need no second word of the argument, no range tests and, with a table of reciprocals, no division. Their errors
-// stay below 2^-51 of the value, and over all floats the rounded results are those of exp() and log() in double.
+// stay below 2^-51 of the value, and the rounded results are those of exp() and log() in double: of exp for every float from -200 to
+// 200, of log for every z = 1 + exp(x) of a float x, its only arguments. (Of the other floats up to there two have a logarithm that
+// close to the middle between two floats: z = 0x1.cb534cp+13 and 0x1.c09d7cp+27, rounded the other way than by the libm.)
 
 // A constant kept in scalar registers: as an operand of a multiply-add it then costs nothing, where the compiler would copy
 // it into two vector registers first.
@@ -80,8 +82,8 @@ __device__ __forceinline__ float log_rn(float z, const double2* table)
 
 // 1 / b in double for a float b > 0, within two units of the last place: the hardware's reciprocal (an error e of 2^-23) times
 // 1 + e + e^2. A float times it is within 2^-51 of the quotient, which is never that close to the middle between two
-// floats (25-bit numbers; quotients of floats keep 2^-49 of themselves away from these): rounded to float it is the IEEE quotient.
-// Quotients by the same number share it: three operations each instead of eleven.
+// floats (25-bit numbers; quotients of floats keep 2^-49 of themselves away from these): rounded to float it is the IEEE quotient,
+// where that is a normal number. Quotients by the same number share it: three operations each instead of eleven.
 __device__ __forceinline__ double reciprocal_of(float b)
 {
     const double bd = (double)b;
@@ -91,6 +93,14 @@ __device__ __forceinline__ double reciprocal_of(float b)
     return fma(r, fma(e, e, e), r);
 }
 __device__ __forceinline__ float quotient(float a, double reciprocal) { return (float)((double)a * reciprocal); }
+// The IEEE quotient also below the normal numbers, where floats are wider apart and it can itself be the middle between two: there it
+// is divided out.
+__device__ __forceinline__ float quotient_of_any_size(float a, float b, double reciprocal)
+{
+    const double q = (double)a * reciprocal;
+    if (fabs(q) < 0x1p-126 && a != 0.f) return (float)((double)a / (double)b);
+    return (float)q;
+}
 
 // softplus and its derivative, with the one exponential that they share (derivative may be nullptr)
 __device__ __forceinline__ float softplus(float x, const double2* table, float* derivative)
