@@ -125,6 +125,20 @@ def test_sizes_that_are_the_middle_between_two_denormals(oracle):
     assert (ref["depth"][0] > 0).all() and np.array_equal(ref["size_px"][0], size / z) and (size / z < 2.0 ** -126).all()
 
 
+def test_exported_lists_name_the_points_of_any_pattern_of_culled_ones(oracle):
+    """The export searches the chunks of the binning kernels, here of 235 points, for the point of a list entry: none culled, two in
+    five, runs of up to 300, all but one in a hundred, all but the first and all but the last point of every chunk."""
+    n, chunk = 60000, 235
+    sc = scenes.tiny(n=n, w=48, h=40, f=45.0, num_layers=2, list_depth=16, seed=51, views=6, radius=(0.001, 0.02))
+    sc.poses_se3[:] = sc.poses_se3[0]
+    rng = np.random.default_rng(51)
+    at = np.arange(n)
+    runs = np.concatenate([np.full(k, i % 2) for i, k in enumerate(rng.integers(1, 300, 1000))])[:n]
+    drop = np.stack([0 * at, rng.random(n) < 0.4, runs, rng.random(n) > 0.01, at % chunk != 0, at % chunk != chunk - 1]).astype(np.float32)
+    _, ref, _ = _check_forward(oracle, sc, abi.desc_for_scene(sc), dropout=drop)
+    assert (ref["lengths"].max(axis=1) > 0).all() and (n + 255) // 256 == chunk
+
+
 def test_forward_distortion(oracle):
     # non-zero distortion: parity with Saiga's model is unpinned; this checks HIP == oracle for the restated model
     sc = scenes.tiny(n=3000, w=64, h=48, f=60.0, num_layers=3, list_depth=16, seed=10)

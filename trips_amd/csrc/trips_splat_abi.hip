@@ -25,7 +25,7 @@ hipError_t launch_export_points(const float* rec, int rec_floats, const float* p
                                 float* depth, float* size_px, int32_t* max_layer, hipStream_t stream);
 hipError_t launch_sum_i32(const int32_t* v, long long n, unsigned mask, unsigned long long* out, hipStream_t stream);
 hipError_t launch_export_lists(const PyramidGeom& g, int K, const int32_t* lists, const int32_t* retained,
-                               const int32_t* cid_of, int num_points, int points_per_block, int32_t* out_lists, int32_t* out_retained,
+                               const int32_t* cid_of, const int32_t* chunk_valid, int num_points, int points_per_block, int32_t* out_lists, int32_t* out_retained,
                                int32_t* out_lengths, hipStream_t stream);
 }  // namespace trips
 
@@ -716,7 +716,8 @@ int trips_splat_export_lists(TripsCtx* ctx, const TripsSplatDesc* desc, const vo
     const char* sv       = reinterpret_cast<const char*>(saved) + sl.bytes_per_view * (size_t)view;
     hipError_t e = launch_export_lists(g, desc->list_depth, reinterpret_cast<const int32_t*>(sv + sl.lists),
                                        reinterpret_cast<const int32_t*>(sv + sl.retained),
-                                       reinterpret_cast<const int32_t*>(sv + sl.cid_of), desc->num_points,
+                                       reinterpret_cast<const int32_t*>(sv + sl.cid_of),
+                                       reinterpret_cast<const int32_t*>(sv + sl.chunk_valid), desc->num_points,
                                        points_per_chunk(*desc), device_lists, device_retained, device_lengths, stream);
     if (e != hipSuccess) return hip_fail(e, "export copy");
     return TRIPS_OK;
