@@ -78,7 +78,7 @@ def _strip_steps(preact, inputs, cin, coarse_w, coarse_h, batch):
     are resident at once. (Sizes in LDS: the patch, the ring of gradients, the image's share.)"""
     image = 4 if cin <= 4 else 8 if cin <= 8 else 16
     lds = 10 * 34 * (preact + 8) * 2 + 10 * 32 * (inputs + 8) * 2 + 8 * 32 * image * 4
-    per_cu = 2 if 2 * lds <= 160 * 1024 and preact * inputs <= 32 * 32 else 1
+    per_cu = 2 if lds <= 64 * 1280 and inputs == 32 else 1
     strips, steps = (coarse_w + 14) // 15 * batch, 1
     while steps < (coarse_h + 4) // 4 and strips * ((coarse_h + 4 * steps - 2) // (4 * steps - 1)) > 256 * per_cu:
         steps += 1
@@ -87,7 +87,8 @@ def _strip_steps(preact, inputs, cin, coarse_w, coarse_h, batch):
 
 @pytest.mark.parametrize("filters,preact,inputs,w,h,cin,batch", [
     ([16, 32], 32, 32, 30, 800, 4, 24),  # two workgroups per CU
-    ([32, 32], 64, 32, 29, 799, 4, 15),
+    ([32, 32], 64, 32, 29, 799, 4, 24),  # ... with twice the pre-activations
+    ([32, 32], 64, 32, 29, 799, 6, 15),  # ... and more than four image channels: one
     ([16, 48], 32, 64, 30, 800, 3, 15),  # block outputs that start at position 6
     ([32, 48], 64, 64, 30, 799, 4, 15),
 ])

@@ -770,9 +770,10 @@ __global__ __launch_bounds__(256, 4) void backward_points_kernel(const BackwardP
     // flags of their rows) one group ahead, and looked at when the group begins. (The rest of a point's record follows in work_off, in a
     // request of its own: where every point is worked off as it comes, 634 MB read instead of 609 at 6M points in no order.) A step
     // at a time, its layers worked out where they were requested, every step waited for that: 9M points 186 -> 172 us, 6M in no order
-    // 169 -> 166, four views of clusters 271 -> 256, crops 109 -> 106; four steps 164, 170, 258 and 110; two steps of eight channels,
-    // 300k points, 23.0 instead of 22.1. (A step without any work, in the form without the queue, passed over at once: 9M
-    // 170, but 6M 170 and clusters 264.)
+    // 169 -> 166, four views of clusters 271 -> 256, crops 109 -> 106; four steps 164, 170, 258 and 110. One step and two of the present
+    // form: four channels, 6M in no order 169 and 166, clusters 260 and 254, 9M without dropout 249 and 253, four views of 500k at
+    // 512 x 512 99.6 and 101; three, 3M in a ball 115 both ways; six, 1M 59.4 and 61; eight, 300k 22.1 and 23.0; sixteen, 1.4M 96 and
+    // 97.6. (A step without any work, in the form without the queue, passed over at once: 9M 170, but 6M 170 and clusters 264.)
     auto cid_at    = [&](long long pid) { return pid < p.num_points ? p.cid_of[pid] : -1; };
     auto request   = [&](int cid) -> uint2
     {
@@ -960,7 +961,7 @@ __global__ __launch_bounds__(kSumThreads) void backward_sums_kernel(const SumsPa
 // On the first view of a call also, in
 // overwrite mode (`texels`): the descriptor and confidence gradients of the columns that the point pass does not write
 // itself. With the identity index (the forward noted it in the header) those are the columns past the last point;
-// otherwise all of them, the point pass then adds with atomics. `clear_sums`: the block sums that both passes add to
+// otherwise all of them, the point pass then adds with atomics. `clear_sums`: the outputs that backward_sums_kernel adds to
 // (background, every pose row, every intrinsics row).
 __global__ __launch_bounds__(256) void backward_prologue_kernel(const ViewHeader* __restrict__ header, const int32_t* __restrict__ chunk_valid,
                                                                 int bin_groups, int points_per_block, float* __restrict__ rows_inline,
@@ -1056,7 +1057,10 @@ hipError_t launch_tiles(const BackwardParams& p, int blocks, hipStream_t stream)
         default: return hipErrorInvalidValue;                                                                  \
     }
 
-// (four workgroups per CU, each walking its share of the points: every further one leaves another row of sums)
+// (Four workgroups per CU, each walking its share of the points; more leave more rows of sums. us, with 1024, 2048 and 4096, the sums
+// behind the plus: 6M points in no order 166 + 6.5, 170 + 10 and 173 + 16; four views of clusters 254 + 8, 253 + 11 and 292 + 18; 9M in
+// Morton order 253 + 6, 257 + 10 and 253 + 16; four views of 500k at 512 x 512 101 + 6, 110 + 8 and 110 + 8; 1.4M of sixteen channels
+// 96 + 8, 96 + 9 and 99 + 13.)
 int point_pass_blocks(int num_points) { return std::min((num_points + 255) / 256, kCameraRows); }
 
 hipError_t launch_backward_view(const BackwardParams& p, int channels, hipStream_t stream, Profiler* prof)

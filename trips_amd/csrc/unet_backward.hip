@@ -760,7 +760,8 @@ constexpr int strip_lds_bytes(int kc, int nn, int ci)
     return kConvPatchH * kConvPatchW * (kc + kLdsChanPad) * 2 + kRingRows * kConvTileW * (nn + kLdsChanPad) * 2 + kConvTileH * kConvTileW * ci * 4;
 }
 // Workgroups of a CU: two where LDS and registers (the weights take 36 (kc / 32) (nn / 32) of a lane) hold them.
-// (LDS is given out in 128 pieces of 1280 bytes.)
+// (LDS is given out in 128 pieces of 1280 bytes. From five image channels on, whose share of the image has room for eight, 64
+// pre-activations take 82752 bytes, 832 too many.)
 constexpr int strip_resident(int kc, int nn, int ci) { return strip_lds_bytes(kc, nn, ci) <= 64 * 1280 && nn == 32 ? 2 : 1; }
 
 alignas(16) __device__ const _Float16 k_zeros[8] = {};  // what lies outside the image
