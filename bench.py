@@ -31,18 +31,18 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "a41803904653c40c2ff50a1afadee7cebb393eaf67b3030e5e2c5c3f3c686c25"
+PMC_SOURCES_SHA256 = "a5cab9f0d370c90f0c7f4057030e15bdd7e69c6b5504c1664fb3c890411b6cbd"
 PMC_KIB_DEFAULT_WORKLOAD = {
-    "project_bin": (129103, 205081),
-    "bin_scatter": (87647, 177753),
-    "tile_count": (13109, 2296),
-    "tile_scatter": (26080, 88451),
-    "cell_sort": (35350, 42079),
-    "blend": (358872, 194218),
-    "backward_prologue": (50, 265142),
-    "backward_tiles": (434079, 121514),
-    "backward_points": (316658, 234535),
-    "adam_fused": (383767, 498420),
+    "project_bin": (129096, 205242),
+    "bin_scatter": (87654, 177435),
+    "tile_count": (13113, 2296),
+    "tile_scatter": (26050, 88315),
+    "cell_sort": (35349, 42080),
+    "blend": (362495, 193920),
+    "backward_prologue": (50, 265197),
+    "backward_tiles": (433838, 121516),
+    "backward_points": (316611, 234535),
+    "adam_fused": (383756, 498420),
 }
 SPLAT_KERNEL_SOURCES = ("splat_forward.hip", "splat_backward.hip", "misc_kernels.hip", "trips_splat_abi.hip",
                         "splat_internal.h", "trips_math.h", "row16.h")
