@@ -31,7 +31,7 @@ DEFAULT_POINTS = 6_000_000
 # sources whose digest is PMC_SOURCES_SHA256 (kernel_sources_sha256 below): when the sources have changed since the
 # profile, no traffic figure is reported.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
-PMC_SOURCES_SHA256 = "a5cab9f0d370c90f0c7f4057030e15bdd7e69c6b5504c1664fb3c890411b6cbd"
+PMC_SOURCES_SHA256 = "fa8fc67b396845ff52118828ba15d1cb1f0f167a6f2272f4270932c2aa34b152"
 PMC_KIB_DEFAULT_WORKLOAD = {
     "project_bin": (129096, 205242),
     "bin_scatter": (87654, 177435),

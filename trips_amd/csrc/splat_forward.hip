@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kBinThreads) void project_bin_kernel(const ForwardP
     // state 27.6 -> 26, 500k of sixteen channels 51 -> 22; 6M in no order, of which a view culls two in five, 125 both ways.
     // With culled points kept in the loop over the layers instead of leaving before it: 6M in no order 125 -> 114, 4M clustered 91 -> 85
     // a view, 9M 168 -> 160, 1M without the saved state 25.3 -> 23.8 (477 MB at 4.2 TB/s, without the saved state 430 MB at 4.4); three
-    // clouds of 6M in turn, whose inputs then all come from memory, 150 both ways.
+    // clouds of 6M in turn, whose inputs then all come from memory, 146 to 151 before and 1 to 2 more now.
     PointInputs<CPAD> nxt{};
     int next_tex = 0;  // descriptor column of the step after `nxt`'s
     if (begin + (int)threadIdx.x < end)
